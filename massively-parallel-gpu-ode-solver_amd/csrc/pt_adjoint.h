@@ -86,18 +86,37 @@ __device__ __forceinline__ void record_body(const AdjArgs<Sys>& A)
     double* sPAR; int* sPARi;
     stage_shared(a, sPAR, sPARi);
     const int tid = threadIdx.x + blockIdx.x * blockDim.x;
-    if (tid >= a.nActive) return;
-    Lane<Sys, double, false, ALG> L;
-    L.load(a, tid, sPAR, sPARi);
-    store_checkpoint<Sys, ALG>(A, L, 0);
+    using L_t = Lane<Sys, double, false, ALG>;
+    L_t L;
     int untilCk = A.K, k = 0;      // accepted steps to the next checkpoint (no division in the loop)
+    if (tid < a.nActive) {
+        L.load(a, tid, sPAR, sPARi);
+        store_checkpoint<Sys, ALG>(A, L, 0);
+    } else {
+        L.idle();
+    }
+    if constexpr (L_t::kCommonTime) {
+        // checkpoints fall on the same step in every lane of the wavefront
+        auto at = [&] {
+            ++k;
+            if (L.term == 0 && tid < a.nActive) {
+                if (k < A.ckcap) store_checkpoint<Sys, ALG>(A, L, k);
+                else L.status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT;
+            }
+        };
+        if ((blockDim.x & 63) == 0) {
+            if (a.NDO > 0) L.template run_common_time<true>(a, sPAR, sPARi, A.K, untilCk, at);
+            else L.template run_common_time<false>(a, sPAR, sPARi, A.K, untilCk, at);
+        }
+    }
+    if (tid >= a.nActive) return;
     while (L.term == 0) {
         const int before = L.nacc;
         L.step(a, sPAR, sPARi);
         if (L.nacc != before && --untilCk == 0) {
             untilCk = A.K;
             ++k;
-            if (L.term == 0) {
+            if (L.term == 0 && tid < a.nActive) {
                 if (k < A.ckcap) store_checkpoint<Sys, ALG>(A, L, k);
                 else L.status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT;
             }

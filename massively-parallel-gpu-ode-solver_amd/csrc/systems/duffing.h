@@ -16,25 +16,50 @@ struct Duffing : NoCallbacks {
     static constexpr int SD = 2, NCP = 2, NSP = 0, NISP = 0, NE = 0, NA = 1, NIA = 0;
     static constexpr bool HAS_VJP = true;
 
+    static constexpr int NTT = 1;
+    static constexpr bool TT_TIME_ONLY = true;
+
     template <class P>
-    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* cPAR, P*, int*, P*, int*)
+    MPGOS_HD static void TimeTerms(P T, P*, P* tt)
     {
         using mpgos::math::cos;
-        using mpgos::math::fma;
-        const P x = X[0], v = X[1];
-        F[0] = v;
-        F[1] = fma(-cPAR[0], v, cPAR[1] * cos(T)) - fma(x * x, x, x);
+        tt[0] = cos(T);
     }
 
     template <class P>
-    MPGOS_HD static void OdeVJP(int, int, const P* lam, P* X, P T, P* cPAR, P*, int*, P*, int*, P* gX, P* gP)
+    MPGOS_HD static void OdeFunctionTT(int, int, P* F, P* X, P, const P* tt, P* cPAR, P*, int*, P*, int*)
     {
-        using mpgos::math::cos;
+        using mpgos::math::fma;
+        const P x = X[0], v = X[1];
+        F[0] = v;
+        F[1] = fma(-cPAR[0], v, cPAR[1] * tt[0]) - fma(x * x, x, x);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunction(int tid, int NT, P* F, P* X, P T, P* cPAR, P* sPAR, int* sPARi, P* ACC, int* ACCi)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, cPAR, tt);
+        OdeFunctionTT<P>(tid, NT, F, X, T, tt, cPAR, sPAR, sPARi, ACC, ACCi);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeVJPTT(int, int, const P* lam, P* X, P, const P* tt, P* cPAR, P*, int*, P*, int*, P* gX, P* gP)
+    {
         const P x = X[0], v = X[1];
         gX[0] = -(P(1) + P(3) * x * x) * lam[1];
         gX[1] = lam[0] - cPAR[0] * lam[1];
         gP[0] = -v * lam[1];
-        gP[1] = cos(T) * lam[1];
+        gP[1] = tt[0] * lam[1];
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeVJP(int tid, int NT, const P* lam, P* X, P T, P* cPAR, P* sPAR, int* sPARi, P* ACC, int* ACCi, P* gX,
+                                P* gP)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, cPAR, tt);
+        OdeVJPTT<P>(tid, NT, lam, X, T, tt, cPAR, sPAR, sPARi, ACC, ACCi, gX, gP);
     }
 
     template <class P>
@@ -61,27 +86,52 @@ struct DuffingQ : NoCallbacks {
     static constexpr int SD = 3, NCP = 2, NSP = 0, NISP = 0, NE = 0, NA = 0, NIA = 0;
     static constexpr bool HAS_VJP = true;
 
+    static constexpr int NTT = 1;
+    static constexpr bool TT_TIME_ONLY = true;
+
     template <class P>
-    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* cPAR, P*, int*, P*, int*)
+    MPGOS_HD static void TimeTerms(P T, P*, P* tt)
     {
         using mpgos::math::cos;
+        tt[0] = cos(T);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunctionTT(int, int, P* F, P* X, P, const P* tt, P* cPAR, P*, int*, P*, int*)
+    {
         using mpgos::math::fma;
         const P x = X[0], v = X[1];
         F[0] = v;
-        F[1] = fma(-cPAR[0], v, cPAR[1] * cos(T)) - fma(x * x, x, x);
+        F[1] = fma(-cPAR[0], v, cPAR[1] * tt[0]) - fma(x * x, x, x);
         F[2] = x * x;
     }
 
     template <class P>
-    MPGOS_HD static void OdeVJP(int, int, const P* lam, P* X, P T, P* cPAR, P*, int*, P*, int*, P* gX, P* gP)
+    MPGOS_HD static void OdeFunction(int tid, int NT, P* F, P* X, P T, P* cPAR, P* sPAR, int* sPARi, P* ACC, int* ACCi)
     {
-        using mpgos::math::cos;
+        P tt[NTT];
+        TimeTerms<P>(T, cPAR, tt);
+        OdeFunctionTT<P>(tid, NT, F, X, T, tt, cPAR, sPAR, sPARi, ACC, ACCi);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeVJPTT(int, int, const P* lam, P* X, P, const P* tt, P* cPAR, P*, int*, P*, int*, P* gX, P* gP)
+    {
         const P x = X[0], v = X[1];
         gX[0] = -(P(1) + P(3) * x * x) * lam[1] + P(2) * x * lam[2];
         gX[1] = lam[0] - cPAR[0] * lam[1];
         gX[2] = P(0);
         gP[0] = -v * lam[1];
-        gP[1] = cos(T) * lam[1];
+        gP[1] = tt[0] * lam[1];
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeVJP(int tid, int NT, const P* lam, P* X, P T, P* cPAR, P* sPAR, int* sPARi, P* ACC, int* ACCi, P* gX,
+                                P* gP)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, cPAR, tt);
+        OdeVJPTT<P>(tid, NT, lam, X, T, tt, cPAR, sPAR, sPARi, ACC, ACCi, gX, gP);
     }
 
     template <class P>
@@ -99,14 +149,31 @@ struct DuffingEps : NoCallbacks {
     static constexpr int SD = 2, NCP = 3, NSP = 0, NISP = 0, NE = 1, NA = 0, NIA = 0;
     static constexpr bool HAS_VJP = true;
 
+    static constexpr int NTT = 1;
+    static constexpr bool TT_TIME_ONLY = false;
+
     template <class P>
-    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* cPAR, P*, int*, P*, int*)
+    MPGOS_HD static void TimeTerms(P T, P* cPAR, P* tt)
     {
         using mpgos::math::cos;
+        tt[0] = cos(cPAR[2] * T);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunctionTT(int, int, P* F, P* X, P, const P* tt, P* cPAR, P*, int*, P*, int*)
+    {
         using mpgos::math::fma;
         const P x = X[0], v = X[1];
         F[0] = v;
-        F[1] = fma(-cPAR[0], v, cPAR[1] * cos(cPAR[2] * T)) - fma(x * x, x, x);
+        F[1] = fma(-cPAR[0], v, cPAR[1] * tt[0]) - fma(x * x, x, x);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunction(int tid, int NT, P* F, P* X, P T, P* cPAR, P* sPAR, int* sPARi, P* ACC, int* ACCi)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, cPAR, tt);
+        OdeFunctionTT<P>(tid, NT, F, X, T, tt, cPAR, sPAR, sPARi, ACC, ACCi);
     }
 
     template <class P>

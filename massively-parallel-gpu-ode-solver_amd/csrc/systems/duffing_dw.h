@@ -20,12 +20,29 @@ struct DuffingDW {
     static constexpr int SD = 2, NCP = 1, NSP = 1, NISP = 0, NE = 2, NA = 3, NIA = 1;
     static constexpr bool HAS_VJP = false;
 
+    static constexpr int NTT = 1;
+    static constexpr bool TT_TIME_ONLY = true;
+
     template <class P>
-    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* cPAR, P* sPAR, int*, P*, int*)
+    MPGOS_HD static void TimeTerms(P T, P*, P* tt)
     {
         using mpgos::math::cos;
+        tt[0] = cos(T);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunctionTT(int, int, P* F, P* X, P, const P* tt, P* cPAR, P* sPAR, int*, P*, int*)
+    {
         F[0] = X[1];
-        F[1] = X[0] - X[0] * X[0] * X[0] - cPAR[0] * X[1] + sPAR[0] * cos(T);
+        F[1] = X[0] - X[0] * X[0] * X[0] - cPAR[0] * X[1] + sPAR[0] * tt[0];
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunction(int tid, int NT, P* F, P* X, P T, P* cPAR, P* sPAR, int* sPARi, P* ACC, int* ACCi)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, cPAR, tt);
+        OdeFunctionTT<P>(tid, NT, F, X, T, tt, cPAR, sPAR, sPARi, ACC, ACCi);
     }
 
     template <class P>

@@ -11,6 +11,19 @@
 // Systems that support the discrete adjoint also provide
 //   OdeVJP(tid, NT, lam, X, T, cPAR, sPAR, sPARi, ACC, ACCi, gX, gP)
 // setting gX = (dF/dX)^T lam and gP = (dF/dcPAR)^T lam.
+// Systems whose right-hand side contains terms of the time (and the control
+// parameters) alone may name them, so that the solver evaluates them once and
+// reuses them (a step's end is the next step's start; with a fixed step and a
+// time common to a wavefront, its lanes evaluate different times at once):
+//   NTT                                       number of such terms
+//   TT_TIME_ONLY                              true when no parameter enters them
+//   TimeTerms(T, cPAR, tt)                    evaluates them
+//   OdeFunctionTT(tid, NT, F, X, T, tt, ...)  the right-hand side, given them
+//   OdeVJPTT(tid, NT, lam, X, T, tt, ...)     its vector-Jacobian product (with
+//                                             TT_TIME_ONLY and HAS_VJP only)
+// with OdeFunction and OdeVJP the same functions over terms evaluated at T.
+// Such a system leaves T, the time domain and the parameters in its terms
+// alone after Initialization.
 // Every callback is MPGOS_HD so the same definition serves the gfx950 kernels
 // and the host oracle; elementary functions come from mpgos::math so both
 // sides evaluate identical bits.
@@ -28,6 +41,17 @@ struct NoCallbacks {
     template <class P> MPGOS_HD static void ActionAfterSuccessfulTimeStep(int, int, int&, P&, P&, P*, P*, P*, P*, int*, P*, int*) {}
     template <class P> MPGOS_HD static void Initialization(int, int, int&, P&, P&, P*, P*, P*, P*, int*, P*, int*) {}
     template <class P> MPGOS_HD static void Finalization(int, int, int&, P&, P&, P*, P*, P*, P*, int*, P*, int*) {}
+};
+
+// Number of time terms of a system (0 for systems that name none), and whether
+// they depend on the time alone.
+template <class Sys, class = void> struct TimeTermsOf {
+    static constexpr int n = 0;
+    static constexpr bool timeOnly = false;
+};
+template <class Sys> struct TimeTermsOf<Sys, decltype((void)Sys::NTT)> {
+    static constexpr int n = Sys::NTT;
+    static constexpr bool timeOnly = Sys::TT_TIME_ONLY;
 };
 
 } // namespace systems
