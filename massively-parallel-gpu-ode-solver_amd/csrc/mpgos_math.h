@@ -60,6 +60,26 @@ MPGOS_HD MPGOS_INLINE bool isfinite(double x) { return (bits(x) & 0x7ff000000000
 MPGOS_HD MPGOS_INLINE bool isfinite(float x) { return (bits(x) & 0x7f800000u) != 0x7f800000u; }
 MPGOS_HD MPGOS_INLINE bool isnan(double x) { return x != x; }
 
+// x, negated where y is negative
+MPGOS_HD MPGOS_INLINE double flip_sign(double x, double y) { return from_bits(bits(x) ^ (bits(y) & 0x8000000000000000ull)); }
+MPGOS_HD MPGOS_INLINE float flip_sign(float x, float y) { return from_bits32(bits(x) ^ (bits(y) & 0x80000000u)); }
+
+// a * b + k for a constant k (Horner steps): on the device the three-operand
+// form with k in vector registers.  Left to itself the compiler picks the
+// accumulating form and copies k into its destination first, or rebuilds k in
+// scalar registers for every use; a wavefront alone on its SIMD pays 4 cycles for
+// each of these moves, as for an fma.
+MPGOS_HD MPGOS_INLINE double fma_k(double a, double b, double k)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(k));
+    return r;
+#else
+    return fma(a, b, k);
+#endif
+}
+
 // IEEE square root: correctly rounded on the host and on gfx950 (the device
 // expansion of the square root refines the hardware estimate to the correctly
 // rounded result; tests compare both bit for bit).
@@ -80,11 +100,11 @@ MPGOS_HD MPGOS_INLINE double cos_kernel(double r)
 {
     const double z = r * r;
     double c = -0x1.907da367a37cbp-37;
-    c = fma(c, z, 0x1.1eeb68e93b64cp-29);
-    c = fma(c, z, -0x1.27e4fa17da09ep-22);
-    c = fma(c, z, 0x1.a01a019f4eb01p-16);
-    c = fma(c, z, -0x1.6c16c16c16967p-10);
-    c = fma(c, z, 0x1.5555555555555p-5);
+    c = fma_k(c, z, 0x1.1eeb68e93b64cp-29);
+    c = fma_k(c, z, -0x1.27e4fa17da09ep-22);
+    c = fma_k(c, z, 0x1.a01a019f4eb01p-16);
+    c = fma_k(c, z, -0x1.6c16c16c16967p-10);
+    c = fma_k(c, z, 0x1.5555555555555p-5);
     // 1 - z/2 + z^2 c, with the large term kept separate until the end
     const double hz = 0.5 * z;
     const double w = 1.0 - hz;                    // exact for z <= 0.62 up to one rounding
@@ -96,11 +116,11 @@ MPGOS_HD MPGOS_INLINE double sin_kernel(double r)
 {
     const double z = r * r;
     double s = 0x1.5e0b19f8b1451p-33;
-    s = fma(s, z, -0x1.ae600b02b6262p-26);
-    s = fma(s, z, 0x1.71de37968a100p-19);
-    s = fma(s, z, -0x1.a01a019e83aaep-13);
-    s = fma(s, z, 0x1.1111111110bb2p-7);
-    s = fma(s, z, -0x1.5555555555555p-3);
+    s = fma_k(s, z, -0x1.ae600b02b6262p-26);
+    s = fma_k(s, z, 0x1.71de37968a100p-19);
+    s = fma_k(s, z, -0x1.a01a019e83aaep-13);
+    s = fma_k(s, z, 0x1.1111111110bb2p-7);
+    s = fma_k(s, z, -0x1.5555555555555p-3);
     return fma(r * z, s, r);
 }
 
@@ -328,27 +348,26 @@ MPGOS_HD MPGOS_INLINE double pow_ctrl(double x, double y)
 // for bit.  Subnormal R is scaled by 2^1000 first; 0 gives 0, +inf gives
 // +inf, NaN gives NaN.
 namespace detail {
-MPGOS_HD MPGOS_INLINE double root5(double x)
+// z^(1/5) as (q, z): fifth root of a normal x >= 0 as v 2^q; the caller scales
+MPGOS_HD MPGOS_INLINE double root5_parts(double x, int& q)
 {
-    const bool tiny = x < 0x1p-1000;
-    const double xs = tiny ? x * 0x1p1000 : x;
-    const uint64_t b = bits(xs);
+    const uint64_t b = bits(x);
     const int e = (int)(b >> 52) - 1023;
     const double m = from_bits((b & 0x000fffffffffffffull) | 0x3ff0000000000000ull);
-    const int q = (e + 1025) / 5 - 205;          // floor(e / 5)
+    q = (e + 1025) / 5 - 205;                    // floor(e / 5)
     const int r = e - 5 * q;                     // 0 .. 4
     const double z = m * pow2i(r);
     double pm = 0x1.d2cadb0bb3296p-7;            // m^(-1/5), Chebyshev fit on [1, 2]
-    pm = fma(pm, m, -0x1.ca9fab0a0d793p-4);
-    pm = fma(pm, m, 0x1.714a36f55ea3cp-2);
-    pm = fma(pm, m, -0x1.484ddb53b357dp-1);
-    pm = fma(pm, m, 0x1.60d7515a3c0e5p+0);
+    pm = fma_k(pm, m, -0x1.ca9fab0a0d793p-4);
+    pm = fma_k(pm, m, 0x1.714a36f55ea3cp-2);
+    pm = fma_k(pm, m, -0x1.484ddb53b357dp-1);
+    pm = fma_k(pm, m, 0x1.60d7515a3c0e5p+0);
     const double rd = (double)r;
     double pr = 0x1.88970ec6f3ab9p-17;           // 2^(-r/5) at r = 0 .. 4
-    pr = fma(pr, rd, -0x1.c4b4e3b1a9125p-12);
-    pr = fma(pr, rd, 0x1.3a4e88f4a3e7ap-7);
-    pr = fma(pr, rd, -0x1.1be579c2b43dbp-3);
-    pr = fma(pr, rd, 1.0);
+    pr = fma_k(pr, rd, -0x1.c4b4e3b1a9125p-12);
+    pr = fma_k(pr, rd, 0x1.3a4e88f4a3e7ap-7);
+    pr = fma_k(pr, rd, -0x1.1be579c2b43dbp-3);
+    pr = fma_k(pr, rd, 1.0);
     double w = pm * pr;
     for (int i = 0; i < 2; i++) {
         const double w2 = w * w;
@@ -358,10 +377,26 @@ MPGOS_HD MPGOS_INLINE double root5(double x)
     const double w2 = w * w, w4 = w2 * w2;
     const double y = z * w4;
     const double d = fma(-z, w4 * w, 1.0);      // w = z^(-1/5) (1 - d / 5): y = z^(1/5) (1 - 4 d / 5)
-    double v = fma(0.8 * d, y, y) * pow2i(tiny ? q - 200 : q);
+    return fma(0.8 * d, y, y);
+}
+
+MPGOS_HD MPGOS_INLINE double root5(double x)
+{
+    const bool tiny = x < 0x1p-1000;
+    int q;
+    const double v5 = root5_parts(tiny ? x * 0x1p1000 : x, q);
+    double v = v5 * pow2i(tiny ? q - 200 : q);
     v = x == 0.0 ? 0.0 : v;
     v = x > 0x1.fffffffffffffp+1023 ? x : v;
     return x != x ? x : v;
+}
+
+// root5's bits for x in [2^-1000, largest finite]
+MPGOS_HD MPGOS_INLINE double root5_regular(double x)
+{
+    int q;
+    const double v5 = root5_parts(x, q);
+    return v5 * pow2i(q);
 }
 } // namespace detail
 
@@ -370,6 +405,10 @@ MPGOS_HD MPGOS_INLINE double ctrl_root(double x, bool fifth)
     if (fifth) return detail::root5(x);
     return sqrt(sqrt(x));
 }
+
+// ctrl_root(x, true) for x in [2^-1000, largest finite] (the controller's
+// R >= 1 of an accepted step) without the tests for other arguments
+MPGOS_HD MPGOS_INLINE double ctrl_root_regular(double x) { return detail::root5_regular(x); }
 
 // ---------------------------------------------------------------- float versions
 // Used by the FP32 stepping mode: computed through the double routines and
@@ -380,6 +419,7 @@ MPGOS_HD MPGOS_INLINE float exp(float x) { return (float)exp((double)x); }
 MPGOS_HD MPGOS_INLINE float log(float x) { return (float)log((double)x); }
 MPGOS_HD MPGOS_INLINE float pow(float x, float y) { return (float)pow((double)x, (double)y); }
 MPGOS_HD MPGOS_INLINE float pow_ctrl(float x, float y) { return (float)pow_ctrl((double)x, (double)y); }
+MPGOS_HD MPGOS_INLINE float ctrl_root_regular(float x) { return (float)ctrl_root_regular((double)x); }
 MPGOS_HD MPGOS_INLINE float ctrl_root(float x, bool fifth) { return (float)ctrl_root((double)x, fifth); }
 MPGOS_HD MPGOS_INLINE float sqrt(float x) { return (float)sqrt((double)x); }   // exact: double has > 2 * 24 + 2 bits
 

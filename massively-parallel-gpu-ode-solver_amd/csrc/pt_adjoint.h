@@ -88,6 +88,7 @@ __device__ __forceinline__ void record_body(const AdjArgs<Sys>& A)
     const int tid = threadIdx.x + blockIdx.x * blockDim.x;
     using L_t = Lane<Sys, double, false, ALG>;
     L_t L;
+    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
     int untilCk = A.K, k = 0;      // accepted steps to the next checkpoint (no division in the loop)
     if (tid < a.nActive) {
         L.load(a, tid, sPAR, sPARi);
@@ -105,18 +106,21 @@ __device__ __forceinline__ void record_body(const AdjArgs<Sys>& A)
             }
         };
         if ((blockDim.x & 63) == 0) {
-            if (a.NDO > 0) L.template run_common_time<true>(a, sPAR, sPARi, A.K, untilCk, at);
-            else L.template run_common_time<false>(a, sPAR, sPARi, A.K, untilCk, at);
+            if (a.NDO > 0) L.template run_common_time<true>(c, sPAR, sPARi, A.K, untilCk, at);
+            else L.template run_common_time<false>(c, sPAR, sPARi, A.K, untilCk, at);
         }
     }
     if (tid >= a.nActive) return;
-    while (L.term == 0) {
-        const int before = L.nacc;
-        L.step(a, sPAR, sPARi);
-        if (L.nacc != before && --untilCk == 0) {
+    constexpr bool CARRY = L_t::NTT > 0;
+    double tt[Pos<L_t::NTT>::value];
+    L.time_terms(L.t, tt);
+    bool ended = L.term != 0, accepted;
+    while (!ended) {
+        ended = L.template step<true, CARRY>(c, sPAR, sPARi, accepted, tt);
+        if (accepted && --untilCk == 0) {
             untilCk = A.K;
             ++k;
-            if (L.term == 0 && tid < a.nActive) {
+            if (!ended) {
                 if (k < A.ckcap) store_checkpoint<Sys, ALG>(A, L, k);
                 else L.status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT;
             }
@@ -298,7 +302,7 @@ __device__ __forceinline__ bool common_time_reverse(const AdjArgs<Sys>& A, Lane<
                                                     double* bACC, int* bACCi)
 {
     constexpr int SD = Sys::SD, NTT = Lane<Sys, double, false, ALG>::NTT;
-    const Args<Sys, double, double>& a = A.a;
+    const typename Lane<Sys, double, false, ALG>::C a(A.a, false);
     const int K = A.K;
     if ((blockDim.x & 63) != 0 || K > 31 || !(a.dt0 > 0.0)) return false;
     const uint64_t live = __ballot(mine);
@@ -345,7 +349,7 @@ __device__ __forceinline__ bool common_time_reverse(const AdjArgs<Sys>& A, Lane<
         for (int c = 0; c < SD; c++)
             if (LDS_SEG || mine) seg((size_t)(slot * SD + c)) = L.X[c];   // HBM records end with the last instance
         L.rk4(a, h, nx, nullptr, sPAR, sPARi, tt1, ttm, tt4);
-        L.template accept<false>(a, h, dtP, nx, nullptr, EFn, 0, sPAR, sPARi);
+        L.accept(a, h, dtP, nx, nullptr, EFn, false, sPAR, sPARi);
     };
     // a step's record, read a step ahead of its use
     double x[SD];
@@ -436,6 +440,9 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
     const bool ok = mine && (a.status[tid] & MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT) == 0;
     const long long nseg = ok ? (total + A.K - 1) / A.K : 0;
     const int K = A.K;
+    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    constexpr bool CARRY = L_t::NTT > 0;
+    double tt[Pos<L_t::NTT>::value];
     // Restore segment s's checkpoint into the lane.
     auto restore = [&](long long s) {
         const size_t cb = (size_t)s * checkpoint_words<Sys>();
@@ -453,6 +460,7 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
         L.tc = 0.0;
         L.term = 0; L.udt = 0; L.nacc = 0; L.nrej = 0; L.status = 0; L.nev = 0;
         L.doIdx = 0; L.skipped = 0; L.doT = 0.0;
+        L.time_terms(L.t, tt);
     };
     // accepted steps of segment s
     auto count = [&](long long s) { return (int)((total - s * K) < K ? (total - s * K) : K); };
@@ -471,13 +479,9 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
 #pragma unroll
         for (int c = 0; c < SD; c++) xp[c] = L.X[c];
         const double tp = L.t;
-        const int before = L.nacc;
-        // the Cash-Karp step with its controller holds more uniform values
-        // than fit in SGPRs next to the adjoint chain: re-read the argument
-        // block at every attempt instead of spilling it
-        if constexpr (ALG == MPGOS_RKCK45) L.template step<false>(kernel_args<Args<Sys, double, double>>(), sPAR, sPARi);
-        else L.template step<false>(a, sPAR, sPARi);
-        if (L.nacc != before) {
+        bool accepted;
+        if (L.template step<false, CARRY>(c, sPAR, sPARi, accepted, tt)) L.term = 1;
+        if (accepted) {
             const size_t sb = (size_t)slot(flip, j) * (SD + 2);
 #pragma unroll
             for (int c = 0; c < SD; c++) seg(sb + c) = xp[c];

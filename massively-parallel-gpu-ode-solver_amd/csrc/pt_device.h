@@ -178,10 +178,54 @@ __device__ __forceinline__ void advance_by_lane_kahan(float& t, float& c, float 
                  : "+v"(t), "+v"(c), "=&s"(save), "=&v"(y), "=&v"(d) : "v"(h) : "scc");
 }
 
+// What a step reads of the argument block.  The control limits and tolerances
+// are put into vector registers once, before the step loop: in scalar registers
+// they and the step's constants exceed the 102 there are, and the compiler
+// reloads them from memory or rebuilds constants inside the loop (a lone
+// wavefront pays for every such instruction and waits for every load).
+template <class Sys, class P, class CP>
+struct StepArgs {
+    static constexpr int SD = Sys::SD, NE = Sys::NE;
+    CP dt0, dtmin, dtmax, grow, shrink;
+    CP least;                   // steps above it, and tolerances as they should be: the short way through step()
+    CP rtol[SD], atol[SD];
+    P etol[Pos<NE>::value];
+    int edir[Pos<NE>::value];
+    int NT, NDO, doFreq;
+
+    template <class T> static __device__ __forceinline__ T pin(T v)
+    {
+        asm volatile("" : "+v"(v));
+        return v;
+    }
+    __device__ __forceinline__ explicit StepArgs(const Args<Sys, P, CP>& a, bool adaptive)
+    {
+        dt0 = a.dt0; NT = a.NT; NDO = a.NDO; doFreq = a.doFreq;
+        if (adaptive) {
+            dtmin = pin(a.dtmin); dtmax = pin(a.dtmax); grow = pin(a.grow); shrink = pin(a.shrink);
+            CP l = a.dtmin * CP(1.01);
+#pragma unroll
+            for (int i = 0; i < NE; i++)
+                if (!(a.etol[i] >= P(0))) l = CP(__builtin_huge_val());
+            least = pin(l);
+#pragma unroll
+            for (int i = 0; i < SD; i++) { rtol[i] = pin(a.rtol[i]); atol[i] = pin(a.atol[i]); }
+        } else {
+            dtmin = a.dtmin;
+        }
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            etol[i] = pin(a.etol[i]);
+            edir[i] = a.edir[i];
+        }
+    }
+};
+
 template <class Sys, class P, bool KAHAN, int ALG>
 struct Lane {
     using CP = typename std::conditional<KAHAN, double, P>::type;
     using A = Args<Sys, P, CP>;
+    using C = StepArgs<Sys, P, CP>;
     using Sys_t = Sys;
     static constexpr bool kKahan = KAHAN;
     static constexpr int SD = Sys::SD, NCP = Sys::NCP, NE = Sys::NE, NA = Sys::NA, NIA = Sys::NIA;
@@ -326,6 +370,23 @@ struct Lane {
         doT = mpgos_fmin(t + a.doMinDt, TD[1]);
     }
 
+    // min and max of values that are results of arithmetic (never signalling
+    // NaNs): the instruction itself, where the builtin first canonicalises each
+    // operand whose origin it does not see (a v_max per operand).  _abs: of the
+    // magnitudes.
+#define MPGOS_MINMAX(name, ins)                                                                                                  \
+    static __device__ __forceinline__ double name(double x, double y)                                                           \
+    { double r; asm(ins "_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y)); return r; }                                              \
+    static __device__ __forceinline__ float name(float x, float y)                                                              \
+    { float r; asm(ins "_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y)); return r; }
+    MPGOS_MINMAX(lane_min, "v_min")
+    MPGOS_MINMAX(lane_max, "v_max")
+#undef MPGOS_MINMAX
+    static __device__ __forceinline__ double lane_max_abs(double x, double y)
+    { double r; asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(x), "v"(y)); return r; }
+    static __device__ __forceinline__ float lane_max_abs(float x, float y)
+    { float r; asm("v_max_f32 %0, |%1|, |%2|" : "=v"(r) : "v"(x), "v"(y)); return r; }
+
     static __device__ __forceinline__ double mpgos_fmin(double x, double y) { return __builtin_fmin(x, y); }
     static __device__ __forceinline__ float mpgos_fmin(float x, float y) { return __builtin_fminf(x, y); }
     static __device__ __forceinline__ double mpgos_fmax(double x, double y) { return __builtin_fmax(x, y); }
@@ -347,7 +408,7 @@ struct Lane {
     // RK4: PT-STP:6-117, with the time terms at t, t + h/2 and t + h.  Returns
     // next state in `nx`; in Kahan mode `inc` gets the increment
     // dt/6 (k1 + 2k2 + 2k3 + k4).
-    __device__ __forceinline__ void rk4(const A& a, P h, P* nx, P* inc, P* sPAR, int* sPARi, const P* tt1, const P* ttm,
+    __device__ __forceinline__ void rk4(const C& a, P h, P* nx, P* inc, P* sPAR, int* sPARi, const P* tt1, const P* ttm,
                                         const P* tt4)
     {
         using math::fma;
@@ -374,17 +435,20 @@ struct Lane {
         }
     }
 
-    // RKCK45: PT-STP:121-290.  err[] in control precision.
-    __device__ __forceinline__ void rkck45(const A& a, P h, P* nx, P* inc, CP* err, int& isfin, P* sPAR, int* sPARi)
+    // RKCK45: PT-STP:121-290.  err[] in control precision.  tt: the time terms
+    // at t; tt5 receives those at t + h.
+    __device__ __forceinline__ void rkck45(const C& a, P h, P* nx, P* inc, CP* err, P* sPAR, int* sPARi, const P* tt, P* tt5)
     {
         using math::fma;
         P Xs[SD], k1[SD], k2[SD], k3[SD], k4[SD], k5[SD], k6[SD];
-        Sys::template OdeFunction<P>(tid, a.NT, k1, X, t, cPAR, sPAR, sPARi, ACC, ACCi);
+        P ts[Pos<NTT>::value];
+        ode(a.NT, k1, X, t, tt, sPAR, sPARi);
 
         P T = fma(h, P(1.0 / 5.0), t);
 #pragma unroll
         for (int i = 0; i < SD; i++) Xs[i] = fma(h, P(1.0 / 5.0) * k1[i], X[i]);
-        Sys::template OdeFunction<P>(tid, a.NT, k2, Xs, T, cPAR, sPAR, sPARi, ACC, ACCi);
+        time_terms(T, ts);
+        ode(a.NT, k2, Xs, T, ts, sPAR, sPARi);
 
         T = fma(h, P(3.0 / 10.0), t);
 #pragma unroll
@@ -393,7 +457,8 @@ struct Lane {
             s = fma(P(9.0 / 40.0), k2[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        Sys::template OdeFunction<P>(tid, a.NT, k3, Xs, T, cPAR, sPAR, sPARi, ACC, ACCi);
+        time_terms(T, ts);
+        ode(a.NT, k3, Xs, T, ts, sPAR, sPARi);
 
         T = fma(h, P(3.0 / 5.0), t);
 #pragma unroll
@@ -403,7 +468,8 @@ struct Lane {
             s = fma(P(6.0 / 5.0), k3[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        Sys::template OdeFunction<P>(tid, a.NT, k4, Xs, T, cPAR, sPAR, sPARi, ACC, ACCi);
+        time_terms(T, ts);
+        ode(a.NT, k4, Xs, T, ts, sPAR, sPARi);
 
         T = t + h;
 #pragma unroll
@@ -414,7 +480,8 @@ struct Lane {
             s = fma(P(35.0 / 27.0), k4[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        Sys::template OdeFunction<P>(tid, a.NT, k5, Xs, T, cPAR, sPAR, sPARi, ACC, ACCi);
+        time_terms(T, tt5);
+        ode(a.NT, k5, Xs, T, tt5, sPAR, sPARi);
 
         T = fma(h, P(7.0 / 8.0), t);
 #pragma unroll
@@ -426,7 +493,8 @@ struct Lane {
             s = fma(P(253.0 / 4096.0), k5[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        Sys::template OdeFunction<P>(tid, a.NT, k6, Xs, T, cPAR, sPAR, sPARi, ACC, ACCi);
+        time_terms(T, ts);
+        ode(a.NT, k6, Xs, T, ts, sPAR, sPARi);
 
 #pragma unroll
         for (int i = 0; i < SD; i++) {
@@ -454,42 +522,52 @@ struct Lane {
                 if (std::is_same<P, double>::value) err[i] = (CP)math::fma((double)h, (double)math::fabs(e), 1e-18);
                 else err[i] = (CP)((double)(h * math::fabs(e)) + 1e-18);   // float*float, then + double literal
             }
-            if (!math::isfinite(nx[i]) || !math::isfinite(err[i])) isfin = 0;
         }
     }
 
     // ------------------------------------------------------------ controllers
-    // PT-CTL:23-86
-    __device__ __forceinline__ void control_rkck45(const A& a, const P* nx, const CP* err, int& update, int& isfin)
+    __device__ __forceinline__ void next_step_size(const C& a, CP fac)
     {
-        CP R = CP(1e30);
+        fac = lane_min(fac, a.grow);
+        fac = lane_max(fac, a.shrink);
+        newDt = dt * fac;
+        newDt = lane_min(newDt, a.dtmax);
+        newDt = lane_max(newDt, a.dtmin);
+    }
+
+    // PT-CTL:23-86, every case of it.  root: R^(1/5) for R >= 2^-1000.
+    __device__ __forceinline__ void control_rkck45(const C& a, const P* nx, const CP* err, const CP* tol, CP R, CP root, int& update)
+    {
+        bool ok = true, fin = true;
 #pragma unroll
         for (int i = 0; i < SD; i++) {
-            const CP tol = mpgos_fmax(a.rtol[i] * mpgos_fmax(math::fabs((CP)nx[i]), math::fabs((CP)X[i])), a.atol[i]);
-            update = update && (err[i] < tol);
-            R = mpgos_fmin(R, tol / err[i]);
+            ok = ok && err[i] < tol[i];
+            fin = fin && math::isfinite(nx[i]) && math::isfinite(err[i]);
         }
-        // one power for both outcomes: lanes of a wavefront that accept and
-        // lanes that reject then share one evaluation
-        CP fac = CP(0.9) * math::ctrl_root(R, update == 1);
-        if (!math::isfinite(fac)) isfin = 0;
-
-        if (isfin == 0) {
-            fac = a.shrink;
-            update = 0;
-            if (dt < a.dtmin * CP(1.01)) { term = 1; status |= MPGOS_STATUS_NONFINITE_MIN_STEP; }
-        } else {
-            if (dt < a.dtmin * CP(1.01)) { update = 1; status |= MPGOS_STATUS_MIN_STEP_REACHED; }
+        if (__builtin_amdgcn_ballot_w64(!(R >= CP(0x1p-100))) != 0) root = math::ctrl_root(R, true);
+        if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
+            const CP fourth = math::ctrl_root(R, false);
+            root = ok ? root : fourth;
         }
-        fac = mpgos_fmin(fac, a.grow);
-        fac = mpgos_fmax(fac, a.shrink);
-        newDt = dt * fac;
-        newDt = mpgos_fmin(newDt, a.dtmax);
-        newDt = mpgos_fmax(newDt, a.dtmin);
+        CP fac = CP(0.9) * root;
+        fin = fin && math::isfinite(fac);
+        const bool smallest = dt < a.dtmin * CP(1.01);
+        if (__builtin_amdgcn_ballot_w64(!fin || smallest) != 0) {
+            if (!fin) {
+                fac = a.shrink;
+                ok = false;
+                if (smallest) { term = 1; status |= MPGOS_STATUS_NONFINITE_MIN_STEP; }
+            } else if (smallest) {
+                ok = true;
+                status |= MPGOS_STATUS_MIN_STEP_REACHED;
+            }
+        }
+        update = ok ? 1 : 0;
+        next_step_size(a, fac);
     }
 
     // PT-EVT:5-45
-    __device__ __forceinline__ void event_control(const A& a, const P* EFn, int& update)
+    __device__ __forceinline__ void event_control(const C& a, const P* EFn, int& update)
     {
         CP evDt = dt;
         int corrected = 0;
@@ -511,57 +589,120 @@ struct Lane {
     }
 
     // ------------------------------------------------------------ one attempted step
-    // One iteration of the loop at PT-SOL:197-394.  DENSE = false compiles the
+    // One iteration of the loop at PT-SOL:197-394; returns whether the instance
+    // has ended, `accepted` whether the step was.  DENSE = false compiles the
     // dense-output bookkeeping out (the adjoint's re-steps, which run with
-    // NDO = 0), so that the step has no branch on it.
-    template <bool DENSE = true>
-    __device__ __forceinline__ void step(const A& a, P* sPAR, int* sPARi)
+    // NDO = 0), so that the step has no branch on it.  CARRY: tt holds the time
+    // terms at t (time_terms(t, tt) before the first step); else they are
+    // evaluated anew.
+    template <bool DENSE = true, bool CARRY = false>
+    __device__ __forceinline__ bool step(const C& a, P* sPAR, int* sPARi, bool& accepted, P* tt = nullptr)
     {
         const int NT = a.NT;
-        int update = 1, isfin = 1, endReached = 0;
+        int update = 1, isfin = 1;
+        bool stop;
         dt = newDt;
         CP remaining;
         if (KAHAN) remaining = (CP)TD[1] - ((CP)t - (CP)tc);
         else remaining = (CP)(TD[1] - t);
-        if (dt > remaining) { dt = remaining; endReached = 1; }
+        const bool endReached = dt > remaining;
+        if (endReached) dt = remaining;
 
         const P h = (P)dt;
         P nx[SD], inc[KAHAN ? SD : 1];
-        if (ALG == MPGOS_RK4) {
-            P tt1[Pos<NTT>::value], ttm[Pos<NTT>::value], tt4[Pos<NTT>::value];
+        P tt1[Pos<NTT>::value], ttm[Pos<NTT>::value], ttEnd[Pos<NTT>::value];
+        if constexpr (CARRY) {
+#pragma unroll
+            for (int i = 0; i < NTT; i++) tt1[i] = tt[i];
+        } else {
             time_terms(t, tt1);
+        }
+        P EFn[Pos<NE>::value];
+        P dtP = h;
+        if constexpr (ALG == MPGOS_RK4) {
             time_terms(t + P(0.5) * h, ttm);
-            time_terms(t + h, tt4);
-            rk4(a, h, nx, inc, sPAR, sPARi, tt1, ttm, tt4);
+            time_terms(t + h, ttEnd);
+            rk4(a, h, nx, inc, sPAR, sPARi, tt1, ttm, ttEnd);
 #pragma unroll
             for (int i = 0; i < SD; i++)
                 if (!math::isfinite(nx[i])) isfin = 0;
             // PT-CTL:5-20
             if (isfin == 0) { term = 1; status |= MPGOS_STATUS_NONFINITE_RK4; }
             newDt = a.dt0;
+            if (NE > 0) Sys::template EventFunction<P>(tid, NT, EFn, t + h, dtP, TD, nx, cPAR, sPAR, sPARi, ACC, ACCi);
+            accepted = settle<CARRY>(a, h, dtP, nx, inc, EFn, update, sPAR, sPARi, tt, ttEnd);
+            stop = term != 0;
         } else {
-            CP err[SD];
-            rkck45(a, h, nx, inc, err, isfin, sPAR, sPARi);
-            control_rkck45(a, nx, err, update, isfin);
+            CP err[SD], tol[SD];
+            rkck45(a, h, nx, inc, err, sPAR, sPARi, tt1, ttEnd);
+            if (NE > 0) Sys::template EventFunction<P>(tid, NT, EFn, t + h, dtP, TD, nx, cPAR, sPAR, sPARi, ACC, ACCi);
+            // Nearly always every lane of the wavefront has an accepted, finite
+            // step above the smallest size with no event near: u < 0 in one
+            // comparison and one branch per wavefront, and no execution mask.
+            // Each u >= 0 (or NaN) sends the wavefront the general way, which
+            // decides every case as the reference does.  A comparison whose
+            // result a scalar instruction or branch waits for costs a lone
+            // wavefront 20 cycles, a branch 10 to 20 more, a vector
+            // instruction 4; so the tests are folded into arithmetic:
+            //   err_i < tol_i           <=>  err_i - tol_i < 0
+            //   no event near           <=   |EF| tolerance - (EFn with the sign of EF) <= 0
+            //   everything finite       <=>  adding 0 * value leaves u as it is
+            // Whole Solves against one masked way for all cases: 256 relief
+            // valves 520 -> 325 us, 50001 Lorenz instances 2660 -> 2140 us,
+            // 262144 in the sorted form 3.22 -> 2.93 ms, 20000 Duffing instances
+            // with events 129 -> 116 ms, Cash-Karp adjoint of 10007 4.50 -> 3.76 ms.
+            CP R = CP(1e30), u = a.least - dt;
+#pragma unroll
+            for (int i = 0; i < SD; i++) {
+                tol[i] = lane_max(a.rtol[i] * lane_max_abs((CP)nx[i], (CP)X[i]), a.atol[i]);
+                u = lane_max(u, err[i] - tol[i]);
+                R = lane_min(R, tol[i] / err[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < NE; i++) u = lane_max(u, (CP)(a.etol[i] - math::flip_sign(EFn[i], EF[i])));
+#pragma unroll
+            for (int i = 0; i < SD; i++) u = math::fma((CP)nx[i], CP(0), math::fma(err[i], CP(0), u));
+            const uint64_t unusual = __builtin_amdgcn_ballot_w64(!(u < CP(0)));
+            const CP root = math::ctrl_root_regular(R);
+            if (__builtin_expect(unusual == 0, 1)) {
+                next_step_size(a, CP(0.9) * root);
+#pragma unroll
+                for (int i = 0; i < NTT; i++) if (CARRY) tt[i] = ttEnd[i];
+                accept(a, h, dtP, nx, inc, EFn, false, sPAR, sPARi);
+                accepted = true;
+                stop = false;
+            } else {
+                control_rkck45(a, nx, err, tol, R, root, update);
+                accepted = settle<CARRY>(a, h, dtP, nx, inc, EFn, update, sPAR, sPARi, tt, ttEnd);
+                stop = term != 0;
+            }
         }
-
-        P EFn[Pos<NE>::value];
-        P dtP = h;
-        if (NE > 0) {
-            Sys::template EventFunction<P>(tid, NT, EFn, t + h, dtP, TD, nx, cPAR, sPAR, sPARi, ACC, ACCi);
-            event_control(a, EFn, update);
+        if (DENSE && __builtin_expect(a.NDO > 0, 0)) {
+            if (accepted) dense_output(a, endReached);
         }
+        return stop || (accepted && (endReached || udt == 1));
+    }
 
-        if (update == 1) accept<DENSE>(a, h, dtP, nx, inc, EFn, endReached, sPAR, sPARi);
+    // After the controller: event step control, then the accepted or rejected step.
+    template <bool CARRY>
+    __device__ __forceinline__ bool settle(const C& a, P h, P& dtP, const P* nx, const P* inc, P* EFn, int update, P* sPAR,
+                                           int* sPARi, P* tt, const P* ttEnd)
+    {
+        if (NE > 0) event_control(a, EFn, update);
+        if constexpr (CARRY) {
+            // t + h becomes t when the step is accepted
+#pragma unroll
+            for (int i = 0; i < NTT; i++) tt[i] = update == 1 ? ttEnd[i] : tt[i];
+        }
+        if (update == 1) accept(a, h, dtP, nx, inc, EFn, true, sPAR, sPARi);
         else nrej++;
+        return update == 1;
     }
 
     // The accepted part of the loop body (PT-SOL:323-394): t and x take the
-    // step's values, then the user's action, event detection, dense output and
-    // termination.
-    template <bool DENSE>
-    __device__ __forceinline__ void accept(const A& a, P h, P& dtP, const P* nx, const P* inc, P* EFn, int endReached, P* sPAR,
-                                           int* sPARi)
+    // step's values, then the user's action and event detection (dense output and
+    // termination follow).
+    __device__ __forceinline__ void accept(const C& a, P h, P& dtP, const P* nx, const P* inc, P* EFn, bool near, P* sPAR, int* sPARi)
     {
         const int NT = a.NT;
         if (KAHAN) {
@@ -576,42 +717,46 @@ struct Lane {
         }
         Sys::template ActionAfterSuccessfulTimeStep<P>(tid, NT, udt, t, dtP, TD, X, cPAR, sPAR, sPARi, ACC, ACCi);
         if (NE > 0) {
+            if (near) {
 #pragma unroll
-            for (int i = 0; i < NE; i++) {
-                const P tol = a.etol[i];
-                if ((EF[i] > tol && math::fabs(EFn[i]) < tol && a.edir[i] <= 0) ||
-                    (EF[i] < -tol && math::fabs(EFn[i]) < tol && a.edir[i] >= 0)) {
-                    const A& c = kernel_args<A>();   // rare path: fields loaded here
-                    if (nev < c.evcap) {
-                        const long long base = (long long)nev * (SD + 1);
-                        c.evlog[tid + base * NT] = t;
+                for (int i = 0; i < NE; i++) {
+                    const P tol = a.etol[i];
+                    if ((EF[i] > tol && math::fabs(EFn[i]) < tol && a.edir[i] <= 0) ||
+                        (EF[i] < -tol && math::fabs(EFn[i]) < tol && a.edir[i] >= 0)) {
+                        const A& c = kernel_args<A>();   // rare path: fields loaded here
+                        if (nev < c.evcap) {
+                            const long long base = (long long)nev * (SD + 1);
+                            c.evlog[tid + base * NT] = t;
 #pragma unroll
-                        for (int j = 0; j < SD; j++) c.evlog[tid + (base + 1 + j) * NT] = X[j];
-                        c.evlogidx[tid + (long long)nev * NT] = i;
+                            for (int j = 0; j < SD; j++) c.evlog[tid + (base + 1 + j) * NT] = X[j];
+                            c.evlogidx[tid + (long long)nev * NT] = i;
+                        }
+                        nev++;
+                        Sys::template ActionAfterEventDetection<P>(tid, NT, i, udt, t, dtP, TD, X, cPAR, sPAR, sPARi, ACC, ACCi);
                     }
-                    nev++;
-                    Sys::template ActionAfterEventDetection<P>(tid, NT, i, udt, t, dtP, TD, X, cPAR, sPAR, sPARi, ACC, ACCi);
                 }
             }
             Sys::template EventFunction<P>(tid, NT, EFn, t, dtP, TD, X, cPAR, sPAR, sPARi, ACC, ACCi);
 #pragma unroll
             for (int i = 0; i < NE; i++) EF[i] = EFn[i];
         }
-        if (DENSE && a.NDO > 0) {
-            // PT-DO:40-58 then PT-DO:5-37
-            int upd;
-            if (doIdx < a.NDO && doT < t && skipped >= a.doFreq - 1) upd = 1;
-            else upd = 0;
-            if (doIdx < a.NDO && (endReached == 1 || udt == 1)) upd = 1;
-            if (upd) {
-                if constexpr (kCommonTime) store_dense(kernel_args_joined<A>());
-                else store_dense(kernel_args<A>());
-            }
-            else skipped++;
-        }
-        if (endReached == 1 || udt == 1) term = 1;
         dt = (CP)dtP;   // a callback may have changed dT; it reaches Finalization (PT-SOL:398-410)
         nacc++;
+    }
+
+    // PT-DO:40-58 then PT-DO:5-37
+    __device__ __forceinline__ void dense_output(const C& a, bool endReached)
+    {
+        int upd;
+        if (doIdx < a.NDO && doT < t && skipped >= a.doFreq - 1) upd = 1;
+        else upd = 0;
+        if (doIdx < a.NDO && (endReached || udt == 1)) upd = 1;
+        if (upd) {
+            if constexpr (kCommonTime) store_dense(kernel_args_joined<A>());
+            else store_dense(kernel_args<A>());
+        } else {
+            skipped++;
+        }
     }
 
     // ------------------------------------------------------------ common time
@@ -635,7 +780,7 @@ struct Lane {
     // calls at(until) after every `every` accepted steps, the first after
     // `until`.
     template <bool DENSE, class F>
-    __device__ __forceinline__ void run_common_time(const A& a, P* sPAR, int* sPARi, int every, int& until, F&& at)
+    __device__ __forceinline__ void run_common_time(const C& a, P* sPAR, int* sPARi, int every, int& until, F&& at)
     {
         constexpr int PTS = KAHAN ? 3 : 2, BLK = KAHAN ? 21 : 31;
         const uint64_t live = __ballot(term == 0);
@@ -682,7 +827,8 @@ struct Lane {
                     rk4(a, h, nx, inc, sPAR, sPARi, tt1, ttm, tt4);
 #pragma unroll
                     for (int i = 0; i < SD; i++) zero = math::fma(nx[i], P(0), zero);
-                    accept<DENSE>(a, h, dtP, nx, inc, EFn, 0, sPAR, sPARi);
+                    accept(a, h, dtP, nx, inc, EFn, false, sPAR, sPARi);
+                    if (DENSE) dense_output(a, false);
                     ended |= udt;
 #pragma unroll
                     for (int i = 0; i < NTT; i++) tt1[i] = tt4[i];
@@ -780,40 +926,40 @@ __device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys,
     const int n = (SLICED && a.listLenDev) ? (int)*a.listLenDev : a.listLen;
     using L_t = Lane<Sys, P, KAHAN, ALG>;
     L_t L;
+    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
     const int id = i < n ? (a.list ? a.list[i] : i) : 0;
     constexpr bool COMMON = !SLICED && L_t::kCommonTime;
+    // a step's end is the next one's start (in the compensated form it is not t + h)
+    constexpr bool CARRY = L_t::NTT > 0 && !KAHAN;
+    P tt[Pos<L_t::NTT>::value];
     if constexpr (COMMON) {
         if (i < n) L.load(a, id, sPAR, sPARi);
         else L.idle();
         // whole wavefronts only (the lanes of a wavefront work together)
         if ((blockDim.x & 63) == 0) {
             int until = 0;
-            if (a.NDO > 0) L.template run_common_time<true>(a, sPAR, sPARi, 0, until, [] {});
-            else L.template run_common_time<false>(a, sPAR, sPARi, 0, until, [] {});
+            if (a.NDO > 0) L.template run_common_time<true>(c, sPAR, sPARi, 0, until, [] {});
+            else L.template run_common_time<false>(c, sPAR, sPARi, 0, until, [] {});
         }
     }
     if (i < n) {
-        // With event functions the step keeps more uniform values live (event
-        // tolerances, direction tests) than there are SGPRs, and the
-        // compiler spills argument fields to VGPR lanes and reloads them as
-        // whole 16-register tuples inside the loop; re-reading the argument
-        // block at every step instead keeps the loop free of spills (fewer
-        // instructions per step, which bounds a lone lane).  Without events
-        // the loop does not spill and keeps its hoisted arguments.
-        auto step_args = [&]() -> const typename L_t::A& {
-            if constexpr (Sys::NE > 0) return kernel_args<typename L_t::A>();
-            else return a;
-        };
         if constexpr (SLICED) {
             // the loop only steps; finishing or suspending follows it, so
             // the step loop keeps the plain form's registers
             L.begin(a, id, sPAR, sPARi);
-            do L.step(step_args(), sPAR, sPARi);
-            while (!L.stop());
+            L.time_terms(L.t, tt);
+            // the budget is the same for every lane
+            int left = a.slice;
+            bool ended, accepted;
+            do ended = L.template step<true, CARRY>(c, sPAR, sPARi, accepted, tt);
+            while (!ended && --left > 0);
+            if (ended) L.term = 1;
             L.release(kernel_args<typename L_t::A>(), sPAR, sPARi);
         } else {
             if constexpr (!COMMON) L.load(a, id, sPAR, sPARi);
-            while (L.term == 0) L.step(step_args(), sPAR, sPARi);
+            L.time_terms(L.t, tt);
+            bool ended = L.term != 0, accepted;
+            while (!ended) ended = L.template step<true, CARRY>(c, sPAR, sPARi, accepted, tt);
             if constexpr (COMMON) L.finish(kernel_args_joined<typename L_t::A>(), sPAR, sPARi);
             else L.finish(kernel_args<typename L_t::A>(), sPAR, sPARi);
         }
@@ -855,6 +1001,7 @@ __device__ __forceinline__ void persistent_body(const Args<Sys, P, typename Lane
     const unsigned lane = __lane_id();
 
     L_t L;
+    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
     bool busy = false;
     const unsigned D = (unsigned)a.solo;
     if (tid == 0) {
@@ -942,13 +1089,15 @@ __device__ __forceinline__ void persistent_body(const Args<Sys, P, typename Lane
         for (int m = 0; m < a.roundSteps; m++) {
             if (!__any(busy)) break;
             if (busy) {
-                L.step(a, sPAR, sPARi);
+                bool accepted;
+                const bool ended = L.step(c, sPAR, sPARi, accepted);
+                if (ended) L.term = 1;
                 if constexpr (SLICED) {
                     if (L.stop()) {
                         L.release(kernel_args<typename L_t::A>(), sPAR, sPARi);
                         busy = false;
                     }
-                } else if (L.term) {
+                } else if (ended) {
                     L.finish(kernel_args<typename L_t::A>(), sPAR, sPARi);
                     busy = false;
                 }
