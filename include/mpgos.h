@@ -334,13 +334,14 @@ enum {
     MPGOS_PB_SHARED_GLOBAL_VARIABLES,
     MPGOS_PB_SHARED_COUPLING_MATRICES,
     /* New (no reference counterpart): which coupling kernel runs.  0 automatic
-     * (the dense-contraction MFMA kernel for a full FP64 matrix with UPS a
-     * multiple of 32 in [32, 256], else lane per pair), 1 lane per pair (any
-     * storage form; SPB as created), 2 dense contraction (8 systems per
-     * workgroup, 2*UPS threads).  Results are bit-identical between them. */
+     * (the dense-contraction MFMA kernel for full FP64 matrices up to 256
+     * units; lane per pair for all other matrices, and for up to 8 units when
+     * the systems alone fill the device), 1 lane per pair (any storage form;
+     * SPB as created), 2 dense contraction (UPS a multiple of 32 in [32, 256];
+     * 4 or 8 systems per workgroup).  Results are bit-identical between them. */
     MPGOS_PB_COUPLING_KERNEL,
-    /* New: units per lane of the dense-contraction kernel, 4 (2*UPS threads,
-     * the default) or 2 (4*UPS threads).  A launch shape only. */
+    /* New: 2 or 4, a launch-shape hint that is accepted and has no effect any
+     * more (the dense-contraction kernel chooses its split itself). */
     MPGOS_PB_MFMA_UNITS_PER_LANE,
     MPGOS_PB_NUM_OPTIONS
 };

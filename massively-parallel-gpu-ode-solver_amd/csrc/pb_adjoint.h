@@ -35,7 +35,7 @@
 // returns the same bits as the lane form.
 #pragma once
 
-#include "pb_device.h"
+#include "pb_dense.h"
 
 namespace mpgos {
 namespace pb {
@@ -446,21 +446,6 @@ __device__ __forceinline__ double rk_a(int s, int l)
                                 {-11.0 / 54.0, 5.0 / 2.0, -70.0 / 27.0, 35.0 / 27.0, 0},
                                 {1631.0 / 55296.0, 175.0 / 512.0, 575.0 / 13824.0, 44275.0 / 110592.0, 253.0 / 4096.0}};
     return l < s ? A[s][l] : 0.0;
-}
-
-template <int ALG>
-__device__ __forceinline__ double rk_stage_time(int s, double t, double h)
-{
-    using math::fma;
-    if (ALG == MPGOS_RK4) return s == 0 ? t : (s == 3 ? t + h : t + 0.5 * h);
-    switch (s) {
-    case 0: return t;
-    case 1: return fma(1.0 / 5.0, h, t);
-    case 2: return fma(3.0 / 10.0, h, t);
-    case 3: return fma(3.0 / 5.0, h, t);
-    case 4: return t + h;
-    default: return fma(7.0 / 8.0, h, t);
-    }
 }
 
 // LDS of the dense-contraction reverse pass: system scopes, the B operand and

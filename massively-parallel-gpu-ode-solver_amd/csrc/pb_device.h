@@ -1,6 +1,5 @@
 // Per-block coupled-systems solver for gfx950: one workgroup integrates SPB
-// systems of UPS coupled units; a lane owns PAIRS (system, unit) pairs of one
-// unit (PAIRS = 1 in the lane-per-pair form, 2 in the dense-contraction form).
+// systems of UPS coupled units, a lane owns one (system, unit) pair.
 //
 // Semantics follow the reference's per-block kernels
 // (SourceCodes/CoupledSystmes_PerBlock_Solver.cuh, single-system form at
@@ -24,19 +23,11 @@
 // form of the reference's expressions, so the host oracle reproduces every bit.
 //
 // Two coupling forms:
-//  * lane-per-pair (any storage form): each lane forms its own dot product,
-//    coupling matrix from L2 (or LDS), coupling terms double-buffered in LDS
-//    (one barrier per stage);
-//  * dense contraction (full matrix, FP64, UPS a multiple of 32 up to 256, 8
-//    systems per workgroup, 4 pairs per lane): the products C . [CPT_s0 ..
-//    CPT_s7] of all 8 systems run on v_mfma_f64_4x4x4f64 (mfma_contract44:
-//    four 4 x 4 x 4 blocks per instruction take the four 4-row slices of a
-//    16-unit tile against 4 systems; two chains per tile cover the 8
-//    systems).  The instruction accumulates its four products as a chain of
-//    fused multiply-adds in k order, so chaining the column blocks in order
-//    equals the sequential fma(M[u][col], CPT[col], v) over col = 0 .. UPS-1
-//    of the lane-per-pair form bit for bit.  Results go through LDS to the
-//    lane that owns the pair (two barriers per stage).
+//  * lane-per-pair (any storage form and precision, this file): each lane forms
+//    its own dot product, coupling matrix from L2 (or LDS), coupling terms
+//    double-buffered in LDS (one barrier per stage);
+//  * dense contraction (full FP64 matrix, pb_dense.h): the products of all
+//    systems of a workgroup on the matrix cores, with the same bits.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -64,19 +55,10 @@ __device__ __forceinline__ void lds_barrier()
 }
 
 constexpr int kMaxBlock = 1024;
-constexpr int kMfmaSystems = 8;          // systems per workgroup of the dense-contraction form
-constexpr int kMfmaPairs = 4;            // default pairs per lane of the dense-contraction form (2 * UPS threads)
+constexpr int kMfmaSystems = 8;          // systems per workgroup of the dense-contraction reverse pass
+constexpr int kMfmaPairs = 4;            // its pairs per lane (2 * UPS threads)
 
-// Tiles of the dense-contraction form that a wave contracts together: all of
-// its PAIRS / 2 tiles when the lane's unit states and stage vectors leave room
-// in the registers (UD * PAIRS <= 8), else one at a time.  Only the first way
-// keeps leading matrix pairs in LDS.
-template <class Sys, int PAIRS>
-__host__ __device__ constexpr int mfma_tiles_together() { return PAIRS >= 4 && Sys::UD * PAIRS <= 8 ? PAIRS / 2 : 1; }
-template <class Sys, int PAIRS>
-__host__ __device__ constexpr bool mfma_lds_matrix() { return mfma_tiles_together<Sys, PAIRS>() > 1; }
-
-// LDS of the dense-contraction form: the B operand (coupling terms) and the
+// LDS of the dense-contraction reverse pass: the B operand (coupling terms) and the
 // contraction results, one row of UPS + 2 doubles per (coupling, block
 // system).  A wave's writes and reads of one system's consecutive units fall
 // in consecutive banks; rows 4 banks apart (UPS a multiple of 16) put the B
@@ -91,7 +73,7 @@ __host__ __device__ inline size_t mfma_index(int i, int s, int u, int UPS)
     return ((size_t)i * kMfmaSystems + s) * mfma_row(UPS) + u;
 }
 
-enum Coupling { kLaneCoupling = 0, kMfmaCoupling = 1 };
+enum Coupling { kLaneCoupling = 0, kDenseCoupling = 1 };
 
 // CP: precision of the step size, tolerances and controller (FP64 in the
 // FLOAT_KAHAN mode, else P).
@@ -105,7 +87,7 @@ struct Args {
     P* DOx;                   // unit index + component * NU + k * NU * UD
     // global scope
     P* gPAR; int* gPARi; int* cIndex; P* cMat;
-    const P* cTile;           // dense-contraction form: the matrix in column-block pairs per lane (null: read cMat)
+    const P* cTile;           // dense-contraction form: the matrix in column-block pairs per lane
     int ldsPairs;             // dense-contraction form: leading column-block pairs of every tile of cTile held in LDS
     long long* nacc; long long* nrej; int* status;
     int NS, UPS, SPB, nActive, NDO, CBW, CCI, cMatSize, sharedGlobals, sharedMatrix;
@@ -158,31 +140,22 @@ template <class P> __device__ __forceinline__ P dmax(P a, P b);
 template <> __device__ __forceinline__ double dmax<double>(double a, double b) { return __builtin_fmax(a, b); }
 template <> __device__ __forceinline__ float dmax<float>(float a, float b) { return __builtin_fmaxf(a, b); }
 
-// LDS bytes: system scopes, coupling terms (two [system][unit][coupling]
-// buffers in the lane-per-pair form; one [coupling][unit][16] B-operand
-// buffer plus a [coupling][unit][system] result buffer in the dense form),
-// optional global parameters and coupling matrix copies.
+// LDS of the lane-per-pair form: system scopes, two [system][unit][coupling]
+// buffers of coupling terms, optional copies of the global parameters and
+// coupling matrices.
 struct LdsLayout {
-    size_t cpt, coup, g, gi, m, mt, total;
+    size_t cpt, g, gi, m, total;
 };
 
 template <class Sys, class P, bool KAHAN = false>
-__host__ __device__ inline LdsLayout lds_layout(int cpl, int SPB, int UPS, int sharedGlobals, int sharedMatrix,
-                                                int cMatSize, int ldsPairs = 0)
+__host__ __device__ inline LdsLayout lds_layout(int SPB, int UPS, int sharedGlobals, int sharedMatrix, int cMatSize)
 {
     constexpr int NCp = Pos<Sys::NC>::value;
     LdsLayout L;
     size_t o = (size_t)SPB * sizeof(SysScope<Sys, P, KAHAN>);
     o = (o + 15) & ~(size_t)15;
     L.cpt = o;
-    if (cpl == kMfmaCoupling) {
-        o += (size_t)NCp * kMfmaSystems * mfma_row(UPS) * sizeof(P);
-        L.coup = o;
-        o += (size_t)NCp * kMfmaSystems * mfma_row(UPS) * sizeof(P);
-    } else {
-        o += 2 * (size_t)SPB * UPS * NCp * sizeof(P);
-        L.coup = o;
-    }
+    o += 2 * (size_t)SPB * UPS * NCp * sizeof(P);
     L.g = o;
     if (sharedGlobals) o += (size_t)Sys::NGP * sizeof(P);
     o = (o + 15) & ~(size_t)15;
@@ -190,10 +163,7 @@ __host__ __device__ inline LdsLayout lds_layout(int cpl, int SPB, int UPS, int s
     if (sharedMatrix) o += (size_t)Sys::NC * cMatSize * sizeof(P);
     L.gi = o;
     if (sharedGlobals) o += (size_t)Sys::NiGP * sizeof(int);
-    o = (o + 15) & ~(size_t)15;
-    L.mt = o;
-    if (cpl == kMfmaCoupling) o += (size_t)NCp * (UPS / 16) * ldsPairs * 64 * 16;
-    L.total = o;
+    L.total = (o + 15) & ~(size_t)15;
     return L;
 }
 
@@ -450,7 +420,7 @@ __device__ __forceinline__ void mfma_contract44(const double* M, const double* c
 // i.e. the A operand of lane l for column blocks 2 cp and 2 cp + 1 side by
 // side (the same values, so the contraction's results are unchanged).
 template <int Unused = 0>
-__global__ void tile_pair_matrix(const double* M, double* Mt, int UPS, int NC)
+__global__ void tile_pair_matrix_old(const double* M, double* Mt, int UPS, int NC)
 {
     const size_t n = (size_t)NC * UPS * UPS;
     const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -464,18 +434,15 @@ __global__ void tile_pair_matrix(const double* M, double* Mt, int UPS, int NC)
     Mt[k] = M[(size_t)i * UPS * UPS + t * 16 + (l & 15) + (size_t)(4 * (2 * cp + j) + (l >> 4)) * UPS];
 }
 
-// One workgroup = SPB systems.  A system has UPS / PAIRS lanes; lane t belongs
-// to block system lsys = t / (UPS / PAIRS) and owns the PAIRS units
-// u0 + p * (UPS / PAIRS), u0 = t % (UPS / PAIRS), so the system-scope scalars
-// (time, step) are shared by the lane's pairs and global accesses to unit-scope
-// arrays stay coalesced.
+// One workgroup = SPB systems: lane t owns unit t % UPS of block system t / UPS,
+// so global accesses to unit-scope arrays are coalesced.
 //
 // KAHAN (P = float): FLOAT_KAHAN mode.  Unit states, stages, right-hand sides
 // and coupling terms in FP32; the state and the time are accumulated with Kahan
 // compensation (x += dt * sum b_j k_j and t += dt as compensated sums); the
 // step size, the error norm (from the FP32 stages in FP64 arithmetic), the
 // controller and the event step control in FP64.
-template <class Sys, class P, int ALG, int PAIRS, int CPL, bool REC = false, bool KAHAN = false>
+template <class Sys, class P, int ALG, bool REC = false, bool KAHAN = false>
 __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>& a)
 {
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NSP = Sys::NSP, NGP = Sys::NGP, NiGP = Sys::NiGP;
@@ -487,27 +454,23 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
     using math::fma;
 
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
-    const int ldsPairs = mfma_lds_matrix<Sys, PAIRS>() ? a.ldsPairs : 0;
-    const LdsLayout L = lds_layout<Sys, P, KAHAN>(CPL, a.SPB, a.UPS, a.sharedGlobals, a.sharedMatrix, a.cMatSize, ldsPairs);
+    const LdsLayout L = lds_layout<Sys, P, KAHAN>(a.SPB, a.UPS, a.sharedGlobals, a.sharedMatrix, a.cMatSize);
     S* sys = reinterpret_cast<S*>(mpgos_pb_lds);
     P* cptBuf = reinterpret_cast<P*>(mpgos_pb_lds + L.cpt);
-    P* coupBuf = reinterpret_cast<P*>(mpgos_pb_lds + L.coup);
     const int cptStride = a.SPB * a.UPS * NCp;
 
     const int UPS = a.UPS, NS = a.NS, SPB = a.SPB;
-    const int lanesPerSys = UPS / PAIRS;
     const int tid = threadIdx.x;
-    const int lsys = tid / lanesPerSys;
-    const int u0 = tid - lsys * lanesPerSys;
-    const bool lane = lsys < SPB;                              // lane owns PAIRS (system, unit) pairs
-    const bool leader = lane && u0 == 0;
+    const int lsys = tid / UPS;
+    const int u = tid - lsys * UPS;
+    const bool lane = lsys < SPB;                              // lane owns a (system, unit) pair
+    const bool leader = lane && u == 0;
     const size_t NU = (size_t)NS * UPS;
     const int gsys = blockIdx.x * SPB + lsys;
     const bool exists = lane && gsys < NS;
     const bool active = exists && gsys < a.nActive;
     S* const my = lane ? &sys[lsys] : &sys[0];
-    auto uid = [&](int p) { return u0 + p * lanesPerSys; };
-    auto gu = [&](int p) { return (size_t)gsys * UPS + uid(p); };   // unit-scope index
+    const size_t gu = (size_t)gsys * UPS + u;                  // unit-scope index
 
     // ---- global scope (LDS when SharedGlobalVariables / SharedCouplingMatrices)
     P* gPAR = a.gPAR;
@@ -525,23 +488,6 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         P* lm = reinterpret_cast<P*>(mpgos_pb_lds + L.m);
         for (int i = tid; i < NC * a.cMatSize; i += blockDim.x) lm[i] = a.cMat[i];
         M = lm;
-    }
-    if (CPL == kMfmaCoupling)   // B operand: rows of absent systems stay zero
-        for (int i = tid; i < NCp * kMfmaSystems * mfma_row(UPS); i += blockDim.x) cptBuf[i] = P(0);
-    const double* Ml = nullptr;
-    if (CPL == kMfmaCoupling && ldsPairs > 0) {
-        // the leading ldsPairs column-block pairs of every tile of the tiled
-        // matrix, for the whole Solve (16 bytes per lane and pair)
-        using Q = double2;
-        Q* lm = reinterpret_cast<Q*>(mpgos_pb_lds + L.mt);
-        const Q* src = reinterpret_cast<const Q*>(a.cTile);
-        const int lp = ldsPairs, pairs = UPS >> 3;
-        const int n = NCp * (UPS >> 4) * lp * 64;
-        for (int k = tid; k < n; k += blockDim.x) {
-            const int r = k >> 6;
-            lm[k] = src[((size_t)(r / lp) * pairs + r % lp) * 64 + (k & 63)];
-        }
-        Ml = reinterpret_cast<const double*>(lm);
     }
     int cIndex[NCp];
 #pragma unroll
@@ -568,26 +514,22 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
     }
 
     // ---- unit scope in registers
-    P X[PAIRS][UD], uPAR[PAIRS][Pos<NUP>::value], uACC[PAIRS][Pos<NUA>::value], EF[PAIRS][Pos<NE>::value];
-    P Xc[PAIRS][KAHAN ? UD : 1];                 // Kahan compensation of the unit states
-    P CPF[PAIRS][NCp];
-    int uACCi[PAIRS][Pos<NiUA>::value];
+    P X[UD], uPAR[Pos<NUP>::value], uACC[Pos<NUA>::value], EF[Pos<NE>::value];
+    P Xc[KAHAN ? UD : 1];                 // Kahan compensation of the unit states
+    P CPF[NCp];
+    int uACCi[Pos<NiUA>::value];
+    if (exists) {
 #pragma unroll
-    for (int p = 0; p < PAIRS; p++) {
-        if (exists) {
-            const size_t g = gu(p);
+        for (int c = 0; c < UD; c++) { X[c] = a.X[gu + c * NU]; if (KAHAN) Xc[c] = P(0); }
 #pragma unroll
-            for (int c = 0; c < UD; c++) { X[p][c] = a.X[g + c * NU]; if (KAHAN) Xc[p][c] = P(0); }
+        for (int c = 0; c < NUP; c++) uPAR[c] = a.uPAR[gu + c * NU];
 #pragma unroll
-            for (int c = 0; c < NUP; c++) uPAR[p][c] = a.uPAR[g + c * NU];
+        for (int c = 0; c < NUA; c++) uACC[c] = a.uACC[gu + c * NU];
 #pragma unroll
-            for (int c = 0; c < NUA; c++) uACC[p][c] = a.uACC[g + c * NU];
-#pragma unroll
-            for (int c = 0; c < NiUA; c++) uACCi[p][c] = a.uACCi[g + c * NU];
-        }
-#pragma unroll
-        for (int i = 0; i < NC; i++) CPF[p][i] = P(0);
+        for (int c = 0; c < NiUA; c++) uACCi[c] = a.uACCi[gu + c * NU];
     }
+#pragma unroll
+    for (int i = 0; i < NC; i++) CPF[i] = P(0);
     __syncthreads();
 
     // the step size as the user callbacks see it (FP32 copy in the Kahan mode)
@@ -595,18 +537,12 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         if constexpr (KAHAN) return my->dtP;
         else return my->dt;
     };
-#define MPGOS_PB_USER(p, TT, DTT) TT, DTT, my->TD, X[p], uPAR[p], my->sPAR, gPAR, gPARi, uACC[p], uACCi[p], my->sACC, my->sACCi
+#define MPGOS_PB_USER(TT, DTT) TT, DTT, my->TD, X, uPAR, my->sPAR, gPAR, gPARi, uACC, uACCi, my->sACC, my->sACCi
     // ---- initialisation (PB-SOL:2465-2528)
-    if (active) {
-#pragma unroll
-        for (int p = 0; p < PAIRS; p++) Sys::template Initialization<P>(gsys, uid(p), my->DOidx, MPGOS_PB_USER(p, my->t, udt()));
-    }
+    if (active) Sys::template Initialization<P>(gsys, u, my->DOidx, MPGOS_PB_USER(my->t, udt()));
     __syncthreads();
     if (NE > 0) {
-        if (active) {
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++) Sys::template EventFunction<P>(gsys, uid(p), EF[p], MPGOS_PB_USER(p, my->t, udt()));
-        }
+        if (active) Sys::template EventFunction<P>(gsys, u, EF, MPGOS_PB_USER(my->t, udt()));
         __syncthreads();
     }
     if (a.NDO > 0) {
@@ -614,9 +550,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         if (active && my->DOidx < a.NDO) {
             const int k = my->DOidx;
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) a.DOx[gu(p) + c * NU + (size_t)k * NU * UD] = X[p][c];
+            for (int c = 0; c < UD; c++) a.DOx[gu + c * NU + (size_t)k * NU * UD] = X[c];
             if (leader) a.DOt[gsys + (size_t)k * NS] = my->t;
         }
         __syncthreads();
@@ -630,54 +564,20 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
 
     if (REC && active) {        // checkpoint 0: the initial unit states
 #pragma unroll
-        for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-            for (int c = 0; c < UD; c++) a.recX[(size_t)c * NU + gu(p)] = X[p][c];
+        for (int c = 0; c < UD; c++) a.recX[(size_t)c * NU + gu] = X[c];
     }
 
     int buf = 0;
-    // right-hand sides of this lane's pairs at (Y[p], T), then the coupling terms
-    auto rhs = [&](P (*F)[UD], P (*Y)[UD], const P T) {
+    // right-hand sides of this lane's pair at (Y, T), then the coupling terms
+    auto rhs = [&](P* F, P* Y, const P T) {
         const bool run = lane && my->term == 0;
-        if constexpr (CPL == kMfmaCoupling) {
-            if (run) {
-#pragma unroll
-                for (int p = 0; p < PAIRS; p++) {
-                    P cp[NCp];
-                    Sys::template OdeFunction<P>(gsys, uid(p), F[p], Y[p], T, uPAR[p], my->sPAR, gPAR, gPARi, uACC[p], uACCi[p],
-                                                 my->sACC, my->sACCi, cp, CPF[p]);
-#pragma unroll
-                    for (int i = 0; i < NC; i++) cptBuf[mfma_index(i, lsys, uid(p), UPS)] = cp[i];
-                }
-            }
-            __syncthreads();
-            if (a.sharedMatrix) mfma_contract44<NC, false>(M, cptBuf, coupBuf, UPS, SPB);
-            else mfma_contract44<NC, true, 8, mfma_tiles_together<Sys, PAIRS>()>(M, cptBuf, coupBuf, UPS, SPB, (const double*)a.cTile, Ml,
-                                                                                 ldsPairs);
-            __syncthreads();
-            if (run) {
-#pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                    for (int i = 0; i < NC; i++)
-                        U::add(cIndex[i], my->strength[i] * CPF[p][i], coupBuf[mfma_index(i, lsys, uid(p), UPS)], F[p]);
-            }
-        } else {
-            P* cpt = cptBuf + (size_t)buf * cptStride;
-            if (run) {
-#pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-                    Sys::template OdeFunction<P>(gsys, uid(p), F[p], Y[p], T, uPAR[p], my->sPAR, gPAR, gPARi, uACC[p], uACCi[p],
-                                                 my->sACC, my->sACCi, cpt + (size_t)(lsys * UPS + uid(p)) * NCp, CPF[p]);
-            }
-            __syncthreads();
-            if (run) {
-#pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-                    U::couple(a, M, cIndex, my->strength, cpt + (size_t)lsys * UPS * NCp, uid(p), CPF[p], F[p]);
-            }
-            buf ^= 1;
-        }
+        P* cpt = cptBuf + (size_t)buf * cptStride;
+        if (run)
+            Sys::template OdeFunction<P>(gsys, u, F, Y, T, uPAR, my->sPAR, gPAR, gPARi, uACC, uACCi, my->sACC, my->sACCi,
+                                         cpt + (size_t)(lsys * UPS + u) * NCp, CPF);
+        __syncthreads();
+        if (run) U::couple(a, M, cIndex, my->strength, cpt + (size_t)lsys * UPS * NCp, u, CPF, F);
+        buf ^= 1;
     };
 
     for (;;) {
@@ -696,133 +596,92 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         }
         __syncthreads();
         const P h = (P)my->dt, t = my->t;
-        P next[PAIRS][UD], inc[PAIRS][KAHAN ? UD : 1];
-        CP err[PAIRS][UD];
+        P next[UD], inc[KAHAN ? UD : 1];
+        CP err[UD];
         bool isfin = true;
         if (ALG == MPGOS_RK4) {
             // PB-STP:2016-2224
-            P k[PAIRS][UD], Y[PAIRS][UD];
+            P k[UD], Y[UD];
             rhs(next, X, t);
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) Y[p][c] = fma(next[p][c] * P(0.5), h, X[p][c]);
+            for (int c = 0; c < UD; c++) Y[c] = fma(next[c] * P(0.5), h, X[c]);
             const P t2 = t + P(0.5) * h;
             rhs(k, Y, t2);
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) { next[p][c] = fma(P(2), k[p][c], next[p][c]); Y[p][c] = fma(k[p][c] * P(0.5), h, X[p][c]); }
+            for (int c = 0; c < UD; c++) { next[c] = fma(P(2), k[c], next[c]); Y[c] = fma(k[c] * P(0.5), h, X[c]); }
             rhs(k, Y, t2);
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) { next[p][c] = fma(P(2.0), k[p][c], next[p][c]); Y[p][c] = fma(k[p][c], h, X[p][c]); }
+            for (int c = 0; c < UD; c++) { next[c] = fma(P(2.0), k[c], next[c]); Y[c] = fma(k[c], h, X[c]); }
             rhs(k, Y, t + h);
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) {
-                    if (KAHAN) { inc[p][c] = h * (next[p][c] + k[p][c]) * P(1.0 / 6.0); next[p][c] = X[p][c] + inc[p][c]; }
-                    else next[p][c] = fma(h * (next[p][c] + k[p][c]), P(1.0 / 6.0), X[p][c]);
-                    if (!math::isfinite(next[p][c])) isfin = false;
-                }
+            for (int c = 0; c < UD; c++) {
+                if (KAHAN) { inc[c] = h * (next[c] + k[c]) * P(1.0 / 6.0); next[c] = X[c] + inc[c]; }
+                else next[c] = fma(h * (next[c] + k[c]), P(1.0 / 6.0), X[c]);
+                if (!math::isfinite(next[c])) isfin = false;
+            }
         } else {
             // PB-STP:2227-2544
-            P k1[PAIRS][UD], k2[PAIRS][UD], k3[PAIRS][UD], k4[PAIRS][UD], k5[PAIRS][UD], k6[PAIRS][UD], Y[PAIRS][UD];
+            P k1[UD], k2[UD], k3[UD], k4[UD], k5[UD], k6[UD], Y[UD];
             rhs(k1, X, t);
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) Y[p][c] = fma(k1[p][c] * P(1.0 / 5.0), h, X[p][c]);
+            for (int c = 0; c < UD; c++) Y[c] = fma(k1[c] * P(1.0 / 5.0), h, X[c]);
             rhs(k2, Y, fma(P(1.0 / 5.0), h, t));
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) Y[p][c] = fma(fma(k2[p][c], P(9.0 / 40.0), k1[p][c] * P(3.0 / 40.0)), h, X[p][c]);
+            for (int c = 0; c < UD; c++) Y[c] = fma(fma(k2[c], P(9.0 / 40.0), k1[c] * P(3.0 / 40.0)), h, X[c]);
             rhs(k3, Y, fma(P(3.0 / 10.0), h, t));
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    Y[p][c] = fma(fma(k3[p][c], P(6.0 / 5.0), fma(k2[p][c], P(-9.0 / 10.0), k1[p][c] * P(3.0 / 10.0))), h, X[p][c]);
+            for (int c = 0; c < UD; c++)
+                Y[c] = fma(fma(k3[c], P(6.0 / 5.0), fma(k2[c], P(-9.0 / 10.0), k1[c] * P(3.0 / 10.0))), h, X[c]);
             rhs(k4, Y, fma(P(3.0 / 5.0), h, t));
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    Y[p][c] = fma(fma(k4[p][c], P(35.0 / 27.0), fma(k3[p][c], P(-70.0 / 27.0), fma(k2[p][c], P(5.0 / 2.0),
-                                  k1[p][c] * P(-11.0 / 54.0)))), h, X[p][c]);
+            for (int c = 0; c < UD; c++)
+                Y[c] = fma(fma(k4[c], P(35.0 / 27.0), fma(k3[c], P(-70.0 / 27.0), fma(k2[c], P(5.0 / 2.0),
+                              k1[c] * P(-11.0 / 54.0)))), h, X[c]);
             rhs(k5, Y, t + h);
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    Y[p][c] = fma(fma(k5[p][c], P(253.0 / 4096.0), fma(k4[p][c], P(44275.0 / 110592.0), fma(k3[p][c], P(575.0 / 13824.0),
-                                  fma(k2[p][c], P(175.0 / 512.0), k1[p][c] * P(1631.0 / 55296.0))))), h, X[p][c]);
+            for (int c = 0; c < UD; c++)
+                Y[c] = fma(fma(k5[c], P(253.0 / 4096.0), fma(k4[c], P(44275.0 / 110592.0), fma(k3[c], P(575.0 / 13824.0),
+                              fma(k2[c], P(175.0 / 512.0), k1[c] * P(1631.0 / 55296.0))))), h, X[c]);
             rhs(k6, Y, fma(P(7.0 / 8.0), h, t));
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) {
-                    const P sum = fma(k6[p][c], P(512.0 / 1771.0), fma(k4[p][c], P(125.0 / 594.0), fma(k3[p][c], P(250.0 / 621.0),
-                                      k1[p][c] * P(37.0 / 378.0))));
-                    if (KAHAN) {
-                        inc[p][c] = sum * h;
-                        next[p][c] = X[p][c] + inc[p][c];
-                        // FP64 error norm over the FP32 stages
-                        double e = (double)k1[p][c] * (37.0 / 378.0 - 2825.0 / 27648.0);
-                        e = math::fma((double)k3[p][c], 250.0 / 621.0 - 18575.0 / 48384.0, e);
-                        e = math::fma((double)k4[p][c], 125.0 / 594.0 - 13525.0 / 55296.0, e);
-                        e = math::fma((double)k5[p][c], 0.0 - 277.0 / 14336.0, e);
-                        e = math::fma((double)k6[p][c], 512.0 / 1771.0 - 1.0 / 4.0, e);
-                        err[p][c] = math::fma((double)h, math::fabs(e), 1e-18);
-                    } else {
-                        next[p][c] = fma(sum, h, X[p][c]);
-                        P e = k1[p][c] * P(37.0 / 378.0 - 2825.0 / 27648.0);
-                        e = fma(k3[p][c], P(250.0 / 621.0 - 18575.0 / 48384.0), e);
-                        e = fma(k4[p][c], P(125.0 / 594.0 - 13525.0 / 55296.0), e);
-                        e = fma(k5[p][c], P(0.0 - 277.0 / 14336.0), e);
-                        e = fma(k6[p][c], P(512.0 / 1771.0 - 1.0 / 4.0), e);
-                        err[p][c] = (CP)fma(h, math::fabs(e), P(1e-18));
-                    }
-                    if (!math::isfinite(next[p][c]) || !math::isfinite(err[p][c])) isfin = false;
+            for (int c = 0; c < UD; c++) {
+                const P sum = fma(k6[c], P(512.0 / 1771.0), fma(k4[c], P(125.0 / 594.0), fma(k3[c], P(250.0 / 621.0),
+                                  k1[c] * P(37.0 / 378.0))));
+                if (KAHAN) {
+                    inc[c] = sum * h;
+                    next[c] = X[c] + inc[c];
+                    // FP64 error norm over the FP32 stages
+                    double e = (double)k1[c] * (37.0 / 378.0 - 2825.0 / 27648.0);
+                    e = math::fma((double)k3[c], 250.0 / 621.0 - 18575.0 / 48384.0, e);
+                    e = math::fma((double)k4[c], 125.0 / 594.0 - 13525.0 / 55296.0, e);
+                    e = math::fma((double)k5[c], 0.0 - 277.0 / 14336.0, e);
+                    e = math::fma((double)k6[c], 512.0 / 1771.0 - 1.0 / 4.0, e);
+                    err[c] = math::fma((double)h, math::fabs(e), 1e-18);
+                } else {
+                    next[c] = fma(sum, h, X[c]);
+                    P e = k1[c] * P(37.0 / 378.0 - 2825.0 / 27648.0);
+                    e = fma(k3[c], P(250.0 / 621.0 - 18575.0 / 48384.0), e);
+                    e = fma(k4[c], P(125.0 / 594.0 - 13525.0 / 55296.0), e);
+                    e = fma(k5[c], P(0.0 - 277.0 / 14336.0), e);
+                    e = fma(k6[c], P(512.0 / 1771.0 - 1.0 / 4.0), e);
+                    err[c] = (CP)fma(h, math::fabs(e), P(1e-18));
                 }
+                if (!math::isfinite(next[c]) || !math::isfinite(err[c])) isfin = false;
+            }
         }
         if (lane && my->term == 0 && !isfin) my->isfin = 0;
         // ---- controller (PB-CTL:424-542)
         if (ALG == MPGOS_RKCK45) {
             const bool part = lane && my->term == 0;
-            CP R = CP(1e30);                    // the reduction's start value, also for lanes not taking part
-            int upd = 1;
             if (part) {
+                CP R = CP(1e30);
+                int upd = 1;
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                    for (int c = 0; c < UD; c++) {
-                        const CP tol = dmax<CP>(a.rtol[c] * dmax<CP>(math::fabs((CP)next[p][c]), math::fabs((CP)X[p][c])), a.atol[c]);
-                        upd = upd & (err[p][c] < tol);
-                        R = dmin<CP>(R, tol / err[p][c]);
-                    }
-            }
-            // systems on aligned power-of-two groups of lanes (or whole waves):
-            // reduce in the group with lane shuffles, then one LDS atomic per
-            // group instead of one per lane (same-address atomics serialise).
-            // min and AND do not depend on the order, so the bits are those of
-            // the per-lane atomics.  Only where the lane's stage vectors leave
-            // registers for it (the two-tile dense-contraction kernels: ring of
-            // 256 two-component units 107.2 -> 106.5 ms; with three components
-            // the extra registers spilled, 125.8 -> 131.3 ms).
-            const int grp = !(CPL == kMfmaCoupling && mfma_tiles_together<Sys, PAIRS>() > 1) ? 0
-                            : lanesPerSys >= 64 ? (lanesPerSys % 64 == 0 ? 64 : 0)
-                                                : ((lanesPerSys & (lanesPerSys - 1)) == 0 ? lanesPerSys : 0);
-            if (grp > 1) {
-                for (int m = 1; m < grp; m <<= 1) {
-                    R = dmin<CP>(R, __shfl_xor(R, m));
-                    upd &= __shfl_xor(upd, m);
+                for (int c = 0; c < UD; c++) {
+                    const CP tol = dmax<CP>(a.rtol[c] * dmax<CP>(math::fabs((CP)next[c]), math::fabs((CP)X[c])), a.atol[c]);
+                    upd = upd & (err[c] < tol);
+                    R = dmin<CP>(R, tol / err[c]);
                 }
-            }
-            if (part && (grp == 0 || (tid & (grp - 1)) == 0)) {
                 atomicAnd(&my->update, upd);
                 atomicMin(&my->ratioBits, order_bits<CP>(R));
             }
@@ -855,26 +714,23 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         }
         __syncthreads();
         // ---- events (PB-SOL:2618-2655, PB-EVT:215-268)
-        P EFn[PAIRS][Pos<NE>::value];
+        P EFn[Pos<NE>::value];
         if (NE > 0) {
             const P tn = my->t + (P)my->dt;
             if (lane && my->term == 0) {
                 bool corr = false;
                 CP ev = my->dt;
+                // the event function of the candidate state, at the end of the step
+                Sys::template EventFunction<P>(gsys, u, EFn, tn, (P)my->newDt, my->TD, next, uPAR, my->sPAR, gPAR,
+                                               gPARi, uACC, uACCi, my->sACC, my->sACCi);
+                if (my->update == 1) {
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++) {
-                    // the event function of the candidate state, at the end of the step
-                    Sys::template EventFunction<P>(gsys, uid(p), EFn[p], tn, (P)my->newDt, my->TD, next[p], uPAR[p], my->sPAR, gPAR,
-                                                   gPARi, uACC[p], uACCi[p], my->sACC, my->sACCi);
-                    if (my->update == 1) {
-#pragma unroll
-                        for (int i = 0; i < NE; i++) {
-                            const P tol = a.etol[i];
-                            if ((EF[p][i] > tol && EFn[p][i] < -tol && a.edir[i] <= 0) ||
-                                (EF[p][i] < -tol && EFn[p][i] > tol && a.edir[i] >= 0)) {
-                                ev = dmin<CP>(ev, -(CP)EF[p][i] / ((CP)EFn[p][i] - (CP)EF[p][i]) * my->dt);
-                                corr = true;
-                            }
+                    for (int i = 0; i < NE; i++) {
+                        const P tol = a.etol[i];
+                        if ((EF[i] > tol && EFn[i] < -tol && a.edir[i] <= 0) ||
+                            (EF[i] < -tol && EFn[i] > tol && a.edir[i] >= 0)) {
+                            ev = dmin<CP>(ev, -(CP)EF[i] / ((CP)EFn[i] - (CP)EF[i]) * my->dt);
+                            corr = true;
                         }
                     }
                 }
@@ -895,18 +751,16 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         const int upd = my->update;
         if (lane && upd == 1) {
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) {
-                    if (KAHAN) {   // compensated x += inc
-                        const P y = inc[p][c] - Xc[p][c];
-                        const P sx = X[p][c] + y;
-                        Xc[p][c] = (sx - X[p][c]) - y;
-                        X[p][c] = sx;
-                    } else {
-                        X[p][c] = next[p][c];
-                    }
+            for (int c = 0; c < UD; c++) {
+                if (KAHAN) {   // compensated x += inc
+                    const P y = inc[c] - Xc[c];
+                    const P sx = X[c] + y;
+                    Xc[c] = (sx - X[c]) - y;
+                    X[c] = sx;
+                } else {
+                    X[c] = next[c];
                 }
+            }
             if (REC) {
                 const long long n = my->nacc;            // accepted steps before this one
                 if (leader) {
@@ -917,9 +771,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
                     const long long k = (n + 1) / a.recK;
                     if (k < a.recCkCap) {
 #pragma unroll
-                        for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                            for (int c = 0; c < UD; c++) a.recX[((size_t)k * UD + c) * NU + gu(p)] = X[p][c];
+                        for (int c = 0; c < UD; c++) a.recX[((size_t)k * UD + c) * NU + gu] = X[c];
                     } else if (leader) {
                         my->status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW;
                     }
@@ -939,34 +791,27 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         }
         __syncthreads();
         if (lane && upd == 1) {
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-                Sys::template ActionAfterSuccessfulTimeStep<P>(gsys, uid(p), my->udt, MPGOS_PB_USER(p, my->t, udt()));
+            Sys::template ActionAfterSuccessfulTimeStep<P>(gsys, u, my->udt, MPGOS_PB_USER(my->t, udt()));
         }
         __syncthreads();
         if (NE > 0) {
             if (lane && upd == 1) {
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                    for (int i = 0; i < NE; i++) {
-                        const P tol = a.etol[i];
-                        if ((EF[p][i] > tol && math::fabs(EFn[p][i]) < tol && a.edir[i] <= 0) ||
-                            (EF[p][i] < -tol && math::fabs(EFn[p][i]) < tol && a.edir[i] >= 0))
-                            Sys::template ActionAfterEventDetection<P>(gsys, uid(p), i, my->udt, MPGOS_PB_USER(p, my->t, udt()));
-                    }
+                for (int i = 0; i < NE; i++) {
+                    const P tol = a.etol[i];
+                    if ((EF[i] > tol && math::fabs(EFn[i]) < tol && a.edir[i] <= 0) ||
+                        (EF[i] < -tol && math::fabs(EFn[i]) < tol && a.edir[i] >= 0))
+                        Sys::template ActionAfterEventDetection<P>(gsys, u, i, my->udt, MPGOS_PB_USER(my->t, udt()));
+                }
+            }
+            __syncthreads();
+            if (lane && upd == 1) {
+                Sys::template EventFunction<P>(gsys, u, EFn, MPGOS_PB_USER(my->t, (P)my->newDt));
             }
             __syncthreads();
             if (lane && upd == 1) {
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++) Sys::template EventFunction<P>(gsys, uid(p), EFn[p], MPGOS_PB_USER(p, my->t, (P)my->newDt));
-            }
-            __syncthreads();
-            if (lane && upd == 1) {
-#pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                    for (int i = 0; i < NE; i++) EF[p][i] = EFn[p][i];
+                for (int i = 0; i < NE; i++) EF[i] = EFn[i];
             }
         }
         // ---- dense output (PB-DO:312-395)
@@ -984,9 +829,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
             if (lane && my->updDO == 1 && upd == 1) {
                 const int k = my->DOidx;
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                    for (int c = 0; c < UD; c++) a.DOx[gu(p) + c * NU + (size_t)k * NU * UD] = X[p][c];
+                for (int c = 0; c < UD; c++) a.DOx[gu + c * NU + (size_t)k * NU * UD] = X[c];
                 if (leader) a.DOt[gsys + (size_t)k * NS] = my->t;
             }
             __syncthreads();
@@ -1018,21 +861,17 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
     __syncthreads();
     // ---- finalisation and write-back (PB-SOL:2814-2887)
     if (active) {
-#pragma unroll
-        for (int p = 0; p < PAIRS; p++) Sys::template Finalization<P>(gsys, uid(p), my->DOidx, MPGOS_PB_USER(p, my->t, udt()));
+        Sys::template Finalization<P>(gsys, u, my->DOidx, MPGOS_PB_USER(my->t, udt()));
     }
     __syncthreads();
     if (exists) {
+        const size_t g = gu;
 #pragma unroll
-        for (int p = 0; p < PAIRS; p++) {
-            const size_t g = gu(p);
+        for (int c = 0; c < UD; c++) a.X[g + c * NU] = X[c];
 #pragma unroll
-            for (int c = 0; c < UD; c++) a.X[g + c * NU] = X[p][c];
+        for (int c = 0; c < NUA; c++) a.uACC[g + c * NU] = uACC[c];
 #pragma unroll
-            for (int c = 0; c < NUA; c++) a.uACC[g + c * NU] = uACC[p][c];
-#pragma unroll
-            for (int c = 0; c < NiUA; c++) a.uACCi[g + c * NU] = uACCi[p][c];
-        }
+        for (int c = 0; c < NiUA; c++) a.uACCi[g + c * NU] = uACCi[c];
     }
     if (leader && active) {
         S& s = sys[lsys];
@@ -1053,29 +892,15 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
 template <class Sys, class P, int ALG, int MAXT, bool KAHAN = false>
 __global__ void __launch_bounds__(MAXT) pb_kernel(Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP> a)
 {
-    pb_body<Sys, P, ALG, 1, kLaneCoupling, false, KAHAN>(a);
+    pb_body<Sys, P, ALG, false, KAHAN>(a);
 }
 
 // Record pass of the discrete adjoint (FP64): the forward integration plus
-// checkpoints (lane-per-pair or dense-contraction form).
+// checkpoints.
 template <class Sys, int ALG, int MAXT>
 __global__ void __launch_bounds__(MAXT) pb_record_kernel(Args<Sys, double> a)
 {
-    pb_body<Sys, double, ALG, 1, kLaneCoupling, true>(a);
-}
-template <class Sys, int ALG>
-__global__ void __launch_bounds__(512) pb_record_mfma_kernel(Args<Sys, double> a)
-{
-    pb_body<Sys, double, ALG, 4, kMfmaCoupling, true>(a);
-}
-
-// Dense-contraction form: SPB = 8, PAIRS units per lane, 8 * UPS / PAIRS
-// threads (UPS a multiple of 32 up to 256, so every wave is full).
-template <class Sys, class P, int ALG, int PAIRS>
-__global__ void __launch_bounds__(8 * 256 / PAIRS) pb_mfma_kernel(Args<Sys, P> a)
-{
-    if constexpr (std::is_same<P, double>::value)
-        pb_body<Sys, P, ALG, PAIRS, kMfmaCoupling>(a);
+    pb_body<Sys, double, ALG, true>(a);
 }
 
 } // namespace pb

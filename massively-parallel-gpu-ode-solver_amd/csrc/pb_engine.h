@@ -21,6 +21,7 @@
 
 #include "mpgos.h"
 #include "pb_adjoint.h"
+#include "pb_dense.h"
 #include "pb_device.h"
 #include "pt_engine.h"   // Buffer, set_error, MPGOS_HIP_TRY
 
@@ -68,11 +69,12 @@ public:
     hipStream_t strm = nullptr;
     hipEvent_t syncEvent = nullptr, evStart = nullptr, evStop = nullptr;
     size_t ldsMax = 0;
+    int cus = 1;              // compute units of the device
 
     int nActive = 0, sharedGlobals = 1, sharedMatrix = 0, doFreq = 1;
     int couplingKernel = 0;   // 0 automatic, 1 lane-per-pair, 2 dense contraction (MFMA)
     int lastForm = -1;        // coupling form of the last launch
-    int mfmaPairs = 4;        // units per lane of the dense-contraction form (2 or 4)
+    int mfmaPairs = 4;        // accepted (2 or 4); the dense-contraction form chooses its own split
     double dt0 = 1e-2, dtmax = 1.0e6, dtmin = 1.0e-12, grow = 5.0, shrink = 0.1, doMinDt = 0.0;
     std::vector<double> rtol, atol, etol;
     std::vector<int> edir;
@@ -88,8 +90,8 @@ public:
     double* recX = nullptr; double* recT = nullptr; double* recH = nullptr; double* seg = nullptr; double* cMatT = nullptr;
     double* stg = nullptr; double* gSp = nullptr;
     double* cTile = nullptr;                // pair-tiled copies (tile_pair_matrix) of the dense coupling matrices
-    double* cTileT = nullptr;               // and of their transposes (adjoint sweep)
-    size_t cTileN = 0, cTileTN = 0;
+    double* cTileR = nullptr; double* cTileT = nullptr;   // and for the adjoint: of them, of their transposes
+    size_t cTileRN = 0, cTileTN = 0;
     size_t recXn = 0, recTn = 0, recHn = 0, segn = 0, cMatTn = 0, stgn = 0, gSpn = 0;
     int adjK = 0, adjCap = 0, adjStepCap = 0;
 
@@ -97,7 +99,7 @@ public:
     {
         if (strm) (void)hipStreamSynchronize(strm);
         lamB.release(); gUB.release(); gSB.release();
-        for (double* q : {recX, recT, recH, seg, cMatT, stg, gSp, cTile, cTileT})
+        for (double* q : {recX, recT, recH, seg, cMatT, stg, gSp, cTile, cTileR, cTileT})
             if (q) (void)hipFree(q);
         for (auto* b : {&X, &uPAR, &uACC, &TD, &T, &sPAR, &sACC, &strength, &DOt, &DOx, &gPAR, &cMat}) b->release();
         for (auto* b : {&uACCi, &sACCi, &DOidx, &gPARi, &cIndex, &status}) b->release();
@@ -130,6 +132,7 @@ public:
         hipDeviceProp_t prop;
         MPGOS_HIP_TRY(hipGetDeviceProperties(&prop, device));
         ldsMax = prop.sharedMemPerBlock;
+        cus = std::max(1, prop.multiProcessorCount);
         const size_t NU = (size_t)NS * UPS;
         int rc;
         if ((rc = X.alloc(UD * NU)) || (rc = uPAR.alloc(NUP * NU)) || (rc = uACC.alloc(NUA * NU)) ||
@@ -140,6 +143,11 @@ public:
             (rc = cIndex.alloc(NC)) || (rc = cMat.alloc((size_t)NC * cMatSize)) || (rc = status.alloc(NS)) ||
             (rc = nacc.alloc(NS)) || (rc = nrej.alloc(NS)))
             return rc;
+        if (dense_possible() && hipMalloc((void**)&cTile, (size_t)NC * dense_matrix_size(UPS) * sizeof(double)) != hipSuccess) {
+            cTile = nullptr;
+            set_error("per-block: allocation of the tiled coupling matrix failed");
+            return MPGOS_E_MEMORY;
+        }
         if (kAdjoint && ((rc = lamB.alloc(UD * NU)) || (rc = gUB.alloc(NUP * NU)) || (rc = gSB.alloc((size_t)NSP * NS))))
             return rc;
         cMatOriginal.assign((size_t)NC * UPS * UPS, P(0));
@@ -429,39 +437,92 @@ public:
         return a;
     }
 
-    // the dense-contraction (MFMA) form applies to full FP64 matrices with UPS a
-    // multiple of 32 in [32, 256] (2 * UPS threads fill whole waves);
-    // CouplingKernel 0 picks it when it applies
-    bool mfma_applies() const
+    // Full FP64 coupling matrices of up to 256 units can run in the
+    // dense-contraction form (pb_dense.h).
+    bool dense_possible() const
     {
-        return std::is_same<P, double>::value && CCI == 0 && CBW == 0 && UPS % 32 == 0 && UPS >= 32 && UPS <= 256;
+        return std::is_same<P, double>::value && NC > 0 && CCI == 0 && CBW == 0 && UPS <= kDenseMaxUnits;
     }
+    // what CouplingKernel 2 accepts
+    bool dense_request_valid() const
+    {
+        return std::is_same<P, double>::value && CCI == 0 && CBW == 0 && UPS % 32 == 0 && UPS <= 256;
+    }
+    // Workgroups of the dense form with 4 systems that a CU holds at once (its
+    // registers allow 16 wavefronts with one tile each, 8 with two).
+    int dense_per_cu() const
+    {
+        const int tiles = dense_tiles(UPS);
+        return tiles > 8 ? 1 : 16 / tiles;
+    }
+    // 4 systems per workgroup while the card holds all workgroups at once, else
+    // 8: the second four share the matrix operand, but a wavefront's step takes
+    // 1.3 to 1.7 times as long.  Measured, ms with 4 | 8 systems (ring of Duffing
+    // oscillators, one period): 1024 x 256 units 8.7 | 11.5, 4096 x 256 33.3 |
+    // 23.9, 1000 x 100 2.3 | 3.8, 4096 x 100 7.2 | 6.2, 4096 x 128 10.1 | 8.6,
+    // 8192 x 12 1.1 | 1.6, 65536 x 16 5.7 | 5.3.
+    bool dense_four() const { return (long)(NS + 3) / 4 <= (long)dense_per_cu() * cus; }
+    // Automatic choice.  Up to 8 units the dense form computes at least as many
+    // padded rows as real ones; it is the faster one only while the card is not
+    // full (2048 x 4 units: 0.9 against 1.4 ms; 65536 x 4: 4.9 against 2.4 ms;
+    // 65536 x 8: 5.1 against 5.0 ms; 65536 x 12: 5.2 against 9.7 ms).
     int coupling_form() const
     {
         if (couplingKernel == 1) return kLaneCoupling;
-        if (couplingKernel == 2) return kMfmaCoupling;
-        return mfma_applies() ? kMfmaCoupling : kLaneCoupling;
+        if (couplingKernel == 2 && NC > 0) return kDenseCoupling;
+        return dense_possible() && (UPS > 8 || dense_four()) ? kDenseCoupling : kLaneCoupling;
     }
 
-    size_t lds_bytes(int cpl, int spb, int sm, int ldsPairs = 0) const
+    size_t lds_bytes(int spb, int sm) const
     {
-        return lds_layout<Sys, P, KAHAN>(cpl, spb, UPS, sharedGlobals, sm, cMatSize, ldsPairs).total;
+        return lds_layout<Sys, P, KAHAN>(spb, UPS, sharedGlobals, sm, cMatSize).total;
     }
 
-    // Dense-contraction form with the tiled matrix: the leading column-block
-    // pairs of every tile that fit into the LDS the workgroup leaves free (a
-    // multiple of 2 pairs, one group of the two-tile contraction loop; at
-    // most all).  At U = 256: 6 of 32 pairs, 96 KiB.  (Letting the results
-    // overwrite the coupling terms after a barrier made room for 8 pairs but
-    // ran 1.4 % slower.)
-    int lds_pairs(int spb) const
+    // Dense-contraction form.  A workgroup's LDS beyond its coupling terms takes
+    // the leading column-block pairs of every tile, as many as fit next to the
+    // other workgroups that its CU is to hold (4096 x 100 units, 8 systems: 6.2 ms
+    // with 4 of 14 pairs and three workgroups per CU, 7.8 ms with all pairs and
+    // one; 1000 x 100, 4 systems: 4.6 ms with all, 5.4 ms with none).
+    template <int NSL, int TT, bool REC, bool QUIET>
+    int launch_dense(Args<Sys, double>& a)
     {
-        const size_t perPair = (size_t)std::max(NC, 1) * (UPS / 16) * 64 * 16;
-        const size_t base = lds_bytes(kMfmaCoupling, spb, 0, 1) - perPair;
-        if (base >= ldsMax) return 0;
-        int lp = (int)std::min<size_t>((ldsMax - base) / perPair, (size_t)(UPS / 8));
-        lp -= lp % 2;
-        return lp;
+        constexpr int spb = 4 * NSL;
+        auto bytes = [&](int pairs) { return dense_layout<DenseScope<Sys>, NC, NGP, NiGP>(spb, UPS, sharedGlobals, pairs).total; };
+        const int grid = (NS + spb - 1) / spb;
+        const int perCu = std::max(1, std::min((grid + cus - 1) / cus, NSL == 1 ? dense_per_cu() : std::max(1, dense_per_cu() * 3 / 4)));
+        const size_t perPair = (size_t)NC * dense_tiles(UPS) * 64 * 16, room = ldsMax / perCu;
+        int lp = room > bytes(0) ? (int)std::min<size_t>((room - bytes(0)) / perPair, (size_t)dense_pairs(UPS)) : 0;
+        lp -= lp % kDenseGroup;
+        a.SPB = spb;
+        a.ldsPairs = lp;
+        a.cTile = cTile;
+        const int threads = 64 * ((dense_tiles(UPS) + TT - 1) / TT);
+        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_dense_kernel<Sys, MPGOS_RK4, NSL, TT, REC, QUIET>), dim3(grid), dim3(threads), bytes(lp), strm, a);
+        else hipLaunchKernelGGL((pb_dense_kernel<Sys, MPGOS_RKCK45, NSL, TT, REC, QUIET>), dim3(grid), dim3(threads), bytes(lp), strm, a);
+        return MPGOS_OK;
+    }
+    template <int NSL, int TT, bool REC>
+    int launch_dense(Args<Sys, double>& a)
+    {
+        constexpr bool quiet = NE == 0 && systems::no_step_action<Sys, systems::PBNoCallbacks>();
+        if constexpr (quiet) {
+            if (NDO == 0) return launch_dense<NSL, TT, REC, true>(a);
+        }
+        return launch_dense<NSL, TT, REC, false>(a);
+    }
+    template <bool REC>
+    int launch_dense(Args<Sys, double>& a)
+    {
+        // the matrices in column-block pairs per lane, refreshed every Solve
+        // (a kernel on the solver's stream, so graph capture records it)
+        if (int rc = tile_pairs((const double*)cMat.d, cTile)) return rc;
+        auto fits = [&](int spb) { return dense_layout<DenseScope<Sys>, NC, NGP, NiGP>(spb, UPS, sharedGlobals, 0).total <= ldsMax; };
+        if (!fits(4)) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
+        const bool four = dense_four() || !fits(8);
+        // two tiles per wavefront above 8 tiles: they share the coupling terms
+        // (4096 x 256: 23.9 against 25.9 ms), below one (4096 x 128: 8.6 against 9.6 ms)
+        if (dense_tiles(UPS) > 8) return four ? launch_dense<1, 2, REC>(a) : launch_dense<2, 2, REC>(a);
+        return four ? launch_dense<1, 1, REC>(a) : launch_dense<2, 1, REC>(a);
     }
 
     // PB-IF:1949-1965
@@ -469,74 +530,56 @@ public:
     {
         MPGOS_HIP_TRY(hipSetDevice(device));
         Args<Sys, P, CP> a = make_args();
-        const int cpl = coupling_form();
-        if (cpl == kMfmaCoupling && !mfma_applies()) {
-            set_error("per-block: the dense-contraction coupling kernel needs a full FP64 coupling matrix and UPS a multiple of 32 up to 256");
-            return MPGOS_E_ARG;
+        if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
+        lastForm = coupling_form();
+        if constexpr (!KAHAN && std::is_same<P, double>::value && NC > 0) {
+            if (lastForm == kDenseCoupling) {
+                MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
+                if (int rc = launch_dense<false>(a)) return rc;
+                MPGOS_HIP_TRY(hipGetLastError());
+                MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
+                return MPGOS_OK;
+            }
         }
-        const int spb = cpl == kMfmaCoupling ? kMfmaSystems : SPB;
-        a.SPB = spb;
         // the coupling matrix goes to LDS only when asked for and when it fits
-        a.sharedMatrix = sharedMatrix && lds_bytes(cpl, spb, 1) <= ldsMax ? 1 : 0;
-        const bool tiled = !KAHAN && cpl == kMfmaCoupling && !a.sharedMatrix && std::is_same<P, double>::value;
-        if (tiled && (mfmaPairs == 2 ? mfma_lds_matrix<Sys, 2>() : mfma_lds_matrix<Sys, 4>())) a.ldsPairs = lds_pairs(spb);
-        const size_t lds = lds_bytes(cpl, spb, a.sharedMatrix, a.ldsPairs);
+        a.sharedMatrix = sharedMatrix && lds_bytes(SPB, 1) <= ldsMax ? 1 : 0;
+        const size_t lds = lds_bytes(SPB, a.sharedMatrix);
         if (lds > ldsMax) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
-        const int threads = cpl == kMfmaCoupling ? kMfmaSystems * UPS / mfmaPairs : ((SPB * UPS + 63) / 64) * 64;
-        const int grid = NS / spb + (NS % spb == 0 ? 0 : 1);
-        lastForm = cpl;
+        const int threads = ((SPB * UPS + 63) / 64) * 64;
+        const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
         MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-        if constexpr (KAHAN) {   // lane-per-pair form only
-            if (threads <= 256) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, 256, true>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, 256, true>), dim3(grid), dim3(threads), lds, strm, a);
-            } else {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, kMaxBlock, true>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, kMaxBlock, true>), dim3(grid), dim3(threads), lds, strm, a);
-            }
+        if (threads <= 256) {
+            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+            else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
         } else {
-            if (tiled) {
-                // the matrices in column-block pairs per lane, refreshed every Solve
-                // (a kernel on the solver's stream, so graph capture records it)
-                if (int rc = tile_pairs((const double*)cMat.d, cTile, cTileN)) return rc;
-                a.cTile = (const P*)cTile;
-            }
-            if (cpl == kMfmaCoupling && mfmaPairs == 2) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_mfma_kernel<Sys, P, MPGOS_RK4, 2>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_mfma_kernel<Sys, P, MPGOS_RKCK45, 2>), dim3(grid), dim3(threads), lds, strm, a);
-            } else if (cpl == kMfmaCoupling) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_mfma_kernel<Sys, P, MPGOS_RK4, 4>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_mfma_kernel<Sys, P, MPGOS_RKCK45, 4>), dim3(grid), dim3(threads), lds, strm, a);
-            } else if (threads <= 256) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a);
-            } else {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
-            }
+            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+            else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
         }
         MPGOS_HIP_TRY(hipGetLastError());
         MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
         return MPGOS_OK;
     }
 
-    // The pair-tiled copy of NC full UPS x UPS matrices at src (column-major),
-    // written by a kernel on the solver's stream (allocated on first use; the
-    // size never changes for a solver, so no buffer in use is freed).
-    int tile_pairs(const double* src, double*& dst, size_t& have)
+    static int refuse_dense()
+    {
+        set_error("per-block: the dense-contraction coupling kernel needs a full FP64 coupling matrix and UPS a multiple of 32 up to 256");
+        return MPGOS_E_ARG;
+    }
+
+    // The pair-tiled copy of the NC full matrices at src (column-major),
+    // written by a kernel on the solver's stream.
+    int tile_pairs(const double* src, double* dst)
+    {
+        const size_t n = (size_t)NC * dense_matrix_size(UPS);
+        hipLaunchKernelGGL(tile_pair_matrix<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, strm, src, dst, UPS, NC);
+        MPGOS_HIP_TRY(hipGetLastError());
+        return MPGOS_OK;
+    }
+    int tile_pairs_reverse(const double* src, double*& dst, size_t& have)
     {
         const size_t n = (size_t)NC * UPS * UPS;
-        if (n > have) {
-            if (dst) { MPGOS_HIP_TRY(hipStreamSynchronize(strm)); (void)hipFree(dst); }
-            dst = nullptr; have = 0;
-            if (hipMalloc((void**)&dst, n * sizeof(double)) != hipSuccess) {
-                dst = nullptr;
-                set_error("per-block: allocation of the tiled coupling matrix failed");
-                return MPGOS_E_MEMORY;
-            }
-            have = n;
-        }
-        hipLaunchKernelGGL(tile_pair_matrix<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, strm, src, dst, UPS, NC);
+        if (int rc = grow_device(dst, have, n, "tiled coupling matrix")) return rc;
+        hipLaunchKernelGGL(tile_pair_matrix_old<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, strm, src, dst, UPS, NC);
         MPGOS_HIP_TRY(hipGetLastError());
         return MPGOS_OK;
     }
@@ -574,24 +617,23 @@ public:
             adjK = K; adjCap = ckcap; adjStepCap = stepcap;
             Args<Sys, double> a = make_args();
             a.recX = recX; a.recT = recT; a.recH = recH; a.recK = K; a.recCkCap = ckcap; a.recStepCap = stepcap;
-            const int cpl = coupling_form();
-            const int spb = cpl == kMfmaCoupling ? kMfmaSystems : SPB;
-            a.SPB = spb;
-            a.sharedMatrix = sharedMatrix && lds_bytes(cpl, spb, 1) <= ldsMax ? 1 : 0;
-            if (cpl == kMfmaCoupling && !a.sharedMatrix && mfma_lds_matrix<Sys, 4>()) a.ldsPairs = lds_pairs(spb);
-            const size_t lds = lds_bytes(cpl, spb, a.sharedMatrix, a.ldsPairs);
-            if (lds > ldsMax) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
-            const int threads = cpl == kMfmaCoupling ? kMfmaSystems * UPS / 4 : ((SPB * UPS + 63) / 64) * 64;
-            const int grid = NS / spb + (NS % spb == 0 ? 0 : 1);
-            MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-            if (cpl == kMfmaCoupling && !a.sharedMatrix) {
-                if ((rc = tile_pairs((const double*)cMat.d, cTile, cTileN))) return rc;
-                a.cTile = cTile;
+            if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
+            if constexpr (NC > 0) {
+                if (coupling_form() == kDenseCoupling) {
+                    MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
+                    if ((rc = launch_dense<true>(a))) return rc;
+                    MPGOS_HIP_TRY(hipGetLastError());
+                    MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
+                    return MPGOS_OK;
+                }
             }
-            if (cpl == kMfmaCoupling) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_mfma_kernel<Sys, MPGOS_RK4>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_record_mfma_kernel<Sys, MPGOS_RKCK45>), dim3(grid), dim3(threads), lds, strm, a);
-            } else if (threads <= 256) {
+            a.sharedMatrix = sharedMatrix && lds_bytes(SPB, 1) <= ldsMax ? 1 : 0;
+            const size_t lds = lds_bytes(SPB, a.sharedMatrix);
+            if (lds > ldsMax) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
+            const int threads = ((SPB * UPS + 63) / 64) * 64;
+            const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
+            MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
+            if (threads <= 256) {
                 if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a);
                 else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a);
             } else {
@@ -617,14 +659,11 @@ public:
             MPGOS_HIP_TRY(hipSetDevice(device));
             const size_t NU = (size_t)NS * UPS;
             MPGOS_HIP_TRY(hipStreamSynchronize(strm));
-            const int cpl = coupling_form();
-            if (cpl == kMfmaCoupling && !mfma_applies()) {
-                set_error("per-block: the dense-contraction coupling kernel needs a full FP64 coupling matrix and UPS a multiple of 32 up to 256");
-                return MPGOS_E_ARG;
-            }
+            if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
+            const int cpl = couplingKernel != 1 && dense_request_valid() ? kDenseCoupling : kLaneCoupling;
             const int ST = algorithm == MPGOS_RK4 ? 4 : 6;
             int rc;
-            if (cpl == kMfmaCoupling) {
+            if (cpl == kDenseCoupling) {
                 if ((rc = grow_device(stg, stgn, (size_t)adjK * ST * (UD + NC) * NU, "stage buffer"))) return rc;
             } else if ((rc = grow_device(seg, segn, (size_t)adjK * UD * NU, "segment buffer"))) {
                 return rc;
@@ -645,7 +684,7 @@ public:
             A.seg = seg; A.stg = stg; A.gSp = nullptr; A.lam = lamB.d; A.gU = gUB.d; A.gS = gSB.d; A.cMatT = cMatT;
             A.cTileT = nullptr;
             lastForm = cpl;
-            if (cpl == kMfmaCoupling) {
+            if (cpl == kDenseCoupling) {
                 // one replay and one sweep launch per round; rounds = the largest
                 // segment count of a system whose record did not overflow
                 a.SPB = kMfmaSystems;
@@ -667,8 +706,8 @@ public:
                 const int grid = NS / kMfmaSystems + (NS % kMfmaSystems == 0 ? 0 : 1);
                 const int fgrid = (int)((NU + 255) / 256);
                 MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-                if ((rc = tile_pairs((const double*)cMat.d, cTile, cTileN)) || (rc = tile_pairs(cMatT, cTileT, cTileTN))) return rc;
-                a.cTile = cTile;
+                if ((rc = tile_pairs_reverse((const double*)cMat.d, cTileR, cTileRN)) || (rc = tile_pairs_reverse(cMatT, cTileT, cTileTN))) return rc;
+                a.cTile = cTileR;
                 A.cTileT = cTileT;
                 for (int r = 0; r < rounds; r++) {
                     if (algorithm == MPGOS_RK4) {

@@ -14,15 +14,6 @@
 namespace mpgos {
 namespace systems {
 
-struct PBNoCallbacks {
-#define MPGOS_PB_ARGS P*, P*, P*, int*, P*, int*, P*, int*
-    template <class P> MPGOS_HD static void EventFunction(int, int, P*, P, P, P*, P*, MPGOS_PB_ARGS) {}
-    template <class P> MPGOS_HD static void ActionAfterEventDetection(int, int, int, int&, P&, P&, P*, P*, MPGOS_PB_ARGS) {}
-    template <class P> MPGOS_HD static void ActionAfterSuccessfulTimeStep(int, int, int&, P&, P&, P*, P*, MPGOS_PB_ARGS) {}
-    template <class P> MPGOS_HD static void Finalization(int, int, int&, P&, P&, P*, P*, MPGOS_PB_ARGS) {}
-#undef MPGOS_PB_ARGS
-};
-
 // Ring of forced hardening Duffing units with a dense coupling matrix on the
 // velocity equation:  x_u'' + k_u x_u' + x_u + x_u^3 = B cos t + sum_v C_uv x_v.
 // uPAR = (k), sPAR = (B); coupling 0 takes CPT = x (coupling terms) with
@@ -33,17 +24,35 @@ struct RingDuffing : PBNoCallbacks {
     static constexpr const char* name = "ring_duffing";
     static constexpr int UD = 2, NC = 1, NUP = 1, NSP = 1, NGP = 0, NiGP = 0, NUA = 0, NiUA = 0, NSA = 0, NiSA = 0, NE = 0;
 
+    static constexpr int NTT = 1;
+    static constexpr bool TT_TIME_ONLY = true;
+
     template <class P>
-    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* uPAR, P* sPAR, P*, int*, P*, int*, P*, int*, P* CPT,
-                                     P* CPF)
+    MPGOS_HD static void TimeTerms(P T, P*, P* tt)
     {
         using mpgos::math::cos;
+        tt[0] = cos(T);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunctionTT(int, int, P* F, P* X, P, const P* tt, P* uPAR, P* sPAR, P*, int*, P*, int*, P*, int*,
+                                       P* CPT, P* CPF)
+    {
         using mpgos::math::fma;
         const P x = X[0], v = X[1];
         F[0] = v;
-        F[1] = fma(-uPAR[0], v, sPAR[0] * cos(T)) - fma(x * x, x, x);
+        F[1] = fma(-uPAR[0], v, sPAR[0] * tt[0]) - fma(x * x, x, x);
         CPT[0] = x;
         CPF[0] = P(1.0);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunction(int sid, int uid, P* F, P* X, P T, P* uPAR, P* sPAR, P* gPAR, int* gPARi, P* uACC, int* uACCi,
+                                     P* sACC, int* sACCi, P* CPT, P* CPF)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, sPAR, tt);
+        OdeFunctionTT<P>(sid, uid, F, X, T, tt, uPAR, sPAR, gPAR, gPARi, uACC, uACCi, sACC, sACCi, CPT, CPF);
     }
 
     template <class P>
@@ -61,31 +70,57 @@ struct RingDuffingQ : PBNoCallbacks {
     static constexpr const char* name = "ring_duffing_q";
     static constexpr int UD = 3, NC = 1, NUP = 1, NSP = 1, NGP = 0, NiGP = 0, NUA = 0, NiUA = 0, NSA = 0, NiSA = 0, NE = 0;
 
+    static constexpr int NTT = 1;
+    static constexpr bool TT_TIME_ONLY = true;
+
     template <class P>
-    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* uPAR, P* sPAR, P*, int*, P*, int*, P*, int*, P* CPT,
-                                     P* CPF)
+    MPGOS_HD static void TimeTerms(P T, P*, P* tt)
     {
         using mpgos::math::cos;
+        tt[0] = cos(T);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeFunctionTT(int, int, P* F, P* X, P, const P* tt, P* uPAR, P* sPAR, P*, int*, P*, int*, P*, int*,
+                                       P* CPT, P* CPF)
+    {
         using mpgos::math::fma;
         const P x = X[0], v = X[1];
         F[0] = v;
-        F[1] = fma(-uPAR[0], v, sPAR[0] * cos(T)) - fma(x * x, x, x);
+        F[1] = fma(-uPAR[0], v, sPAR[0] * tt[0]) - fma(x * x, x, x);
         F[2] = x * x;
         CPT[0] = x;
         CPF[0] = P(1.0);
     }
 
     template <class P>
-    MPGOS_HD static void OdeVJP(int, int, const P* kbF, const P* kbCPT, const P*, P* X, P T, P* uPAR, P*, P*, int*, P*, int*,
-                                P*, int*, P* gX, P* gU, P* gS)
+    MPGOS_HD static void OdeFunction(int sid, int uid, P* F, P* X, P T, P* uPAR, P* sPAR, P* gPAR, int* gPARi, P* uACC, int* uACCi,
+                                     P* sACC, int* sACCi, P* CPT, P* CPF)
     {
-        using mpgos::math::cos;
+        P tt[NTT];
+        TimeTerms<P>(T, sPAR, tt);
+        OdeFunctionTT<P>(sid, uid, F, X, T, tt, uPAR, sPAR, gPAR, gPARi, uACC, uACCi, sACC, sACCi, CPT, CPF);
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeVJPTT(int, int, const P* kbF, const P* kbCPT, const P*, P* X, P, const P* tt, P* uPAR, P*, P*, int*, P*,
+                                  int*, P*, int*, P* gX, P* gU, P* gS)
+    {
         const P x = X[0], v = X[1];
         gX[0] = -(P(1) + P(3) * x * x) * kbF[1] + P(2) * x * kbF[2] + kbCPT[0];
         gX[1] = kbF[0] - uPAR[0] * kbF[1];
         gX[2] = P(0);
         gU[0] = -v * kbF[1];
-        gS[0] = cos(T) * kbF[1];
+        gS[0] = tt[0] * kbF[1];
+    }
+
+    template <class P>
+    MPGOS_HD static void OdeVJP(int sid, int uid, const P* kbF, const P* kbCPT, const P* kbCPF, P* X, P T, P* uPAR, P* sPAR, P* gPAR,
+                                int* gPARi, P* uACC, int* uACCi, P* sACC, int* sACCi, P* gX, P* gU, P* gS)
+    {
+        P tt[NTT];
+        TimeTerms<P>(T, sPAR, tt);
+        OdeVJPTT<P>(sid, uid, kbF, kbCPT, kbCPF, X, T, tt, uPAR, sPAR, gPAR, gPARi, uACC, uACCi, sACC, sACCi, gX, gU, gS);
     }
 
     template <class P>

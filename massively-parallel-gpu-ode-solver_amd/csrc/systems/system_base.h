@@ -22,12 +22,16 @@
 //   OdeVJPTT(tid, NT, lam, X, T, tt, ...)     its vector-Jacobian product (with
 //                                             TT_TIME_ONLY and HAS_VJP only)
 // with OdeFunction and OdeVJP the same functions over terms evaluated at T.
+// Per-block systems take (sid, uid) for (tid, NT) and the system parameters for
+// cPAR, with the argument lists of their OdeFunction and OdeVJP.
 // Such a system leaves T, the time domain and the parameters in its terms
 // alone after Initialization.
 // Every callback is MPGOS_HD so the same definition serves the gfx950 kernels
 // and the host oracle; elementary functions come from mpgos::math so both
 // sides evaluate identical bits.
 #pragma once
+
+#include <type_traits>
 
 #include "../mpgos_math.h"
 
@@ -42,6 +46,25 @@ struct NoCallbacks {
     template <class P> MPGOS_HD static void Initialization(int, int, int&, P&, P&, P*, P*, P*, P*, int*, P*, int*) {}
     template <class P> MPGOS_HD static void Finalization(int, int, int&, P&, P&, P*, P*, P*, P*, int*, P*, int*) {}
 };
+
+// The same for per-block systems (callback argument lists in pb_ring.h).
+struct PBNoCallbacks {
+#define MPGOS_PB_ARGS P*, P*, P*, int*, P*, int*, P*, int*
+    template <class P> MPGOS_HD static void EventFunction(int, int, P*, P, P, P*, P*, MPGOS_PB_ARGS) {}
+    template <class P> MPGOS_HD static void ActionAfterEventDetection(int, int, int, int&, P&, P&, P*, P*, MPGOS_PB_ARGS) {}
+    template <class P> MPGOS_HD static void ActionAfterSuccessfulTimeStep(int, int, int&, P&, P&, P*, P*, MPGOS_PB_ARGS) {}
+    template <class P> MPGOS_HD static void Finalization(int, int, int&, P&, P&, P*, P*, MPGOS_PB_ARGS) {}
+#undef MPGOS_PB_ARGS
+};
+
+// Whether a system leaves ActionAfterSuccessfulTimeStep to Base (NoCallbacks or
+// PBNoCallbacks).
+template <class Sys, class Base> constexpr bool no_step_action()
+{
+    if constexpr (std::is_base_of<Base, Sys>::value)
+        return &Sys::template ActionAfterSuccessfulTimeStep<double> == &Base::template ActionAfterSuccessfulTimeStep<double>;
+    else return false;
+}
 
 // Number of time terms of a system (0 for systems that name none), and whether
 // they depend on the time alone.

@@ -63,7 +63,7 @@ class PBOption(enum.IntEnum):
     SharedGlobalVariables = 12
     SharedCouplingMatrices = 13
     CouplingKernel = 14          # new: 0 automatic, 1 lane per pair, 2 dense contraction (MFMA)
-    MfmaUnitsPerLane = 15        # new: 4 (default) or 2 units per lane in the dense-contraction kernel
+    MfmaUnitsPerLane = 15        # new: 2 or 4, accepted without effect (the dense-contraction kernel chooses its split)
 
 
 class _PBDims(ctypes.Structure):

@@ -1,0 +1,71 @@
+"""The dense-contraction form of the per-block solver at the edges of its
+layout, bit for bit against the oracle and the lane-per-pair form: unit counts
+around the 16-unit tiles (one unit, one tile, padded tiles, one and two tiles
+per wavefront), system counts around its 4 and 8 systems per workgroup with
+inactive systems at the end, both algorithms; the form with events, user
+termination, accessories and dense output at an odd unit count; and the system
+counts from which a workgroup holds 8 systems."""
+import numpy as np
+import pytest
+
+from mpgos import workloads as W
+from mpgos.enums import Algorithms
+from test_gpu_perblock import assert_pb_bitwise, run_pb_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _ring(ns, ups, alg, end, off):
+    s = W.config4_ring(ns=ns, ups=ups, periods=1, algorithm=alg)
+    s["TD"][1] = np.linspace(0.5 * end, end, ns)
+    s["n_active"] = ns - off
+    if alg == Algorithms.RK4:
+        s["options"]["dt0"] = 0.01
+    return s
+
+
+@pytest.mark.parametrize("ups,ns,off", [(1, 5, 0), (9, 4, 1), (13, 8, 0), (16, 9, 2), (17, 3, 0), (100, 6, 1), (128, 4, 3),
+                                        (129, 7, 5), (250, 5, 0), (256, 2, 0)])
+@pytest.mark.parametrize("alg", [Algorithms.RKCK45, Algorithms.RK4], ids=["rkck45", "rk4"])
+def test_unit_counts(oracle, ups, ns, off, alg):
+    import pyoracle
+    s = _ring(ns, ups, alg, 1.0, off)
+    print(f"dense form {ns} x {ups} alg={int(alg)}", flush=True)
+    ref = pyoracle.run_pb("ring_duffing", s)
+    assert len(np.unique(ref["nacc"][:ns - off])) > 1 or ns - off < 3
+    assert_pb_bitwise(run_pb_gpu(s), ref, "automatic")
+    assert_pb_bitwise(run_pb_gpu(s, kernel=1), ref, "lane per pair")
+    assert_pb_bitwise(run_pb_gpu(s, shared_matrix=1, shared_globals=0), ref, "options")
+
+
+@pytest.mark.parametrize("ns,ups", [(1027, 129), (2053, 113), (16390, 12)])
+def test_eight_systems_per_workgroup(oracle, ns, ups):
+    import pyoracle
+    s = _ring(ns, ups, Algorithms.RKCK45, 0.25, 3)
+    print(f"dense form {ns} x {ups}", flush=True)
+    ref = pyoracle.run_pb("ring_duffing", s)
+    assert_pb_bitwise(run_pb_gpu(s), ref, "automatic")
+
+
+@pytest.mark.parametrize("ns,ups,ndo", [(5, 14, 64), (3, 150, 7), (1025, 130, 3), (2050, 114, 0)])
+def test_events_and_dense_output(oracle, ns, ups, ndo):
+    import pyoracle
+    base = W.tutorial_ring_dw(ns=25, ups=ups)
+    s = W.new_pb_spec("ring_dw", Algorithms.RKCK45, ns, ups, ndo=ndo)
+    for k in ("rtol", "atol", "edir", "options", "gPAR", "cIndex"):
+        s[k] = base[k]
+    for key in ("TD", "T", "sPAR", "sACC", "sACCi", "strength", "DOidx"):
+        s[key] = np.ascontiguousarray(np.resize(base[key].T, (ns,) + base[key].T.shape[1:]).T)
+    for key in ("X", "uPAR", "uACC", "uACCi"):
+        s[key] = np.ascontiguousarray(np.resize(base[key].T, (ns * ups,) + base[key].T.shape[1:]).T)
+    ring = np.zeros((ups, ups))
+    for r in range(ups):
+        ring[r, (r + 1) % ups] = ring[r, (r - 1) % ups] = 1.0
+    s["cMat"] = np.concatenate([W.store_coupling(ring, 0, 0)] * 2)
+    if ns > 100:
+        s["TD"][1] = 2.0
+    print(f"ring_dw {ns} x {ups}", flush=True)
+    ref = pyoracle.run_pb("ring_dw", s)
+    assert_pb_bitwise(run_pb_gpu(s), ref, "automatic")
+    if ns < 100:
+        assert (ref["uACCi"] == 2).any() and (ref["T"] < s["TD"][1]).any()
