@@ -8,7 +8,7 @@
 // (frozen step sequence; the error controller and event step control are not
 // differentiated; user actions that change the state are not replayed).
 //
-// Record pass (pb_record_kernel in pb_device.h): the forward integration
+// Record pass (pb_record_kernel in pb_device.h, pb_dense_kernel): the forward integration
 // storing the unit states every K accepted steps and (t_n, h_n) of every
 // accepted step.
 // Reverse pass (pb_reverse_kernel), lane per (system, unit), SPB systems per
@@ -49,7 +49,7 @@ struct AdjArgs {
     double* gU;           // out: dL/d(unit parameters)             [NUP][NU]
     double* gS;           // out: dL/d(system parameters)           [NSP][NS]
     const double* cMatT;  // transposed coupling matrices in the stored form of cMat
-    const double* cTileT; // their pair-tiled copy (dense-contraction form; null: read cMatT)
+    const double* cTileT; // their pair-tiled copy (dense-contraction form)
 };
 
 // sum over the matrix row u of M_i (any storage form) against vals[col * NCp + i]
@@ -448,428 +448,442 @@ __device__ __forceinline__ double rk_a(int s, int l)
     return l < s ? A[s][l] : 0.0;
 }
 
-// LDS of the dense-contraction reverse pass: system scopes, the B operand and
-// the contraction results (rows of mfma_row(UPS) doubles per coupling and
-// block system, mfma_index), the system-parameter gradient partials and two
-// block-wide counters.
-struct RevMfmaLayout { size_t cptB, coup, red, blk, total; };
-
-template <class Sys>
-__host__ __device__ inline RevMfmaLayout reverse_mfma_layout(int UPS)
-{
-    constexpr int NCp = Pos<Sys::NC>::value, NSPp = Pos<Sys::NSP>::value, SPB = kMfmaSystems;
-    RevMfmaLayout L;
-    size_t o = ((size_t)SPB * sizeof(RevScope<Sys>) + 15) & ~(size_t)15;
-    L.cptB = o;
-    o += (size_t)NCp * SPB * mfma_row(UPS) * sizeof(double);
-    L.coup = o;
-    o += (size_t)NCp * SPB * mfma_row(UPS) * sizeof(double);
-    L.red = o;
-    o += (size_t)SPB * UPS * NSPp * sizeof(double);
-    L.blk = o;
-    o += 2 * sizeof(int);
-    L.total = o;
-    return L;
-}
-
-// Reverse pass in the dense-contraction form (full FP64 coupling matrix, UPS a
-// multiple of 32 up to 256): 8 systems per workgroup, 4 units per lane
-// (2 * UPS threads), every coupling product on v_mfma_f64_4x4x4f64 (mfma_contract44) --
-// M CPT(Y) in the segment replay, M^T w (cMatT) in the adjoint sweep.  Round r
-// handles the r-th segment from the end of every system in two launches:
-//   pb_replay_mfma_kernel: restore checkpoint k = nseg - 1 - r and replay the
+// Reverse pass in the dense-contraction form (full FP64 coupling matrices, up
+// to 256 units): the layout of pb_dense.h, every coupling product on
+// v_mfma_f64_4x4x4f64 -- M CPT(Y) in the segment replay, M^T w in the adjoint
+// sweep.  Round r handles the r-th segment from the end of every system in two
+// launches:
+//   pb_replay_kernel: restore checkpoint k = nseg - 1 - r and replay the
 //     segment's recorded steps, keeping each stage's input Y_s and coupling
 //     values v_s in the stage buffer
 //       stg[(((j * ST + s) * (UD + NC)) + c) * NU + unit],  j < K;
-//   pb_sweep_mfma_kernel: the adjoint sweep through the segment from the
-//     stage buffer (no forward coupling product again; CPF_s from the unit's
+//   pb_sweep_kernel: the adjoint sweep through the segment from the stage
+//     buffer (no forward coupling product again; CPF_s from the unit's
 //     right-hand side at (Y_s, T_s)); dL/dx, the unit-parameter gradient and
 //     the per-unit system-parameter partials carry over between rounds in HBM
 //     (lam, gU, gSp);
 // pb_reverse_finish_kernel sums the partials per system in unit order.  Two
-// kernels instead of one keep the stage-vector registers of the replay and the
-// adjoint registers of the sweep from being live together.  Sums run in the
-// same order as in the lane form (the accumulation chain of the MFMA
-// instruction is a sequential fused multiply-add in column order), so both
-// forms return the same bits.
-template <class Sys, int PAIRS>
-struct MfmaRevCtx {
-    static constexpr int SPB = kMfmaSystems;
-    // tiles a wave contracts together in the replay and sweep kernels: all of
-    // them for every system (these kernels hold fewer values across the
-    // contraction than the forward step; ring with a quadrature state,
-    // reverse 352 -> 321 ms against one tile at a time)
-    static constexpr int TPW = PAIRS >= 4 ? PAIRS / 2 : 1;
+// kernels instead of one keep the stage vectors of the replay and the adjoints
+// of the sweep from being live together, and let each hold its own matrix (M,
+// M^T) in LDS.  Sums run in the same order as in the lane form, so both forms
+// return the same bits.
+//
+// What bounds it: the latency of a step (1024 x 128 units: two wavefronts per
+// SIMD) and, with 8 systems of 256 units, the registers (89 of the sweep's
+// values per lane spill).  Reverse pass of two periods of 1024 x 128 units
+// 24.6 -> 7.9 ms, one period of 300 x 256 25.6 -> 14.6, 4096 x 128 21.1 -> 14.6,
+// 4096 x 256 57.1 -> 51.9 ms against products through LDS with 8 systems per
+// workgroup; 1000 x 100 units 40.5 -> 3.4 ms against one lane per unit.
+template <class Sys, int NSL, int TT>
+struct DenseRev {
+    static constexpr int NC = Sys::NC, SPB = 4 * NSL, NTT = TimeTermsOf<Sys>::n, PER = 64 / SPB;
     using Scope = RevScope<Sys>;
-    Scope* sys; double* cptB; double* coup; int* blk;
-    int lanesPerSys, lsys, u0, gsys, k, len, maxlen;
-    bool leader, active;
+    using Place = DensePlace<NSL, TT>;
+    Scope* sys; double* cptBuf; const double* Ml;
+    int cptStride, maxlen;
     size_t NU;
-    unsigned gu0;
-    Scope* my;
+    Place at;
+    bool active[NSL];
+    int k[NSL], len[NSL];
 
-    // lane mapping, system scope and this round's segment of each system
+    // LDS, system scope and this round's segment of each system
     // (k = nseg - 1 - r, len steps; maxlen over the workgroup)
-    __device__ __forceinline__ void setup(const Args<Sys, double>& a, unsigned char* lds, int r)
+    __device__ __forceinline__ DenseRev(const Args<Sys, double>& a, const double* Mt, unsigned char* lds, int r)
+        : at(a.UPS, a.NS)
     {
-        const RevMfmaLayout L = reverse_mfma_layout<Sys>(a.UPS);
+        const DenseLayout L = dense_layout<Scope, NC, 0, 0>(SPB, a.UPS, 0, a.ldsPairs);
         sys = reinterpret_cast<Scope*>(lds);
-        cptB = reinterpret_cast<double*>(lds + L.cptB);
-        coup = reinterpret_cast<double*>(lds + L.coup);
-        blk = reinterpret_cast<int*>(lds + L.blk);
-        const int tid = threadIdx.x, UPS = a.UPS, NS = a.NS, K = a.recK;
-        lanesPerSys = UPS / PAIRS;
-        lsys = tid / lanesPerSys;                     // < SPB (blockDim.x = SPB * UPS / PAIRS)
-        u0 = tid - lsys * lanesPerSys;
-        leader = u0 == 0;
-        gsys = blockIdx.x * SPB + lsys;
-        active = gsys < NS && gsys < a.nActive;
-        NU = (size_t)NS * UPS;
-        gu0 = (unsigned)gsys * (unsigned)UPS + (unsigned)u0;
-        my = &sys[lsys];
-        for (int i = tid; i < Pos<Sys::NC>::value * kMfmaSystems * mfma_row(UPS); i += blockDim.x) cptB[i] = 0.0;
-        if (tid == 0) blk[1] = 0;
-        if (leader) {
-            my->status = 0; my->k = -1; my->len = 0;
-            if (active) {
-                for (int i = 0; i < Sys::NSP; i++) my->sPAR[i] = a.sPAR[gsys + i * NS];
-                for (int i = 0; i < Sys::NSA; i++) my->sACC[i] = a.sACC[gsys + i * NS];
-                for (int i = 0; i < Sys::NiSA; i++) my->sACCi[i] = a.sACCi[gsys + i * NS];
-                for (int i = 0; i < Sys::NC; i++) my->strength[i] = a.strength[gsys + i * NS];
-                my->nacc = a.nacc[gsys];
-                my->status = a.status[gsys];
-                const bool ok = (my->status & MPGOS_STATUS_CHECKPOINT_OVERFLOW) == 0;
-                const int nseg = ok ? (int)((my->nacc + K - 1) / K) : 0;
-                const int kk = nseg - 1 - r;
-                my->k = kk;
-                my->len = kk >= 0 ? (int)((my->nacc - (long long)kk * K) < K ? (my->nacc - (long long)kk * K) : K) : 0;
+        cptBuf = reinterpret_cast<double*>(lds + L.cpt);
+        Ml = reinterpret_cast<const double*>(lds + L.mt);
+        int* blk = reinterpret_cast<int*>(lds + L.blk);
+        cptStride = NC * SPB * dense_row(a.UPS);
+        NU = (size_t)a.NS * a.UPS;
+        const int K = a.recK;
+        if (threadIdx.x == 0) blk[0] = 0;
+#pragma unroll
+        for (int s = 0; s < NSL; s++) {
+            const int g = at.gsys(s);
+            active[s] = g < a.NS && g < a.nActive;
+            if (!at.leads(s)) continue;
+            Scope& y = sys[at.sys(s)];
+            y.status = 0; y.k = -1; y.len = 0;
+            for (int i = 0; i < Sys::NSP; i++) y.sPAR[i] = active[s] ? a.sPAR[g + i * a.NS] : 0.0;
+            if (active[s]) {
+                for (int i = 0; i < Sys::NSA; i++) y.sACC[i] = a.sACC[g + i * a.NS];
+                for (int i = 0; i < Sys::NiSA; i++) y.sACCi[i] = a.sACCi[g + i * a.NS];
+                for (int i = 0; i < NC; i++) y.strength[i] = a.strength[g + i * a.NS];
+                y.nacc = a.nacc[g];
+                y.status = a.status[g];
+                const bool ok = (y.status & MPGOS_STATUS_CHECKPOINT_OVERFLOW) == 0;
+                const int kk = (ok ? (int)((y.nacc + K - 1) / K) : 0) - 1 - r;
+                y.k = kk;
+                y.len = kk >= 0 ? (int)((y.nacc - (long long)kk * K) < K ? (y.nacc - (long long)kk * K) : K) : 0;
             }
         }
         __syncthreads();
-        if (leader) atomicMax(&blk[1], my->len);
+        if (threadIdx.x < SPB) atomicMax(&blk[0], sys[threadIdx.x].len);
         __syncthreads();
-        maxlen = blk[1];
-        k = my->k;
-        len = my->len;
+        maxlen = blk[0];
+        if (maxlen == 0) return;                       // workgroup-uniform
+#pragma unroll
+        for (int s = 0; s < NSL; s++) {
+            k[s] = sys[at.sys(s)].k;
+            len[s] = active[s] ? sys[at.sys(s)].len : 0;
+        }
+        for (int i = threadIdx.x; i < 2 * cptStride; i += blockDim.x) cptBuf[i] = 0.0;   // padded units and absent systems stay zero
+        dense_stage_matrix(Mt, lds + L.mt, NC, a.UPS, a.ldsPairs);
+        __syncthreads();
     }
-    __device__ __forceinline__ int uid(int p) const { return u0 + p * lanesPerSys; }
-    __device__ __forceinline__ unsigned at(int p) const { return gu0 + (unsigned)(p * lanesPerSys); }
+    __device__ __forceinline__ bool has(int s, int q) const { return len[s] > 0 && at.has(q); }
+    __device__ __forceinline__ unsigned unit(int s, int q) const { return (unsigned)at.gsys(s) * (unsigned)at.UPS + (unsigned)at.unit(q); }
     // row r of a unit-scope array [rows][NU]: wave-uniform row base, 32-bit lane offset
-    __device__ __forceinline__ double* row(double* base, size_t r) const { return base + r * NU; }
+    template <class T>
+    __device__ __forceinline__ T* row(T* base, size_t r) const { return base + r * NU; }
+    // (t, h) of step j of each of the lane's systems, 0 where it has none
+    __device__ __forceinline__ void step_times(const Args<Sys, double>& a, int j, double* t, double* h) const
+    {
+#pragma unroll
+        for (int s = 0; s < NSL; s++) {
+            const bool run = j >= 0 && j < len[s];
+            const size_t n = ((size_t)k[s] * a.recK + j) * a.NS + at.gsys(s);
+            t[s] = run ? a.recT[n] : 0.0;
+            h[s] = run ? a.recH[n] : 0.0;
+        }
+    }
+    // the time terms of a step's stages as in the forward pass: lane l
+    // evaluates stage e * PER + l / SPB of system l % SPB
+    template <int ALG, int N>
+    __device__ __forceinline__ void time_terms(const double* t, const double* h, double (&tt)[N][Pos<NTT>::value]) const
+    {
+        if constexpr (NTT > 0) {
+            double t0 = t[0], h0 = h[0];
+            if constexpr (NSL > 1) {
+                // opaque values: a select between array elements would become an
+                // indexed load, which moves the arrays to scratch memory
+                double t1 = t[NSL - 1], h1 = h[NSL - 1];
+                asm("" : "+v"(t0), "+v"(h0), "+v"(t1), "+v"(h1));
+                const bool own = (at.l % SPB) < 4;
+                t0 = own ? t0 : t1;
+                h0 = own ? h0 : h1;
+            }
+#pragma unroll
+            for (int e = 0; e < N; e++)
+                Sys::template TimeTerms<double>(rk_stage_time<ALG>(e * PER + at.l / SPB, t0, h0), sys[at.l % SPB].sPAR, tt[e]);
+        }
+    }
+    template <int N>
+    __device__ __forceinline__ void stage_terms(int stage, int s, const double (&tterm)[N][Pos<NTT>::value], double* tt) const
+    {
+#pragma unroll
+        for (int i = 0; i < NTT; i++) tt[i] = __shfl(tterm[stage / PER][i], (stage % PER) * SPB + at.sys(s));
+    }
 };
 
-template <class Sys, int ALG, int PAIRS>
-__device__ void pb_replay_mfma_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A, int r)
+#define MPGOS_PB_EACH(s, q) _Pragma("unroll") for (int s = 0; s < NSL; s++) _Pragma("unroll") for (int q = 0; q < TT; q++)
+
+template <class Sys, int ALG, int NSL, int TT>
+__device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A, int r)
 {
     using P = double;
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NUA = Sys::NUA, NiUA = Sys::NiUA;
-    constexpr int NCp = Pos<NC>::value, NUPp = Pos<NUP>::value;
-    constexpr int ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC, SPB = kMfmaSystems;
+    constexpr int NCp = Pos<NC>::value, NTT = TimeTermsOf<Sys>::n, ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC;
     using math::fma;
-    using U = Unit<Sys, P>;
+    using R = DenseRev<Sys, NSL, TT>;
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
-    MfmaRevCtx<Sys, PAIRS> C;
-    C.setup(a, mpgos_pb_lds, r);
-    if (C.maxlen == 0) return;                         // workgroup-uniform
-    const int UPS = a.UPS, NS = a.NS, K = a.recK;
-    const int gsys = C.gsys, lsys = C.lsys, k = C.k, len = C.len;
-    const bool active = C.active;
-    auto* my = C.my;
-    double* cptB = C.cptB;
-    double* coup = C.coup;
+    const R C(a, a.cTile, mpgos_pb_lds, r);
+    if (C.maxlen == 0) return;
+    DenseContraction<NC, NSL, TT> product(a.cTile, C.Ml, a.ldsPairs, a.UPS);
+    const int RS = dense_row(a.UPS);
 
     int cIndex[NCp];
 #pragma unroll
     for (int i = 0; i < NC; i++) cIndex[i] = a.cIndex[i];
-    P uPAR[PAIRS][NUPp], uACC[PAIRS][Pos<NUA>::value], X[PAIRS][UD];
-    int uACCi[PAIRS][Pos<NiUA>::value];
+    P uPAR[NSL][TT][Pos<NUP>::value], uACC[NSL][TT][Pos<NUA>::value], X[NSL][TT][UD];
+    int uACCi[NSL][TT][Pos<NiUA>::value];
+    MPGOS_PB_EACH(s, q) {
+        const bool ld = C.has(s, q);
+        const unsigned u = C.unit(s, q);
 #pragma unroll
-    for (int p = 0; p < PAIRS; p++) {
-        const bool ld = active && len > 0;
+        for (int c = 0; c < NUP; c++) uPAR[s][q][c] = ld ? C.row(a.uPAR, c)[u] : P(0);
 #pragma unroll
-        for (int c = 0; c < NUP; c++) uPAR[p][c] = ld ? C.row(a.uPAR, c)[C.at(p)] : P(0);
+        for (int c = 0; c < NUA; c++) uACC[s][q][c] = ld ? C.row(a.uACC, c)[u] : P(0);
 #pragma unroll
-        for (int c = 0; c < NUA; c++) uACC[p][c] = ld ? C.row(a.uACC, c)[C.at(p)] : P(0);
+        for (int c = 0; c < NiUA; c++) uACCi[s][q][c] = ld ? C.row(a.uACCi, c)[u] : 0;
 #pragma unroll
-        for (int c = 0; c < NiUA; c++) uACCi[p][c] = ld ? a.uACCi[C.at(p) + c * C.NU] : 0;
-#pragma unroll
-        for (int c = 0; c < UD; c++) X[p][c] = ld ? C.row(a.recX, (size_t)k * UD + c)[C.at(p)] : P(0);
+        for (int c = 0; c < UD; c++) X[s][q][c] = ld ? a.recX[((size_t)C.k[s] * UD + c) * C.NU + u] : P(0);
     }
-    P* gPAR = a.gPAR;
-    int* gPARi = a.gPARi;
 
-    // right-hand sides of the lane's units at (Y, T) plus the coupling terms;
-    // v receives the coupling values (M CPT)_u.  The barriers order LDS only,
-    // so the stage-buffer stores stay in flight across them.
-    auto rhs = [&](bool run, P (*F)[UD], P (*Y)[UD], const P T, P (*v)[NCp]) {
-        P CPF[PAIRS][NCp];
-        if (run) {
+    int buf = 0;
+    P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value];
+    P t[NSL], h[NSL], tn[NSL], hn[NSL];
+    // right-hand sides of the lane's units at (Y, T) plus the coupling terms of
+    // stage st of step j; Y and the coupling values (M CPT)_u are kept.  The
+    // barriers order LDS only, so the stage-buffer stores stay in flight.
+    auto rhs = [&](int st, int j, P (*F)[TT][UD], P (*Y)[TT][UD]) {
+        P CPF[NSL][TT][NCp], v[NCp][NSL][TT], tt[NSL][Pos<NTT>::value];
+        P* cpt = C.cptBuf + (size_t)buf * C.cptStride;
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++) {
+        for (int s = 0; s < NSL; s++) C.stage_terms(st, s, tterm, tt[s]);
+        product.prefetch();
+        MPGOS_PB_EACH(s, q) {
+            if (j < C.len[s] && C.at.has(q)) {
                 P cp[NCp];
-                Sys::template OdeFunction<P>(gsys, C.uid(p), F[p], Y[p], T, uPAR[p], my->sPAR, gPAR, gPARi, uACC[p], uACCi[p],
-                                             my->sACC, my->sACCi, cp, CPF[p]);
 #pragma unroll
-                for (int i = 0; i < NC; i++) cptB[mfma_index(i, lsys, C.uid(p), UPS)] = cp[i];
+                for (int i = 0; i < NC; i++) cp[i] = CPF[s][q][i] = P(0);
+                auto& y = C.sys[C.at.sys(s)];
+                const P T = rk_stage_time<ALG>(st, t[s], h[s]);
+                if constexpr (NTT > 0)
+                    Sys::template OdeFunctionTT<P>(C.at.gsys(s), C.at.unit(q), F[s][q], Y[s][q], T, tt[s], uPAR[s][q], y.sPAR, a.gPAR, a.gPARi,
+                                                   uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, cp, CPF[s][q]);
+                else
+                    Sys::template OdeFunction<P>(C.at.gsys(s), C.at.unit(q), F[s][q], Y[s][q], T, uPAR[s][q], y.sPAR, a.gPAR, a.gPARi,
+                                                 uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, cp, CPF[s][q]);
+#pragma unroll
+                for (int i = 0; i < NC; i++) cpt[(i * R::SPB + C.at.sys(s)) * RS + C.at.unit(q)] = cp[i];
+                const size_t base = ((size_t)j * ST + st) * SW;
+#pragma unroll
+                for (int c = 0; c < UD; c++) C.row(A.stg, base + c)[C.unit(s, q)] = Y[s][q][c];
             }
         }
         lds_barrier();
-        mfma_contract44<NC, true, 8, MfmaRevCtx<Sys, PAIRS>::TPW>(a.cMat, cptB, coup, UPS, SPB, a.cTile);
-        lds_barrier();
-        if (run) {
+        product.run(cpt, v);
+        MPGOS_PB_EACH(s, q) {
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
+            for (int i = 0; i < NC; i++)
+                Unit<Sys, P>::add(cIndex[i], C.sys[C.at.sys(s)].strength[i] * CPF[s][q][i], v[i][s][q], F[s][q]);
+            if (j < C.len[s] && C.at.has(q)) {
+                const size_t base = ((size_t)j * ST + st) * SW;
 #pragma unroll
-                for (int i = 0; i < NC; i++) {
-                    v[p][i] = coup[mfma_index(i, lsys, C.uid(p), UPS)];
-                    U::add(cIndex[i], my->strength[i] * CPF[p][i], v[p][i], F[p]);
-                }
+                for (int i = 0; i < NC; i++) C.row(A.stg, base + UD + i)[C.unit(s, q)] = v[i][s][q];
+            }
+        }
+        buf ^= 1;
+    };
+    auto fill = [&](P (*Y)[TT][UD], auto&& value) {
+        MPGOS_PB_EACH(s, q) {
+#pragma unroll
+            for (int c = 0; c < UD; c++) Y[s][q][c] = value(s, q, c);
         }
     };
+    C.step_times(a, 0, tn, hn);
     for (int j = 0; j < C.maxlen; j++) {
-        const bool run = active && j < len;
-        P t = P(0), h = P(0);
-        if (run) {
-            const size_t n = (size_t)k * K + j;
-            t = a.recT[n * NS + gsys];
-            h = a.recH[n * NS + gsys];
-        }
-        auto keep = [&](int s, P (*Y)[UD], P (*v)[NCp]) {
-            if (run) {
-                const size_t base = ((size_t)j * ST + s) * SW;
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++) {
-#pragma unroll
-                    for (int c = 0; c < UD; c++) C.row(A.stg, base + c)[C.at(p)] = Y[p][c];
-#pragma unroll
-                    for (int i = 0; i < NC; i++) C.row(A.stg, base + UD + i)[C.at(p)] = v[p][i];
-                }
-            }
-        };
-        // the forward pass's stage arithmetic (pb_body)
-        P v[PAIRS][NCp], next[PAIRS][UD], Y[PAIRS][UD];
+        for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
+        C.step_times(a, j + 1, tn, hn);                 // one step ahead
+        C.template time_terms<ALG>(t, h, tterm);
+        // the forward pass's stage arithmetic (pb_dense_body)
+        P next[NSL][TT][UD], k[NSL][TT][UD], Y[NSL][TT][UD];
         if (ALG == MPGOS_RK4) {
-            P k1[PAIRS][UD];
-            rhs(run, next, X, t, v);
-            keep(0, X, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) Y[p][c] = fma(next[p][c] * P(0.5), h, X[p][c]);
-            const P t2 = t + P(0.5) * h;
-            rhs(run, k1, Y, t2, v);
-            keep(1, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) { next[p][c] = fma(P(2), k1[p][c], next[p][c]); Y[p][c] = fma(k1[p][c] * P(0.5), h, X[p][c]); }
-            rhs(run, k1, Y, t2, v);
-            keep(2, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) { next[p][c] = fma(P(2.0), k1[p][c], next[p][c]); Y[p][c] = fma(k1[p][c], h, X[p][c]); }
-            rhs(run, k1, Y, t + h, v);
-            keep(3, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) next[p][c] = fma(h * (next[p][c] + k1[p][c]), P(1.0 / 6.0), X[p][c]);
+            rhs(0, j, next, X);
+            fill(Y, [&](int s, int q, int c) { return fma(next[s][q][c] * P(0.5), h[s], X[s][q][c]); });
+            rhs(1, j, k, Y);
+            fill(next, [&](int s, int q, int c) { return fma(P(2), k[s][q][c], next[s][q][c]); });
+            fill(Y, [&](int s, int q, int c) { return fma(k[s][q][c] * P(0.5), h[s], X[s][q][c]); });
+            rhs(2, j, k, Y);
+            fill(next, [&](int s, int q, int c) { return fma(P(2.0), k[s][q][c], next[s][q][c]); });
+            fill(Y, [&](int s, int q, int c) { return fma(k[s][q][c], h[s], X[s][q][c]); });
+            rhs(3, j, k, Y);
+            fill(next, [&](int s, int q, int c) { return fma(h[s] * (next[s][q][c] + k[s][q][c]), P(1.0 / 6.0), X[s][q][c]); });
         } else {
-            P k1[PAIRS][UD], k2[PAIRS][UD], k3[PAIRS][UD], k4[PAIRS][UD], k5[PAIRS][UD], k6[PAIRS][UD];
-            rhs(run, k1, X, t, v);
-            keep(0, X, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) Y[p][c] = fma(k1[p][c] * P(1.0 / 5.0), h, X[p][c]);
-            rhs(run, k2, Y, fma(P(1.0 / 5.0), h, t), v);
-            keep(1, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++) Y[p][c] = fma(fma(k2[p][c], P(9.0 / 40.0), k1[p][c] * P(3.0 / 40.0)), h, X[p][c]);
-            rhs(run, k3, Y, fma(P(3.0 / 10.0), h, t), v);
-            keep(2, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    Y[p][c] = fma(fma(k3[p][c], P(6.0 / 5.0), fma(k2[p][c], P(-9.0 / 10.0), k1[p][c] * P(3.0 / 10.0))), h, X[p][c]);
-            rhs(run, k4, Y, fma(P(3.0 / 5.0), h, t), v);
-            keep(3, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    Y[p][c] = fma(fma(k4[p][c], P(35.0 / 27.0), fma(k3[p][c], P(-70.0 / 27.0), fma(k2[p][c], P(5.0 / 2.0),
-                                  k1[p][c] * P(-11.0 / 54.0)))), h, X[p][c]);
-            rhs(run, k5, Y, t + h, v);
-            keep(4, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    Y[p][c] = fma(fma(k5[p][c], P(253.0 / 4096.0), fma(k4[p][c], P(44275.0 / 110592.0), fma(k3[p][c], P(575.0 / 13824.0),
-                                  fma(k2[p][c], P(175.0 / 512.0), k1[p][c] * P(1631.0 / 55296.0))))), h, X[p][c]);
-            rhs(run, k6, Y, fma(P(7.0 / 8.0), h, t), v);
-            keep(5, Y, v);
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++)
-#pragma unroll
-                for (int c = 0; c < UD; c++)
-                    next[p][c] = fma(fma(k6[p][c], P(512.0 / 1771.0), fma(k4[p][c], P(125.0 / 594.0), fma(k3[p][c], P(250.0 / 621.0),
-                                     k1[p][c] * P(37.0 / 378.0)))), h, X[p][c]);
+            P k1[NSL][TT][UD], k2[NSL][TT][UD], k3[NSL][TT][UD], sum6[NSL][TT][UD];
+            rhs(0, j, k1, X);
+            fill(Y, [&](int s, int q, int c) { return fma(k1[s][q][c] * P(1.0 / 5.0), h[s], X[s][q][c]); });
+            rhs(1, j, k2, Y);
+            fill(Y, [&](int s, int q, int c) { return fma(fma(k2[s][q][c], P(9.0 / 40.0), k1[s][q][c] * P(3.0 / 40.0)), h[s], X[s][q][c]); });
+            rhs(2, j, k3, Y);
+            fill(Y, [&](int s, int q, int c) {
+                return fma(fma(k3[s][q][c], P(6.0 / 5.0), fma(k2[s][q][c], P(-9.0 / 10.0), k1[s][q][c] * P(3.0 / 10.0))), h[s], X[s][q][c]);
+            });
+            rhs(3, j, k, Y);
+            fill(Y, [&](int s, int q, int c) {
+                return fma(fma(k[s][q][c], P(35.0 / 27.0), fma(k3[s][q][c], P(-70.0 / 27.0), fma(k2[s][q][c], P(5.0 / 2.0),
+                           k1[s][q][c] * P(-11.0 / 54.0)))), h[s], X[s][q][c]);
+            });
+            fill(sum6, [&](int s, int q, int c) {
+                return fma(k[s][q][c], P(44275.0 / 110592.0), fma(k3[s][q][c], P(575.0 / 13824.0),
+                           fma(k2[s][q][c], P(175.0 / 512.0), k1[s][q][c] * P(1631.0 / 55296.0))));
+            });
+            fill(next, [&](int s, int q, int c) {
+                return fma(k[s][q][c], P(125.0 / 594.0), fma(k3[s][q][c], P(250.0 / 621.0), k1[s][q][c] * P(37.0 / 378.0)));
+            });
+            rhs(4, j, k, Y);
+            fill(Y, [&](int s, int q, int c) { return fma(fma(k[s][q][c], P(253.0 / 4096.0), sum6[s][q][c]), h[s], X[s][q][c]); });
+            rhs(5, j, k, Y);
+            fill(next, [&](int s, int q, int c) { return fma(fma(k[s][q][c], P(512.0 / 1771.0), next[s][q][c]), h[s], X[s][q][c]); });
         }
-        if (run) {
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
+        for (int s = 0; s < NSL; s++) {
+            if (j < C.len[s]) {
 #pragma unroll
-                for (int c = 0; c < UD; c++) X[p][c] = next[p][c];
+                for (int q = 0; q < TT; q++)
+#pragma unroll
+                    for (int c = 0; c < UD; c++) X[s][q][c] = next[s][q][c];
+            }
         }
     }
 }
 
-template <class Sys, int ALG, int PAIRS>
-__device__ void pb_sweep_mfma_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A, int r)
+template <class Sys, int ALG, int NSL, int TT>
+__device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A, int r)
 {
     using P = double;
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NSP = Sys::NSP, NUA = Sys::NUA, NiUA = Sys::NiUA;
-    constexpr int NCp = Pos<NC>::value, NUPp = Pos<NUP>::value, NSPp = Pos<NSP>::value;
-    constexpr int ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC, SPB = kMfmaSystems;
+    constexpr int NCp = Pos<NC>::value, NUPp = Pos<NUP>::value, NSPp = Pos<NSP>::value, NTT = TimeTermsOf<Sys>::n;
+    constexpr int ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC;
     using math::fma;
+    using R = DenseRev<Sys, NSL, TT>;
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
-    MfmaRevCtx<Sys, PAIRS> C;
-    C.setup(a, mpgos_pb_lds, r);
-    if (C.maxlen == 0) return;                         // workgroup-uniform
-    const int UPS = a.UPS, NS = a.NS, K = a.recK;
-    const int gsys = C.gsys, lsys = C.lsys, k = C.k, len = C.len;
-    const bool active = C.active;
-    const bool mine = active && len > 0;               // this round has a segment of this system
-    auto* my = C.my;
-    double* cptB = C.cptB;
-    double* coup = C.coup;
+    const R C(a, A.cTileT, mpgos_pb_lds, r);
+    if (C.maxlen == 0) return;
+    DenseContraction<NC, NSL, TT> product(A.cTileT, C.Ml, a.ldsPairs, a.UPS);
+    const int RS = dense_row(a.UPS);
 
     int cIndex[NCp];
 #pragma unroll
     for (int i = 0; i < NC; i++) cIndex[i] = a.cIndex[i];
     // adjoint state carried between rounds; round 0 starts the gradients at zero
-    P uPAR[PAIRS][NUPp], uACC[PAIRS][Pos<NUA>::value], lam[PAIRS][UD], muU[PAIRS][NUPp], muS[PAIRS][NSPp];
-    int uACCi[PAIRS][Pos<NiUA>::value];
-#pragma unroll
-    for (int p = 0; p < PAIRS; p++) {
+    P uPAR[NSL][TT][NUPp], uACC[NSL][TT][Pos<NUA>::value], lam[NSL][TT][UD], muU[NSL][TT][NUPp], muS[NSL][TT][NSPp];
+    int uACCi[NSL][TT][Pos<NiUA>::value];
+    MPGOS_PB_EACH(s, q) {
+        const bool ld = C.has(s, q);
+        const unsigned u = C.unit(s, q);
 #pragma unroll
         for (int c = 0; c < NUP; c++) {
-            uPAR[p][c] = mine ? C.row(a.uPAR, c)[C.at(p)] : P(0);
-            muU[p][c] = (mine && r > 0) ? C.row(A.gU, c)[C.at(p)] : P(0);
+            uPAR[s][q][c] = ld ? C.row(a.uPAR, c)[u] : P(0);
+            muU[s][q][c] = (ld && r > 0) ? C.row(A.gU, c)[u] : P(0);
         }
 #pragma unroll
-        for (int c = 0; c < NUA; c++) uACC[p][c] = mine ? C.row(a.uACC, c)[C.at(p)] : P(0);
+        for (int c = 0; c < NUA; c++) uACC[s][q][c] = ld ? C.row(a.uACC, c)[u] : P(0);
 #pragma unroll
-        for (int c = 0; c < NiUA; c++) uACCi[p][c] = mine ? a.uACCi[C.at(p) + c * C.NU] : 0;
+        for (int c = 0; c < NiUA; c++) uACCi[s][q][c] = ld ? C.row(a.uACCi, c)[u] : 0;
 #pragma unroll
-        for (int c = 0; c < UD; c++) lam[p][c] = mine ? C.row(A.lam, c)[C.at(p)] : P(0);
+        for (int c = 0; c < UD; c++) lam[s][q][c] = ld ? C.row(A.lam, c)[u] : P(0);
 #pragma unroll
-        for (int c = 0; c < NSP; c++) muS[p][c] = (mine && r > 0) ? C.row(A.gSp, c)[C.at(p)] : P(0);
+        for (int c = 0; c < NSP; c++) muS[s][q][c] = (ld && r > 0) ? C.row(A.gSp, c)[u] : P(0);
     }
-    P* gPAR = a.gPAR;
-    int* gPARi = a.gPARi;
-
-    for (int j = C.maxlen - 1; j >= 0; j--) {
-        const bool run = active && j < len;
-        P t = P(0), h = P(0);
-        if (run) {
-            const size_t n = (size_t)k * K + j;
-            t = a.recT[n * NS + gsys];
-            h = a.recH[n * NS + gsys];
+    // a stage's inputs and coupling values, loaded one stage ahead
+    P ahead[NSL][TT][SW];
+    auto fetch = [&](int j, int st) {
+        const size_t base = ((size_t)j * ST + st) * SW;
+        MPGOS_PB_EACH(s, q) {
+            const bool ld = j >= 0 && j < C.len[s] && C.at.has(q);
+#pragma unroll
+            for (int c = 0; c < SW; c++) ahead[s][q][c] = ld ? C.row(A.stg, base + c)[C.unit(s, q)] : P(0);
         }
-        P kb[ST][PAIRS][UD];
+    };
+
+    int buf = 0;
+    P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value];
+    P t[NSL], h[NSL], tn[NSL], hn[NSL];
+    C.step_times(a, C.maxlen - 1, tn, hn);
+    fetch(C.maxlen - 1, ST - 1);
+    for (int j = C.maxlen - 1; j >= 0; j--) {
 #pragma unroll
-        for (int s = 0; s < ST; s++)
+        for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
+        C.step_times(a, j - 1, tn, hn);                 // one step ahead
+        C.template time_terms<ALG>(t, h, tterm);
+        P kb[ST][NSL][TT][UD];
 #pragma unroll
-            for (int p = 0; p < PAIRS; p++)
+        for (int st = 0; st < ST; st++)
+            MPGOS_PB_EACH(s, q) {
 #pragma unroll
-                for (int c = 0; c < UD; c++) kb[s][p][c] = h * rk_b<ALG>(s) * lam[p][c];
+                for (int c = 0; c < UD; c++) kb[st][s][q][c] = h[s] * rk_b<ALG>(st) * lam[s][q][c];
+            }
 #pragma unroll
-        for (int s = ST - 1; s >= 0; s--) {
-            const P Ts = rk_stage_time<ALG>(s, t, h);
-            const size_t base = ((size_t)j * ST + s) * SW;
-            P kbCPF[PAIRS][NCp];
-            if (run) {
+        for (int st = ST - 1; st >= 0; st--) {
+            P Y[NSL][TT][UD], kbCPF[NSL][TT][NCp], tt[NSL][Pos<NTT>::value], w[NCp][NSL][TT];
+            P* wb = C.cptBuf + (size_t)buf * C.cptStride;
 #pragma unroll
-                for (int p = 0; p < PAIRS; p++) {
-                    P Y[UD], F[UD], cp[NCp], cpf[NCp];
+            for (int s = 0; s < NSL; s++) C.stage_terms(st, s, tterm, tt[s]);
+            MPGOS_PB_EACH(s, q) {
 #pragma unroll
-                    for (int c = 0; c < UD; c++) Y[c] = C.row(A.stg, base + c)[C.at(p)];
-                    Sys::template OdeFunction<P>(gsys, C.uid(p), F, Y, Ts, uPAR[p], my->sPAR, gPAR, gPARi, uACC[p], uACCi[p],
-                                                 my->sACC, my->sACCi, cp, cpf);
+                for (int c = 0; c < UD; c++) Y[s][q][c] = ahead[s][q][c];
+                if (j < C.len[s] && C.at.has(q)) {
+                    P F[UD], cp[NCp], cpf[NCp];
+#pragma unroll
+                    for (int i = 0; i < NC; i++) cpf[i] = P(0);
+                    auto& y = C.sys[C.at.sys(s)];
+                    const P T = rk_stage_time<ALG>(st, t[s], h[s]);
+                    if constexpr (NTT > 0)
+                        Sys::template OdeFunctionTT<P>(C.at.gsys(s), C.at.unit(q), F, Y[s][q], T, tt[s], uPAR[s][q], y.sPAR, a.gPAR, a.gPARi,
+                                                       uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, cp, cpf);
+                    else
+                        Sys::template OdeFunction<P>(C.at.gsys(s), C.at.unit(q), F, Y[s][q], T, uPAR[s][q], y.sPAR, a.gPAR, a.gPARi,
+                                                     uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, cp, cpf);
 #pragma unroll
                     for (int i = 0; i < NC; i++) {
                         P g = P(0);
 #pragma unroll
                         for (int c = 0; c < UD; c++)
-                            if (c == cIndex[i]) g = kb[s][p][c];
-                        cptB[mfma_index(i, lsys, C.uid(p), UPS)] = my->strength[i] * cpf[i] * g;
-                        kbCPF[p][i] = my->strength[i] * C.row(A.stg, base + UD + i)[C.at(p)] * g;
+                            if (c == cIndex[i]) g = kb[st][s][q][c];
+                        wb[(i * R::SPB + C.at.sys(s)) * RS + C.at.unit(q)] = y.strength[i] * cpf[i] * g;
+                        kbCPF[s][q][i] = y.strength[i] * ahead[s][q][UD + i] * g;
                     }
                 }
             }
-            __syncthreads();
-            mfma_contract44<NC, true, 8, MfmaRevCtx<Sys, PAIRS>::TPW>(A.cMatT, cptB, coup, UPS, SPB, A.cTileT);
-            __syncthreads();
-#pragma unroll
-            for (int p = 0; p < PAIRS; p++) {
+            if (st > 0) fetch(j, st - 1);
+            else fetch(j - 1, ST - 1);
+            product.prefetch();
+            lds_barrier();
+            product.run(wb, w);
+            buf ^= 1;
+            MPGOS_PB_EACH(s, q) {
                 P gy[UD];
-                if (run) {
-                    P Y[UD], kbCPT[NCp], gU[NUPp], gS[NSPp];
+                if (j < C.len[s] && C.at.has(q)) {
+                    P kbCPT[NCp], gU[NUPp], gS[NSPp];
 #pragma unroll
-                    for (int c = 0; c < UD; c++) Y[c] = C.row(A.stg, base + c)[C.at(p)];
+                    for (int i = 0; i < NC; i++) kbCPT[i] = w[i][s][q];
+                    auto& y = C.sys[C.at.sys(s)];
+                    const P T = rk_stage_time<ALG>(st, t[s], h[s]);
+                    if constexpr (NTT > 0)
+                        Sys::template OdeVJPTT<P>(C.at.gsys(s), C.at.unit(q), kb[st][s][q], kbCPT, kbCPF[s][q], Y[s][q], T, tt[s], uPAR[s][q],
+                                                  y.sPAR, a.gPAR, a.gPARi, uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, gy, gU, gS);
+                    else
+                        Sys::template OdeVJP<P>(C.at.gsys(s), C.at.unit(q), kb[st][s][q], kbCPT, kbCPF[s][q], Y[s][q], T, uPAR[s][q], y.sPAR,
+                                                a.gPAR, a.gPARi, uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, gy, gU, gS);
 #pragma unroll
-                    for (int i = 0; i < NC; i++) kbCPT[i] = coup[mfma_index(i, lsys, C.uid(p), UPS)];
-                    Sys::template OdeVJP<P>(gsys, C.uid(p), kb[s][p], kbCPT, kbCPF[p], Y, Ts, uPAR[p], my->sPAR, gPAR, gPARi,
-                                            uACC[p], uACCi[p], my->sACC, my->sACCi, gy, gU, gS);
+                    for (int c = 0; c < NUP; c++) muU[s][q][c] += gU[c];
 #pragma unroll
-                    for (int c = 0; c < NUP; c++) muU[p][c] += gU[c];
-#pragma unroll
-                    for (int c = 0; c < NSP; c++) muS[p][c] += gS[c];
+                    for (int c = 0; c < NSP; c++) muS[s][q][c] += gS[c];
                 } else {
 #pragma unroll
                     for (int c = 0; c < UD; c++) gy[c] = P(0);
                 }
 #pragma unroll
-                for (int c = 0; c < UD; c++) lam[p][c] += gy[c];
+                for (int c = 0; c < UD; c++) lam[s][q][c] += gy[c];
 #pragma unroll
                 for (int l = 0; l < ST; l++)
-                    if (l < s && rk_a<ALG>(s, l) != P(0)) {
+                    if (l < st && rk_a<ALG>(st, l) != P(0)) {
 #pragma unroll
-                        for (int c = 0; c < UD; c++) kb[l][p][c] = fma(h * rk_a<ALG>(s, l), gy[c], kb[l][p][c]);
+                        for (int c = 0; c < UD; c++) kb[l][s][q][c] = fma(h[s] * rk_a<ALG>(st, l), gy[c], kb[l][s][q][c]);
                     }
             }
         }
     }
-    if (mine) {
+    MPGOS_PB_EACH(s, q) {
+        if (C.has(s, q)) {
+            const unsigned u = C.unit(s, q);
 #pragma unroll
-        for (int p = 0; p < PAIRS; p++) {
+            for (int c = 0; c < UD; c++) C.row(A.lam, c)[u] = lam[s][q][c];
 #pragma unroll
-            for (int c = 0; c < UD; c++) C.row(A.lam, c)[C.at(p)] = lam[p][c];
+            for (int c = 0; c < NUP; c++) C.row(A.gU, c)[u] = muU[s][q][c];
 #pragma unroll
-            for (int c = 0; c < NUP; c++) C.row(A.gU, c)[C.at(p)] = muU[p][c];
-#pragma unroll
-            for (int c = 0; c < NSP; c++) C.row(A.gSp, c)[C.at(p)] = muS[p][c];
+            for (int c = 0; c < NSP; c++) C.row(A.gSp, c)[u] = muS[s][q][c];
         }
     }
 }
+#undef MPGOS_PB_EACH
 
-template <class Sys, int ALG, int PAIRS>
-__global__ void __launch_bounds__(kMfmaSystems * 256 / PAIRS) pb_replay_mfma_kernel(Args<Sys, double> a, AdjArgs<Sys> A, int r)
+template <class Sys, int ALG, int NSL, int TT>
+__global__ void __launch_bounds__(512, 2) pb_replay_kernel(Args<Sys, double> a, AdjArgs<Sys> A, int r)
 {
-    pb_replay_mfma_body<Sys, ALG, PAIRS>(a, A, r);
+    pb_replay_body<Sys, ALG, NSL, TT>(a, A, r);
 }
 
-template <class Sys, int ALG, int PAIRS>
-__global__ void __launch_bounds__(kMfmaSystems * 256 / PAIRS) pb_sweep_mfma_kernel(Args<Sys, double> a, AdjArgs<Sys> A, int r)
+template <class Sys, int ALG, int NSL, int TT>
+__global__ void __launch_bounds__(512, 2) pb_sweep_kernel(Args<Sys, double> a, AdjArgs<Sys> A, int r)
 {
-    pb_sweep_mfma_body<Sys, ALG, PAIRS>(a, A, r);
+    pb_sweep_body<Sys, ALG, NSL, TT>(a, A, r);
 }
 
 // Outputs of the dense-contraction reverse pass, one thread per unit: systems

@@ -55,12 +55,13 @@ __host__ __device__ constexpr int dense_pairs(int UPS) { return ((UPS + 8 * kDen
 __host__ __device__ constexpr int dense_row(int UPS) { return dense_pairs(UPS) * 8 + 2; }
 __host__ __device__ constexpr size_t dense_matrix_size(int UPS) { return (size_t)dense_tiles(UPS) * dense_pairs(UPS) * 128; }
 
-// The pair-tiled copy of the dense coupling matrices: for matrix i, tile t,
-// column-block pair cp, lane l and j in {0, 1},
+// The pair-tiled copy of the dense coupling matrices (of their transposes for
+// the adjoint sweep): for matrix i, tile t, column-block pair cp, lane l and j
+// in {0, 1},
 //   Mt[(((i * tiles + t) * pairs + cp) * 64 + l) * 2 + j] = M_i[row + col * UPS],
 //   row = 16 t + l % 16, col = 4 (2 cp + j) + l / 16,
 // and -0 where row or col lies outside the matrix.
-template <int Unused = 0>
+template <bool TRANSPOSED>
 __global__ void tile_pair_matrix(const double* M, double* Mt, int UPS, int NC)
 {
     const int tiles = dense_tiles(UPS), pairs = dense_pairs(UPS);
@@ -72,7 +73,8 @@ __global__ void tile_pair_matrix(const double* M, double* Mt, int UPS, int NC)
     const int cp = (int)(r % pairs); r /= pairs;
     const int t = (int)(r % tiles);
     const int i = (int)(r / tiles);
-    const int row = t * 16 + (l & 15), col = 4 * (2 * cp + j) + (l >> 4);
+    int row = t * 16 + (l & 15), col = 4 * (2 * cp + j) + (l >> 4);
+    if (TRANSPOSED) { const int x = row; row = col; col = x; }
     Mt[k] = row < UPS && col < UPS ? M[(size_t)i * UPS * UPS + row + (size_t)col * UPS] : -0.0;
 }
 

@@ -55,24 +55,6 @@ __device__ __forceinline__ void lds_barrier()
 }
 
 constexpr int kMaxBlock = 1024;
-constexpr int kMfmaSystems = 8;          // systems per workgroup of the dense-contraction reverse pass
-constexpr int kMfmaPairs = 4;            // its pairs per lane (2 * UPS threads)
-
-// LDS of the dense-contraction reverse pass: the B operand (coupling terms) and the
-// contraction results, one row of UPS + 2 doubles per (coupling, block
-// system).  A wave's writes and reads of one system's consecutive units fall
-// in consecutive banks; rows 4 banks apart (UPS a multiple of 16) put the B
-// reads of a column block (4 columns x 4 systems, two columns per half-wave)
-// in 8 distinct bank pairs per half-wave and spread the result stores (4
-// systems x 16 rows of a tile) evenly over the 32 banks (UPS + 4, 8 banks
-// apart, stored them 4 ways conflicting: twice the measured bank conflicts,
-// 1.4 % slower).
-__host__ __device__ constexpr int mfma_row(int UPS) { return UPS + 2; }
-__host__ __device__ inline size_t mfma_index(int i, int s, int u, int UPS)
-{
-    return ((size_t)i * kMfmaSystems + s) * mfma_row(UPS) + u;
-}
-
 enum Coupling { kLaneCoupling = 0, kDenseCoupling = 1 };
 
 // CP: precision of the step size, tolerances and controller (FP64 in the
@@ -219,220 +201,6 @@ struct Unit {
         }
     }
 };
-
-// Dense contraction of the coupling terms of the block's systems: for every
-// coupling i, unit u and system s < SPB (at most 8),
-//   coup[mfma_index(i, s, u)] = sum_col M_i[u + col * UPS] * cptB[mfma_index(i, s, col)]
-// accumulated in column order, on v_mfma_f64_4x4x4f64 (called by every lane of
-// the workgroup: the instruction needs all 64 lanes of a wave; UPS is a
-// multiple of 16).  The instruction computes four independent
-// 4 x 4 x 4 products per instruction (block b = lanes with (lane / 4) % 4 == b:
-// A[i][k] in lane i + 4b + 16k, B[k][j] in lane j + 4b + 16k, D[i][j] in lane
-// j + 4b + 16i) and accumulates its four products as a fused multiply-add
-// chain in k order (both probed on the MI355X).  The four blocks take the four
-// 4-row slices of a 16-unit tile against the same 4 systems, so the A operand
-// is lane (row = lane % 16, column = lane / 16) and every B column is a system:
-// two chains per tile (systems 0..3 and 4..7, independent, so one tile per
-// pass keeps two in flight).  Output (unit 4 ((lane / 4) % 4) + lane / 16 of
-// the tile, system lane % 4 (+ 4)) in one register per chain.
-//
-// The M tile values of a pass stream from L2 (a 256-unit matrix is 512 KiB) in
-// groups of G column blocks.  GLOBAL_M: M is in global memory, read with
-// global loads (a generic pointer gives flat loads, which also count as LDS
-// operations, so the wait for a group's B operands from LDS would wait for all
-// of its M loads too); otherwise M is in LDS.  Mt: the pair-tiled copy of M
-// (tile_pair_matrix), read instead of M; Ml, ldsPairs: the leading ldsPairs
-// column-block pairs of every tile of Mt, copied into LDS.  TPW: the tiles a
-// wave contracts together when the launch gives every wave exactly TPW tiles
-// (2 * UPS threads at TPW = 2).
-template <int NC, bool GLOBAL_M = true, int G = 8, int TPW = 1>
-__device__ __forceinline__ void mfma_contract44(const double* M, const double* cptB, double* coup, int UPS, int SPB,
-                                                const double* Mt = nullptr, const double* Ml = nullptr, int ldsPairs = 0)
-{
-    using GPtr = const __attribute__((address_space(1))) double*;
-    struct alignas(16) Pair { double x, y; };
-    using GP = const __attribute__((address_space(1))) Pair*;
-    using LP = const __attribute__((address_space(3))) Pair*;
-    const int l = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int nw = blockDim.x >> 6;
-    const int tiles = UPS >> 4;
-    const int r16 = l & 15, k4 = l >> 4, sys = l & 3;
-    const int drow = 4 * ((l >> 2) & 3) + (l >> 4);
-    const int blocks = UPS >> 2;                        // a multiple of G (UPS is a multiple of 32)
-    const size_t colStride = (size_t)4 * UPS;
-    const int RS = mfma_row(UPS);
-    auto store = [&](int i, int t, double acc0, double acc1) {
-        if (sys < SPB) coup[mfma_index(i, sys, t * 16 + drow, UPS)] = acc0;
-        if (sys + 4 < SPB) coup[mfma_index(i, sys + 4, t * 16 + drow, UPS)] = acc1;
-    };
-    // pair-tiled copy (tile_pair_matrix): one 16-byte load per lane brings the
-    // lane's A values of two column blocks, half the vector-memory
-    // instructions of column-major reads.  Per tile, row and system the MFMAs
-    // run in column order, as in the column-major loop at the end.
-    if (GLOBAL_M && Mt && TPW > 1 && tiles == TPW * nw) {
-        // every tile of the wave (w, w + nw, ...) at once, G / TPW column
-        // blocks per tile and group: one B read per column block and chain
-        // serves all of them, and the 2 TPW accumulator chains are
-        // independent.  The leading ldsPairs pairs of every tile (a multiple
-        // of G / (2 TPW)) come from the workgroup's LDS copy (Ml, same
-        // layout), which takes their loads off the vector-memory path; the
-        // global groups are read two buffers deep, the first during the LDS
-        // part.
-        constexpr int TT = TPW > 1 ? TPW : 2;
-        constexpr int GB = G / TT;                      // column blocks per tile and group
-        static_assert(GB % 2 == 0, "whole pairs per group");
-        double res[Pos<NC>::value][TT][2];
-#pragma unroll
-        for (int i = 0; i < NC; i++) {
-            const double* Bi = cptB + mfma_index(i, sys, k4, UPS);
-            double (&acc)[TT][2] = res[i];
-#pragma unroll
-            for (int k = 0; k < TT; k++) acc[k][0] = acc[k][1] = 0.0;
-            auto group = [&](const double (*a)[GB], int c0) {
-#pragma unroll
-                for (int d = 0; d < GB; d++) {
-                    const double b0 = Bi[(c0 + d) * 4], b1 = Bi[(c0 + d) * 4 + 4 * RS];
-#pragma unroll
-                    for (int k = 0; k < TT; k++) {
-                        acc[k][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[k][d], b0, acc[k][0], 0, 0, 0);
-                        acc[k][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[k][d], b1, acc[k][1], 0, 0, 0);
-                    }
-                }
-            };
-            const Pair* At = reinterpret_cast<const Pair*>(Mt) + ((size_t)i * tiles + w) * (size_t)blocks * 32 + l;
-            const size_t gs = (size_t)nw * blocks * 32;          // the wave's next tile
-            auto load = [&](double (*a)[GB], int c0) {
-#pragma unroll
-                for (int k = 0; k < TT; k++)
-#pragma unroll
-                    for (int d = 0; d < GB; d += 2) {
-                        const GP q = (GP)(At + k * gs + (size_t)((c0 + d) >> 1) * 64);
-                        a[k][d] = q->x;
-                        a[k][d + 1] = q->y;
-                    }
-            };
-            const int cg = Ml ? 2 * ldsPairs : 0;
-            const int n = (blocks - cg) / GB;
-            double a0[TT][GB], a1[TT][GB];
-            if (n > 0) load(a0, cg);
-            if (Ml) {
-                const Pair* Lt = reinterpret_cast<const Pair*>(Ml) + ((size_t)i * tiles + w) * (size_t)ldsPairs * 64 + l;
-                const size_t ls = (size_t)nw * ldsPairs * 64;
-                for (int cp = 0; cp < ldsPairs; cp += GB / 2) {
-                    double a[TT][GB];
-#pragma unroll
-                    for (int k = 0; k < TT; k++)
-#pragma unroll
-                        for (int d = 0; d < GB; d += 2) {
-                            const LP q = (LP)(Lt + k * ls + (size_t)(cp + (d >> 1)) * 64);
-                            a[k][d] = q->x;
-                            a[k][d + 1] = q->y;
-                        }
-                    group(a, 2 * cp);
-                }
-            }
-            if (n > 0) {
-                // every load in the loop body is unconditional, so the wait
-                // before a group's MFMAs counts only that group's loads
-                int g = 0;
-                for (; g + 2 < n; g += 2) {
-                    load(a1, cg + (g + 1) * GB);
-                    group(a0, cg + g * GB);
-                    load(a0, cg + (g + 2) * GB);
-                    group(a1, cg + (g + 1) * GB);
-                }
-                if (g + 1 < n) {
-                    load(a1, cg + (g + 1) * GB);
-                    group(a0, cg + g * GB);
-                    group(a1, cg + (g + 1) * GB);
-                } else {
-                    group(a0, cg + g * GB);
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NC; i++)
-#pragma unroll
-            for (int k = 0; k < TT; k++) store(i, w + k * nw, res[i][k][0], res[i][k][1]);
-        return;
-    }
-    if (GLOBAL_M && Mt) {
-        // one tile at a time, G column blocks per group (coup and cptB are
-        // distinct here)
-        for (int t = w; t < tiles; t += nw) {
-#pragma unroll
-            for (int i = 0; i < NC; i++) {
-                const double* Bi = cptB + mfma_index(i, sys, k4, UPS);
-                const Pair* At = reinterpret_cast<const Pair*>(Mt + ((size_t)i * tiles + t) * (size_t)blocks * 64) + l;
-                double acc0 = 0.0, acc1 = 0.0;          // systems 0..3, 4..7
-                for (int c0 = 0; c0 < blocks; c0 += G) {
-                    double a0[G];
-#pragma unroll
-                    for (int d = 0; d < G; d += 2) {
-                        const GP q = (GP)(At + (size_t)((c0 + d) >> 1) * 64);
-                        a0[d] = q->x;
-                        a0[d + 1] = q->y;
-                    }
-#pragma unroll
-                    for (int d = 0; d < G; d++) {
-                        const double b0 = Bi[(c0 + d) * 4], b1 = Bi[(c0 + d) * 4 + 4 * RS];
-                        acc0 = __builtin_amdgcn_mfma_f64_4x4x4f64(a0[d], b0, acc0, 0, 0, 0);
-                        acc1 = __builtin_amdgcn_mfma_f64_4x4x4f64(a0[d], b1, acc1, 0, 0, 0);
-                    }
-                }
-                store(i, t, acc0, acc1);
-            }
-        }
-        return;
-    }
-    // one 16-unit tile per pass; its two system halves are two independent chains
-    for (int t = w; t < tiles; t += nw) {
-#pragma unroll
-        for (int i = 0; i < NC; i++) {
-            const double* Ai = M + (size_t)i * UPS * UPS + t * 16 + r16 + (size_t)k4 * UPS;
-            const double* Bi = cptB + mfma_index(i, sys, k4, UPS);
-            auto ldA = [&](int blk) -> double {
-                if constexpr (GLOBAL_M) return *(GPtr)(Ai + (size_t)blk * colStride);
-                else return Ai[(size_t)blk * colStride];
-            };
-            double acc0 = 0.0, acc1 = 0.0;              // systems 0..3, 4..7
-            for (int c0 = 0; c0 < blocks; c0 += G) {
-                double a0[G];
-#pragma unroll
-                for (int d = 0; d < G; d++) a0[d] = ldA(c0 + d);
-#pragma unroll
-                for (int d = 0; d < G; d++) {
-                    const double b0 = Bi[(c0 + d) * 4], b1 = Bi[(c0 + d) * 4 + 4 * RS];
-                    acc0 = __builtin_amdgcn_mfma_f64_4x4x4f64(a0[d], b0, acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f64_4x4x4f64(a0[d], b1, acc1, 0, 0, 0);
-                }
-            }
-            store(i, t, acc0, acc1);
-        }
-    }
-}
-
-// The pair-tiled copy of the dense coupling matrices read by mfma_contract44:
-// for matrix i, 16-unit tile t, column-block pair cp, lane l and j in {0, 1},
-//   Mt[(((i * tiles + t) * blocks / 2 + cp) * 64 + l) * 2 + j]
-//     = M_i[t * 16 + l % 16 + (4 * (2 cp + j) + l / 16) * UPS],
-// i.e. the A operand of lane l for column blocks 2 cp and 2 cp + 1 side by
-// side (the same values, so the contraction's results are unchanged).
-template <int Unused = 0>
-__global__ void tile_pair_matrix_old(const double* M, double* Mt, int UPS, int NC)
-{
-    const size_t n = (size_t)NC * UPS * UPS;
-    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const int tiles = UPS >> 4, pairs = UPS >> 3;
-    const int j = (int)(k & 1), l = (int)((k >> 1) & 63);
-    size_t r = k >> 7;
-    const int cp = (int)(r % pairs); r /= pairs;
-    const int t = (int)(r % tiles);
-    const int i = (int)(r / tiles);
-    Mt[k] = M[(size_t)i * UPS * UPS + t * 16 + (l & 15) + (size_t)(4 * (2 * cp + j) + (l >> 4)) * UPS];
-}
 
 // One workgroup = SPB systems: lane t owns unit t % UPS of block system t / UPS,
 // so global accesses to unit-scope arrays are coalesced.

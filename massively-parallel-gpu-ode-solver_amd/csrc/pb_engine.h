@@ -90,8 +90,8 @@ public:
     double* recX = nullptr; double* recT = nullptr; double* recH = nullptr; double* seg = nullptr; double* cMatT = nullptr;
     double* stg = nullptr; double* gSp = nullptr;
     double* cTile = nullptr;                // pair-tiled copies (tile_pair_matrix) of the dense coupling matrices
-    double* cTileR = nullptr; double* cTileT = nullptr;   // and for the adjoint: of them, of their transposes
-    size_t cTileRN = 0, cTileTN = 0;
+    double* cTileT = nullptr;               // and of their transposes (adjoint sweep)
+    size_t cTileTN = 0;
     size_t recXn = 0, recTn = 0, recHn = 0, segn = 0, cMatTn = 0, stgn = 0, gSpn = 0;
     int adjK = 0, adjCap = 0, adjStepCap = 0;
 
@@ -99,7 +99,7 @@ public:
     {
         if (strm) (void)hipStreamSynchronize(strm);
         lamB.release(); gUB.release(); gSB.release();
-        for (double* q : {recX, recT, recH, seg, cMatT, stg, gSp, cTile, cTileR, cTileT})
+        for (double* q : {recX, recT, recH, seg, cMatT, stg, gSp, cTile, cTileT})
             if (q) (void)hipFree(q);
         for (auto* b : {&X, &uPAR, &uACC, &TD, &T, &sPAR, &sACC, &strength, &DOt, &DOx, &gPAR, &cMat}) b->release();
         for (auto* b : {&uACCi, &sACCi, &DOidx, &gPARi, &cIndex, &status}) b->release();
@@ -478,21 +478,31 @@ public:
         return lds_layout<Sys, P, KAHAN>(spb, UPS, sharedGlobals, sm, cMatSize).total;
     }
 
-    // Dense-contraction form.  A workgroup's LDS beyond its coupling terms takes
-    // the leading column-block pairs of every tile, as many as fit next to the
-    // other workgroups that its CU is to hold (4096 x 100 units, 8 systems: 6.2 ms
-    // with 4 of 14 pairs and three workgroups per CU, 7.8 ms with all pairs and
-    // one; 1000 x 100, 4 systems: 4.6 ms with all, 5.4 ms with none).
+    // The leading column-block pairs of every tile that a workgroup of the dense
+    // form keeps in LDS: as many as fit beside its other data (base bytes) and
+    // the other workgroups that its CU is to hold (4096 x 100 units, 8 systems:
+    // 6.2 ms with 4 of 14 pairs and three workgroups per CU, 7.8 ms with all
+    // pairs and one; 1000 x 100, 4 systems: 4.6 ms with all, 5.4 ms with none).
+    int dense_lds_pairs(size_t base, int perCu) const
+    {
+        const size_t perPair = (size_t)NC * dense_tiles(UPS) * 64 * 16, room = ldsMax / (size_t)std::max(1, perCu);
+        const int lp = room > base ? (int)std::min<size_t>((room - base) / perPair, (size_t)dense_pairs(UPS)) : 0;
+        return lp - lp % kDenseGroup;
+    }
+    // workgroups of the reverse kernels per CU (2 wavefronts per SIMD)
+    int dense_reverse_per_cu() const
+    {
+        const int tiles = dense_tiles(UPS);
+        return tiles > 8 ? 1 : std::max(1, 8 / tiles);
+    }
+
     template <int NSL, int TT, bool REC, bool QUIET>
     int launch_dense(Args<Sys, double>& a)
     {
         constexpr int spb = 4 * NSL;
         auto bytes = [&](int pairs) { return dense_layout<DenseScope<Sys>, NC, NGP, NiGP>(spb, UPS, sharedGlobals, pairs).total; };
         const int grid = (NS + spb - 1) / spb;
-        const int perCu = std::max(1, std::min((grid + cus - 1) / cus, NSL == 1 ? dense_per_cu() : std::max(1, dense_per_cu() * 3 / 4)));
-        const size_t perPair = (size_t)NC * dense_tiles(UPS) * 64 * 16, room = ldsMax / perCu;
-        int lp = room > bytes(0) ? (int)std::min<size_t>((room - bytes(0)) / perPair, (size_t)dense_pairs(UPS)) : 0;
-        lp -= lp % kDenseGroup;
+        const int lp = dense_lds_pairs(bytes(0), std::min((grid + cus - 1) / cus, NSL == 1 ? dense_per_cu() : std::max(1, dense_per_cu() * 3 / 4)));
         a.SPB = spb;
         a.ldsPairs = lp;
         a.cTile = cTile;
@@ -515,7 +525,7 @@ public:
     {
         // the matrices in column-block pairs per lane, refreshed every Solve
         // (a kernel on the solver's stream, so graph capture records it)
-        if (int rc = tile_pairs((const double*)cMat.d, cTile)) return rc;
+        if (int rc = tile_pairs<false>(cTile)) return rc;
         auto fits = [&](int spb) { return dense_layout<DenseScope<Sys>, NC, NGP, NiGP>(spb, UPS, sharedGlobals, 0).total <= ldsMax; };
         if (!fits(4)) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
         const bool four = dense_four() || !fits(8);
@@ -566,20 +576,13 @@ public:
         return MPGOS_E_ARG;
     }
 
-    // The pair-tiled copy of the NC full matrices at src (column-major),
-    // written by a kernel on the solver's stream.
-    int tile_pairs(const double* src, double* dst)
+    // The pair-tiled copy of the NC full matrices on the device (or of their
+    // transposes), written by a kernel on the solver's stream.
+    template <bool TRANSPOSED>
+    int tile_pairs(double* dst)
     {
         const size_t n = (size_t)NC * dense_matrix_size(UPS);
-        hipLaunchKernelGGL(tile_pair_matrix<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, strm, src, dst, UPS, NC);
-        MPGOS_HIP_TRY(hipGetLastError());
-        return MPGOS_OK;
-    }
-    int tile_pairs_reverse(const double* src, double*& dst, size_t& have)
-    {
-        const size_t n = (size_t)NC * UPS * UPS;
-        if (int rc = grow_device(dst, have, n, "tiled coupling matrix")) return rc;
-        hipLaunchKernelGGL(tile_pair_matrix_old<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, strm, src, dst, UPS, NC);
+        hipLaunchKernelGGL(tile_pair_matrix<TRANSPOSED>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, strm, (const double*)cMat.d, dst, UPS, NC);
         MPGOS_HIP_TRY(hipGetLastError());
         return MPGOS_OK;
     }
@@ -660,14 +663,18 @@ public:
             const size_t NU = (size_t)NS * UPS;
             MPGOS_HIP_TRY(hipStreamSynchronize(strm));
             if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
-            const int cpl = couplingKernel != 1 && dense_request_valid() ? kDenseCoupling : kLaneCoupling;
-            const int ST = algorithm == MPGOS_RK4 ? 4 : 6;
-            int rc;
-            if (cpl == kDenseCoupling) {
-                if ((rc = grow_device(stg, stgn, (size_t)adjK * ST * (UD + NC) * NU, "stage buffer"))) return rc;
-            } else if ((rc = grow_device(seg, segn, (size_t)adjK * UD * NU, "segment buffer"))) {
-                return rc;
+            lastForm = coupling_form();
+            if constexpr (NC > 0) {
+                if (lastForm == kDenseCoupling) {
+                    const int rc = reverse_dense();
+                    // what only the automatic choice sent here fits the lane
+                    // form's smaller segment buffer
+                    if (rc != MPGOS_E_MEMORY || dense_request_valid()) return rc;
+                    lastForm = kLaneCoupling;
+                }
             }
+            int rc;
+            if ((rc = grow_device(seg, segn, (size_t)adjK * UD * NU, "segment buffer"))) return rc;
             // transposed coupling matrices in the stored form (from the host mirror)
             std::vector<double> mt((size_t)NC * cMatSize, 0.0);
             for (int i = 0; i < NC; i++)
@@ -681,48 +688,8 @@ public:
             Args<Sys, double> a = make_args();
             a.recX = recX; a.recT = recT; a.recH = recH; a.recK = adjK; a.recCkCap = adjCap; a.recStepCap = adjStepCap;
             AdjArgs<Sys> A;
-            A.seg = seg; A.stg = stg; A.gSp = nullptr; A.lam = lamB.d; A.gU = gUB.d; A.gS = gSB.d; A.cMatT = cMatT;
+            A.seg = seg; A.stg = nullptr; A.gSp = nullptr; A.lam = lamB.d; A.gU = gUB.d; A.gS = gSB.d; A.cMatT = cMatT;
             A.cTileT = nullptr;
-            lastForm = cpl;
-            if (cpl == kDenseCoupling) {
-                // one replay and one sweep launch per round; rounds = the largest
-                // segment count of a system whose record did not overflow
-                a.SPB = kMfmaSystems;
-                const size_t lds = reverse_mfma_layout<Sys>(UPS).total;
-                if (lds > ldsMax) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
-                if ((rc = grow_device(gSp, gSpn, (size_t)(NSP > 0 ? NSP : 1) * NU, "system-parameter partials"))) return rc;
-                A.gSp = gSp;
-                std::vector<long long> nh((size_t)NS);
-                std::vector<int> sh((size_t)NS);
-                MPGOS_HIP_TRY(hipMemcpy(nh.data(), nacc.d, nh.size() * sizeof(long long), hipMemcpyDeviceToHost));
-                MPGOS_HIP_TRY(hipMemcpy(sh.data(), status.d, sh.size() * sizeof(int), hipMemcpyDeviceToHost));
-                int rounds = 0;
-                for (int i = 0; i < nActive && i < NS; i++)
-                    if ((sh[i] & MPGOS_STATUS_CHECKPOINT_OVERFLOW) == 0) {
-                        const long long nseg = (nh[i] + adjK - 1) / adjK;
-                        if (nseg > rounds) rounds = (int)nseg;
-                    }
-                const int threads = kMfmaSystems * UPS / kMfmaPairs;
-                const int grid = NS / kMfmaSystems + (NS % kMfmaSystems == 0 ? 0 : 1);
-                const int fgrid = (int)((NU + 255) / 256);
-                MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-                if ((rc = tile_pairs_reverse((const double*)cMat.d, cTileR, cTileRN)) || (rc = tile_pairs_reverse(cMatT, cTileT, cTileTN))) return rc;
-                a.cTile = cTileR;
-                A.cTileT = cTileT;
-                for (int r = 0; r < rounds; r++) {
-                    if (algorithm == MPGOS_RK4) {
-                        hipLaunchKernelGGL((pb_replay_mfma_kernel<Sys, MPGOS_RK4, kMfmaPairs>), dim3(grid), dim3(threads), lds, strm, a, A, r);
-                        hipLaunchKernelGGL((pb_sweep_mfma_kernel<Sys, MPGOS_RK4, kMfmaPairs>), dim3(grid), dim3(threads), lds, strm, a, A, r);
-                    } else {
-                        hipLaunchKernelGGL((pb_replay_mfma_kernel<Sys, MPGOS_RKCK45, kMfmaPairs>), dim3(grid), dim3(threads), lds, strm, a, A, r);
-                        hipLaunchKernelGGL((pb_sweep_mfma_kernel<Sys, MPGOS_RKCK45, kMfmaPairs>), dim3(grid), dim3(threads), lds, strm, a, A, r);
-                    }
-                }
-                hipLaunchKernelGGL((pb_reverse_finish_kernel<Sys>), dim3(fgrid), dim3(256), 0, strm, a, A);
-                MPGOS_HIP_TRY(hipGetLastError());
-                MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
-                return MPGOS_OK;
-            }
             const size_t lds = reverse_layout<Sys>(SPB, UPS).total;
             if (lds > ldsMax) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
             const int threads = ((SPB * UPS + 63) / 64) * 64;
@@ -738,6 +705,66 @@ public:
             MPGOS_HIP_TRY(hipGetLastError());
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;
+        }
+    }
+
+    // Reverse pass in the dense-contraction form: one replay and one sweep
+    // launch per round; rounds = the largest segment count of a system whose
+    // record did not overflow.
+    int reverse_dense()
+    {
+        const size_t NU = (size_t)NS * UPS;
+        const int ST = algorithm == MPGOS_RK4 ? 4 : 6;
+        int rc;
+        if ((rc = grow_device(stg, stgn, (size_t)adjK * ST * (UD + NC) * NU, "stage buffer")) ||
+            (rc = grow_device(gSp, gSpn, (size_t)(NSP > 0 ? NSP : 1) * NU, "system-parameter partials")) ||
+            (rc = grow_device(cTileT, cTileTN, (size_t)NC * dense_matrix_size(UPS), "tiled coupling matrix")))
+            return rc;
+        std::vector<long long> nh((size_t)NS);
+        std::vector<int> sh((size_t)NS);
+        MPGOS_HIP_TRY(hipMemcpy(nh.data(), nacc.d, nh.size() * sizeof(long long), hipMemcpyDeviceToHost));
+        MPGOS_HIP_TRY(hipMemcpy(sh.data(), status.d, sh.size() * sizeof(int), hipMemcpyDeviceToHost));
+        int rounds = 0;
+        for (int i = 0; i < nActive && i < NS; i++)
+            if ((sh[i] & MPGOS_STATUS_CHECKPOINT_OVERFLOW) == 0) {
+                const long long nseg = (nh[i] + adjK - 1) / adjK;
+                if (nseg > rounds) rounds = (int)nseg;
+            }
+        Args<Sys, double> a = make_args();
+        a.recX = recX; a.recT = recT; a.recH = recH; a.recK = adjK; a.recCkCap = adjCap; a.recStepCap = adjStepCap;
+        AdjArgs<Sys> A;
+        A.seg = nullptr; A.stg = stg; A.gSp = gSp; A.lam = lamB.d; A.gU = gUB.d; A.gS = gSB.d; A.cMatT = nullptr; A.cTileT = cTileT;
+        auto fits = [&](int spb) { return dense_layout<RevScope<Sys>, NC, 0, 0>(spb, UPS, 0, 0).total <= ldsMax; };
+        if (!fits(4)) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
+        MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
+        if ((rc = tile_pairs<false>(cTile)) || (rc = tile_pairs<true>(cTileT))) return rc;
+        a.cTile = cTile;
+        const bool four = dense_four() || !fits(8);
+        if (dense_tiles(UPS) > 8) { if (four) launch_reverse<1, 2>(a, A, rounds); else launch_reverse<2, 2>(a, A, rounds); }
+        else if (four) launch_reverse<1, 1>(a, A, rounds);
+        else launch_reverse<2, 1>(a, A, rounds);
+        hipLaunchKernelGGL((pb_reverse_finish_kernel<Sys>), dim3((unsigned)((NU + 255) / 256)), dim3(256), 0, strm, a, A);
+        MPGOS_HIP_TRY(hipGetLastError());
+        MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
+        return MPGOS_OK;
+    }
+    template <int NSL, int TT>
+    void launch_reverse(Args<Sys, double>& a, const AdjArgs<Sys>& A, int rounds)
+    {
+        constexpr int spb = 4 * NSL;
+        auto bytes = [&](int pairs) { return dense_layout<RevScope<Sys>, NC, 0, 0>(spb, UPS, 0, pairs).total; };
+        const int grid = (NS + spb - 1) / spb, threads = 64 * ((dense_tiles(UPS) + TT - 1) / TT);
+        a.SPB = spb;
+        a.ldsPairs = dense_lds_pairs(bytes(0), std::min((grid + cus - 1) / cus, dense_reverse_per_cu()));
+        const size_t lds = bytes(a.ldsPairs);
+        for (int r = 0; r < rounds; r++) {
+            if (algorithm == MPGOS_RK4) {
+                hipLaunchKernelGGL((pb_replay_kernel<Sys, MPGOS_RK4, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+                hipLaunchKernelGGL((pb_sweep_kernel<Sys, MPGOS_RK4, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+            } else {
+                hipLaunchKernelGGL((pb_replay_kernel<Sys, MPGOS_RKCK45, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+                hipLaunchKernelGGL((pb_sweep_kernel<Sys, MPGOS_RKCK45, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+            }
         }
     }
 

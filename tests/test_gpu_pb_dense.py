@@ -10,6 +10,7 @@ import pytest
 
 from mpgos import workloads as W
 from mpgos.enums import Algorithms
+from mpgos.perblock import PB, PBOption, PBProblemSolver
 from test_gpu_perblock import assert_pb_bitwise, run_pb_gpu
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +70,37 @@ def test_events_and_dense_output(oracle, ns, ups, ndo):
     assert_pb_bitwise(run_pb_gpu(s), ref, "automatic")
     if ns < 100:
         assert (ref["uACCi"] == 2).any() and (ref["T"] < s["TD"][1]).any()
+
+
+@pytest.mark.parametrize("ns,ups,off,K,alg", [(5, 1, 0, 3, Algorithms.RKCK45), (4, 13, 1, 5, Algorithms.RK4),
+                                              (9, 100, 2, 64, Algorithms.RKCK45), (6, 131, 0, 7, Algorithms.RK4),
+                                              (3, 256, 0, 9, Algorithms.RKCK45), (1027, 129, 3, 4, Algorithms.RKCK45),
+                                              (2053, 113, 0, 6, Algorithms.RKCK45)])
+def test_adjoint_equals_lane_form(ns, ups, off, K, alg):
+    """Reverse pass at the same edges: gradients bit for bit those of the
+    lane-per-pair form, a checkpoint interval that does not divide the steps."""
+    s = W.config4_ring(ns=ns, ups=ups, periods=1, algorithm=alg, system="ring_duffing_q")
+    end = 0.25 if ns > 100 else 1.0
+    s["TD"][1] = np.linspace(0.5 * end, end, ns)
+    s["n_active"] = ns - off
+    if alg == Algorithms.RK4:
+        s["options"]["dt0"] = 0.02
+    w = W.Stream(W.SEED, 320).normal(3 * ns * ups).reshape(3, -1)
+    print(f"adjoint {ns} x {ups} K={K} alg={int(alg)}", flush=True)
+    outs = []
+    for kernel in (1, 0):
+        p = PBProblemSolver("ring_duffing_q", ns, ups, alg)
+        try:
+            W.load_pb(p, s)
+            p.SolverOption(PBOption.CouplingKernel, kernel)
+            outs.append([np.array(x) for x in p.adjoint(w, K, 400 // K + 2, 400)])
+            p.SynchroniseFromDeviceToHost(PB.Status)
+            p.InsertSynchronisationPoint()
+            p.SynchroniseSolver()
+            assert not (p.host_array(PB.Status) & 16).any()
+        finally:
+            p.close()
+    for a, b in zip(*outs):
+        a, b = (x.reshape(x.shape[0], ns, -1)[:, :ns - off] for x in (a, b))
+        assert np.isfinite(a).all() and np.abs(a).max() > 0
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
