@@ -474,8 +474,9 @@ __device__ __forceinline__ double rk_a(int s, int l)
 // 24.6 -> 7.9 ms, one period of 300 x 256 25.6 -> 14.6, 4096 x 128 21.1 -> 14.6,
 // 4096 x 256 57.1 -> 51.9 ms against products through LDS with 8 systems per
 // workgroup; 1000 x 100 units 40.5 -> 3.4 ms against one lane per unit.
-template <class Sys, int NSL, int TT>
+template <class Sys, int NSL, int MT>
 struct DenseRev {
+    static constexpr int TT = dense_tt(MT);
     static constexpr int NC = Sys::NC, SPB = 4 * NSL, NTT = TimeTermsOf<Sys>::n, PER = 64 / SPB;
     using Scope = RevScope<Sys>;
     using Place = DensePlace<NSL, TT>;
@@ -485,6 +486,7 @@ struct DenseRev {
     Place at;
     bool active[NSL];
     int k[NSL], len[NSL];
+    double strength[NSL][Pos<NC>::value];
 
     // LDS, system scope and this round's segment of each system
     // (k = nseg - 1 - r, len steps; maxlen over the workgroup)
@@ -529,6 +531,8 @@ struct DenseRev {
         for (int s = 0; s < NSL; s++) {
             k[s] = sys[at.sys(s)].k;
             len[s] = active[s] ? sys[at.sys(s)].len : 0;
+#pragma unroll
+            for (int i = 0; i < NC; i++) strength[s][i] = sys[at.sys(s)].strength[i];
         }
         for (int i = threadIdx.x; i < 2 * cptStride; i += blockDim.x) cptBuf[i] = 0.0;   // padded units and absent systems stay zero
         dense_stage_matrix(Mt, lds + L.mt, NC, a.UPS, a.ldsPairs);
@@ -572,27 +576,30 @@ struct DenseRev {
         }
     }
     template <int N>
-    __device__ __forceinline__ void stage_terms(int stage, int s, const double (&tterm)[N][Pos<NTT>::value], double* tt) const
+    __device__ __forceinline__ void stage_terms(int stage, const double (&tterm)[N][Pos<NTT>::value], double (&tt)[NSL][Pos<NTT>::value]) const
     {
 #pragma unroll
-        for (int i = 0; i < NTT; i++) tt[i] = __shfl(tterm[stage / PER][i], (stage % PER) * SPB + at.sys(s));
+        for (int s = 0; s < NSL; s++)
+#pragma unroll
+            for (int i = 0; i < NTT; i++) tt[s][i] = __shfl(tterm[stage / PER][i], (stage % PER) * SPB + at.sys(s));
     }
 };
 
 #define MPGOS_PB_EACH(s, q) _Pragma("unroll") for (int s = 0; s < NSL; s++) _Pragma("unroll") for (int q = 0; q < TT; q++)
 
-template <class Sys, int ALG, int NSL, int TT>
+template <class Sys, int ALG, int NSL, int MT>
 __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A, int r)
 {
+    constexpr int TT = dense_tt(MT);
     using P = double;
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NUA = Sys::NUA, NiUA = Sys::NiUA;
     constexpr int NCp = Pos<NC>::value, NTT = TimeTermsOf<Sys>::n, ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC;
     using math::fma;
-    using R = DenseRev<Sys, NSL, TT>;
+    using R = DenseRev<Sys, NSL, MT>;
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
     const R C(a, a.cTile, mpgos_pb_lds, r);
     if (C.maxlen == 0) return;
-    DenseContraction<NC, NSL, TT> product(a.cTile, C.Ml, a.ldsPairs, a.UPS);
+    DenseContraction<Sys, NSL, MT> product(a.cTile, C.Ml, a.ldsPairs, a.UPS);
     const int RS = dense_row(a.UPS);
 
     int cIndex[NCp];
@@ -614,16 +621,14 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
     }
 
     int buf = 0;
-    P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value];
+    P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value], tt[NSL][Pos<NTT>::value];
     P t[NSL], h[NSL], tn[NSL], hn[NSL];
     // right-hand sides of the lane's units at (Y, T) plus the coupling terms of
     // stage st of step j; Y and the coupling values (M CPT)_u are kept.  The
     // barriers order LDS only, so the stage-buffer stores stay in flight.
     auto rhs = [&](int st, int j, P (*F)[TT][UD], P (*Y)[TT][UD]) {
-        P CPF[NSL][TT][NCp], v[NCp][NSL][TT], tt[NSL][Pos<NTT>::value];
+        P CPF[NSL][TT][NCp], v[NCp][NSL][TT];
         P* cpt = C.cptBuf + (size_t)buf * C.cptStride;
-#pragma unroll
-        for (int s = 0; s < NSL; s++) C.stage_terms(st, s, tterm, tt[s]);
         product.prefetch();
         MPGOS_PB_EACH(s, q) {
             if (j < C.len[s] && C.at.has(q)) {
@@ -645,12 +650,13 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
                 for (int c = 0; c < UD; c++) C.row(A.stg, base + c)[C.unit(s, q)] = Y[s][q][c];
             }
         }
+        if (st + 1 < ST) C.stage_terms(st + 1, tterm, tt);
         lds_barrier();
         product.run(cpt, v);
         MPGOS_PB_EACH(s, q) {
 #pragma unroll
             for (int i = 0; i < NC; i++)
-                Unit<Sys, P>::add(cIndex[i], C.sys[C.at.sys(s)].strength[i] * CPF[s][q][i], v[i][s][q], F[s][q]);
+                Unit<Sys, P>::add(cIndex[i], C.strength[s][i] * CPF[s][q][i], v[i][s][q], F[s][q]);
             if (j < C.len[s] && C.at.has(q)) {
                 const size_t base = ((size_t)j * ST + st) * SW;
 #pragma unroll
@@ -671,6 +677,7 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
         for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
         C.step_times(a, j + 1, tn, hn);                 // one step ahead
         C.template time_terms<ALG>(t, h, tterm);
+        C.stage_terms(0, tterm, tt);
         // the forward pass's stage arithmetic (pb_dense_body)
         P next[NSL][TT][UD], k[NSL][TT][UD], Y[NSL][TT][UD];
         if (ALG == MPGOS_RK4) {
@@ -723,19 +730,20 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
     }
 }
 
-template <class Sys, int ALG, int NSL, int TT>
+template <class Sys, int ALG, int NSL, int MT>
 __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A, int r)
 {
+    constexpr int TT = dense_tt(MT);
     using P = double;
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NSP = Sys::NSP, NUA = Sys::NUA, NiUA = Sys::NiUA;
     constexpr int NCp = Pos<NC>::value, NUPp = Pos<NUP>::value, NSPp = Pos<NSP>::value, NTT = TimeTermsOf<Sys>::n;
     constexpr int ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC;
     using math::fma;
-    using R = DenseRev<Sys, NSL, TT>;
+    using R = DenseRev<Sys, NSL, MT>;
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
     const R C(a, A.cTileT, mpgos_pb_lds, r);
     if (C.maxlen == 0) return;
-    DenseContraction<NC, NSL, TT> product(A.cTileT, C.Ml, a.ldsPairs, a.UPS);
+    DenseContraction<Sys, NSL, MT> product(A.cTileT, C.Ml, a.ldsPairs, a.UPS);
     const int RS = dense_row(a.UPS);
 
     int cIndex[NCp];
@@ -773,7 +781,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
     };
 
     int buf = 0;
-    P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value];
+    P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value], tt[NSL][Pos<NTT>::value];
     P t[NSL], h[NSL], tn[NSL], hn[NSL];
     C.step_times(a, C.maxlen - 1, tn, hn);
     fetch(C.maxlen - 1, ST - 1);
@@ -782,6 +790,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
         for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
         C.step_times(a, j - 1, tn, hn);                 // one step ahead
         C.template time_terms<ALG>(t, h, tterm);
+        C.stage_terms(ST - 1, tterm, tt);
         P kb[ST][NSL][TT][UD];
 #pragma unroll
         for (int st = 0; st < ST; st++)
@@ -791,10 +800,8 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
             }
 #pragma unroll
         for (int st = ST - 1; st >= 0; st--) {
-            P Y[NSL][TT][UD], kbCPF[NSL][TT][NCp], tt[NSL][Pos<NTT>::value], w[NCp][NSL][TT];
+            P Y[NSL][TT][UD], kbCPF[NSL][TT][NCp], w[NCp][NSL][TT];
             P* wb = C.cptBuf + (size_t)buf * C.cptStride;
-#pragma unroll
-            for (int s = 0; s < NSL; s++) C.stage_terms(st, s, tterm, tt[s]);
             MPGOS_PB_EACH(s, q) {
 #pragma unroll
                 for (int c = 0; c < UD; c++) Y[s][q][c] = ahead[s][q][c];
@@ -816,8 +823,8 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
 #pragma unroll
                         for (int c = 0; c < UD; c++)
                             if (c == cIndex[i]) g = kb[st][s][q][c];
-                        wb[(i * R::SPB + C.at.sys(s)) * RS + C.at.unit(q)] = y.strength[i] * cpf[i] * g;
-                        kbCPF[s][q][i] = y.strength[i] * ahead[s][q][UD + i] * g;
+                        wb[(i * R::SPB + C.at.sys(s)) * RS + C.at.unit(q)] = C.strength[s][i] * cpf[i] * g;
+                        kbCPF[s][q][i] = C.strength[s][i] * ahead[s][q][UD + i] * g;
                     }
                 }
             }
@@ -858,6 +865,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
                         for (int c = 0; c < UD; c++) kb[l][s][q][c] = fma(h[s] * rk_a<ALG>(st, l), gy[c], kb[l][s][q][c]);
                     }
             }
+            if (st > 0) C.stage_terms(st - 1, tterm, tt);
         }
     }
     MPGOS_PB_EACH(s, q) {
@@ -874,16 +882,16 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
 }
 #undef MPGOS_PB_EACH
 
-template <class Sys, int ALG, int NSL, int TT>
+template <class Sys, int ALG, int NSL, int MT>
 __global__ void __launch_bounds__(512, 2) pb_replay_kernel(Args<Sys, double> a, AdjArgs<Sys> A, int r)
 {
-    pb_replay_body<Sys, ALG, NSL, TT>(a, A, r);
+    pb_replay_body<Sys, ALG, NSL, MT>(a, A, r);
 }
 
-template <class Sys, int ALG, int NSL, int TT>
+template <class Sys, int ALG, int NSL, int MT>
 __global__ void __launch_bounds__(512, 2) pb_sweep_kernel(Args<Sys, double> a, AdjArgs<Sys> A, int r)
 {
-    pb_sweep_body<Sys, ALG, NSL, TT>(a, A, r);
+    pb_sweep_body<Sys, ALG, NSL, MT>(a, A, r);
 }
 
 // Outputs of the dense-contraction reverse pass, one thread per unit: systems

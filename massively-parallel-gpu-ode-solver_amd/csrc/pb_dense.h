@@ -45,6 +45,11 @@ namespace pb {
 using systems::TimeTermsOf;
 
 constexpr int kDenseMaxUnits = 256;
+// Kernels for up to MT = 4, 8 and 16 tiles: one tile per wavefront up to 8, else
+// two, so at most 8 wavefronts; the wavefronts per SIMD that they aim at.
+__host__ __device__ constexpr int dense_tt(int MT) { return MT > 8 ? 2 : 1; }
+__host__ __device__ constexpr int dense_waves(int MT) { return MT / dense_tt(MT); }
+__host__ __device__ constexpr int dense_per_simd(int NSL, int MT) { return MT > 8 ? 2 : (MT > 4 ? 4 : 5) - NSL; }
 constexpr int kDenseGroup = 2;             // column-block pairs per tile and load group
 __host__ __device__ constexpr int dense_tiles(int UPS) { return (UPS + 15) >> 4; }
 // column-block pairs of a tile, whole load groups
@@ -131,10 +136,74 @@ struct DensePlace {
 // acc[i][s][k] = sum over columns of M_i of the wave's tiles against the coupling
 // terms of the workgroup's systems (cptB: rows [coupling][system]), accumulated
 // in column order.  Mt: tiled matrices in global memory, Ml: their leading
-// ldsPairs pairs in LDS.  The wave's loads of the first global group are issued
-// by prefetch() before the barrier.
+// ldsPairs pairs in LDS.
+//
+// One matrix, one tile per wave (up to 128 units) and few enough results per
+// lane: the tile stays in registers (4 to 32 column blocks of one double per
+// lane) for the whole Solve, and a stage reads only the coupling terms from
+// LDS.  One period, from the streamed form: 1000 x 64 units 1.56 -> 1.36 ms,
+// 2000 x 7 0.92 -> 0.81, 4096 x 64 3.0 -> 2.7, 1024 x 128 2.7 -> 2.6, 1000 x 100
+// 2.4 (unchanged); the adjoint of 1024 x 128 units over two periods 12.2 -> 11.1 ms.
+// What remains of a step of 1000 x 100 units (6.7 us): the products of two
+// wavefronts on a SIMD (6 x 28 x 2 of 16 cycles, 2.4 us), right-hand sides,
+// barriers and the controller (2.9 us without any products), and the first reads
+// of each stage.
+template <class Sys, int NSL, int MT>
+__host__ __device__ constexpr bool dense_resident() { return Sys::NC == 1 && dense_tt(MT) == 1 && NSL * Sys::UD <= 4; }
+
+template <int NSL, int MT>
+struct ResidentContraction {
+    using LD = const __attribute__((address_space(3))) double*;
+    static constexpr int kBlocks = 4 * MT;   // column blocks of 16 MT units
+    double a[kBlocks];
+    int nb, RS, l;
+
+    __device__ __forceinline__ ResidentContraction(const double* Mt, const double*, int, int UPS)
+    {
+        l = threadIdx.x & 63;
+        nb = 2 * dense_pairs(UPS);           // a multiple of 4
+        RS = dense_row(UPS);
+        const double2* At = reinterpret_cast<const double2*>(Mt) + (size_t)wave_index() * dense_pairs(UPS) * 64 + l;
+#pragma unroll
+        for (int p = 0; p < kBlocks / 2; p++) {
+            const double2 v = 2 * p < nb ? At[p * 64] : double2{0.0, 0.0};
+            a[2 * p] = v.x;
+            a[2 * p + 1] = v.y;
+        }
+    }
+    __device__ __forceinline__ void prefetch() {}
+    __device__ __forceinline__ void run(const double* cptB, double (&acc)[1][NSL][1]) const
+    {
+        const LD B = (LD)(cptB + (l & 3) * RS + (l >> 4));
+        double b[2][4][NSL];
+        auto terms = [&](int g) {
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+#pragma unroll
+                for (int s = 0; s < NSL; s++) b[g & 1][d][s] = B[(4 * g + d) * 4 + s * 4 * RS];
+        };
+#pragma unroll
+        for (int s = 0; s < NSL; s++) acc[0][s][0] = 0.0;
+        terms(0);
+#pragma unroll
+        for (int g = 0; g < kBlocks / 4; g++) {
+            const bool more = 4 * (g + 1) < nb;
+            if (more) terms(g + 1);
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+#pragma unroll
+                for (int s = 0; s < NSL; s++)
+                    acc[0][s][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[4 * g + d], b[g & 1][d][s], acc[0][s][0], 0, 0, 0);
+            if (!more) break;
+        }
+    }
+};
+
+// Otherwise both operands are streamed: A from LDS and L2, one group of pairs
+// ahead (the wave's loads of the first global group are issued by prefetch()
+// before the barrier).
 template <int NC, int NSL, int TT>
-struct DenseContraction {
+struct StreamedContraction {
     struct alignas(16) Pair { double x, y; };
     using GP = const __attribute__((address_space(1))) Pair*;
     using LP = const __attribute__((address_space(3))) Pair*;
@@ -145,7 +214,7 @@ struct DenseContraction {
     int gs, gi, ls, li, lp, pairs, RS, bi, l, nt;
     double a0[TT][2 * G];
 
-    __device__ __forceinline__ DenseContraction(const double* Mt, const double* Ml, int ldsPairs, int UPS)
+    __device__ __forceinline__ StreamedContraction(const double* Mt, const double* Ml, int ldsPairs, int UPS)
     {
         const int w = wave_index(), nw = blockDim.x >> 6, tiles = dense_tiles(UPS);
         l = threadIdx.x & 63;
@@ -242,6 +311,10 @@ struct DenseContraction {
     }
 };
 
+template <class Sys, int NSL, int MT>
+using DenseContraction = typename std::conditional<dense_resident<Sys, NSL, MT>(), ResidentContraction<NSL, MT>,
+                                                   StreamedContraction<Sys::NC, NSL, dense_tt(MT)>>::type;
+
 // Copies the leading ldsPairs pairs of every tile of the tiled matrices into LDS.
 __device__ __forceinline__ void dense_stage_matrix(const double* Mt, unsigned char* lds, int NC, int UPS, int ldsPairs)
 {
@@ -285,9 +358,10 @@ __device__ __forceinline__ double rk_stage_time(int s, double t, double h)
 }
 
 // QUIET: no events, no user action after a step and no dense output (a.NDO == 0)
-template <class Sys, int ALG, int NSL, int TT, bool REC, bool QUIET>
+template <class Sys, int ALG, int NSL, int MT, bool REC, bool QUIET>
 __device__ void pb_dense_body(const Args<Sys, double>& a)
 {
+    constexpr int TT = dense_tt(MT);
     using P = double;
     using CP = double;
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NSP = Sys::NSP, NGP = Sys::NGP, NiGP = Sys::NiGP;
@@ -322,7 +396,7 @@ __device__ void pb_dense_body(const Args<Sys, double>& a)
     }
     for (int i = tid; i < 2 * cptStride; i += blockDim.x) cptBuf[i] = P(0);   // padded units and absent systems stay zero
     dense_stage_matrix(a.cTile, mpgos_pb_lds + L.mt, NC, UPS, a.ldsPairs);
-    DenseContraction<NC, NSL, TT> product(a.cTile, reinterpret_cast<const double*>(mpgos_pb_lds + L.mt), a.ldsPairs, UPS);
+    DenseContraction<Sys, NSL, MT> product(a.cTile, reinterpret_cast<const double*>(mpgos_pb_lds + L.mt), a.ldsPairs, UPS);
     int cIndex[NCp];
 #pragma unroll
     for (int i = 0; i < NC; i++) cIndex[i] = a.cIndex[i];
@@ -489,15 +563,28 @@ __device__ void pb_dense_body(const Args<Sys, double>& a)
     int buf = 0;
     // right-hand sides of this lane's units at (Y, T), then the coupling terms
     constexpr int PER = 64 / SPB;        // stages whose time terms one evaluation covers
-    P tterm[(ST + PER - 1) / PER][Pos<NTT>::value];
-    auto rhs = [&](int stage, P (*F)[TT][UD], P (*Y)[TT][UD], const P* T, const bool* run) {
-        P* cpt = cptBuf + (size_t)buf * cptStride;
-        P CPF[NSL][TT][NCp];
-        P tt[NSL][Pos<NTT>::value];
+    P tterm[(ST + PER - 1) / PER][Pos<NTT>::value], tt[NSL][Pos<NTT>::value];
+    auto fetch_terms = [&](int stage) {
 #pragma unroll
         for (int s = 0; s < NSL; s++)
 #pragma unroll
             for (int i = 0; i < NTT; i++) tt[s][i] = __shfl(tterm[stage / PER][i], (stage % PER) * SPB + at.sys(s));
+    };
+    // coupling strengths and, where no user code can change them during the
+    // steps, system parameters in registers: a stage waits for LDS only where
+    // it needs the other units' coupling terms
+    constexpr bool keepPar = QUIET && NSP <= 4;
+    P strength[NSL][NCp], par[NSL][Pos<NSP>::value];
+#pragma unroll
+    for (int s = 0; s < NSL; s++) {
+#pragma unroll
+        for (int i = 0; i < NC; i++) strength[s][i] = MPGOS_PB_MY(s).strength[i];
+#pragma unroll
+        for (int i = 0; i < NSP; i++) par[s][i] = keepPar ? MPGOS_PB_MY(s).sPAR[i] : P(0);
+    }
+    auto rhs = [&](int stage, P (*F)[TT][UD], P (*Y)[TT][UD], const P* T, const bool* run) {
+        P* cpt = cptBuf + (size_t)buf * cptStride;
+        P CPF[NSL][TT][NCp];
         product.prefetch();
         each([&](int s, int k) {
             if (run[s] && at.has(k)) {
@@ -505,22 +592,24 @@ __device__ void pb_dense_body(const Args<Sys, double>& a)
 #pragma unroll
                 for (int i = 0; i < NC; i++) cp[i] = CPF[s][k][i] = P(0);
                 S& y = MPGOS_PB_MY(s);
+                P* sPAR = keepPar ? par[s] : y.sPAR;
                 if constexpr (NTT > 0)
-                    Sys::template OdeFunctionTT<P>(at.gsys(s), at.unit(k), F[s][k], Y[s][k], T[s], tt[s], uPAR[s][k], y.sPAR, gPAR,
+                    Sys::template OdeFunctionTT<P>(at.gsys(s), at.unit(k), F[s][k], Y[s][k], T[s], tt[s], uPAR[s][k], sPAR, gPAR,
                                                    gPARi, uACC[s][k], uACCi[s][k], y.sACC, y.sACCi, cp, CPF[s][k]);
                 else
-                    Sys::template OdeFunction<P>(at.gsys(s), at.unit(k), F[s][k], Y[s][k], T[s], uPAR[s][k], y.sPAR, gPAR, gPARi,
+                    Sys::template OdeFunction<P>(at.gsys(s), at.unit(k), F[s][k], Y[s][k], T[s], uPAR[s][k], sPAR, gPAR, gPARi,
                                                  uACC[s][k], uACCi[s][k], y.sACC, y.sACCi, cp, CPF[s][k]);
 #pragma unroll
                 for (int i = 0; i < NC; i++) cpt[(i * SPB + at.sys(s)) * RS + at.unit(k)] = cp[i];
             }
         });
+        if (stage + 1 < ST) fetch_terms(stage + 1);
         lds_barrier();
         P v[NCp][NSL][TT];
         product.run(cpt, v);
         each([&](int s, int k) {
 #pragma unroll
-            for (int i = 0; i < NC; i++) U::add(cIndex[i], MPGOS_PB_MY(s).strength[i] * CPF[s][k][i], v[i][s][k], F[s][k]);
+            for (int i = 0; i < NC; i++) U::add(cIndex[i], strength[s][i] * CPF[s][k][i], v[i][s][k], F[s][k]);
         });
         buf ^= 1;
     };
@@ -546,6 +635,7 @@ __device__ void pb_dense_body(const Args<Sys, double>& a)
             for (int e = 0; e * PER < ST; e++)
                 Sys::template TimeTerms<P>(rk_stage_time<ALG>(e * PER + at.l / SPB, sys[at.l % SPB].t, sys[at.l % SPB].dt),
                                            sys[at.l % SPB].sPAR, tterm[e]);
+            fetch_terms(0);
         }
         P next[NSL][TT][UD], err[NSL][TT][UD];
         auto stage_time = [&](int st) {
@@ -886,13 +976,12 @@ __device__ void pb_dense_body(const Args<Sys, double>& a)
 #undef MPGOS_PB_MY
 }
 
-// At most 8 wavefronts: up to 8 tiles one each (TT 1), up to 16 two each.  The
-// register limits: 4 wavefronts per SIMD with one result per lane (98 VGPRs
-// used), 3 with two systems and one tile, else 2.
-template <class Sys, int ALG, int NSL, int TT, bool REC, bool QUIET>
-__global__ void __launch_bounds__(512, TT == 1 ? 5 - NSL : 2) pb_dense_kernel(Args<Sys, double> a)
+// Wavefronts per SIMD that the registers have to allow: one result per lane 4
+// with at most 4 tiles and 3 with 8; two results 3 and 2; else 2.
+template <class Sys, int ALG, int NSL, int MT, bool REC, bool QUIET>
+__global__ void __launch_bounds__(64 * dense_waves(MT), dense_per_simd(NSL, MT)) pb_dense_kernel(Args<Sys, double> a)
 {
-    pb_dense_body<Sys, ALG, NSL, TT, REC, QUIET>(a);
+    pb_dense_body<Sys, ALG, NSL, MT, REC, QUIET>(a);
 }
 
 } // namespace pb

@@ -448,20 +448,22 @@ public:
     {
         return std::is_same<P, double>::value && CCI == 0 && CBW == 0 && UPS % 32 == 0 && UPS <= 256;
     }
-    // Workgroups of the dense form with 4 systems that a CU holds at once (its
-    // registers allow 16 wavefronts with one tile each, 8 with two).
-    int dense_per_cu() const
-    {
-        const int tiles = dense_tiles(UPS);
-        return tiles > 8 ? 1 : 16 / tiles;
-    }
+    int dense_mt() const { return dense_tiles(UPS) <= 4 ? 4 : dense_tiles(UPS) <= 8 ? 8 : 16; }
+    int dense_threads() const { return 64 * ((dense_tiles(UPS) + dense_tt(dense_mt()) - 1) / dense_tt(dense_mt())); }
+    // workgroups that a CU holds at once, perSimd wavefronts on each SIMD
+    int dense_per_cu(int perSimd) const { return std::max(1, 4 * perSimd / (dense_threads() / 64)); }
     // 4 systems per workgroup while the card holds all workgroups at once, else
     // 8: the second four share the matrix operand, but a wavefront's step takes
     // 1.3 to 1.7 times as long.  Measured, ms with 4 | 8 systems (ring of Duffing
     // oscillators, one period): 1024 x 256 units 8.7 | 11.5, 4096 x 256 33.3 |
-    // 23.9, 1000 x 100 2.3 | 3.8, 4096 x 100 7.2 | 6.2, 4096 x 128 10.1 | 8.6,
+    // 23.9, 1000 x 100 2.3 | 3.8, 4096 x 100 9.2 | 7.8, 4096 x 128 10.1 | 8.6,
     // 8192 x 12 1.1 | 1.6, 65536 x 16 5.7 | 5.3.
-    bool dense_four() const { return (long)(NS + 3) / 4 <= (long)dense_per_cu() * cus; }
+    bool dense_four() const { return (long)(NS + 3) / 4 <= (long)dense_per_cu(dense_per_simd(1, dense_mt())) * cus; }
+    template <class Scope>
+    bool dense_fits(int spb, int sharedG) const
+    {
+        return dense_layout<Scope, NC, NGP, NiGP>(spb, UPS, sharedG, 0).total <= ldsMax;
+    }
     // Automatic choice.  Up to 8 units the dense form computes at least as many
     // padded rows as real ones; it is the faster one only while the card is not
     // full (2048 x 4 units: 0.9 against 1.4 ms; 65536 x 4: 4.9 against 2.4 ms;
@@ -470,7 +472,10 @@ public:
     {
         if (couplingKernel == 1) return kLaneCoupling;
         if (couplingKernel == 2 && NC > 0) return kDenseCoupling;
-        return dense_possible() && (UPS > 8 || dense_four()) ? kDenseCoupling : kLaneCoupling;
+        if constexpr (std::is_same<P, double>::value) {
+            if (dense_possible() && (UPS > 8 || dense_four()) && dense_fits<DenseScope<Sys>>(4, sharedGlobals)) return kDenseCoupling;
+        }
+        return kLaneCoupling;
     }
 
     size_t lds_bytes(int spb, int sm) const
@@ -479,46 +484,40 @@ public:
     }
 
     // The leading column-block pairs of every tile that a workgroup of the dense
-    // form keeps in LDS: as many as fit beside its other data (base bytes) and
-    // the other workgroups that its CU is to hold (4096 x 100 units, 8 systems:
-    // 6.2 ms with 4 of 14 pairs and three workgroups per CU, 7.8 ms with all
-    // pairs and one; 1000 x 100, 4 systems: 4.6 ms with all, 5.4 ms with none).
-    int dense_lds_pairs(size_t base, int perCu) const
+    // form keeps in LDS where it streams the matrix: as many as fit beside its
+    // other data (base bytes) and the other workgroups that its CU is to hold
+    // (1000 x 100 units, 4 systems: 4.6 ms with all 14, 5.4 ms with none).
+    int dense_lds_pairs(size_t base, int grid, int perSimd) const
     {
+        const int perCu = std::min((grid + cus - 1) / cus, dense_per_cu(perSimd));
         const size_t perPair = (size_t)NC * dense_tiles(UPS) * 64 * 16, room = ldsMax / (size_t)std::max(1, perCu);
         const int lp = room > base ? (int)std::min<size_t>((room - base) / perPair, (size_t)dense_pairs(UPS)) : 0;
         return lp - lp % kDenseGroup;
     }
-    // workgroups of the reverse kernels per CU (2 wavefronts per SIMD)
-    int dense_reverse_per_cu() const
-    {
-        const int tiles = dense_tiles(UPS);
-        return tiles > 8 ? 1 : std::max(1, 8 / tiles);
-    }
 
-    template <int NSL, int TT, bool REC, bool QUIET>
+    template <int NSL, int MT, bool REC, bool QUIET>
     int launch_dense(Args<Sys, double>& a)
     {
         constexpr int spb = 4 * NSL;
         auto bytes = [&](int pairs) { return dense_layout<DenseScope<Sys>, NC, NGP, NiGP>(spb, UPS, sharedGlobals, pairs).total; };
         const int grid = (NS + spb - 1) / spb;
-        const int lp = dense_lds_pairs(bytes(0), std::min((grid + cus - 1) / cus, NSL == 1 ? dense_per_cu() : std::max(1, dense_per_cu() * 3 / 4)));
+        const int lp = dense_resident<Sys, NSL, MT>() ? 0 : dense_lds_pairs(bytes(0), grid, dense_per_simd(NSL, MT));
         a.SPB = spb;
         a.ldsPairs = lp;
         a.cTile = cTile;
-        const int threads = 64 * ((dense_tiles(UPS) + TT - 1) / TT);
-        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_dense_kernel<Sys, MPGOS_RK4, NSL, TT, REC, QUIET>), dim3(grid), dim3(threads), bytes(lp), strm, a);
-        else hipLaunchKernelGGL((pb_dense_kernel<Sys, MPGOS_RKCK45, NSL, TT, REC, QUIET>), dim3(grid), dim3(threads), bytes(lp), strm, a);
+        const int threads = dense_threads();
+        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_dense_kernel<Sys, MPGOS_RK4, NSL, MT, REC, QUIET>), dim3(grid), dim3(threads), bytes(lp), strm, a);
+        else hipLaunchKernelGGL((pb_dense_kernel<Sys, MPGOS_RKCK45, NSL, MT, REC, QUIET>), dim3(grid), dim3(threads), bytes(lp), strm, a);
         return MPGOS_OK;
     }
-    template <int NSL, int TT, bool REC>
+    template <int NSL, int MT, bool REC>
     int launch_dense(Args<Sys, double>& a)
     {
         constexpr bool quiet = NE == 0 && systems::no_step_action<Sys, systems::PBNoCallbacks>();
         if constexpr (quiet) {
-            if (NDO == 0) return launch_dense<NSL, TT, REC, true>(a);
+            if (NDO == 0) return launch_dense<NSL, MT, REC, true>(a);
         }
-        return launch_dense<NSL, TT, REC, false>(a);
+        return launch_dense<NSL, MT, REC, false>(a);
     }
     template <bool REC>
     int launch_dense(Args<Sys, double>& a)
@@ -526,13 +525,17 @@ public:
         // the matrices in column-block pairs per lane, refreshed every Solve
         // (a kernel on the solver's stream, so graph capture records it)
         if (int rc = tile_pairs<false>(cTile)) return rc;
-        auto fits = [&](int spb) { return dense_layout<DenseScope<Sys>, NC, NGP, NiGP>(spb, UPS, sharedGlobals, 0).total <= ldsMax; };
-        if (!fits(4)) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
-        const bool four = dense_four() || !fits(8);
+        if (!dense_fits<DenseScope<Sys>>(4, sharedGlobals)) { set_error("per-block: system scope and coupling terms exceed the LDS of a workgroup"); return MPGOS_E_ARG; }
+        const bool four = dense_four() || !dense_fits<DenseScope<Sys>>(8, sharedGlobals);
         // two tiles per wavefront above 8 tiles: they share the coupling terms
-        // (4096 x 256: 23.9 against 25.9 ms), below one (4096 x 128: 8.6 against 9.6 ms)
-        if (dense_tiles(UPS) > 8) return four ? launch_dense<1, 2, REC>(a) : launch_dense<2, 2, REC>(a);
-        return four ? launch_dense<1, 1, REC>(a) : launch_dense<2, 1, REC>(a);
+        // (4096 x 256: 23.9 against 25.9 ms), below one (4096 x 128: 8.6 against
+        // 9.6 ms); up to 4 tiles the registers leave room for one more wavefront
+        // per SIMD (4096 x 64: 2.7 against 3.4 ms, 8192 x 32: 2.0 against 2.7 ms)
+        switch (dense_mt()) {
+        case 4: return four ? launch_dense<1, 4, REC>(a) : launch_dense<2, 4, REC>(a);
+        case 8: return four ? launch_dense<1, 8, REC>(a) : launch_dense<2, 8, REC>(a);
+        default: return four ? launch_dense<1, 16, REC>(a) : launch_dense<2, 16, REC>(a);
+        }
     }
 
     // PB-IF:1949-1965
@@ -734,36 +737,35 @@ public:
         a.recX = recX; a.recT = recT; a.recH = recH; a.recK = adjK; a.recCkCap = adjCap; a.recStepCap = adjStepCap;
         AdjArgs<Sys> A;
         A.seg = nullptr; A.stg = stg; A.gSp = gSp; A.lam = lamB.d; A.gU = gUB.d; A.gS = gSB.d; A.cMatT = nullptr; A.cTileT = cTileT;
-        auto fits = [&](int spb) { return dense_layout<RevScope<Sys>, NC, 0, 0>(spb, UPS, 0, 0).total <= ldsMax; };
-        if (!fits(4)) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
+        if (!dense_fits<RevScope<Sys>>(4, 0)) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
         MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
         if ((rc = tile_pairs<false>(cTile)) || (rc = tile_pairs<true>(cTileT))) return rc;
         a.cTile = cTile;
-        const bool four = dense_four() || !fits(8);
-        if (dense_tiles(UPS) > 8) { if (four) launch_reverse<1, 2>(a, A, rounds); else launch_reverse<2, 2>(a, A, rounds); }
-        else if (four) launch_reverse<1, 1>(a, A, rounds);
-        else launch_reverse<2, 1>(a, A, rounds);
+        const bool four = dense_four() || !dense_fits<RevScope<Sys>>(8, 0);
+        if (dense_mt() > 8) { if (four) launch_reverse<1, 16>(a, A, rounds); else launch_reverse<2, 16>(a, A, rounds); }
+        else if (four) launch_reverse<1, 8>(a, A, rounds);
+        else launch_reverse<2, 8>(a, A, rounds);
         hipLaunchKernelGGL((pb_reverse_finish_kernel<Sys>), dim3((unsigned)((NU + 255) / 256)), dim3(256), 0, strm, a, A);
         MPGOS_HIP_TRY(hipGetLastError());
         MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
         return MPGOS_OK;
     }
-    template <int NSL, int TT>
+    template <int NSL, int MT>
     void launch_reverse(Args<Sys, double>& a, const AdjArgs<Sys>& A, int rounds)
     {
         constexpr int spb = 4 * NSL;
         auto bytes = [&](int pairs) { return dense_layout<RevScope<Sys>, NC, 0, 0>(spb, UPS, 0, pairs).total; };
-        const int grid = (NS + spb - 1) / spb, threads = 64 * ((dense_tiles(UPS) + TT - 1) / TT);
+        const int grid = (NS + spb - 1) / spb, threads = dense_threads();
         a.SPB = spb;
-        a.ldsPairs = dense_lds_pairs(bytes(0), std::min((grid + cus - 1) / cus, dense_reverse_per_cu()));
+        a.ldsPairs = dense_resident<Sys, NSL, MT>() ? 0 : dense_lds_pairs(bytes(0), grid, 2);
         const size_t lds = bytes(a.ldsPairs);
         for (int r = 0; r < rounds; r++) {
             if (algorithm == MPGOS_RK4) {
-                hipLaunchKernelGGL((pb_replay_kernel<Sys, MPGOS_RK4, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
-                hipLaunchKernelGGL((pb_sweep_kernel<Sys, MPGOS_RK4, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+                hipLaunchKernelGGL((pb_replay_kernel<Sys, MPGOS_RK4, NSL, MT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+                hipLaunchKernelGGL((pb_sweep_kernel<Sys, MPGOS_RK4, NSL, MT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
             } else {
-                hipLaunchKernelGGL((pb_replay_kernel<Sys, MPGOS_RKCK45, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
-                hipLaunchKernelGGL((pb_sweep_kernel<Sys, MPGOS_RKCK45, NSL, TT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+                hipLaunchKernelGGL((pb_replay_kernel<Sys, MPGOS_RKCK45, NSL, MT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
+                hipLaunchKernelGGL((pb_sweep_kernel<Sys, MPGOS_RKCK45, NSL, MT>), dim3(grid), dim3(threads), lds, strm, a, A, r);
             }
         }
     }
