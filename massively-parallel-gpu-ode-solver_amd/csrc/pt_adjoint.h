@@ -78,21 +78,23 @@ __device__ __forceinline__ void store_checkpoint(const AdjArgs<Sys>& A, const La
     for (int i = 0; i < Sys::NIA; i++) A.ckpt[(base + SD + 2 + NE + Sys::NA + i) * NT + L.tid] = (double)L.ACCi[i];
 }
 
-template <class Sys, int ALG>
+template <class Sys, int ALG, int GROUP>
 __device__ __forceinline__ void record_body(const AdjArgs<Sys>& A)
 {
     static_assert(offsetof(AdjArgs<Sys>, a) == 0, "Lane's rare paths read the Args at the start of the kernel arguments");
     const Args<Sys, double, double>& a = A.a;
     double* sPAR; int* sPARi;
     stage_shared(a, sPAR, sPARi);
-    const int tid = threadIdx.x + blockIdx.x * blockDim.x;
+    const int tid = threadIdx.x / GROUP + blockIdx.x * (blockDim.x / GROUP);
+    const bool stores = GROUP == 1 || threadIdx.x % GROUP == 0;
     using L_t = Lane<Sys, double, false, ALG>;
     L_t L;
-    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    if constexpr (GROUP > 1) c.template set_nodes<GROUP>();
     int untilCk = A.K, k = 0;      // accepted steps to the next checkpoint (no division in the loop)
     if (tid < a.nActive) {
         L.load(a, tid, sPAR, sPARi);
-        store_checkpoint<Sys, ALG>(A, L, 0);
+        if (stores) store_checkpoint<Sys, ALG>(A, L, 0);
     } else {
         L.idle();
     }
@@ -111,22 +113,22 @@ __device__ __forceinline__ void record_body(const AdjArgs<Sys>& A)
         }
     }
     if (tid >= a.nActive) return;
-    constexpr bool CARRY = L_t::NTT > 0;
+    constexpr bool CARRY = L_t::NTT > 0 && GROUP == 1;
     double tt[Pos<L_t::NTT>::value];
-    L.time_terms(L.t, tt);
+    if (CARRY) L.time_terms(L.t, tt);
     bool ended = L.term != 0, accepted;
     while (!ended) {
-        ended = L.template step<true, CARRY>(c, sPAR, sPARi, accepted, tt);
+        ended = L.template step<true, CARRY, GROUP>(c, sPAR, sPARi, accepted, tt);
         if (accepted && --untilCk == 0) {
             untilCk = A.K;
             ++k;
             if (!ended) {
-                if (k < A.ckcap) store_checkpoint<Sys, ALG>(A, L, k);
-                else L.status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT;
+                if (k >= A.ckcap) L.status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT;
+                else if (stores) store_checkpoint<Sys, ALG>(A, L, k);
             }
         }
     }
-    L.finish(a, sPAR, sPARi);
+    if (stores) L.finish(a, sPAR, sPARi);
 }
 
 // ---------------------------------------------------------------- reverse steps
@@ -199,11 +201,16 @@ __device__ __forceinline__ void reverse_rk4(int tid, int NT, const double* x, do
     Vjp<Sys, TT>::template apply<NCPA>(tid, NT, kb, xx, t, cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy, tt1);
 }
 
-// Cash-Karp (stages as in Lane::rkck45, 5th-order weights b).
-template <class Sys>
+// Cash-Karp (stages as in Lane::rkck45, 5th-order weights b).  Time terms are
+// evaluated once per stage, with several lanes per instance (GROUP, node) once or
+// twice per step.
+template <class Sys, int GROUP>
 __device__ __forceinline__ void reverse_rkck45(int tid, int NT, const double* x, double t, double h, double* cPAR,
-                                               double* sPAR, int* sPARi, double* ACC, int* ACCi, double* lam, double* mu)
+                                               double* sPAR, int* sPARi, double* ACC, int* ACCi, double* lam, double* mu,
+                                               const double* node)
 {
+    constexpr bool TT = TimeTermsOf<Sys>::timeOnly;
+    constexpr int NTT = TimeTermsOf<Sys>::n;
     using math::fma;
     constexpr int SD = Sys::SD, NCPA = Pos<Sys::NCP>::value;
     constexpr double a21 = 1.0 / 5.0;
@@ -216,22 +223,44 @@ __device__ __forceinline__ void reverse_rkck45(int tid, int NT, const double* x,
 
     double y[6][SD], k[5][SD];
     const double T[6] = {t, fma(h, 1.0 / 5.0, t), fma(h, 3.0 / 10.0, t), fma(h, 3.0 / 5.0, t), t + h, fma(h, 7.0 / 8.0, t)};
+    double tt[6][Pos<NTT>::value];
+    if constexpr (TT && GROUP > 1) {
+        double all[group_evals<GROUP>()][Pos<NTT>::value];
+#pragma unroll
+        for (int e = 0; e < group_evals<GROUP>(); e++) Sys::template TimeTerms<double>(fma(h, node[e], t), cPAR, all[e]);
+        auto take = [&](auto J) {
+#pragma unroll
+            for (int i = 0; i < NTT; i++) tt[J.value][i] = group_value<GROUP, J.value % GROUP>(all[J.value / GROUP][i]);
+        };
+        take(std::integral_constant<int, 0>{}); take(std::integral_constant<int, 1>{}); take(std::integral_constant<int, 2>{});
+        take(std::integral_constant<int, 3>{}); take(std::integral_constant<int, 4>{}); take(std::integral_constant<int, 5>{});
+    } else if constexpr (TT) {
+#pragma unroll
+        for (int j = 0; j < 6; j++) Sys::template TimeTerms<double>(T[j], cPAR, tt[j]);
+    }
+    auto ode = [&](double* F, int j) {
+        if constexpr (TT) Sys::template OdeFunctionTT<double>(tid, NT, F, y[j], T[j], tt[j], cPAR, sPAR, sPARi, ACC, ACCi);
+        else Sys::template OdeFunction<double>(tid, NT, F, y[j], T[j], cPAR, sPAR, sPARi, ACC, ACCi);
+    };
+    auto vjp = [&](int j, double* kb, double* gy) {
+        Vjp<Sys, TT>::template apply<NCPA>(tid, NT, kb, y[j], T[j], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy, tt[j]);
+    };
 #pragma unroll
     for (int c = 0; c < SD; c++) y[0][c] = x[c];
-    Sys::template OdeFunction<double>(tid, NT, k[0], y[0], T[0], cPAR, sPAR, sPARi, ACC, ACCi);
+    ode(k[0], 0);
 #pragma unroll
     for (int c = 0; c < SD; c++) y[1][c] = fma(h, a21 * k[0][c], x[c]);
-    Sys::template OdeFunction<double>(tid, NT, k[1], y[1], T[1], cPAR, sPAR, sPARi, ACC, ACCi);
+    ode(k[1], 1);
 #pragma unroll
     for (int c = 0; c < SD; c++) y[2][c] = fma(h, fma(a32, k[1][c], a31 * k[0][c]), x[c]);
-    Sys::template OdeFunction<double>(tid, NT, k[2], y[2], T[2], cPAR, sPAR, sPARi, ACC, ACCi);
+    ode(k[2], 2);
 #pragma unroll
     for (int c = 0; c < SD; c++) y[3][c] = fma(h, fma(a43, k[2][c], fma(a42, k[1][c], a41 * k[0][c])), x[c]);
-    Sys::template OdeFunction<double>(tid, NT, k[3], y[3], T[3], cPAR, sPAR, sPARi, ACC, ACCi);
+    ode(k[3], 3);
 #pragma unroll
     for (int c = 0; c < SD; c++)
         y[4][c] = fma(h, fma(a54, k[3][c], fma(a53, k[2][c], fma(a52, k[1][c], a51 * k[0][c]))), x[c]);
-    Sys::template OdeFunction<double>(tid, NT, k[4], y[4], T[4], cPAR, sPAR, sPARi, ACC, ACCi);
+    ode(k[4], 4);
 #pragma unroll
     for (int c = 0; c < SD; c++)
         y[5][c] = fma(h, fma(a65, k[4][c], fma(a64, k[3][c], fma(a63, k[2][c], fma(a62, k[1][c], a61 * k[0][c])))), x[c]);
@@ -244,36 +273,36 @@ __device__ __forceinline__ void reverse_rkck45(int tid, int NT, const double* x,
         kb[0][c] = b1 * hl; kb[1][c] = 0.0; kb[2][c] = b3 * hl; kb[3][c] = b4 * hl; kb[4][c] = 0.0; kb[5][c] = b6 * hl;
     }
     // stage 6 -> contributes to k1..k5
-    Vjp<Sys>::template apply<NCPA>(tid, NT, kb[5], y[5], T[5], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy);
+    vjp(5, kb[5], gy);
 #pragma unroll
     for (int c = 0; c < SD; c++) {
         const double g = h * gy[c];
         kb[0][c] = fma(a61, g, kb[0][c]); kb[1][c] = fma(a62, g, kb[1][c]); kb[2][c] = fma(a63, g, kb[2][c]);
         kb[3][c] = fma(a64, g, kb[3][c]); kb[4][c] = fma(a65, g, kb[4][c]);
     }
-    Vjp<Sys>::template apply<NCPA>(tid, NT, kb[4], y[4], T[4], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy);
+    vjp(4, kb[4], gy);
 #pragma unroll
     for (int c = 0; c < SD; c++) {
         const double g = h * gy[c];
         kb[0][c] = fma(a51, g, kb[0][c]); kb[1][c] = fma(a52, g, kb[1][c]); kb[2][c] = fma(a53, g, kb[2][c]);
         kb[3][c] = fma(a54, g, kb[3][c]);
     }
-    Vjp<Sys>::template apply<NCPA>(tid, NT, kb[3], y[3], T[3], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy);
+    vjp(3, kb[3], gy);
 #pragma unroll
     for (int c = 0; c < SD; c++) {
         const double g = h * gy[c];
         kb[0][c] = fma(a41, g, kb[0][c]); kb[1][c] = fma(a42, g, kb[1][c]); kb[2][c] = fma(a43, g, kb[2][c]);
     }
-    Vjp<Sys>::template apply<NCPA>(tid, NT, kb[2], y[2], T[2], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy);
+    vjp(2, kb[2], gy);
 #pragma unroll
     for (int c = 0; c < SD; c++) {
         const double g = h * gy[c];
         kb[0][c] = fma(a31, g, kb[0][c]); kb[1][c] = fma(a32, g, kb[1][c]);
     }
-    Vjp<Sys>::template apply<NCPA>(tid, NT, kb[1], y[1], T[1], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy);
+    vjp(1, kb[1], gy);
 #pragma unroll
     for (int c = 0; c < SD; c++) kb[0][c] = fma(a21, h * gy[c], kb[0][c]);
-    Vjp<Sys>::template apply<NCPA>(tid, NT, kb[0], y[0], T[0], cPAR, sPAR, sPARi, ACC, ACCi, lam, mu, gy);
+    vjp(0, kb[0], gy);
 }
 
 // LDS bytes of the shared-parameter staging (16-byte aligned); the segment
@@ -397,7 +426,7 @@ __device__ __forceinline__ bool common_time_reverse(const AdjArgs<Sys>& A, Lane<
     return true;
 }
 
-template <class Sys, int ALG, bool LDS_SEG>
+template <class Sys, int ALG, bool LDS_SEG, int GROUP>
 __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
 {
     constexpr int SD = Sys::SD, NCP = Sys::NCP, NA = Sys::NA, NIA = Sys::NIA;
@@ -407,7 +436,7 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
     stage_shared(a, sPAR, sPARi);
     using L_t = Lane<Sys, double, false, ALG>;
     constexpr bool COMMON = L_t::kCommonTime && Sys::HAS_VJP;
-    const int tid = threadIdx.x + blockIdx.x * blockDim.x;
+    const int tid = threadIdx.x / GROUP + blockIdx.x * (blockDim.x / GROUP);
     const bool mine = tid < a.nActive;
     if (!COMMON && !mine) return;      // with COMMON whole wavefronts stay together
     const int NT = a.NT;
@@ -440,8 +469,9 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
     const bool ok = mine && (a.status[tid] & MPGOS_STATUS_CHECKPOINT_OVERFLOW_BIT) == 0;
     const long long nseg = ok ? (total + A.K - 1) / A.K : 0;
     const int K = A.K;
-    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
-    constexpr bool CARRY = L_t::NTT > 0;
+    typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    if constexpr (GROUP > 1) c.template set_nodes<GROUP>();
+    constexpr bool CARRY = L_t::NTT > 0 && GROUP == 1;
     double tt[Pos<L_t::NTT>::value];
     // Restore segment s's checkpoint into the lane.
     auto restore = [&](long long s) {
@@ -460,7 +490,7 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
         L.tc = 0.0;
         L.term = 0; L.udt = 0; L.nacc = 0; L.nrej = 0; L.status = 0; L.nev = 0;
         L.doIdx = 0; L.skipped = 0; L.doT = 0.0;
-        L.time_terms(L.t, tt);
+        if (CARRY) L.time_terms(L.t, tt);
     };
     // accepted steps of segment s
     auto count = [&](long long s) { return (int)((total - s * K) < K ? (total - s * K) : K); };
@@ -480,7 +510,7 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
         for (int c = 0; c < SD; c++) xp[c] = L.X[c];
         const double tp = L.t;
         bool accepted;
-        if (L.template step<false, CARRY>(c, sPAR, sPARi, accepted, tt)) L.term = 1;
+        if (L.template step<false, CARRY, GROUP>(c, sPAR, sPARi, accepted, tt)) L.term = 1;
         if (accepted) {
             const size_t sb = (size_t)slot(flip, j) * (SD + 2);
 #pragma unroll
@@ -512,7 +542,7 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
         if (ALG == MPGOS_RK4)
             reverse_rk4<Sys>(tid, NT, x, tn, hn, bPAR, sPAR, sPARi, bACC, bACCi, lam, mu);
         else
-            reverse_rkck45<Sys>(tid, NT, x, tn, hn, bPAR, sPAR, sPARi, bACC, bACCi, lam, mu);
+            reverse_rkck45<Sys, GROUP>(tid, NT, x, tn, hn, bPAR, sPAR, sPARi, bACC, bACCi, lam, mu, c.node);
     };
     bool swept = false;
     if constexpr (COMMON) {
@@ -554,11 +584,12 @@ __device__ __forceinline__ void reverse_body(const AdjArgs<Sys>& A)
     for (int c = 0; c < NCP; c++) A.gp[c * NT + tid] = ok ? mu[c] : __builtin_nan("");
 }
 
-template <class Sys, int ALG>
-__global__ void __launch_bounds__(kMaxBlock) adjoint_record_kernel(AdjArgs<Sys> A) { record_body<Sys, ALG>(A); }
+// GROUP: lanes per instance (Cash-Karp and systems with time terms only, else 1)
+template <class Sys, int ALG, int GROUP = 1>
+__global__ void __launch_bounds__(kMaxBlock) adjoint_record_kernel(AdjArgs<Sys> A) { record_body<Sys, ALG, GROUP>(A); }
 
-template <class Sys, int ALG, bool LDS_SEG>
-__global__ void __launch_bounds__(kMaxBlock) adjoint_reverse_kernel(AdjArgs<Sys> A) { reverse_body<Sys, ALG, LDS_SEG>(A); }
+template <class Sys, int ALG, bool LDS_SEG, int GROUP = 1>
+__global__ void __launch_bounds__(kMaxBlock) adjoint_reverse_kernel(AdjArgs<Sys> A) { reverse_body<Sys, ALG, LDS_SEG, GROUP>(A); }
 
 } // namespace pt
 } // namespace mpgos

@@ -77,6 +77,7 @@ struct Args {
     int NT, nActive, NDO, evcap, preferShared;
     int doFreq;
     int roundSteps;           // persistent form: attempted steps between compactions
+    int octets;               // sorted form's last launch: workgroups [0, octets) give an instance 8 lanes
     int solo;                 // persistent form: list entries [0, solo) run one per workgroup (workgroups [0, solo))
     CP dt0, dtmax, dtmin, grow, shrink;
     P doMinDt;
@@ -178,6 +179,53 @@ __device__ __forceinline__ void advance_by_lane_kahan(float& t, float& c, float 
                  : "+v"(t), "+v"(c), "=&s"(save), "=&v"(y), "=&v"(d) : "v"(h) : "scc");
 }
 
+// ---- several lanes per instance
+// With fewer instances than keep the card busy, GROUP (4 or 8) neighbouring
+// lanes hold one instance: all of them make its steps, on the same values, and
+// the time terms of a Cash-Karp step's six stages, whose times are known when
+// the step starts, are evaluated one stage per lane (two with 4 lanes) and
+// exchanged within the group, in one or two evaluations per step instead of
+// five.  The values are those that a single lane would compute.  A lone
+// wavefront is bound by the instructions of its step; the step of a double-well
+// Duffing oscillator has 455 FP64 instructions with one lane and 345 with 8.
+// 20000 uneven Duffing instances 116 -> 67 ms, 10007 Cash-Karp adjoints 3.76 ->
+// 2.82 ms, 4000 double wells 127 -> 92 us.
+template <int GROUP> __host__ __device__ constexpr int group_evals() { return GROUP > 1 ? (6 + GROUP - 1) / GROUP : 1; }
+
+// Word that lane J of the lane's group of GROUP holds.
+template <int GROUP, int J>
+__device__ __forceinline__ int group_word(int v)
+{
+    constexpr int j = J & 3, quad = j | j << 2 | j << 4 | j << 6;
+    int q = __builtin_amdgcn_update_dpp(0, v, quad, 0xf, 0xf, true);            // lane j of each 4 lanes
+    if (GROUP == 8)                                                             // the other 4 take it mirrored
+        q = __builtin_amdgcn_update_dpp(q, q, 0x141, 0xf, J < 4 ? 0xa : 0x5, false);
+    return q;
+}
+template <int GROUP, int J> __device__ __forceinline__ float group_value(float v)
+{
+    return __builtin_bit_cast(float, group_word<GROUP, J>(__builtin_bit_cast(int, v)));
+}
+template <int GROUP, int J> __device__ __forceinline__ double group_value(double v)
+{
+    const uint64_t b = math::bits(v);
+    const uint32_t lo = (uint32_t)group_word<GROUP, J>((int)(uint32_t)b), hi = (uint32_t)group_word<GROUP, J>((int)(uint32_t)(b >> 32));
+    return math::from_bits(((uint64_t)hi << 32) | lo);
+}
+// The node c of the stage whose terms the lane evaluates in evaluation e: its
+// time is fma(h, c, t), as in the stepper (t itself for c = 0, t + h for c = 1).
+template <int GROUP, class P>
+__device__ __forceinline__ P stage_node(int e)
+{
+    const int j = e * GROUP + (int)(threadIdx.x & (GROUP - 1));
+    P c = P(7.0 / 8.0);
+    c = j == 0 ? P(0) : c;
+    c = j == 1 ? P(1.0 / 5.0) : c;
+    c = j == 2 ? P(3.0 / 10.0) : c;
+    c = j == 3 ? P(3.0 / 5.0) : c;
+    return j == 4 ? P(1) : c;
+}
+
 // What a step reads of the argument block.  The control limits and tolerances
 // are put into vector registers once, before the step loop: in scalar registers
 // they and the step's constants exceed the 102 there are, and the compiler
@@ -192,6 +240,7 @@ struct StepArgs {
     P etol[Pos<NE>::value];
     int edir[Pos<NE>::value];
     int NT, NDO, doFreq;
+    P node[2];                  // several lanes per instance: stage_node of this lane
 
     template <class T> static __device__ __forceinline__ T pin(T v)
     {
@@ -218,6 +267,11 @@ struct StepArgs {
             etol[i] = pin(a.etol[i]);
             edir[i] = a.edir[i];
         }
+    }
+    template <int GROUP> __device__ __forceinline__ void set_nodes()
+    {
+#pragma unroll
+        for (int e = 0; e < group_evals<GROUP>(); e++) node[e] = pin(stage_node<GROUP, P>(e));
     }
 };
 
@@ -437,17 +491,37 @@ struct Lane {
 
     // RKCK45: PT-STP:121-290.  err[] in control precision.  tt: the time terms
     // at t; tt5 receives those at t + h.
+    template <int GROUP>
     __device__ __forceinline__ void rkck45(const C& a, P h, P* nx, P* inc, CP* err, P* sPAR, int* sPARi, const P* tt, P* tt5)
     {
         using math::fma;
         P Xs[SD], k1[SD], k2[SD], k3[SD], k4[SD], k5[SD], k6[SD];
         P ts[Pos<NTT>::value];
-        ode(a.NT, k1, X, t, tt, sPAR, sPARi);
+        P all[group_evals<GROUP>()][Pos<NTT>::value];
+        if constexpr (GROUP > 1) {
+#pragma unroll
+            for (int e = 0; e < group_evals<GROUP>(); e++) time_terms(fma(h, a.node[e], t), all[e]);
+        }
+        // the time terms of stage J, at T
+        auto terms = [&](auto J, P T, P* r) {
+            if constexpr (GROUP > 1) {
+#pragma unroll
+                for (int i = 0; i < NTT; i++) r[i] = group_value<GROUP, J.value % GROUP>(all[J.value / GROUP][i]);
+            } else {
+                time_terms(T, r);
+            }
+        };
+        if constexpr (GROUP > 1) {
+            terms(std::integral_constant<int, 0>{}, t, ts);
+            ode(a.NT, k1, X, t, ts, sPAR, sPARi);
+        } else {
+            ode(a.NT, k1, X, t, tt, sPAR, sPARi);
+        }
 
         P T = fma(h, P(1.0 / 5.0), t);
 #pragma unroll
         for (int i = 0; i < SD; i++) Xs[i] = fma(h, P(1.0 / 5.0) * k1[i], X[i]);
-        time_terms(T, ts);
+        terms(std::integral_constant<int, 1>{}, T, ts);
         ode(a.NT, k2, Xs, T, ts, sPAR, sPARi);
 
         T = fma(h, P(3.0 / 10.0), t);
@@ -457,7 +531,7 @@ struct Lane {
             s = fma(P(9.0 / 40.0), k2[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        time_terms(T, ts);
+        terms(std::integral_constant<int, 2>{}, T, ts);
         ode(a.NT, k3, Xs, T, ts, sPAR, sPARi);
 
         T = fma(h, P(3.0 / 5.0), t);
@@ -468,7 +542,7 @@ struct Lane {
             s = fma(P(6.0 / 5.0), k3[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        time_terms(T, ts);
+        terms(std::integral_constant<int, 3>{}, T, ts);
         ode(a.NT, k4, Xs, T, ts, sPAR, sPARi);
 
         T = t + h;
@@ -480,7 +554,7 @@ struct Lane {
             s = fma(P(35.0 / 27.0), k4[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        time_terms(T, tt5);
+        terms(std::integral_constant<int, 4>{}, T, tt5);
         ode(a.NT, k5, Xs, T, tt5, sPAR, sPARi);
 
         T = fma(h, P(7.0 / 8.0), t);
@@ -493,7 +567,7 @@ struct Lane {
             s = fma(P(253.0 / 4096.0), k5[i], s);
             Xs[i] = fma(h, s, X[i]);
         }
-        time_terms(T, ts);
+        terms(std::integral_constant<int, 5>{}, T, ts);
         ode(a.NT, k6, Xs, T, ts, sPAR, sPARi);
 
 #pragma unroll
@@ -594,8 +668,8 @@ struct Lane {
     // dense-output bookkeeping out (the adjoint's re-steps, which run with
     // NDO = 0), so that the step has no branch on it.  CARRY: tt holds the time
     // terms at t (time_terms(t, tt) before the first step); else they are
-    // evaluated anew.
-    template <bool DENSE = true, bool CARRY = false>
+    // evaluated anew.  GROUP: several lanes per instance (RKCK45, no CARRY).
+    template <bool DENSE = true, bool CARRY = false, int GROUP = 1>
     __device__ __forceinline__ bool step(const C& a, P* sPAR, int* sPARi, bool& accepted, P* tt = nullptr)
     {
         const int NT = a.NT;
@@ -614,7 +688,7 @@ struct Lane {
         if constexpr (CARRY) {
 #pragma unroll
             for (int i = 0; i < NTT; i++) tt1[i] = tt[i];
-        } else {
+        } else if constexpr (GROUP == 1) {
             time_terms(t, tt1);
         }
         P EFn[Pos<NE>::value];
@@ -634,7 +708,7 @@ struct Lane {
             stop = term != 0;
         } else {
             CP err[SD], tol[SD];
-            rkck45(a, h, nx, inc, err, sPAR, sPARi, tt1, ttEnd);
+            rkck45<GROUP>(a, h, nx, inc, err, sPAR, sPARi, tt1, ttEnd);
             if (NE > 0) Sys::template EventFunction<P>(tid, NT, EFn, t + h, dtP, TD, nx, cPAR, sPAR, sPARi, ACC, ACCi);
             // Nearly always every lane of the wavefront has an accepted, finite
             // step above the smallest size with no event near: u < 0 in one
@@ -916,21 +990,25 @@ __device__ __forceinline__ void stage_shared(const Args<Sys, P, CP>& a, P*& sPAR
     }
 }
 
-// Reference form: lane = instance, whole integration in one launch.
-template <class Sys, class P, bool KAHAN, int ALG, bool SLICED = false>
-__device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP>& a)
+// Reference form: lane = instance, whole integration in one launch.  GROUP: that
+// many lanes per instance (whole wavefronts; its first lane stores).  Instances
+// list[first + ...) in the order of the lanes of workgroups `block0` and later.
+template <class Sys, class P, bool KAHAN, int ALG, bool SLICED = false, int GROUP = 1>
+__device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP>& a, int block0 = 0, int first = 0)
 {
     P* sPAR; int* sPARi;
     stage_shared(a, sPAR, sPARi);
-    const int i = threadIdx.x + blockIdx.x * blockDim.x;
+    const int i = first + (int)(threadIdx.x / GROUP) + ((int)blockIdx.x - block0) * (int)(blockDim.x / GROUP);
     const int n = (SLICED && a.listLenDev) ? (int)*a.listLenDev : a.listLen;
     using L_t = Lane<Sys, P, KAHAN, ALG>;
     L_t L;
-    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    if constexpr (GROUP > 1) c.template set_nodes<GROUP>();
+    const bool stores = GROUP == 1 || threadIdx.x % GROUP == 0;
     const int id = i < n ? (a.list ? a.list[i] : i) : 0;
     constexpr bool COMMON = !SLICED && L_t::kCommonTime;
     // a step's end is the next one's start (in the compensated form it is not t + h)
-    constexpr bool CARRY = L_t::NTT > 0 && !KAHAN;
+    constexpr bool CARRY = L_t::NTT > 0 && !KAHAN && GROUP == 1;
     P tt[Pos<L_t::NTT>::value];
     if constexpr (COMMON) {
         if (i < n) L.load(a, id, sPAR, sPARi);
@@ -947,22 +1025,37 @@ __device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys,
             // the loop only steps; finishing or suspending follows it, so
             // the step loop keeps the plain form's registers
             L.begin(a, id, sPAR, sPARi);
-            L.time_terms(L.t, tt);
+            if (CARRY) L.time_terms(L.t, tt);
             // the budget is the same for every lane
             int left = a.slice;
             bool ended, accepted;
-            do ended = L.template step<true, CARRY>(c, sPAR, sPARi, accepted, tt);
+            do ended = L.template step<true, CARRY, GROUP>(c, sPAR, sPARi, accepted, tt);
             while (!ended && --left > 0);
             if (ended) L.term = 1;
-            L.release(kernel_args<typename L_t::A>(), sPAR, sPARi);
+            if (stores) L.release(kernel_args<typename L_t::A>(), sPAR, sPARi);
         } else {
             if constexpr (!COMMON) L.load(a, id, sPAR, sPARi);
-            L.time_terms(L.t, tt);
+            if (CARRY) L.time_terms(L.t, tt);
             bool ended = L.term != 0, accepted;
-            while (!ended) ended = L.template step<true, CARRY>(c, sPAR, sPARi, accepted, tt);
+            while (!ended) ended = L.template step<true, CARRY, GROUP>(c, sPAR, sPARi, accepted, tt);
+            if (!stores) return;
             if constexpr (COMMON) L.finish(kernel_args_joined<typename L_t::A>(), sPAR, sPARi);
             else L.finish(kernel_args<typename L_t::A>(), sPAR, sPARi);
         }
+    }
+}
+
+// Sorted form's long launch: the first a.octets workgroups give their instances
+// (the longest ones) 8 lanes each.
+template <class Sys, class P, bool KAHAN, int ALG>
+__device__ __forceinline__ void mixed_body(const Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP>& a)
+{
+    if ((int)blockIdx.x < a.octets) {
+        // before the others that share its SIMD: it decides when the launch ends
+        __builtin_amdgcn_s_setprio(2);
+        plain_body<Sys, P, KAHAN, ALG, true, 8>(a);
+    } else {
+        plain_body<Sys, P, KAHAN, ALG, true>(a, a.octets, a.octets * (int)(blockDim.x / 8));
     }
 }
 

@@ -51,6 +51,9 @@ inline int bound_check(const char* fn, const char* what, int v, int lo, int hi)
 
 namespace pt {
 
+// forms with several lanes per instance (RKCK45, systems with time terms)
+constexpr int kOctetMode = 4, kQuadMode = 5, kMixedMode = 6;
+
 // Kernel entry points.  WPE is the waves-per-EU hint of the register-budget
 // variant (1 = no constraint); MODE 0 = plain, 1 = persistent.
 template <class Sys, class P, bool KAHAN, int ALG, int MODE, int WPE>
@@ -58,10 +61,12 @@ __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(
 solve_kernel(Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP> a)
 {
     // MODE + 2: the same forms with the time-sliced lane lifecycle
-    if (MODE == MPGOS_KERNEL_PLAIN) plain_body<Sys, P, KAHAN, ALG>(a);
-    else if (MODE == MPGOS_KERNEL_PERSISTENT) persistent_body<Sys, P, KAHAN, ALG>(a);
-    else if (MODE == MPGOS_KERNEL_PLAIN + 2) plain_body<Sys, P, KAHAN, ALG, true>(a);
-    else persistent_body<Sys, P, KAHAN, ALG, true>(a);
+    if constexpr (MODE == MPGOS_KERNEL_PLAIN) plain_body<Sys, P, KAHAN, ALG>(a);
+    else if constexpr (MODE == MPGOS_KERNEL_PERSISTENT) persistent_body<Sys, P, KAHAN, ALG>(a);
+    else if constexpr (MODE == MPGOS_KERNEL_PLAIN + 2) plain_body<Sys, P, KAHAN, ALG, true>(a);
+    else if constexpr (MODE == MPGOS_KERNEL_PERSISTENT + 2) persistent_body<Sys, P, KAHAN, ALG, true>(a);
+    else if constexpr (MODE == kMixedMode) mixed_body<Sys, P, KAHAN, ALG>(a);
+    else plain_body<Sys, P, KAHAN, ALG, false, MODE == kOctetMode ? 8 : 4>(a);
 }
 
 // Virtual interface the C ABI talks to; one implementation per (system, precision).
@@ -533,6 +538,37 @@ public:
         }
     }
 
+    // Several lanes per instance (pt_device.h): RKCK45 systems with time terms,
+    // in whole wavefronts, as long as every wavefront has a SIMD to itself; a
+    // second one on a SIMD costs more than the shared evaluations save.  The
+    // launch variants other than the default are the user's choice of
+    // registers and keep one lane per instance.  Duffing oscillators with a
+    // quadrature state, Solve | reverse pass in ms with 1, 4 and 8 lanes:
+    //   8192 instances  1.11 | 2.38   0.84 | 1.79   0.77 | 1.65
+    //  10007            1.14 | 2.43   0.86 | 1.81   1.07 | 2.59
+    //  16384            1.12 | 2.43   0.89 | 1.85   1.20 | 3.72
+    //  20000            1.14 | 2.47   1.25 | 2.89   1.61 | 4.63
+    static constexpr bool kGroups = TimeTermsOf<Sys>::n > 0;
+    int lanes_per_instance(int n, int B) const
+    {
+        if (!kGroups || algorithm != MPGOS_RKCK45 || variant != 0 || B % 64 != 0) return 1;
+        const long simds = 4L * numCU;
+        return 8L * n <= 64 * simds ? 8 : 4L * n <= 64 * simds ? 4 : 1;
+    }
+    // Workgroups of the sorted form's last launch that give an instance 8 lanes:
+    // the longest instances, as many as leave every wavefront a SIMD to itself,
+    // and on three quarters of the SIMDs where the card is full all the same.
+    // Uneven Duffing oscillators with logged events, ms with 0, 512, 712 and 1024
+    // such wavefronts: 20000 instances 107.9, 66.1, 61.9, 62.0; 65536 35.9, 21.6,
+    // 18.5, 26.3; 131072 34.9, 28.8, 25.2, 31.6.
+    int octet_blocks(int B) const
+    {
+        if (!kGroups || algorithm != MPGOS_RKCK45 || variant != 0 || B % 64 != 0) return 0;
+        const int simds = 4 * numCU, waves = (nActive + 63) / 64;
+        const int octets = std::min(std::max(simds - waves, simds * 3 / 4), (nActive + 7) / 8);
+        return (octets * 64 + B - 1) / B;
+    }
+
     KernelFn kernel(bool sliced = false) const
     {
         const bool plain = kernelMode != MPGOS_KERNEL_PERSISTENT;
@@ -542,6 +578,11 @@ public:
                                      : pick_variant<MPGOS_RK4, MPGOS_KERNEL_PERSISTENT + 2>(variant);
             return plain ? pick_variant<MPGOS_RK4, MPGOS_KERNEL_PLAIN>(variant)
                          : pick_variant<MPGOS_RK4, MPGOS_KERNEL_PERSISTENT>(variant);
+        }
+        if constexpr (kGroups) {
+            const int g = sliced || !plain ? 1 : lanes_per_instance(NT, blockSize);
+            if (g == 8) return solve_kernel<Sys, P, KAHAN, MPGOS_RKCK45, kOctetMode, 1>;
+            if (g == 4) return solve_kernel<Sys, P, KAHAN, MPGOS_RKCK45, kQuadMode, 1>;
         }
         if (sliced) return plain ? pick_variant<MPGOS_RKCK45, MPGOS_KERNEL_PLAIN + 2>(variant)
                                  : pick_variant<MPGOS_RKCK45, MPGOS_KERNEL_PERSISTENT + 2>(variant);
@@ -562,7 +603,8 @@ public:
     {
         const int B = block();
         if (kernelMode == MPGOS_KERNEL_PLAIN) {
-            grid = NT / B + (NT % B == 0 ? 0 : 1);   // PT-IF:344
+            const int per = B / lanes_per_instance(NT, B);   // instances of a workgroup
+            grid = NT / per + (NT % per == 0 ? 0 : 1);   // PT-IF:344
             return MPGOS_OK;
         }
         if (kernelMode == MPGOS_KERNEL_RELAUNCH || kernelMode == MPGOS_KERNEL_SORTED) {   // lists are at most nActive long
@@ -653,6 +695,14 @@ public:
                            r.counts, sortHist, r.listB);
         b.list = r.listB; b.listOut = nullptr; b.listLenDev = r.counts; b.outCount = nullptr;
         b.slice = 0x7fffffff; b.sortKey = nullptr;
+        if constexpr (kGroups) {
+            if (const int octets = octet_blocks(B)) {
+                b.octets = octets;
+                const int rest = nActive - octets * (B / 8);
+                grid = octets + (rest > 0 ? (rest + B - 1) / B : 0);
+                fn = solve_kernel<Sys, P, KAHAN, MPGOS_RKCK45, kMixedMode, 1>;
+            }
+        }
         hipLaunchKernelGGL(fn, dim3(grid), dim3(B), lds, strm, b);
         MPGOS_HIP_TRY(hipGetLastError());
         return MPGOS_OK;
@@ -916,11 +966,17 @@ public:
             AdjArgs<Sys> A;
             adjoint_args(A);
             const int B = blockSize;
-            const int grid = NT / B + (NT % B == 0 ? 0 : 1);
+            const int group = lanes_per_instance(NT, B), per = B / group;
+            const int grid = NT / per + (NT % per == 0 ? 0 : 1);
             const size_t lds = preferShared ? (size_t)NSP * sizeof(P) + (size_t)NISP * sizeof(int) : 0;
             MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((adjoint_record_kernel<Sys, MPGOS_RK4>), dim3(grid), dim3(B), lds, strm, A);
-            else hipLaunchKernelGGL((adjoint_record_kernel<Sys, MPGOS_RKCK45>), dim3(grid), dim3(B), lds, strm, A);
+            void (*fn)(AdjArgs<Sys>) = adjoint_record_kernel<Sys, MPGOS_RKCK45>;
+            if (algorithm == MPGOS_RK4) fn = adjoint_record_kernel<Sys, MPGOS_RK4>;
+            if constexpr (kGroups) {
+                if (group == 8) fn = adjoint_record_kernel<Sys, MPGOS_RKCK45, 8>;
+                if (group == 4) fn = adjoint_record_kernel<Sys, MPGOS_RKCK45, 4>;
+            }
+            hipLaunchKernelGGL(fn, dim3(grid), dim3(B), lds, strm, A);
             MPGOS_HIP_TRY(hipGetLastError());
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;
@@ -949,7 +1005,8 @@ public:
             A.a.NDO = 0;       // the recomputation writes nothing but the segment buffer
             A.a.evcap = 0;
             const int B = blockSize;
-            const int grid = NT / B + (NT % B == 0 ? 0 : 1);
+            const int group = lanes_per_instance(NT, B), per = B / group;
+            const int grid = NT / per + (NT % per == 0 ? 0 : 1);
             const bool ldsSeg = segment_in_lds(adjK);
             const size_t lds = adjoint_shared_bytes<Sys>(preferShared) + (ldsSeg ? segment_lds_bytes(adjK) : 0);
             if (!ldsSeg && segCount < (size_t)adjK * (SD + 2) * NT) {
@@ -957,13 +1014,13 @@ public:
                 return MPGOS_E_STATE;
             }
             MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-            if (ldsSeg) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((adjoint_reverse_kernel<Sys, MPGOS_RK4, true>), dim3(grid), dim3(B), lds, strm, A);
-                else hipLaunchKernelGGL((adjoint_reverse_kernel<Sys, MPGOS_RKCK45, true>), dim3(grid), dim3(B), lds, strm, A);
-            } else {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((adjoint_reverse_kernel<Sys, MPGOS_RK4, false>), dim3(grid), dim3(B), lds, strm, A);
-                else hipLaunchKernelGGL((adjoint_reverse_kernel<Sys, MPGOS_RKCK45, false>), dim3(grid), dim3(B), lds, strm, A);
+            void (*fn)(AdjArgs<Sys>) = ldsSeg ? adjoint_reverse_kernel<Sys, MPGOS_RKCK45, true> : adjoint_reverse_kernel<Sys, MPGOS_RKCK45, false>;
+            if (algorithm == MPGOS_RK4) fn = ldsSeg ? adjoint_reverse_kernel<Sys, MPGOS_RK4, true> : adjoint_reverse_kernel<Sys, MPGOS_RK4, false>;
+            if constexpr (kGroups) {
+                if (group == 8) fn = ldsSeg ? adjoint_reverse_kernel<Sys, MPGOS_RKCK45, true, 8> : adjoint_reverse_kernel<Sys, MPGOS_RKCK45, false, 8>;
+                if (group == 4) fn = ldsSeg ? adjoint_reverse_kernel<Sys, MPGOS_RKCK45, true, 4> : adjoint_reverse_kernel<Sys, MPGOS_RKCK45, false, 4>;
             }
+            hipLaunchKernelGGL(fn, dim3(grid), dim3(B), lds, strm, A);
             MPGOS_HIP_TRY(hipGetLastError());
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;

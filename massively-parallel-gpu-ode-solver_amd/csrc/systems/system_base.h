@@ -14,7 +14,8 @@
 // Systems whose right-hand side contains terms of the time (and the control
 // parameters) alone may name them, so that the solver evaluates them once and
 // reuses them (a step's end is the next step's start; with a fixed step and a
-// time common to a wavefront, its lanes evaluate different times at once):
+// time common to a wavefront, its lanes evaluate different times at once; with
+// few instances, several lanes make one's steps and evaluate a stage's terms each):
 //   NTT                                       number of such terms
 //   TT_TIME_ONLY                              true when no parameter enters them
 //   TimeTerms(T, cPAR, tt)                    evaluates them
@@ -25,7 +26,8 @@
 // Per-block systems take (sid, uid) for (tid, NT) and the system parameters for
 // cPAR, with the argument lists of their OdeFunction and OdeVJP.
 // Such a system leaves T, the time domain and the parameters in its terms
-// alone after Initialization.
+// alone after Initialization, and its callbacks change only what they are
+// given for the instance (several lanes may make the same steps of one).
 // Every callback is MPGOS_HD so the same definition serves the gfx950 kernels
 // and the host oracle; elementary functions come from mpgos::math so both
 // sides evaluate identical bits.
