@@ -28,6 +28,7 @@
 namespace mpgos {
 namespace pb {
 
+using pt::Arena;
 using pt::Buffer;
 
 class SolverBase {
@@ -82,6 +83,8 @@ public:
     Buffer<P> X, uPAR, uACC, TD, T, sPAR, sACC, strength, DOt, DOx, gPAR, cMat;
     Buffer<int> uACCi, sACCi, DOidx, gPARi, cIndex, status;
     Buffer<long long> nacc, nrej;
+    Arena arena;                   // of all buffers
+    size_t allIn = 0, allOut = 0;  // its bytes that a transfer of All moves up and down
     std::vector<P> cMatOriginal;   // the full matrices as set (GetHost), NC * UPS * UPS
 
     // discrete adjoint (FP64 systems with OdeVJP)
@@ -98,12 +101,9 @@ public:
     ~Solver() override
     {
         if (strm) (void)hipStreamSynchronize(strm);
-        lamB.release(); gUB.release(); gSB.release();
         for (double* q : {recX, recT, recH, seg, cMatT, stg, gSp, cTile, cTileT})
             if (q) (void)hipFree(q);
-        for (auto* b : {&X, &uPAR, &uACC, &TD, &T, &sPAR, &sACC, &strength, &DOt, &DOx, &gPAR, &cMat}) b->release();
-        for (auto* b : {&uACCi, &sACCi, &DOidx, &gPARi, &cIndex, &status}) b->release();
-        nacc.release(); nrej.release();
+        arena.release();
         if (syncEvent) (void)hipEventDestroy(syncEvent);
         if (evStart) (void)hipEventDestroy(evStart);
         if (evStop) (void)hipEventDestroy(evStop);
@@ -135,28 +135,32 @@ public:
         cus = std::max(1, prop.multiProcessorCount);
         const size_t NU = (size_t)NS * UPS;
         int rc;
-        if ((rc = X.alloc(UD * NU)) || (rc = uPAR.alloc(NUP * NU)) || (rc = uACC.alloc(NUA * NU)) ||
-            (rc = uACCi.alloc(NiUA * NU)) || (rc = TD.alloc(2 * (size_t)NS)) || (rc = T.alloc(NS)) ||
-            (rc = sPAR.alloc((size_t)NSP * NS)) || (rc = sACC.alloc((size_t)NSA * NS)) || (rc = sACCi.alloc((size_t)NiSA * NS)) ||
-            (rc = strength.alloc((size_t)NC * NS)) || (rc = DOidx.alloc(NS)) || (rc = DOt.alloc((size_t)NDO * NS)) ||
-            (rc = DOx.alloc((size_t)NDO * UD * NU)) || (rc = gPAR.alloc(NGP)) || (rc = gPARi.alloc(NiGP)) ||
-            (rc = cIndex.alloc(NC)) || (rc = cMat.alloc((size_t)NC * cMatSize)) || (rc = status.alloc(NS)) ||
-            (rc = nacc.alloc(NS)) || (rc = nrej.alloc(NS)))
-            return rc;
+        // in the order of a transfer of All: what goes both ways, then the outputs
+        const size_t ns_ = (size_t)NS;
+        X.place(arena, UD * NU); uPAR.place(arena, NUP * NU); uACC.place(arena, NUA * NU); uACCi.place(arena, NiUA * NU);
+        TD.place(arena, 2 * ns_); T.place(arena, ns_); sPAR.place(arena, NSP * ns_); sACC.place(arena, NSA * ns_);
+        sACCi.place(arena, NiSA * ns_); strength.place(arena, NC * ns_); DOidx.place(arena, ns_); DOt.place(arena, (size_t)NDO * ns_);
+        DOx.place(arena, (size_t)NDO * UD * NU); gPAR.place(arena, NGP); gPARi.place(arena, NiGP); cIndex.place(arena, NC);
+        cMat.place(arena, (size_t)NC * cMatSize);
+        allIn = arena.n;
+        nacc.place(arena, ns_); nrej.place(arena, ns_); status.place(arena, ns_);
+        allOut = arena.n;
+        if (kAdjoint) { lamB.place(arena, UD * NU); gUB.place(arena, NUP * NU); gSB.place(arena, NSP * ns_); }
+        if ((rc = arena.alloc())) return rc;
+        for (auto* q : {&X, &uPAR, &uACC, &TD, &T, &sPAR, &sACC, &strength, &DOt, &DOx, &gPAR, &cMat, &lamB, &gUB, &gSB}) q->bind(arena);
+        for (auto* q : {&uACCi, &sACCi, &DOidx, &gPARi, &cIndex, &status}) q->bind(arena);
+        nacc.bind(arena); nrej.bind(arena);
         if (dense_possible() && hipMalloc((void**)&cTile, (size_t)NC * dense_matrix_size(UPS) * sizeof(double)) != hipSuccess) {
             cTile = nullptr;
             set_error("per-block: allocation of the tiled coupling matrix failed");
             return MPGOS_E_MEMORY;
         }
-        if (kAdjoint && ((rc = lamB.alloc(UD * NU)) || (rc = gUB.alloc(NUP * NU)) || (rc = gSB.alloc((size_t)NSP * NS))))
-            return rc;
         cMatOriginal.assign((size_t)NC * UPS * UPS, P(0));
         rtol.assign(UD, 1e-8);
         atol.assign(UD, 1e-8);
         etol.assign(NE, 1e-6);
         edir.assign(NE, 0);
-        if ((rc = copy(status, true)) || (rc = copy(nacc, true)) || (rc = copy(nrej, true))) return rc;
-        return sync(MPGOS_PB_ALL, true);
+        return arena.copy(allOut, true, strm);
     }
 
     int dims(mpgos_pb_dims* d) const override
@@ -374,12 +378,7 @@ public:
         int rc = MPGOS_OK;
         switch (var) {
         case MPGOS_PB_ALL:
-            for (int v = MPGOS_PB_TIME_DOMAIN; v <= MPGOS_PB_DENSE_STATE; v++) {
-                if (v == MPGOS_PB_DENSE_OUTPUT) continue;
-                if ((rc = sync(v, to_device))) return rc;
-            }
-            if (!to_device && ((rc = copy(nacc, false)) || (rc = copy(nrej, false)) || (rc = copy(status, false)))) return rc;
-            return MPGOS_OK;
+            return arena.copy(to_device ? allIn : allOut, to_device, strm);
         case MPGOS_PB_DENSE_OUTPUT:
             if ((rc = copy(DOidx, to_device)) || (rc = copy(DOt, to_device)) || (rc = copy(DOx, to_device))) return rc;
             return MPGOS_OK;
