@@ -469,11 +469,11 @@ __device__ __forceinline__ double rk_a(int s, int l)
 // return the same bits.
 //
 // What bounds it: the latency of a step (1024 x 128 units: two wavefronts per
-// SIMD) and, with 8 systems of 256 units, the registers (89 of the sweep's
+// SIMD) and, with 8 systems of 256 units, the registers (78 of the sweep's
 // values per lane spill).  Reverse pass of two periods of 1024 x 128 units
-// 24.6 -> 7.9 ms, one period of 300 x 256 25.6 -> 14.6, 4096 x 128 21.1 -> 14.6,
-// 4096 x 256 57.1 -> 51.9 ms against products through LDS with 8 systems per
-// workgroup; 1000 x 100 units 40.5 -> 3.4 ms against one lane per unit.
+// 24.6 -> 7.3 ms, one period of 300 x 256 25.6 -> 14.6, 4096 x 128 21.1 -> 14.3,
+// 4096 x 256 57.1 -> 49.8 ms against products through LDS with 8 systems per
+// workgroup; 1000 x 100 units 40.5 -> 3.0 ms against one lane per unit.
 template <class Sys, int NSL, int MT>
 struct DenseRev {
     static constexpr int TT = dense_tt(MT);
@@ -769,7 +769,10 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
 #pragma unroll
         for (int c = 0; c < NSP; c++) muS[s][q][c] = (ld && r > 0) ? C.row(A.gSp, c)[u] : P(0);
     }
-    // a stage's inputs and coupling values, loaded one stage ahead
+    // a stage's inputs and coupling values, loaded one stage ahead where the
+    // registers hold them (with 4 results per lane they would be spilled:
+    // reverse pass of 4096 x 256 units 54.6 against 49.8 ms)
+    constexpr bool AHEAD = NSL * TT < 4;
     P ahead[NSL][TT][SW];
     auto fetch = [&](int j, int st) {
         const size_t base = ((size_t)j * ST + st) * SW;
@@ -784,7 +787,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
     P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value], tt[NSL][Pos<NTT>::value];
     P t[NSL], h[NSL], tn[NSL], hn[NSL];
     C.step_times(a, C.maxlen - 1, tn, hn);
-    fetch(C.maxlen - 1, ST - 1);
+    if (AHEAD) fetch(C.maxlen - 1, ST - 1);
     for (int j = C.maxlen - 1; j >= 0; j--) {
 #pragma unroll
         for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
@@ -802,6 +805,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
         for (int st = ST - 1; st >= 0; st--) {
             P Y[NSL][TT][UD], kbCPF[NSL][TT][NCp], w[NCp][NSL][TT];
             P* wb = C.cptBuf + (size_t)buf * C.cptStride;
+            if (!AHEAD) fetch(j, st);
             MPGOS_PB_EACH(s, q) {
 #pragma unroll
                 for (int c = 0; c < UD; c++) Y[s][q][c] = ahead[s][q][c];
@@ -828,8 +832,10 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
                     }
                 }
             }
-            if (st > 0) fetch(j, st - 1);
-            else fetch(j - 1, ST - 1);
+            if (AHEAD) {
+                if (st > 0) fetch(j, st - 1);
+                else fetch(j - 1, ST - 1);
+            }
             product.prefetch();
             lds_barrier();
             product.run(wb, w);
