@@ -43,7 +43,7 @@ namespace pb {
 template <class Sys>
 struct AdjArgs {
     double* seg;          // [K][UD][NU] (lane form)
-    double* stg;          // [K][stages][UD + NC][NU] stage inputs and coupling values (dense-contraction form)
+    double* stg;          // [K * rev_rows][NU] stage buffer (dense-contraction form)
     double* gSp;          // [NSP][NU] per-unit partials of dL/d(system parameters) (dense-contraction form)
     double* lam;          // in: dL/dx(end), out: dL/dx(start)      [UD][NU]
     double* gU;           // out: dL/d(unit parameters)             [NUP][NU]
@@ -448,18 +448,36 @@ __device__ __forceinline__ double rk_a(int s, int l)
     return l < s ? A[s][l] : 0.0;
 }
 
+// Input of stage st > 0 by the forward pass's arithmetic: x and the stages before.
+template <int ALG, int UD, int ST>
+__device__ __forceinline__ double rk_stage_input(int st, int c, double h, const double (&x)[UD], const double (&k)[ST][UD])
+{
+    using math::fma;
+    if (ALG == MPGOS_RK4) return fma(st == 3 ? k[2][c] : k[st - 1][c] * 0.5, h, x[c]);
+    double r = 0.0;
+    switch (st) {
+    case 1: r = k[0][c] * (1.0 / 5.0); break;
+    case 2: r = fma(k[1][c], 9.0 / 40.0, k[0][c] * (3.0 / 40.0)); break;
+    case 3: r = fma(k[2][c], 6.0 / 5.0, fma(k[1][c], -9.0 / 10.0, k[0][c] * (3.0 / 10.0))); break;
+    case 4: r = fma(k[ST - 3][c], 35.0 / 27.0, fma(k[2][c], -70.0 / 27.0, fma(k[1][c], 5.0 / 2.0, k[0][c] * (-11.0 / 54.0)))); break;
+    default:
+        r = fma(k[ST - 2][c], 253.0 / 4096.0, fma(k[ST - 3][c], 44275.0 / 110592.0, fma(k[2][c], 575.0 / 13824.0,
+                fma(k[1][c], 175.0 / 512.0, k[0][c] * (1631.0 / 55296.0)))));
+    }
+    return fma(r, h, x[c]);
+}
+
 // Reverse pass in the dense-contraction form (full FP64 coupling matrices, up
 // to 256 units): the layout of pb_dense.h, every coupling product on
 // v_mfma_f64_4x4x4f64 -- M CPT(Y) in the segment replay, M^T w in the adjoint
 // sweep.  Round r handles the r-th segment from the end of every system in two
 // launches:
 //   pb_replay_kernel: restore checkpoint k = nseg - 1 - r and replay the
-//     segment's recorded steps, keeping each stage's input Y_s and coupling
-//     values v_s in the stage buffer
-//       stg[(((j * ST + s) * (UD + NC)) + c) * NU + unit],  j < K;
+//     segment's recorded steps, keeping each stage's coupling values v_s, and
+//     the step's state or each stage's input Y_s, in the stage buffer of rows
+//     [row][NU], rev_rows() of them per step;
 //   pb_sweep_kernel: the adjoint sweep through the segment from the stage
-//     buffer (no forward coupling product again; CPF_s from the unit's
-//     right-hand side at (Y_s, T_s)); dL/dx, the unit-parameter gradient and
+//     buffer (no forward coupling product again); dL/dx, the unit-parameter gradient and
 //     the per-unit system-parameter partials carry over between rounds in HBM
 //     (lam, gU, gSp);
 // pb_reverse_finish_kernel sums the partials per system in unit order.  Two
@@ -471,16 +489,34 @@ __device__ __forceinline__ double rk_a(int s, int l)
 // What bounds it: the latency of a step (1024 x 128 units: two wavefronts per
 // SIMD) and, with 8 systems of 256 units, the registers (78 of the sweep's
 // values per lane spill).  Reverse pass of two periods of 1024 x 128 units
-// 24.6 -> 7.3 ms, one period of 300 x 256 25.6 -> 14.6, 4096 x 128 21.1 -> 14.3,
+// 24.6 -> 6.8 ms, one period of 300 x 256 25.6 -> 14.6, 4096 x 128 21.1 -> 14.3,
 // 4096 x 256 57.1 -> 49.8 ms against products through LDS with 8 systems per
-// workgroup; 1000 x 100 units 40.5 -> 3.0 ms against one lane per unit.
+// workgroup; 1000 x 100 units 40.5 -> 2.9 ms against one lane per unit.
+// Stage buffer: with one result per lane the step's state and the stages'
+// coupling values, from which the sweep makes the stage inputs again (all of them
+// stay in its registers); with more the inputs themselves.  At 1024 x 128 units of
+// the ring with a quadrature state a step moves 9 rows, 9.4 MB each way, instead
+// of 24, 25 MB: reverse pass of two periods 7.1 -> 6.8 ms, smaller ones unchanged
+// (the sweep makes up for it with the right-hand sides it evaluates).
+template <class Sys>
+__host__ __device__ inline size_t rev_lds_bytes(int SPB, int UPS, int ldsPairs)
+{
+    return dense_layout<RevScope<Sys>, Sys::NC, 0, 0>(SPB, UPS, 0, ldsPairs).total + 2 * sizeof(double) * (size_t)SPB * 64;
+}
+template <int NSL, int MT> __host__ __device__ constexpr bool rev_remake() { return NSL * dense_tt(MT) == 1; }
+template <class Sys> __host__ __device__ constexpr int rev_rows(bool remake, int ST)
+{
+    return remake ? Sys::UD + ST * Sys::NC : ST * (Sys::UD + Sys::NC);
+}
+
 template <class Sys, int NSL, int MT>
 struct DenseRev {
     static constexpr int TT = dense_tt(MT);
     static constexpr int NC = Sys::NC, SPB = 4 * NSL, NTT = TimeTermsOf<Sys>::n, PER = 64 / SPB;
+    static constexpr int kTimes = 64;
     using Scope = RevScope<Sys>;
     using Place = DensePlace<NSL, TT>;
-    Scope* sys; double* cptBuf; const double* Ml;
+    Scope* sys; double* cptBuf; const double* Ml; double* times;
     int cptStride, maxlen;
     size_t NU;
     Place at;
@@ -497,6 +533,7 @@ struct DenseRev {
         sys = reinterpret_cast<Scope*>(lds);
         cptBuf = reinterpret_cast<double*>(lds + L.cpt);
         Ml = reinterpret_cast<const double*>(lds + L.mt);
+        times = reinterpret_cast<double*>(lds + L.total);
         int* blk = reinterpret_cast<int*>(lds + L.blk);
         cptStride = NC * SPB * dense_row(a.UPS);
         NU = (size_t)a.NS * a.UPS;
@@ -543,15 +580,31 @@ struct DenseRev {
     // row r of a unit-scope array [rows][NU]: wave-uniform row base, 32-bit lane offset
     template <class T>
     __device__ __forceinline__ T* row(T* base, size_t r) const { return base + r * NU; }
-    // (t, h) of step j of each of the lane's systems, 0 where it has none
-    __device__ __forceinline__ void step_times(const Args<Sys, double>& a, int j, double* t, double* h) const
+    // (t, h) of step j of each of the lane's systems, 0 where it has none, from
+    // kTimes steps of them in LDS (read from global memory where they are used,
+    // they wait for the stage buffer's stores as well, which the same counter
+    // counts: replay of 32 steps of 1024 x 128 units 0.30 -> 0.22 ms).  Called by
+    // the whole workgroup.
+    __device__ __forceinline__ void step_times(const Args<Sys, double>& a, int j, int& chunk, double* t, double* h) const
     {
+        if (j >= 0 && j < maxlen && j / kTimes != chunk) {
+            chunk = j / kTimes;
+            __syncthreads();
+            for (int e = threadIdx.x; e < kTimes * SPB; e += blockDim.x) {
+                const int s = e % SPB, jj = chunk * kTimes + e / SPB;
+                const bool run = jj < sys[s].len;
+                const size_t n = ((size_t)sys[s].k * a.recK + jj) * a.NS + ((size_t)blockIdx.x * SPB + s);
+                times[e] = run ? a.recT[n] : 0.0;
+                times[kTimes * SPB + e] = run ? a.recH[n] : 0.0;
+            }
+            __syncthreads();
+        }
 #pragma unroll
         for (int s = 0; s < NSL; s++) {
             const bool run = j >= 0 && j < len[s];
-            const size_t n = ((size_t)k[s] * a.recK + j) * a.NS + at.gsys(s);
-            t[s] = run ? a.recT[n] : 0.0;
-            h[s] = run ? a.recH[n] : 0.0;
+            const int e = (j % kTimes) * SPB + at.sys(s);
+            t[s] = run ? times[e] : 0.0;
+            h[s] = run ? times[kTimes * SPB + e] : 0.0;
         }
     }
     // the time terms of a step's stages as in the forward pass: lane l
@@ -594,6 +647,8 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
     using P = double;
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NUA = Sys::NUA, NiUA = Sys::NiUA;
     constexpr int NCp = Pos<NC>::value, NTT = TimeTermsOf<Sys>::n, ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC;
+    constexpr bool REMAKE = rev_remake<NSL, MT>();
+    constexpr int ROWS = rev_rows<Sys>(REMAKE, ST);
     using math::fma;
     using R = DenseRev<Sys, NSL, MT>;
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
@@ -623,6 +678,7 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
     int buf = 0;
     P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value], tt[NSL][Pos<NTT>::value];
     P t[NSL], h[NSL], tn[NSL], hn[NSL];
+    int chunk = -1;
     // right-hand sides of the lane's units at (Y, T) plus the coupling terms of
     // stage st of step j; Y and the coupling values (M CPT)_u are kept.  The
     // barriers order LDS only, so the stage-buffer stores stay in flight.
@@ -645,9 +701,11 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
                                                  uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, cp, CPF[s][q]);
 #pragma unroll
                 for (int i = 0; i < NC; i++) cpt[(i * R::SPB + C.at.sys(s)) * RS + C.at.unit(q)] = cp[i];
-                const size_t base = ((size_t)j * ST + st) * SW;
+                if (!REMAKE || st == 0) {
+                    const size_t base = REMAKE ? (size_t)j * ROWS : ((size_t)j * ST + st) * SW;
 #pragma unroll
-                for (int c = 0; c < UD; c++) C.row(A.stg, base + c)[C.unit(s, q)] = Y[s][q][c];
+                    for (int c = 0; c < UD; c++) C.row(A.stg, base + c)[C.unit(s, q)] = Y[s][q][c];
+                }
             }
         }
         if (st + 1 < ST) C.stage_terms(st + 1, tterm, tt);
@@ -658,9 +716,9 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
             for (int i = 0; i < NC; i++)
                 Unit<Sys, P>::add(cIndex[i], C.strength[s][i] * CPF[s][q][i], v[i][s][q], F[s][q]);
             if (j < C.len[s] && C.at.has(q)) {
-                const size_t base = ((size_t)j * ST + st) * SW;
+                const size_t base = REMAKE ? (size_t)j * ROWS + UD + st * NC : ((size_t)j * ST + st) * SW + UD;
 #pragma unroll
-                for (int i = 0; i < NC; i++) C.row(A.stg, base + UD + i)[C.unit(s, q)] = v[i][s][q];
+                for (int i = 0; i < NC; i++) C.row(A.stg, base + i)[C.unit(s, q)] = v[i][s][q];
             }
         }
         buf ^= 1;
@@ -671,11 +729,11 @@ __device__ void pb_replay_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A
             for (int c = 0; c < UD; c++) Y[s][q][c] = value(s, q, c);
         }
     };
-    C.step_times(a, 0, tn, hn);
+    C.step_times(a, 0, chunk, tn, hn);
     for (int j = 0; j < C.maxlen; j++) {
 #pragma unroll
         for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
-        C.step_times(a, j + 1, tn, hn);                 // one step ahead
+        C.step_times(a, j + 1, chunk, tn, hn);                 // one step ahead
         C.template time_terms<ALG>(t, h, tterm);
         C.stage_terms(0, tterm, tt);
         // the forward pass's stage arithmetic (pb_dense_body)
@@ -738,6 +796,8 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NSP = Sys::NSP, NUA = Sys::NUA, NiUA = Sys::NiUA;
     constexpr int NCp = Pos<NC>::value, NUPp = Pos<NUP>::value, NSPp = Pos<NSP>::value, NTT = TimeTermsOf<Sys>::n;
     constexpr int ST = ALG == MPGOS_RK4 ? 4 : 6, SW = UD + NC;
+    constexpr bool REMAKE = rev_remake<NSL, MT>();
+    constexpr int ROWS = rev_rows<Sys>(REMAKE, ST), FETCH = REMAKE ? ROWS : SW;
     using math::fma;
     using R = DenseRev<Sys, NSL, MT>;
     extern __shared__ __align__(16) unsigned char mpgos_pb_lds[];
@@ -771,29 +831,67 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
     }
     // a stage's inputs and coupling values, loaded one stage ahead where the
     // registers hold them (with 4 results per lane they would be spilled:
-    // reverse pass of 4096 x 256 units 54.6 against 49.8 ms)
+    // reverse pass of 4096 x 256 units 54.6 against 49.8 ms); REMAKE: a step's
+    // state and coupling values, loaded one step ahead
     constexpr bool AHEAD = NSL * TT < 4;
-    P ahead[NSL][TT][SW];
+    P ahead[NSL][TT][FETCH];
     auto fetch = [&](int j, int st) {
-        const size_t base = ((size_t)j * ST + st) * SW;
+        const size_t base = REMAKE ? (size_t)j * ROWS : ((size_t)j * ST + st) * SW;
         MPGOS_PB_EACH(s, q) {
             const bool ld = j >= 0 && j < C.len[s] && C.at.has(q);
 #pragma unroll
-            for (int c = 0; c < SW; c++) ahead[s][q][c] = ld ? C.row(A.stg, base + c)[C.unit(s, q)] : P(0);
+            for (int c = 0; c < FETCH; c++) ahead[s][q][c] = ld ? C.row(A.stg, base + c)[C.unit(s, q)] : P(0);
         }
     };
 
     int buf = 0;
     P tterm[(ST + R::PER - 1) / R::PER][Pos<NTT>::value], tt[NSL][Pos<NTT>::value];
     P t[NSL], h[NSL], tn[NSL], hn[NSL];
-    C.step_times(a, C.maxlen - 1, tn, hn);
+    int chunk = -1;
+    C.step_times(a, C.maxlen - 1, chunk, tn, hn);
     if (AHEAD) fetch(C.maxlen - 1, ST - 1);
     for (int j = C.maxlen - 1; j >= 0; j--) {
 #pragma unroll
         for (int s = 0; s < NSL; s++) { t[s] = tn[s]; h[s] = hn[s]; }
-        C.step_times(a, j - 1, tn, hn);                 // one step ahead
+        C.step_times(a, j - 1, chunk, tn, hn);                 // one step ahead
         C.template time_terms<ALG>(t, h, tterm);
-        C.stage_terms(ST - 1, tterm, tt);
+        // REMAKE: the stage inputs by the forward pass's arithmetic
+        // (pb_dense_body) from the coupling values; Ys, cpfs, tts of every stage
+        P Ys[REMAKE ? ST : 1][UD], vs[REMAKE ? ST : 1][NCp], cpfs[REMAKE ? ST : 1][NCp], tts[REMAKE ? ST : 1][NSL][Pos<NTT>::value];
+        if constexpr (REMAKE) {
+            P k[ST][UD];
+#pragma unroll
+            for (int st = 0; st < ST; st++) {
+                C.stage_terms(st, tterm, tts[st]);
+#pragma unroll
+                for (int i = 0; i < NC; i++) { vs[st][i] = ahead[0][0][UD + st * NC + i]; cpfs[st][i] = P(0); }
+            }
+#pragma unroll
+            for (int c = 0; c < UD; c++) Ys[0][c] = ahead[0][0][c];
+            fetch(j - 1, 0);
+            const bool run = j < C.len[0] && C.at.has(0);
+#pragma unroll
+            for (int st = 0; st < ST; st++) {
+#pragma unroll
+                for (int c = 0; c < UD; c++)
+                    if (st > 0) Ys[st][c] = rk_stage_input<ALG, UD>(st, c, h[0], Ys[0], k);
+                if (run) {
+                    auto& y = C.sys[C.at.sys(0)];
+                    P cp[NCp];
+                    const P T = rk_stage_time<ALG>(st, t[0], h[0]);
+                    if constexpr (NTT > 0)
+                        Sys::template OdeFunctionTT<P>(C.at.gsys(0), C.at.unit(0), k[st], Ys[st], T, tts[st][0], uPAR[0][0], y.sPAR, a.gPAR,
+                                                       a.gPARi, uACC[0][0], uACCi[0][0], y.sACC, y.sACCi, cp, cpfs[st]);
+                    else
+                        Sys::template OdeFunction<P>(C.at.gsys(0), C.at.unit(0), k[st], Ys[st], T, uPAR[0][0], y.sPAR, a.gPAR, a.gPARi,
+                                                     uACC[0][0], uACCi[0][0], y.sACC, y.sACCi, cp, cpfs[st]);
+#pragma unroll
+                    for (int i = 0; i < NC; i++) Unit<Sys, P>::add(cIndex[i], C.strength[0][i] * cpfs[st][i], vs[st][i], k[st]);
+                }
+            }
+        } else {
+            C.stage_terms(ST - 1, tterm, tt);
+        }
         P kb[ST][NSL][TT][UD];
 #pragma unroll
         for (int st = 0; st < ST; st++)
@@ -806,16 +904,21 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
             P Y[NSL][TT][UD], kbCPF[NSL][TT][NCp], w[NCp][NSL][TT];
             P* wb = C.cptBuf + (size_t)buf * C.cptStride;
             if (!AHEAD) fetch(j, st);
+            if constexpr (REMAKE) {
+#pragma unroll
+                for (int i = 0; i < NTT; i++) tt[0][i] = tts[st][0][i];
+            }
             MPGOS_PB_EACH(s, q) {
 #pragma unroll
-                for (int c = 0; c < UD; c++) Y[s][q][c] = ahead[s][q][c];
+                for (int c = 0; c < UD; c++) Y[s][q][c] = REMAKE ? Ys[REMAKE ? st : 0][c] : ahead[s][q][c];
                 if (j < C.len[s] && C.at.has(q)) {
                     P F[UD], cp[NCp], cpf[NCp];
 #pragma unroll
-                    for (int i = 0; i < NC; i++) cpf[i] = P(0);
+                    for (int i = 0; i < NC; i++) cpf[i] = REMAKE ? cpfs[REMAKE ? st : 0][i] : P(0);
                     auto& y = C.sys[C.at.sys(s)];
                     const P T = rk_stage_time<ALG>(st, t[s], h[s]);
-                    if constexpr (NTT > 0)
+                    if constexpr (REMAKE) {
+                    } else if constexpr (NTT > 0)
                         Sys::template OdeFunctionTT<P>(C.at.gsys(s), C.at.unit(q), F, Y[s][q], T, tt[s], uPAR[s][q], y.sPAR, a.gPAR, a.gPARi,
                                                        uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, cp, cpf);
                     else
@@ -828,11 +931,11 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
                         for (int c = 0; c < UD; c++)
                             if (c == cIndex[i]) g = kb[st][s][q][c];
                         wb[(i * R::SPB + C.at.sys(s)) * RS + C.at.unit(q)] = C.strength[s][i] * cpf[i] * g;
-                        kbCPF[s][q][i] = C.strength[s][i] * ahead[s][q][UD + i] * g;
+                        kbCPF[s][q][i] = C.strength[s][i] * (REMAKE ? vs[REMAKE ? st : 0][i] : ahead[s][q][REMAKE ? 0 : UD + i]) * g;
                     }
                 }
             }
-            if (AHEAD) {
+            if (AHEAD && !REMAKE) {
                 if (st > 0) fetch(j, st - 1);
                 else fetch(j - 1, ST - 1);
             }
@@ -871,7 +974,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
                         for (int c = 0; c < UD; c++) kb[l][s][q][c] = fma(h[s] * rk_a<ALG>(st, l), gy[c], kb[l][s][q][c]);
                     }
             }
-            if (st > 0) C.stage_terms(st - 1, tterm, tt);
+            if (!REMAKE && st > 0) C.stage_terms(st - 1, tterm, tt);
         }
     }
     MPGOS_PB_EACH(s, q) {

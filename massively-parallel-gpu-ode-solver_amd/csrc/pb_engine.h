@@ -718,7 +718,9 @@ public:
         const size_t NU = (size_t)NS * UPS;
         const int ST = algorithm == MPGOS_RK4 ? 4 : 6;
         int rc;
-        if ((rc = grow_device(stg, stgn, (size_t)adjK * ST * (UD + NC) * NU, "stage buffer")) ||
+        const bool four = dense_four() || rev_lds_bytes<Sys>(8, UPS, 0) > ldsMax;
+        const int rows = rev_rows<Sys>(four ? (dense_mt() > 8 ? rev_remake<1, 16>() : rev_remake<1, 8>()) : false, ST);
+        if ((rc = grow_device(stg, stgn, (size_t)adjK * rows * NU, "stage buffer")) ||
             (rc = grow_device(gSp, gSpn, (size_t)(NSP > 0 ? NSP : 1) * NU, "system-parameter partials")) ||
             (rc = grow_device(cTileT, cTileTN, (size_t)NC * dense_matrix_size(UPS), "tiled coupling matrix")))
             return rc;
@@ -736,11 +738,10 @@ public:
         a.recX = recX; a.recT = recT; a.recH = recH; a.recK = adjK; a.recCkCap = adjCap; a.recStepCap = adjStepCap;
         AdjArgs<Sys> A;
         A.seg = nullptr; A.stg = stg; A.gSp = gSp; A.lam = lamB.d; A.gU = gUB.d; A.gS = gSB.d; A.cMatT = nullptr; A.cTileT = cTileT;
-        if (!dense_fits<RevScope<Sys>>(4, 0)) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
+        if (rev_lds_bytes<Sys>(4, UPS, 0) > ldsMax) { set_error("per-block adjoint: reverse-pass LDS exceeds a workgroup's"); return MPGOS_E_ARG; }
         MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
         if ((rc = tile_pairs<false>(cTile)) || (rc = tile_pairs<true>(cTileT))) return rc;
         a.cTile = cTile;
-        const bool four = dense_four() || !dense_fits<RevScope<Sys>>(8, 0);
         if (dense_mt() > 8) { if (four) launch_reverse<1, 16>(a, A, rounds); else launch_reverse<2, 16>(a, A, rounds); }
         else if (four) launch_reverse<1, 8>(a, A, rounds);
         else launch_reverse<2, 8>(a, A, rounds);
@@ -753,7 +754,7 @@ public:
     void launch_reverse(Args<Sys, double>& a, const AdjArgs<Sys>& A, int rounds)
     {
         constexpr int spb = 4 * NSL;
-        auto bytes = [&](int pairs) { return dense_layout<RevScope<Sys>, NC, 0, 0>(spb, UPS, 0, pairs).total; };
+        auto bytes = [&](int pairs) { return rev_lds_bytes<Sys>(spb, UPS, pairs); };
         const int grid = (NS + spb - 1) / spb, threads = dense_threads();
         a.SPB = spb;
         a.ldsPairs = dense_resident<Sys, NSL, MT>() ? 0 : dense_lds_pairs(bytes(0), grid, 2);
