@@ -104,3 +104,34 @@ def test_adjoint_equals_lane_form(ns, ups, off, K, alg):
         a, b = (x.reshape(x.shape[0], ns, -1)[:, :ns - off] for x in (a, b))
         assert np.isfinite(a).all() and np.abs(a).max() > 0
         assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
+@pytest.mark.parametrize("kind", ["subnormal", "huge", "non-finite"])
+def test_extreme_values(oracle, kind):
+    """Subnormal and huge states, coupling terms and matrix entries, and systems
+    with infinities and NaN beside ordinary ones in the same workgroup."""
+    import pyoracle
+    ns, ups = 9, 20
+    rs = W.Stream(W.SEED, 330)
+    s = W.new_pb_spec("pb_linear", Algorithms.RKCK45, ns, ups)
+    s["cMat"] = rs.normal(ups * ups) * 0.1
+    s["uPAR"][0] = rs.uniform(ns * ups, -1.0, 0.3)
+    s["X"][0] = rs.uniform(ns * ups, -1.0, 1.0)
+    s["strength"][0] = 1.0
+    s["TD"][1] = 1.0
+    s["rtol"] = s["atol"] = 1e-6
+    if kind == "subnormal":
+        s["X"][0] *= 1e-310
+        s["cMat"][::7] *= 1e-309
+    elif kind == "huge":
+        s["X"][0] *= 1e150
+        s["cMat"][::5] = -0.0
+        s["strength"][0, 3] = 1e120
+    else:
+        s["X"][0, 2 * ups + 3] = np.inf
+        s["X"][0, 5 * ups] = np.nan
+        s["strength"][0, 7] = np.inf
+    print(f"dense form {kind}", flush=True)
+    ref = pyoracle.run_pb("pb_linear", s)
+    assert_pb_bitwise(run_pb_gpu(s), ref, "automatic")
+    assert_pb_bitwise(run_pb_gpu(s, kernel=1), ref, "lane per pair")
