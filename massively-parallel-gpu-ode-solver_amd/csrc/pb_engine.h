@@ -56,6 +56,51 @@ template <class Sys, class = void> struct HasVjp : std::false_type {};
 template <class Sys>
 struct HasVjp<Sys, decltype((void)&Sys::template OdeVJP<double>)> : std::true_type {};
 
+// Launches of the lane-per-pair kernels.  Plain function templates, so that a
+// library system's kernels can be compiled apart from its solver: the
+// dense-contraction kernels are built with -disable-machine-licm, which a full
+// circular matrix in the lane-per-pair form pays for dearly (1000 systems of 40
+// linear units: 0.32 ms with the default flags, 0.55 ms with it).
+template <class Sys, class P, bool KAHAN>
+void launch_lane(int algorithm, int grid, int threads, size_t lds, hipStream_t strm, const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>& a)
+{
+    if (threads <= 256) {
+        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+        else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+    } else {
+        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+        else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+    }
+}
+
+template <class Sys>
+void launch_lane_record(int algorithm, int grid, int threads, size_t lds, hipStream_t strm, const Args<Sys, double>& a)
+{
+    if constexpr (HasVjp<Sys>::value) {
+        if (threads <= 256) {
+            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a);
+            else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a);
+        } else {
+            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
+            else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
+        }
+    }
+}
+
+template <class Sys>
+void launch_lane_reverse(int algorithm, int grid, int threads, size_t lds, hipStream_t strm, const Args<Sys, double>& a, const AdjArgs<Sys>& A)
+{
+    if constexpr (HasVjp<Sys>::value) {
+        if (threads <= 256) {
+            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a, A);
+            else hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a, A);
+        } else {
+            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RK4, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a, A);
+            else hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RKCK45, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a, A);
+        }
+    }
+}
+
 // KAHAN (P = float): the FLOAT_KAHAN mode (compensated FP32 state and time,
 // FP64 step size, error norm, controller and event step control).
 template <class Sys, class P, bool KAHAN = false>
@@ -560,13 +605,7 @@ public:
         const int threads = ((SPB * UPS + 63) / 64) * 64;
         const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
         MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-        if (threads <= 256) {
-            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
-            else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
-        } else {
-            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
-            else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
-        }
+        launch_lane<Sys, P, KAHAN>(algorithm, grid, threads, lds, strm, a);
         MPGOS_HIP_TRY(hipGetLastError());
         MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
         return MPGOS_OK;
@@ -638,13 +677,7 @@ public:
             const int threads = ((SPB * UPS + 63) / 64) * 64;
             const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
             MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-            if (threads <= 256) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a);
-            } else {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
-                else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
-            }
+            launch_lane_record<Sys>(algorithm, grid, threads, lds, strm, a);
             MPGOS_HIP_TRY(hipGetLastError());
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;
@@ -697,13 +730,7 @@ public:
             const int threads = ((SPB * UPS + 63) / 64) * 64;
             const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
             MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-            if (threads <= 256) {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a, A);
-                else hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a, A);
-            } else {
-                if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RK4, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a, A);
-                else hipLaunchKernelGGL((pb_reverse_kernel<Sys, MPGOS_RKCK45, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a, A);
-            }
+            launch_lane_reverse<Sys>(algorithm, grid, threads, lds, strm, a, A);
             MPGOS_HIP_TRY(hipGetLastError());
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;
