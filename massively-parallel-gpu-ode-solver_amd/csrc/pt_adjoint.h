@@ -380,11 +380,12 @@ __device__ __forceinline__ bool common_time_reverse(const AdjArgs<Sys>& A, Lane<
         L.rk4(a, h, nx, nullptr, sPAR, sPARi, tt1, ttm, tt4);
         L.accept(a, h, dtP, nx, nullptr, EFn, false, sPAR, sPARi);
     };
-    // a step's record, read a step ahead of its use
+    // a step's record, read a step ahead of its use (as above: HBM records end
+    // with the last instance)
     double x[SD];
     auto record = [&](int slot) {
 #pragma unroll
-        for (int c = 0; c < SD; c++) x[c] = seg((size_t)(slot * SD + c));
+        for (int c = 0; c < SD; c++) x[c] = LDS_SEG || mine ? seg((size_t)(slot * SD + c)) : 0.0;
     };
     auto reverse = [&](int j, int next) {
         double tt1[NTT], ttm[NTT], tt4[NTT], xj[SD];
