@@ -899,10 +899,12 @@ struct Lane {
                     }
                     P nx[SD], inc[KAHAN ? SD : 1], EFn[1], dtP = h;
                     rk4(a, h, nx, inc, sPAR, sPARi, tt1, ttm, tt4);
+                    // an instance that has ended stores no more points
+                    const bool open = !DENSE || (zero == P(0) && ended == 0);
 #pragma unroll
                     for (int i = 0; i < SD; i++) zero = math::fma(nx[i], P(0), zero);
                     accept(a, h, dtP, nx, inc, EFn, false, sPAR, sPARi);
-                    if (DENSE) dense_output(a, false);
+                    if (DENSE && open) dense_output(a, false);
                     ended |= udt;
 #pragma unroll
                     for (int i = 0; i < NTT; i++) tt1[i] = tt4[i];
@@ -911,7 +913,7 @@ struct Lane {
                 for (; m + 4 <= j + n; m += 4) { one(m); one(m + 1); one(m + 2); one(m + 3); }
                 for (; m < j + n; m++) one(m);
                 // an instance ended on the way: the ordinary loop makes these
-                // steps again (dense output it has stored is stored again)
+                // steps again (the dense output up to its end is stored again)
                 if (__any(mine && (zero != P(0) || ended != 0))) {
                     *this = before;
                     return;
