@@ -199,8 +199,7 @@ public:
         for (auto* q : {&X, &uPAR, &uACC, &TD, &T, &sPAR, &sACC, &strength, &DOt, &DOx, &gPAR, &cMat, &lamB, &gUB, &gSB}) q->bind(arena);
         for (auto* q : {&uACCi, &sACCi, &DOidx, &gPARi, &cIndex, &status}) q->bind(arena);
         nacc.bind(arena); nrej.bind(arena);
-        if (dense_possible() && hipMalloc((void**)&cTile, (size_t)NC * dense_matrix_size(UPS) * sizeof(double)) != hipSuccess) {
-            cTile = nullptr;
+        if (dense_possible() && !device_alloc(cTile, (size_t)NC * dense_matrix_size(UPS) * sizeof(double))) {
             set_error("per-block: allocation of the tiled coupling matrix failed");
             return MPGOS_E_MEMORY;
         }
@@ -632,12 +631,17 @@ public:
         return MPGOS_OK;
     }
 
+    static void drop_device(double*& p, size_t& have)
+    {
+        if (p) (void)hipFree(p);
+        p = nullptr; have = 0;
+    }
+
     static int grow_device(double*& p, size_t& have, size_t need, const char* what)
     {
         if (need <= have) return MPGOS_OK;
-        if (p) (void)hipFree(p);
-        p = nullptr; have = 0;
-        if (hipMalloc((void**)&p, need * sizeof(double)) != hipSuccess) {
+        drop_device(p, have);
+        if (!device_alloc(p, need * sizeof(double))) {
             set_error(std::string("per-block adjoint: allocation of ") + what + " failed");
             return MPGOS_E_MEMORY;
         }
@@ -709,6 +713,9 @@ public:
                     // what only the automatic choice sent here fits the lane
                     // form's smaller segment buffer
                     if (rc != MPGOS_E_MEMORY || dense_request_valid()) return rc;
+                    drop_device(stg, stgn);
+                    drop_device(gSp, gSpn);
+                    drop_device(cTileT, cTileTN);
                     lastForm = kLaneCoupling;
                 }
             }

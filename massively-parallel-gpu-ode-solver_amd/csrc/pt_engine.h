@@ -49,6 +49,26 @@ inline int bound_check(const char* fn, const char* what, int v, int lo, int hi)
     return MPGOS_OK;
 }
 
+// Allocations whose failure the caller reports: false leaves the pointer null
+// and no error behind (the runtime keeps a call's error until it is asked for,
+// and the check after a later launch would take it for that launch's).
+template <class T>
+bool device_alloc(T*& p, size_t bytes)
+{
+    if (hipMalloc((void**)&p, bytes) == hipSuccess) return true;
+    p = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+template <class T>
+bool host_alloc(T*& p, size_t bytes)
+{
+    if (hipHostMalloc((void**)&p, bytes, hipHostMallocDefault) == hipSuccess) return true;
+    p = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+
 namespace pt {
 
 // forms with several lanes per instance (RKCK45, systems with time terms)
@@ -112,14 +132,12 @@ struct Arena {
     int alloc()
     {
         if (n == 0) return MPGOS_OK;
-        if (hipHostMalloc((void**)&h, n, hipHostMallocDefault) != hipSuccess) {
-            h = nullptr;
+        if (!host_alloc(h, n)) {
             set_error("failed to allocate pinned host memory");
             return MPGOS_E_MEMORY;
         }
         std::memset(h, 0, n);
-        if (hipMalloc((void**)&d, n) != hipSuccess) {
-            d = nullptr;
+        if (!device_alloc(d, n)) {
             set_error("failed to allocate device memory");
             return MPGOS_E_MEMORY;
         }
@@ -165,12 +183,12 @@ struct Buffer {
         n = count;
         own = true;
         if (count == 0) return MPGOS_OK;
-        if (hipHostMalloc((void**)&h, count * sizeof(T), hipHostMallocDefault) != hipSuccess) {
+        if (!host_alloc(h, count * sizeof(T))) {
             set_error("failed to allocate pinned host memory");
             return MPGOS_E_MEMORY;
         }
         std::memset(h, 0, count * sizeof(T));
-        if (hipMalloc((void**)&d, count * sizeof(T)) != hipSuccess) {
+        if (!device_alloc(d, count * sizeof(T))) {
             set_error("failed to allocate device memory");
             return MPGOS_E_MEMORY;
         }
@@ -796,8 +814,8 @@ public:
     int ensure_slice_buffers()
     {
         if (!saved) {
-            if (hipMalloc((void**)&saved, lane_words() * 4 * (size_t)NT) != hipSuccess || hipMalloc((void**)&phase, 4 * (size_t)NT) != hipSuccess ||
-                hipMalloc((void**)&listA, 4 * (size_t)NT) != hipSuccess || hipMalloc((void**)&listB, 4 * (size_t)NT) != hipSuccess) {
+            if (!device_alloc(saved, lane_words() * 4 * (size_t)NT) || !device_alloc(phase, 4 * (size_t)NT) ||
+                !device_alloc(listA, 4 * (size_t)NT) || !device_alloc(listB, 4 * (size_t)NT)) {
                 set_error("time-sliced launches: allocation failed");
                 return MPGOS_E_MEMORY;
             }
@@ -806,7 +824,7 @@ public:
             MPGOS_HIP_TRY(hipStreamSynchronize(strm));
             if (relaunchCounts) (void)hipFree(relaunchCounts);
             relaunchCounts = nullptr; relaunchCountsN = 0;
-            if (hipMalloc((void**)&relaunchCounts, sizeof(unsigned) * (size_t)(relaunchLaunches + 1)) != hipSuccess) {
+            if (!device_alloc(relaunchCounts, sizeof(unsigned) * (size_t)(relaunchLaunches + 1))) {
                 set_error("relaunch form: allocation failed");
                 return MPGOS_E_MEMORY;
             }
@@ -845,7 +863,7 @@ public:
     {
         if (!orderDirty && order) return MPGOS_OK;
         if (!order) {
-            if (hipMalloc((void**)&order, sizeof(int) * (size_t)NT) != hipSuccess) { set_error("QueueOrder: allocation failed"); return MPGOS_E_MEMORY; }
+            if (!device_alloc(order, sizeof(int) * (size_t)NT)) { set_error("QueueOrder: allocation failed"); return MPGOS_E_MEMORY; }
         }
         orderHost.resize((size_t)nActive);
         for (int i = 0; i < nActive; i++) orderHost[(size_t)i] = i;
@@ -873,8 +891,8 @@ public:
             if (int rc = ensure_slice_buffers()) return rc;
         }
         if (kernelMode == MPGOS_KERNEL_SORTED && !sortKey) {
-            if (hipMalloc((void**)&sortKey, sizeof(float) * (size_t)NT) != hipSuccess ||
-                hipMalloc((void**)&sortHist, sizeof(unsigned) * 256) != hipSuccess) {
+            if (!device_alloc(sortKey, sizeof(float) * (size_t)NT) ||
+                !device_alloc(sortHist, sizeof(unsigned) * 256)) {
                 set_error("sorted form: allocation failed");
                 return MPGOS_E_MEMORY;
             }
@@ -1010,13 +1028,13 @@ public:
             if (needC > ckptCount) {
                 if (ckpt) (void)hipFree(ckpt);
                 ckpt = nullptr; ckptCount = 0;
-                if (hipMalloc((void**)&ckpt, needC * sizeof(double)) != hipSuccess) { set_error("adjoint: checkpoint allocation failed"); return MPGOS_E_MEMORY; }
+                if (!device_alloc(ckpt, needC * sizeof(double))) { set_error("adjoint: checkpoint allocation failed"); return MPGOS_E_MEMORY; }
                 ckptCount = needC;
             }
             if (needS > segCount) {
                 if (seg) (void)hipFree(seg);
                 seg = nullptr; segCount = 0;
-                if (hipMalloc((void**)&seg, needS * sizeof(double)) != hipSuccess) { set_error("adjoint: segment allocation failed"); return MPGOS_E_MEMORY; }
+                if (!device_alloc(seg, needS * sizeof(double))) { set_error("adjoint: segment allocation failed"); return MPGOS_E_MEMORY; }
                 segCount = needS;
             }
             adjK = K; adjCap = capacity;
