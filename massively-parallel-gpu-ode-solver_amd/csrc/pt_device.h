@@ -256,6 +256,11 @@ struct StepArgs {
 #pragma unroll
             for (int i = 0; i < NE; i++)
                 if (!(a.etol[i] >= P(0))) l = CP(__builtin_huge_val());
+            // the maximum in step() drops a NaN tolerance, which no error is
+            // below (a NaN rtol alone leaves tol = atol)
+#pragma unroll
+            for (int i = 0; i < SD; i++)
+                if (a.atol[i] != a.atol[i]) l = CP(__builtin_huge_val());
             least = pin(l);
 #pragma unroll
             for (int i = 0; i < SD; i++) { rtol[i] = pin(a.rtol[i]); atol[i] = pin(a.atol[i]); }
