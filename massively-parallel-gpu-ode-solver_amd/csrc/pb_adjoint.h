@@ -951,7 +951,7 @@ __device__ void pb_sweep_body(const Args<Sys, double>& a, const AdjArgs<Sys>& A,
                     for (int i = 0; i < NC; i++) kbCPT[i] = w[i][s][q];
                     auto& y = C.sys[C.at.sys(s)];
                     const P T = rk_stage_time<ALG>(st, t[s], h[s]);
-                    if constexpr (NTT > 0)
+                    if constexpr (TimeTermsOf<Sys>::timeOnly)
                         Sys::template OdeVJPTT<P>(C.at.gsys(s), C.at.unit(q), kb[st][s][q], kbCPT, kbCPF[s][q], Y[s][q], T, tt[s], uPAR[s][q],
                                                   y.sPAR, a.gPAR, a.gPARi, uACC[s][q], uACCi[s][q], y.sACC, y.sACCi, gy, gU, gS);
                     else
