@@ -525,6 +525,17 @@ public:
         return kLaneCoupling;
     }
 
+    // The reverse pass keeps step sizes in LDS beside what the Solve keeps; where
+    // that does not fit, one lane per unit.
+    int reverse_form() const
+    {
+        const int form = coupling_form();
+        if constexpr (kAdjoint && NC > 0) {
+            if (form == kDenseCoupling && couplingKernel != 2 && rev_lds_bytes<Sys>(4, UPS, 0) > ldsMax) return kLaneCoupling;
+        }
+        return form;
+    }
+
     size_t lds_bytes(int spb, int sm) const
     {
         return lds_layout<Sys, P, KAHAN>(spb, UPS, sharedGlobals, sm, cMatSize).total;
@@ -706,7 +717,7 @@ public:
             const size_t NU = (size_t)NS * UPS;
             MPGOS_HIP_TRY(hipStreamSynchronize(strm));
             if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
-            lastForm = coupling_form();
+            lastForm = reverse_form();
             if constexpr (NC > 0) {
                 if (lastForm == kDenseCoupling) {
                     const int rc = reverse_dense();

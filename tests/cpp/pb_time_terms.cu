@@ -3,7 +3,8 @@
 // which only systems with terms of the time alone provide.  Gradient and end
 // state in the matrix-core form, with one and with several results per lane,
 // against one lane per unit, which evaluates no shared terms, bit for bit.
-// Prints "same" and returns 0, or says what differs and returns 1.
+// Prints "same" and returns 0, or says what differs and returns 1.  With an
+// argument: the forms it would choose, without a device.
 #include <cstdio>
 #include <string>
 #include <utility>
@@ -89,8 +90,28 @@ static bool run(int algorithm, int ns, int ups, int kernel, std::vector<unsigned
     return true;
 }
 
-int main()
+// The choice of the reverse pass where the LDS holds the Solve's data and not
+// the step sizes of the reverse pass as well (no device needed).
+static int forms()
 {
+    mpgos::pb::Solver<Named, double> S;
+    S.NS = 40; S.UPS = 100; S.cus = 256;
+    using namespace mpgos::pb;
+    const size_t solve = dense_layout<DenseScope<Named>, 1, 0, 0>(4, 100, 1, 0).total, reverse = rev_lds_bytes<Named>(4, 100, 0);
+    bool ok = reverse > solve;
+    S.ldsMax = reverse;
+    ok = ok && S.coupling_form() == kDenseCoupling && S.reverse_form() == kDenseCoupling;
+    S.ldsMax = solve;
+    ok = ok && S.coupling_form() == kDenseCoupling && S.reverse_form() == kLaneCoupling;
+    S.couplingKernel = 2;                              // asked for: refused later, as too large
+    ok = ok && S.reverse_form() == kDenseCoupling;
+    std::printf(ok ? "forms\n" : "wrong form\n");
+    return ok ? 0 : 1;
+}
+
+int main(int argc, char**)
+{
+    if (argc > 1) return forms();
     for (int algorithm : {MPGOS_RK4, MPGOS_RKCK45})
         for (auto shape : {std::pair<int, int>{5, 20}, {3, 130}, {2100, 130}}) {
             std::vector<unsigned char> a, b;

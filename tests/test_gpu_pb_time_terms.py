@@ -13,3 +13,9 @@ def test_gradient_without_a_time_term_vjp(gpu):
     assert os.path.exists(EXE), "build() compiles tests/cpp/pb_time_terms"
     r = subprocess.run([EXE], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "same", (r.returncode, r.stdout, r.stderr)
+
+
+def test_reverse_pass_that_exceeds_the_lds_runs_one_lane_per_unit():
+    assert os.path.exists(EXE), "build() compiles tests/cpp/pb_time_terms"
+    r = subprocess.run([EXE, "forms"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.strip() == "forms", (r.returncode, r.stdout, r.stderr)
