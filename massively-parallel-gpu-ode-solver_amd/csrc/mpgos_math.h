@@ -64,14 +64,16 @@ MPGOS_HD MPGOS_INLINE bool isnan(double x) { return x != x; }
 MPGOS_HD MPGOS_INLINE double flip_sign(double x, double y) { return from_bits(bits(x) ^ (bits(y) & 0x8000000000000000ull)); }
 MPGOS_HD MPGOS_INLINE float flip_sign(float x, float y) { return from_bits32(bits(x) ^ (bits(y) & 0x80000000u)); }
 
-// a * b + k for a constant k (Horner steps): on the device the three-operand
-// form with k in vector registers.  Left to itself the compiler picks the
-// accumulating form and copies k into its destination first, or rebuilds k in
-// scalar registers for every use; a wavefront alone on its SIMD pays 4 cycles for
-// each of these moves, as for an fma.
+// a * b + k for a constant k (Horner steps).  MPGOS_HORNER_IN_REGISTERS: on the
+// device the three-operand form with k in vector registers.  Left to itself the
+// compiler picks the accumulating form and copies k into its destination first,
+// or rebuilds k in scalar registers for every use; a wavefront alone on its SIMD
+// pays 4 cycles for each of these moves, as for an fma.  The coefficients then
+// hold registers through the step loop, so kernels whose wavefronts share a SIMD
+// are compiled without it (the lane-per-pair kernels of the per-block solver).
 MPGOS_HD MPGOS_INLINE double fma_k(double a, double b, double k)
 {
-#if defined(__HIP_DEVICE_COMPILE__)
+#if defined(__HIP_DEVICE_COMPILE__) && defined(MPGOS_HORNER_IN_REGISTERS)
     double r;
     asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(k));
     return r;

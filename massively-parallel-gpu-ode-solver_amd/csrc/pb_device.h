@@ -153,20 +153,25 @@ template <class Sys, class P>
 struct Unit {
     static constexpr int UD = Sys::UD, NC = Sys::NC, NE = Sys::NE;
 
+    using GP = const __attribute__((address_space(1))) P*;
+    using LP = const __attribute__((address_space(3))) P*;
+
     // v = fma(M(u, k), CPT_k, v) over the columns k = col .. col + N - 1, in
     // order, the matrix values loaded ahead
     template <int N>
-    static __device__ __forceinline__ void dot(const P* Mi, const P* cptSys, int col, int i, int UPS, P& v)
+    static __device__ __forceinline__ void dot(GP Mi, LP cpt, int col, int i, int UPS, P& v)
     {
         P m[N];
 #pragma unroll
         for (int j = 0; j < N; j++) m[j] = Mi[(size_t)(col + j) * UPS];
 #pragma unroll
-        for (int j = 0; j < N; j++) v = math::fma(m[j], cptSys[(col + j) * NC + i], v);
+        for (int j = 0; j < N; j++) v = math::fma(m[j], cpt[(col + j) * NC + i], v);
     }
 
-    // coupling: F[CouplingIndex[i]] += strength_i CPF_i sum_col M_i(u, col) CPT_col[i]
-    template <class A>
+    // coupling: F[CouplingIndex[i]] += strength_i CPF_i sum_col M_i(u, col) CPT_col[i].
+    // GROUPED: full matrices in global memory, the columns in groups (lane_grouped
+    // in pb_engine.h says where); else any storage form, one after the other.
+    template <bool GROUPED, class A>
     static __device__ __forceinline__ void couple(const A& a, const P* M, const int* cIndex, const P* strength,
                                                   const P* cptSys, int u, const P* CPF, P* F)
     {
@@ -174,25 +179,29 @@ struct Unit {
 #pragma unroll
         for (int i = 0; i < NC; i++) {
             P v = P(0);
-            if (a.CCI == 0 && a.CBW == 0) {
-                const P* Mi = M + (size_t)i * UPS * UPS + u;
+            if constexpr (GROUPED) {
+                const GP Mi = (GP)(M + (size_t)i * UPS * UPS + u);
+                const LP cpt = (LP)cptSys;
                 // Bound by the latency of the matrix loads (L2 and beyond), so
-                // eight are in flight at a time.  Against a plain loop over the
-                // columns: 46 x 64 FP32 622 -> 500 us, 500 x 256 FP32 4.80 ->
-                // 3.39 ms, 60 x 300 FP64 16.0 -> 6.3 ms, 200 x 1024 FP64 163 ->
-                // 68 ms.  The last 1 to 3 columns load the last one again in
-                // place of absent ones and skip the product (300 x 7 FP32:
-                // 0.46 -> 0.38 ms against a plain loop for all but the eights).
+                // eight are in flight at a time, as global loads (through a
+                // generic pointer they count as LDS operations too, and the
+                // coupling terms from LDS wait for them: 100 x 128 FP64, RK4,
+                // 1.10 -> 0.84 ms).  Against a plain loop over the columns: 46 x 64
+                // FP32 622 -> 500 us, 500 x 256 FP32 4.80 -> 3.39 ms, 60 x 300
+                // FP64 16.0 -> 6.3 ms, 200 x 1024 FP64 163 -> 68 ms.  The last 1 to
+                // 3 columns load the last one again in place of absent ones and
+                // skip the product (300 x 7 FP32: 0.46 -> 0.38 ms against a plain
+                // loop for all but the eights).
                 int col = 0;
-                for (; col + 8 <= UPS; col += 8) dot<8>(Mi, cptSys, col, i, UPS, v);
-                if (col + 4 <= UPS) { dot<4>(Mi, cptSys, col, i, UPS, v); col += 4; }
+                for (; col + 8 <= UPS; col += 8) dot<8>(Mi, cpt, col, i, UPS, v);
+                if (col + 4 <= UPS) { dot<4>(Mi, cpt, col, i, UPS, v); col += 4; }
                 if (col < UPS) {
                     P m[3], c[3];
 #pragma unroll
                     for (int j = 0; j < 3; j++) {
                         const int k = col + j < UPS ? col + j : UPS - 1;
                         m[j] = Mi[(size_t)k * UPS];
-                        c[j] = cptSys[k * NC + i];
+                        c[j] = cpt[k * NC + i];
                     }
 #pragma unroll
                     for (int j = 0; j < 3; j++) {
@@ -200,6 +209,9 @@ struct Unit {
                         v = col + j < UPS ? w : v;
                     }
                 }
+            } else if (a.CCI == 0 && a.CBW == 0) {
+                const P* Mi = M + (size_t)i * UPS * UPS + u;
+                for (int col = 0; col < UPS; col++) v = math::fma(Mi[(size_t)col * UPS], cptSys[col * NC + i], v);
             } else if (a.CCI == 0) {
                 const int W = 2 * a.CBW + 1;
                 const P* Mi = M + (size_t)i * UPS * W + u;
@@ -245,12 +257,21 @@ struct Unit {
 // compensation (x += dt * sum b_j k_j and t += dt as compensated sums); the
 // step size, the error norm (from the FP32 stages in FP64 arithmetic), the
 // controller and the event step control in FP64.
-template <class Sys, class P, int ALG, bool REC = false, bool KAHAN = false>
+//
+// A lane's registers decide how many wavefronts a SIMD holds, and these kernels
+// sit at the limits (FP32 Cash-Karp of the double-well ring: 128 of the 128 that
+// allow four).  Two loops over the lane's kUnits = 1 units keep its values from
+// being live where they are not needed; written without them the same kernel has
+// 130 registers and three wavefronts: 4000 systems of 10 units 0.26 -> 0.34 ms.
+// The right-hand sides' polynomials keep their coefficients out of registers
+// (MPGOS_HORNER_IN_REGISTERS) for the same reason: with them in registers 141,
+// and a circular matrix of 64 units (FP32, RK4) 0.80 -> 1.50 ms.
+template <class Sys, class P, int ALG, bool GROUPED, bool REC = false, bool KAHAN = false>
 __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>& a)
 {
     constexpr int UD = Sys::UD, NC = Sys::NC, NUP = Sys::NUP, NSP = Sys::NSP, NGP = Sys::NGP, NiGP = Sys::NiGP;
     constexpr int NUA = Sys::NUA, NiUA = Sys::NiUA, NSA = Sys::NSA, NiSA = Sys::NiSA, NE = Sys::NE;
-    constexpr int NCp = Pos<NC>::value;
+    constexpr int NCp = Pos<NC>::value, kUnits = 1;
     using S = SysScope<Sys, P, KAHAN>;
     using CP = typename S::CP;
     using U = Unit<Sys, P>;
@@ -273,7 +294,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
     const bool exists = lane && gsys < NS;
     const bool active = exists && gsys < a.nActive;
     S* const my = lane ? &sys[lsys] : &sys[0];
-    const size_t gu = (size_t)gsys * UPS + u;                  // unit-scope index
+    auto gu = [&]() { return (size_t)gsys * UPS + u; };        // unit-scope index, formed where it is used
 
     // ---- global scope (LDS when SharedGlobalVariables / SharedCouplingMatrices)
     P* gPAR = a.gPAR;
@@ -321,18 +342,22 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
     P Xc[KAHAN ? UD : 1];                 // Kahan compensation of the unit states
     P CPF[NCp];
     int uACCi[Pos<NiUA>::value];
-    if (exists) {
 #pragma unroll
-        for (int c = 0; c < UD; c++) { X[c] = a.X[gu + c * NU]; if (KAHAN) Xc[c] = P(0); }
+    for (int k = 0; k < kUnits; k++) {
+        if (exists) {
+            const size_t g = gu();
 #pragma unroll
-        for (int c = 0; c < NUP; c++) uPAR[c] = a.uPAR[gu + c * NU];
+            for (int c = 0; c < UD; c++) { X[c] = a.X[g + c * NU]; if (KAHAN) Xc[c] = P(0); }
 #pragma unroll
-        for (int c = 0; c < NUA; c++) uACC[c] = a.uACC[gu + c * NU];
+            for (int c = 0; c < NUP; c++) uPAR[c] = a.uPAR[g + c * NU];
 #pragma unroll
-        for (int c = 0; c < NiUA; c++) uACCi[c] = a.uACCi[gu + c * NU];
+            for (int c = 0; c < NUA; c++) uACC[c] = a.uACC[g + c * NU];
+#pragma unroll
+            for (int c = 0; c < NiUA; c++) uACCi[c] = a.uACCi[g + c * NU];
+        }
+#pragma unroll
+        for (int i = 0; i < NC; i++) CPF[i] = P(0);
     }
-#pragma unroll
-    for (int i = 0; i < NC; i++) CPF[i] = P(0);
     __syncthreads();
 
     // the step size as the user callbacks see it (FP32 copy in the Kahan mode)
@@ -353,7 +378,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
         if (active && my->DOidx < a.NDO) {
             const int k = my->DOidx;
 #pragma unroll
-            for (int c = 0; c < UD; c++) a.DOx[gu + c * NU + (size_t)k * NU * UD] = X[c];
+            for (int c = 0; c < UD; c++) a.DOx[gu() + c * NU + (size_t)k * NU * UD] = X[c];
             if (leader) a.DOt[gsys + (size_t)k * NS] = my->t;
         }
         __syncthreads();
@@ -367,7 +392,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
 
     if (REC && active) {        // checkpoint 0: the initial unit states
 #pragma unroll
-        for (int c = 0; c < UD; c++) a.recX[(size_t)c * NU + gu] = X[c];
+        for (int c = 0; c < UD; c++) a.recX[(size_t)c * NU + gu()] = X[c];
     }
 
     int buf = 0;
@@ -379,7 +404,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
             Sys::template OdeFunction<P>(gsys, u, F, Y, T, uPAR, my->sPAR, gPAR, gPARi, uACC, uACCi, my->sACC, my->sACCi,
                                          cpt + (size_t)(lsys * UPS + u) * NCp, CPF);
         __syncthreads();
-        if (run) U::couple(a, M, cIndex, my->strength, cpt + (size_t)lsys * UPS * NCp, u, CPF, F);
+        if (run) U::template couple<GROUPED>(a, M, cIndex, my->strength, cpt + (size_t)lsys * UPS * NCp, u, CPF, F);
         buf ^= 1;
     };
 
@@ -523,17 +548,20 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
             if (lane && my->term == 0) {
                 bool corr = false;
                 CP ev = my->dt;
-                // the event function of the candidate state, at the end of the step
-                Sys::template EventFunction<P>(gsys, u, EFn, tn, (P)my->newDt, my->TD, next, uPAR, my->sPAR, gPAR,
-                                               gPARi, uACC, uACCi, my->sACC, my->sACCi);
-                if (my->update == 1) {
 #pragma unroll
-                    for (int i = 0; i < NE; i++) {
-                        const P tol = a.etol[i];
-                        if ((EF[i] > tol && EFn[i] < -tol && a.edir[i] <= 0) ||
-                            (EF[i] < -tol && EFn[i] > tol && a.edir[i] >= 0)) {
-                            ev = dmin<CP>(ev, -(CP)EF[i] / ((CP)EFn[i] - (CP)EF[i]) * my->dt);
-                            corr = true;
+                for (int k = 0; k < kUnits; k++) {
+                    // the event function of the candidate state, at the end of the step
+                    Sys::template EventFunction<P>(gsys, u, EFn, tn, (P)my->newDt, my->TD, next, uPAR, my->sPAR, gPAR,
+                                                   gPARi, uACC, uACCi, my->sACC, my->sACCi);
+                    if (my->update == 1) {
+#pragma unroll
+                        for (int i = 0; i < NE; i++) {
+                            const P tol = a.etol[i];
+                            if ((EF[i] > tol && EFn[i] < -tol && a.edir[i] <= 0) ||
+                                (EF[i] < -tol && EFn[i] > tol && a.edir[i] >= 0)) {
+                                ev = dmin<CP>(ev, -(CP)EF[i] / ((CP)EFn[i] - (CP)EF[i]) * my->dt);
+                                corr = true;
+                            }
                         }
                     }
                 }
@@ -574,7 +602,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
                     const long long k = (n + 1) / a.recK;
                     if (k < a.recCkCap) {
 #pragma unroll
-                        for (int c = 0; c < UD; c++) a.recX[((size_t)k * UD + c) * NU + gu] = X[c];
+                        for (int c = 0; c < UD; c++) a.recX[((size_t)k * UD + c) * NU + gu()] = X[c];
                     } else if (leader) {
                         my->status |= MPGOS_STATUS_CHECKPOINT_OVERFLOW;
                     }
@@ -632,7 +660,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
             if (lane && my->updDO == 1 && upd == 1) {
                 const int k = my->DOidx;
 #pragma unroll
-                for (int c = 0; c < UD; c++) a.DOx[gu + c * NU + (size_t)k * NU * UD] = X[c];
+                for (int c = 0; c < UD; c++) a.DOx[gu() + c * NU + (size_t)k * NU * UD] = X[c];
                 if (leader) a.DOt[gsys + (size_t)k * NS] = my->t;
             }
             __syncthreads();
@@ -668,7 +696,7 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
     }
     __syncthreads();
     if (exists) {
-        const size_t g = gu;
+        const size_t g = gu();
 #pragma unroll
         for (int c = 0; c < UD; c++) a.X[g + c * NU] = X[c];
 #pragma unroll
@@ -690,20 +718,21 @@ __device__ void pb_body(const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>
 #undef MPGOS_PB_USER
 }
 
-// Lane-per-pair form; MAXT bounds the block size so that blocks of up to 256
+// Lane-per-pair form (GROUPED: a kernel of its own for the full matrices that sum
+// their columns in groups); MAXT bounds the block size so that blocks of up to 256
 // threads get the larger register budget.
-template <class Sys, class P, int ALG, int MAXT, bool KAHAN = false>
+template <class Sys, class P, int ALG, int MAXT, bool GROUPED, bool KAHAN = false>
 __global__ void __launch_bounds__(MAXT) pb_kernel(Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP> a)
 {
-    pb_body<Sys, P, ALG, false, KAHAN>(a);
+    pb_body<Sys, P, ALG, GROUPED, false, KAHAN>(a);
 }
 
 // Record pass of the discrete adjoint (FP64): the forward integration plus
 // checkpoints.
-template <class Sys, int ALG, int MAXT>
+template <class Sys, int ALG, int MAXT, bool GROUPED>
 __global__ void __launch_bounds__(MAXT) pb_record_kernel(Args<Sys, double> a)
 {
-    pb_body<Sys, double, ALG, true>(a);
+    pb_body<Sys, double, ALG, GROUPED, true>(a);
 }
 
 } // namespace pb

@@ -61,29 +61,42 @@ struct HasVjp<Sys, decltype((void)&Sys::template OdeVJP<double>)> : std::true_ty
 // dense-contraction kernels are built with -disable-machine-licm, which a full
 // circular matrix in the lane-per-pair form pays for dearly (1000 systems of 40
 // linear units: 0.32 ms with the default flags, 0.55 ms with it).
-template <class Sys, class P, bool KAHAN>
-void launch_lane(int algorithm, int grid, int threads, size_t lds, hipStream_t strm, const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>& a)
+template <class F>
+void choose_lane(int algorithm, bool grouped, F&& f)   // f(algorithm, grouped), both as types
 {
-    if (threads <= 256) {
-        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
-        else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, 256, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+    using RK4 = std::integral_constant<int, MPGOS_RK4>;
+    using RKCK45 = std::integral_constant<int, MPGOS_RKCK45>;
+    if (algorithm == MPGOS_RK4) {
+        if (grouped) f(RK4{}, std::true_type{});
+        else f(RK4{}, std::false_type{});
     } else {
-        if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RK4, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
-        else hipLaunchKernelGGL((pb_kernel<Sys, P, MPGOS_RKCK45, kMaxBlock, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+        if (grouped) f(RKCK45{}, std::true_type{});
+        else f(RKCK45{}, std::false_type{});
     }
 }
 
+template <class Sys, class P, bool KAHAN>
+void launch_lane(int algorithm, bool grouped, int grid, int threads, size_t lds, hipStream_t strm,
+                 const Args<Sys, P, typename SysScope<Sys, P, KAHAN>::CP>& a)
+{
+    choose_lane(algorithm, grouped, [&](auto alg, auto g) {
+        constexpr int ALG = decltype(alg)::value;
+        constexpr bool G = decltype(g)::value;
+        if (threads <= 256) hipLaunchKernelGGL((pb_kernel<Sys, P, ALG, 256, G, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+        else hipLaunchKernelGGL((pb_kernel<Sys, P, ALG, kMaxBlock, G, KAHAN>), dim3(grid), dim3(threads), lds, strm, a);
+    });
+}
+
 template <class Sys>
-void launch_lane_record(int algorithm, int grid, int threads, size_t lds, hipStream_t strm, const Args<Sys, double>& a)
+void launch_lane_record(int algorithm, bool grouped, int grid, int threads, size_t lds, hipStream_t strm, const Args<Sys, double>& a)
 {
     if constexpr (HasVjp<Sys>::value) {
-        if (threads <= 256) {
-            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, 256>), dim3(grid), dim3(threads), lds, strm, a);
-            else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, 256>), dim3(grid), dim3(threads), lds, strm, a);
-        } else {
-            if (algorithm == MPGOS_RK4) hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RK4, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
-            else hipLaunchKernelGGL((pb_record_kernel<Sys, MPGOS_RKCK45, kMaxBlock>), dim3(grid), dim3(threads), lds, strm, a);
-        }
+        choose_lane(algorithm, grouped, [&](auto alg, auto g) {
+            constexpr int ALG = decltype(alg)::value;
+            constexpr bool G = decltype(g)::value;
+            if (threads <= 256) hipLaunchKernelGGL((pb_record_kernel<Sys, ALG, 256, G>), dim3(grid), dim3(threads), lds, strm, a);
+            else hipLaunchKernelGGL((pb_record_kernel<Sys, ALG, kMaxBlock, G>), dim3(grid), dim3(threads), lds, strm, a);
+        });
     }
 }
 
@@ -536,6 +549,27 @@ public:
         return form;
     }
 
+    // Whether the lane form sums a full matrix's columns in groups (Unit::couple),
+    // which has loads in flight at the price of registers.  Solve time of the
+    // plain loop over that of the groups, mean over 1 to 20000 systems of three
+    // kinds in three precisions (worst of them in brackets):
+    //   4, 5 and 6 units 1.01, 0.95 and 1.03 (0.75): a group of four and a rest
+    //   2, 3, 7 and 8 units 1.08, 1.17, 1.11, 1.10 (0.95), 9 units 1.06 with
+    //     Cash-Karp, 1.02 (0.81) with RK4, 11 to 23 units 1.05 to 1.22, 24 to 64 1.13
+    //     to 1.30, 100 to 1000 1.35 to 2.2
+    // With RK4, one coupling and several components per unit the plain loop is
+    // unrolled well: 1.03 (0.88) for 10 to 64 units, but 1.09 to 1.16 where three
+    // columns are left over.  FP32 Cash-Karp kernels with several couplings lose
+    // one wavefront per SIMD to the registers, which up to 23 units costs more than
+    // the groups give once that many systems are there (4000 systems of 17 units
+    // 0.91, 100 of them 1.22).
+    bool lane_grouped(int sm, int grid, int threads) const
+    {
+        if (CCI != 0 || CBW != 0 || sm || UPS < 2 || (UPS >= 4 && UPS <= 6)) return false;
+        if (algorithm == MPGOS_RK4) return UPS != 9 && (UPS > 64 || UPS <= 8 || UPS % 4 == 3 || NC > 1 || UD == 1);
+        return UPS >= 24 || NC == 1 || sizeof(P) == 8 || (long)grid * (threads / 64) <= 12L * cus;
+    }
+
     size_t lds_bytes(int spb, int sm) const
     {
         return lds_layout<Sys, P, KAHAN>(spb, UPS, sharedGlobals, sm, cMatSize).total;
@@ -619,7 +653,7 @@ public:
         const int threads = ((SPB * UPS + 63) / 64) * 64;
         const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
         MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-        launch_lane<Sys, P, KAHAN>(algorithm, grid, threads, lds, strm, a);
+        launch_lane<Sys, P, KAHAN>(algorithm, lane_grouped(a.sharedMatrix, grid, threads), grid, threads, lds, strm, a);
         MPGOS_HIP_TRY(hipGetLastError());
         MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
         return MPGOS_OK;
@@ -696,7 +730,7 @@ public:
             const int threads = ((SPB * UPS + 63) / 64) * 64;
             const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
             MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
-            launch_lane_record<Sys>(algorithm, grid, threads, lds, strm, a);
+            launch_lane_record<Sys>(algorithm, lane_grouped(a.sharedMatrix, grid, threads), grid, threads, lds, strm, a);
             MPGOS_HIP_TRY(hipGetLastError());
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;

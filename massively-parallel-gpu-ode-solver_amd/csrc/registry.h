@@ -32,10 +32,10 @@
 // object of their own (sys_lane_pb_<name>.hip, default flags), declared with
 // MPGOS_PB_LANE_EXTERN where the factory stands.
 #define MPGOS_PB_LANE(EXTERN, SYS)                                                                                      \
-    EXTERN template void launch_lane<SYS, double, false>(int, int, int, size_t, hipStream_t, const Args<SYS, double>&); \
-    EXTERN template void launch_lane<SYS, float, false>(int, int, int, size_t, hipStream_t, const Args<SYS, float>&);   \
-    EXTERN template void launch_lane<SYS, float, true>(int, int, int, size_t, hipStream_t, const Args<SYS, float, double>&); \
-    EXTERN template void launch_lane_record<SYS>(int, int, int, size_t, hipStream_t, const Args<SYS, double>&);         \
+    EXTERN template void launch_lane<SYS, double, false>(int, bool, int, int, size_t, hipStream_t, const Args<SYS, double>&); \
+    EXTERN template void launch_lane<SYS, float, false>(int, bool, int, int, size_t, hipStream_t, const Args<SYS, float>&);   \
+    EXTERN template void launch_lane<SYS, float, true>(int, bool, int, int, size_t, hipStream_t, const Args<SYS, float, double>&); \
+    EXTERN template void launch_lane_record<SYS>(int, bool, int, int, size_t, hipStream_t, const Args<SYS, double>&);         \
     EXTERN template void launch_lane_reverse<SYS>(int, int, int, size_t, hipStream_t, const Args<SYS, double>&, const AdjArgs<SYS>&);
 #define MPGOS_PB_LANE_KERNELS(SYS) MPGOS_PB_LANE(, SYS)
 #define MPGOS_PB_LANE_EXTERN(SYS) MPGOS_PB_LANE(extern, SYS)

@@ -46,13 +46,19 @@ struct RingDuffing : PBNoCallbacks {
         CPF[0] = P(1.0);
     }
 
+    // spelled out, not through TimeTerms: the cosine evaluated first costs the
+    // lane-per-pair kernels registers (FP32 RK4, banded matrix: 0.15 -> 0.18 ms)
     template <class P>
-    MPGOS_HD static void OdeFunction(int sid, int uid, P* F, P* X, P T, P* uPAR, P* sPAR, P* gPAR, int* gPARi, P* uACC, int* uACCi,
-                                     P* sACC, int* sACCi, P* CPT, P* CPF)
+    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* uPAR, P* sPAR, P*, int*, P*, int*, P*, int*, P* CPT,
+                                     P* CPF)
     {
-        P tt[NTT];
-        TimeTerms<P>(T, sPAR, tt);
-        OdeFunctionTT<P>(sid, uid, F, X, T, tt, uPAR, sPAR, gPAR, gPARi, uACC, uACCi, sACC, sACCi, CPT, CPF);
+        using mpgos::math::cos;
+        using mpgos::math::fma;
+        const P x = X[0], v = X[1];
+        F[0] = v;
+        F[1] = fma(-uPAR[0], v, sPAR[0] * cos(T)) - fma(x * x, x, x);
+        CPT[0] = x;
+        CPF[0] = P(1.0);
     }
 
     template <class P>
@@ -94,12 +100,17 @@ struct RingDuffingQ : PBNoCallbacks {
     }
 
     template <class P>
-    MPGOS_HD static void OdeFunction(int sid, int uid, P* F, P* X, P T, P* uPAR, P* sPAR, P* gPAR, int* gPARi, P* uACC, int* uACCi,
-                                     P* sACC, int* sACCi, P* CPT, P* CPF)
+    MPGOS_HD static void OdeFunction(int, int, P* F, P* X, P T, P* uPAR, P* sPAR, P*, int*, P*, int*, P*, int*, P* CPT,
+                                     P* CPF)
     {
-        P tt[NTT];
-        TimeTerms<P>(T, sPAR, tt);
-        OdeFunctionTT<P>(sid, uid, F, X, T, tt, uPAR, sPAR, gPAR, gPARi, uACC, uACCi, sACC, sACCi, CPT, CPF);
+        using mpgos::math::cos;
+        using mpgos::math::fma;
+        const P x = X[0], v = X[1];
+        F[0] = v;
+        F[1] = fma(-uPAR[0], v, sPAR[0] * cos(T)) - fma(x * x, x, x);
+        F[2] = x * x;
+        CPT[0] = x;
+        CPF[0] = P(1.0);
     }
 
     template <class P>
