@@ -31,9 +31,6 @@
 #include <iostream>
 #include <string>
 
-// polynomial coefficients in registers (mpgos_math.h), unless the program has
-// included the library's functions before
-#define MPGOS_HORNER_IN_REGISTERS
 #include "mpgos.h"
 #include "pt_engine.h"
 

@@ -226,11 +226,26 @@ __device__ __forceinline__ P stage_node(int e)
     return j == 4 ? P(1) : c;
 }
 
+// wavefronts per SIMD from which a kernel is short of registers (128 and 64)
+constexpr int kNarrowWaves = 4;
+
+// Whether a kernel for WPE wavefronts per SIMD has the way for usual steps beside
+// the general one (Lane::step).  With 64 registers and compensated steps the two
+// together spill far more than the general way does: 65536 Lorenz instances
+// 53 us without the short way, 92 us with it; 65536 in the other forms and other
+// systems 1.1 to 1.4 times as long with it.  In the others it pays in most (FP64
+// without it: 0.9 to 1.4 times as long with 64 registers, to 1.5 times with 128).
+template <bool KAHAN, int WPE>
+constexpr bool short_way() { return !(KAHAN && WPE >= 2 * kNarrowWaves); }
+
 // What a step reads of the argument block.  The control limits and tolerances
 // are put into vector registers once, before the step loop: in scalar registers
 // they and the step's constants exceed the 102 there are, and the compiler
 // reloads them from memory or rebuilds constants inside the loop (a lone
-// wavefront pays for every such instruction and waits for every load).
+// wavefront pays for every such instruction and waits for every load).  Kernels
+// that are held to few registers (wide = false) leave them to the compiler: there
+// they and what they push out are spilled at every step (64 registers, 65536
+// Duffing oscillators: 0.75 ms so, 1.04 ms with them pinned).
 template <class Sys, class P, class CP>
 struct StepArgs {
     static constexpr int SD = Sys::SD, NE = Sys::NE;
@@ -242,13 +257,14 @@ struct StepArgs {
     int NT, NDO, doFreq;
     P node[2];                  // several lanes per instance: stage_node of this lane
 
-    template <class T> static __device__ __forceinline__ T pin(T v)
+    template <class T> static __device__ __forceinline__ T in_register(T v)
     {
         asm volatile("" : "+v"(v));
         return v;
     }
-    __device__ __forceinline__ explicit StepArgs(const Args<Sys, P, CP>& a, bool adaptive)
+    __device__ __forceinline__ StepArgs(const Args<Sys, P, CP>& a, bool adaptive, bool wide = true)
     {
+        auto pin = [&](auto v) { return wide ? in_register(v) : v; };
         dt0 = a.dt0; NT = a.NT; NDO = a.NDO; doFreq = a.doFreq;
         if (adaptive) {
             dtmin = pin(a.dtmin); dtmax = pin(a.dtmax); grow = pin(a.grow); shrink = pin(a.shrink);
@@ -276,7 +292,7 @@ struct StepArgs {
     template <int GROUP> __device__ __forceinline__ void set_nodes()
     {
 #pragma unroll
-        for (int e = 0; e < group_evals<GROUP>(); e++) node[e] = pin(stage_node<GROUP, P>(e));
+        for (int e = 0; e < group_evals<GROUP>(); e++) node[e] = in_register(stage_node<GROUP, P>(e));
     }
 };
 
@@ -614,20 +630,12 @@ struct Lane {
         newDt = lane_max(newDt, a.dtmin);
     }
 
-    // PT-CTL:23-86, every case of it.  root: R^(1/5) for R >= 2^-1000.
-    __device__ __forceinline__ void control_rkck45(const C& a, const P* nx, const CP* err, const CP* tol, CP R, CP root, int& update)
+    // PT-CTL:23-86, every case of it.  ok: every err_i < tol_i; root: ctrl_root(R, ok).
+    __device__ __forceinline__ void control_rkck45(const C& a, const P* nx, const CP* err, bool ok, CP root, int& update)
     {
-        bool ok = true, fin = true;
+        bool fin = true;
 #pragma unroll
-        for (int i = 0; i < SD; i++) {
-            ok = ok && err[i] < tol[i];
-            fin = fin && math::isfinite(nx[i]) && math::isfinite(err[i]);
-        }
-        if (__builtin_amdgcn_ballot_w64(!(R >= CP(0x1p-100))) != 0) root = math::ctrl_root(R, true);
-        if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
-            const CP fourth = math::ctrl_root(R, false);
-            root = ok ? root : fourth;
-        }
+        for (int i = 0; i < SD; i++) fin = fin && math::isfinite(nx[i]) && math::isfinite(err[i]);
         CP fac = CP(0.9) * root;
         fin = fin && math::isfinite(fac);
         const bool smallest = dt < a.dtmin * CP(1.01);
@@ -674,7 +682,8 @@ struct Lane {
     // NDO = 0), so that the step has no branch on it.  CARRY: tt holds the time
     // terms at t (time_terms(t, tt) before the first step); else they are
     // evaluated anew.  GROUP: several lanes per instance (RKCK45, no CARRY).
-    template <bool DENSE = true, bool CARRY = false, int GROUP = 1>
+    // SHORT: see short_way.
+    template <bool DENSE = true, bool CARRY = false, int GROUP = 1, bool SHORT = true>
     __device__ __forceinline__ bool step(const C& a, P* sPAR, int* sPARi, bool& accepted, P* tt = nullptr)
     {
         const int NT = a.NT;
@@ -730,30 +739,53 @@ struct Lane {
             // valves 520 -> 325 us, 50001 Lorenz instances 2660 -> 2140 us,
             // 262144 in the sorted form 3.22 -> 2.93 ms, 20000 Duffing instances
             // with events 129 -> 116 ms, Cash-Karp adjoint of 10007 4.50 -> 3.76 ms.
-            CP R = CP(1e30), u = a.least - dt;
+            if constexpr (!SHORT) {
+                CP R = CP(1e30);
+                bool ok = true;
 #pragma unroll
-            for (int i = 0; i < SD; i++) {
-                tol[i] = lane_max(a.rtol[i] * lane_max_abs((CP)nx[i], (CP)X[i]), a.atol[i]);
-                u = lane_max(u, err[i] - tol[i]);
-                R = lane_min(R, tol[i] / err[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < NE; i++) u = lane_max(u, (CP)(a.etol[i] - math::flip_sign(EFn[i], EF[i])));
-#pragma unroll
-            for (int i = 0; i < SD; i++) u = math::fma((CP)nx[i], CP(0), math::fma(err[i], CP(0), u));
-            const uint64_t unusual = __builtin_amdgcn_ballot_w64(!(u < CP(0)));
-            const CP root = math::ctrl_root_regular(R);
-            if (__builtin_expect(unusual == 0, 1)) {
-                next_step_size(a, CP(0.9) * root);
-#pragma unroll
-                for (int i = 0; i < NTT; i++) if (CARRY) tt[i] = ttEnd[i];
-                accept(a, h, dtP, nx, inc, EFn, false, sPAR, sPARi);
-                accepted = true;
-                stop = false;
-            } else {
-                control_rkck45(a, nx, err, tol, R, root, update);
+                for (int i = 0; i < SD; i++) {
+                    tol[i] = mpgos_fmax(a.rtol[i] * mpgos_fmax(math::fabs((CP)nx[i]), math::fabs((CP)X[i])), a.atol[i]);
+                    ok = ok && err[i] < tol[i];
+                    R = mpgos_fmin(R, tol[i] / err[i]);
+                }
+                control_rkck45(a, nx, err, ok, math::ctrl_root(R, ok), update);
                 accepted = settle<CARRY>(a, h, dtP, nx, inc, EFn, update, sPAR, sPARi, tt, ttEnd);
                 stop = term != 0;
+            } else {
+                CP R = CP(1e30), u = a.least - dt;
+#pragma unroll
+                for (int i = 0; i < SD; i++) {
+                    tol[i] = lane_max(a.rtol[i] * lane_max_abs((CP)nx[i], (CP)X[i]), a.atol[i]);
+                    u = lane_max(u, err[i] - tol[i]);
+                    R = lane_min(R, tol[i] / err[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < NE; i++) u = lane_max(u, (CP)(a.etol[i] - math::flip_sign(EFn[i], EF[i])));
+#pragma unroll
+                for (int i = 0; i < SD; i++) u = math::fma((CP)nx[i], CP(0), math::fma(err[i], CP(0), u));
+                const uint64_t unusual = __builtin_amdgcn_ballot_w64(!(u < CP(0)));
+                const CP regular = math::ctrl_root_regular(R);
+                if (__builtin_expect(unusual == 0, 1)) {
+                    next_step_size(a, CP(0.9) * regular);
+#pragma unroll
+                    for (int i = 0; i < NTT; i++) if (CARRY) tt[i] = ttEnd[i];
+                    accept(a, h, dtP, nx, inc, EFn, false, sPAR, sPARi);
+                    accepted = true;
+                    stop = false;
+                } else {
+                    bool ok = true;
+#pragma unroll
+                    for (int i = 0; i < SD; i++) ok = ok && err[i] < tol[i];
+                    CP root = regular;
+                    if (__builtin_amdgcn_ballot_w64(!(R >= CP(0x1p-100))) != 0) root = math::ctrl_root(R, true);
+                    if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
+                        const CP fourth = math::ctrl_root(R, false);
+                        root = ok ? root : fourth;
+                    }
+                    control_rkck45(a, nx, err, ok, root, update);
+                    accepted = settle<CARRY>(a, h, dtP, nx, inc, EFn, update, sPAR, sPARi, tt, ttEnd);
+                    stop = term != 0;
+                }
             }
         }
         if (DENSE && __builtin_expect(a.NDO > 0, 0)) {
@@ -1000,7 +1032,7 @@ __device__ __forceinline__ void stage_shared(const Args<Sys, P, CP>& a, P*& sPAR
 // Reference form: lane = instance, whole integration in one launch.  GROUP: that
 // many lanes per instance (whole wavefronts; its first lane stores).  Instances
 // list[first + ...) in the order of the lanes of workgroups `block0` and later.
-template <class Sys, class P, bool KAHAN, int ALG, bool SLICED = false, int GROUP = 1>
+template <class Sys, class P, bool KAHAN, int ALG, bool SLICED = false, int GROUP = 1, int WPE = 1>
 __device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP>& a, int block0 = 0, int first = 0)
 {
     P* sPAR; int* sPARi;
@@ -1009,7 +1041,7 @@ __device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys,
     const int n = (SLICED && a.listLenDev) ? (int)*a.listLenDev : a.listLen;
     using L_t = Lane<Sys, P, KAHAN, ALG>;
     L_t L;
-    typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    typename L_t::C c(a, ALG == MPGOS_RKCK45, WPE < kNarrowWaves);
     if constexpr (GROUP > 1) c.template set_nodes<GROUP>();
     const bool stores = GROUP == 1 || threadIdx.x % GROUP == 0;
     const int id = i < n ? (a.list ? a.list[i] : i) : 0;
@@ -1036,7 +1068,7 @@ __device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys,
             // the budget is the same for every lane
             int left = a.slice;
             bool ended, accepted;
-            do ended = L.template step<true, CARRY, GROUP>(c, sPAR, sPARi, accepted, tt);
+            do ended = L.template step<true, CARRY, GROUP, short_way<KAHAN, WPE>()>(c, sPAR, sPARi, accepted, tt);
             while (!ended && --left > 0);
             if (ended) L.term = 1;
             if (stores) L.release(kernel_args<typename L_t::A>(), sPAR, sPARi);
@@ -1044,7 +1076,7 @@ __device__ __forceinline__ void plain_body(const Args<Sys, P, typename Lane<Sys,
             if constexpr (!COMMON) L.load(a, id, sPAR, sPARi);
             if (CARRY) L.time_terms(L.t, tt);
             bool ended = L.term != 0, accepted;
-            while (!ended) ended = L.template step<true, CARRY, GROUP>(c, sPAR, sPARi, accepted, tt);
+            while (!ended) ended = L.template step<true, CARRY, GROUP, short_way<KAHAN, WPE>()>(c, sPAR, sPARi, accepted, tt);
             if (!stores) return;
             if constexpr (COMMON) L.finish(kernel_args_joined<typename L_t::A>(), sPAR, sPARi);
             else L.finish(kernel_args<typename L_t::A>(), sPAR, sPARi);
@@ -1079,7 +1111,7 @@ __device__ __forceinline__ void mixed_body(const Args<Sys, P, typename Lane<Sys,
 // Every instance's arithmetic is independent of the lane that runs it, so the
 // results are bit-identical to the plain form.  The workgroup leaves the loop
 // together once the queue is drained and no lane is live (block-uniform test).
-template <class Sys, class P, bool KAHAN, int ALG, bool SLICED = false>
+template <class Sys, class P, bool KAHAN, int ALG, bool SLICED = false, int WPE = 1>
 __device__ __forceinline__ void persistent_body(const Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP>& a)
 {
     using L_t = Lane<Sys, P, KAHAN, ALG>;
@@ -1101,7 +1133,7 @@ __device__ __forceinline__ void persistent_body(const Args<Sys, P, typename Lane
     const unsigned lane = __lane_id();
 
     L_t L;
-    const typename L_t::C c(a, ALG == MPGOS_RKCK45);
+    const typename L_t::C c(a, ALG == MPGOS_RKCK45, WPE < kNarrowWaves);
     bool busy = false;
     const unsigned D = (unsigned)a.solo;
     if (tid == 0) {
@@ -1190,7 +1222,7 @@ __device__ __forceinline__ void persistent_body(const Args<Sys, P, typename Lane
             if (!__any(busy)) break;
             if (busy) {
                 bool accepted;
-                const bool ended = L.step(c, sPAR, sPARi, accepted);
+                const bool ended = L.template step<true, false, 1, short_way<KAHAN, WPE>()>(c, sPAR, sPARi, accepted);
                 if (ended) L.term = 1;
                 if constexpr (SLICED) {
                     if (L.stop()) {

@@ -81,12 +81,33 @@ __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(
 solve_kernel(Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP> a)
 {
     // MODE + 2: the same forms with the time-sliced lane lifecycle
-    if constexpr (MODE == MPGOS_KERNEL_PLAIN) plain_body<Sys, P, KAHAN, ALG>(a);
-    else if constexpr (MODE == MPGOS_KERNEL_PERSISTENT) persistent_body<Sys, P, KAHAN, ALG>(a);
-    else if constexpr (MODE == MPGOS_KERNEL_PLAIN + 2) plain_body<Sys, P, KAHAN, ALG, true>(a);
-    else if constexpr (MODE == MPGOS_KERNEL_PERSISTENT + 2) persistent_body<Sys, P, KAHAN, ALG, true>(a);
+    if constexpr (MODE == MPGOS_KERNEL_PLAIN) plain_body<Sys, P, KAHAN, ALG, false, 1, WPE>(a);
+    else if constexpr (MODE == MPGOS_KERNEL_PERSISTENT) persistent_body<Sys, P, KAHAN, ALG, false, WPE>(a);
+    else if constexpr (MODE == MPGOS_KERNEL_PLAIN + 2) plain_body<Sys, P, KAHAN, ALG, true, 1, WPE>(a);
+    else if constexpr (MODE == MPGOS_KERNEL_PERSISTENT + 2) persistent_body<Sys, P, KAHAN, ALG, true, WPE>(a);
     else if constexpr (MODE == kMixedMode) mixed_body<Sys, P, KAHAN, ALG>(a);
     else plain_body<Sys, P, KAHAN, ALG, false, MODE == kOctetMode ? 8 : 4>(a);
+}
+
+// The kernels of launch variants 2 and 3 (128 and 64 registers).  A plain
+// function template, so that a library system's can be compiled apart, with the
+// polynomials' coefficients out of registers (mpgos_math.h).
+template <class Sys, class P, bool KAHAN>
+auto narrow_kernel(int algorithm, int mode, int variant) -> void (*)(Args<Sys, P, typename Lane<Sys, P, KAHAN, MPGOS_RK4>::CP>)
+{
+    auto pick = [&](auto alg, auto m) -> void (*)(Args<Sys, P, typename Lane<Sys, P, KAHAN, MPGOS_RK4>::CP>) {
+        constexpr int ALG = decltype(alg)::value, MODE = decltype(m)::value;
+        return variant == 2 ? solve_kernel<Sys, P, KAHAN, ALG, MODE, kNarrowWaves> : solve_kernel<Sys, P, KAHAN, ALG, MODE, 2 * kNarrowWaves>;
+    };
+    auto form = [&](auto alg) {
+        switch (mode) {
+        case MPGOS_KERNEL_PLAIN: return pick(alg, std::integral_constant<int, MPGOS_KERNEL_PLAIN>{});
+        case MPGOS_KERNEL_PERSISTENT: return pick(alg, std::integral_constant<int, MPGOS_KERNEL_PERSISTENT>{});
+        case MPGOS_KERNEL_PLAIN + 2: return pick(alg, std::integral_constant<int, MPGOS_KERNEL_PLAIN + 2>{});
+        default: return pick(alg, std::integral_constant<int, MPGOS_KERNEL_PERSISTENT + 2>{});
+        }
+    };
+    return algorithm == MPGOS_RK4 ? form(std::integral_constant<int, MPGOS_RK4>{}) : form(std::integral_constant<int, MPGOS_RKCK45>{});
 }
 
 // Virtual interface the C ABI talks to; one implementation per (system, precision).
@@ -607,8 +628,7 @@ public:
     {
         switch (v) {
         case 1: return solve_kernel<Sys, P, KAHAN, ALG, MODE, 2>;
-        case 2: return solve_kernel<Sys, P, KAHAN, ALG, MODE, 4>;
-        case 3: return solve_kernel<Sys, P, KAHAN, ALG, MODE, 8>;
+        case 2: case 3: return narrow_kernel<Sys, P, KAHAN>(ALG, MODE, v);
         default: return solve_kernel<Sys, P, KAHAN, ALG, MODE, 1>;
         }
     }

@@ -28,6 +28,16 @@
         }                                                                             \
     }
 
+// The kernels of a per-thread system that are held to few registers:
+// MPGOS_PT_NARROW_KERNELS in an object of their own (sys_narrow_<name>.hip),
+// declared with MPGOS_PT_NARROW_EXTERN where the factory stands.
+#define MPGOS_PT_NARROW(EXTERN, SYS)                                                                                          \
+    EXTERN template auto narrow_kernel<SYS, double, false>(int, int, int) -> void (*)(Args<SYS, double, double>);              \
+    EXTERN template auto narrow_kernel<SYS, float, false>(int, int, int) -> void (*)(Args<SYS, float, float>);                 \
+    EXTERN template auto narrow_kernel<SYS, float, true>(int, int, int) -> void (*)(Args<SYS, float, double>);
+#define MPGOS_PT_NARROW_KERNELS(SYS) MPGOS_PT_NARROW(, SYS)
+#define MPGOS_PT_NARROW_EXTERN(SYS) MPGOS_PT_NARROW(extern, SYS)
+
 // The lane-per-pair kernels of a per-block system: MPGOS_PB_LANE_KERNELS in an
 // object of their own (sys_lane_pb_<name>.hip, default flags), declared with
 // MPGOS_PB_LANE_EXTERN where the factory stands.

@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::Affine2)
 MPGOS_PT_FACTORY(affine2, ::mpgos::systems::Affine2)
 } // namespace pt
 } // namespace mpgos

@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::Duffing)
 MPGOS_PT_FACTORY(duffing, ::mpgos::systems::Duffing)
 } // namespace pt
 } // namespace mpgos

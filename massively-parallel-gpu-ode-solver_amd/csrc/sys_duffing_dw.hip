@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::DuffingDW)
 MPGOS_PT_FACTORY(duffing_dw, ::mpgos::systems::DuffingDW)
 } // namespace pt
 } // namespace mpgos

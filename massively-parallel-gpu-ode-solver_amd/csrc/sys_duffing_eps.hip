@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::DuffingEps)
 MPGOS_PT_FACTORY(duffing_eps, ::mpgos::systems::DuffingEps)
 } // namespace pt
 } // namespace mpgos

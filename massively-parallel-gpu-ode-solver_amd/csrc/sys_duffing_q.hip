@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::DuffingQ)
 MPGOS_PT_FACTORY(duffing_q, ::mpgos::systems::DuffingQ)
 } // namespace pt
 } // namespace mpgos

@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::KellerMiksis)
 MPGOS_PT_FACTORY(keller_miksis, ::mpgos::systems::KellerMiksis)
 } // namespace pt
 } // namespace mpgos

@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::KellerMiksisMax)
 MPGOS_PT_FACTORY(keller_miksis_max, ::mpgos::systems::KellerMiksisMax)
 } // namespace pt
 } // namespace mpgos

@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::Lorenz)
 MPGOS_PT_FACTORY(lorenz, ::mpgos::systems::Lorenz)
 } // namespace pt
 } // namespace mpgos

@@ -1,0 +1,9 @@
+// Kernels of the per-thread system keller_miksis_max that are held to few registers.
+#include "registry.h"
+#include "systems/keller_miksis.h"
+
+namespace mpgos {
+namespace pt {
+MPGOS_PT_NARROW_KERNELS(::mpgos::systems::KellerMiksisMax)
+} // namespace pt
+} // namespace mpgos

@@ -5,6 +5,7 @@
 
 namespace mpgos {
 namespace pt {
+MPGOS_PT_NARROW_EXTERN(::mpgos::systems::ReliefValve)
 MPGOS_PT_FACTORY(relief_valve, ::mpgos::systems::ReliefValve)
 } // namespace pt
 } // namespace mpgos
