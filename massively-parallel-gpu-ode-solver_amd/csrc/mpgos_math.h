@@ -71,7 +71,8 @@ MPGOS_HD MPGOS_INLINE float flip_sign(float x, float y) { return from_bits32(bit
 // pays 4 cycles for each of these moves, as for an fma.  The coefficients then
 // hold registers through the step loop, so kernels whose wavefronts share a SIMD
 // are compiled without it (the lane-per-pair kernels of the per-block solver, the
-// per-thread kernels held to 128 or 64 registers, programs with systems of their own).
+// per-thread kernels held to 128 or 64 registers and the persistent RK4 ones,
+// programs with systems of their own).
 MPGOS_HD MPGOS_INLINE double fma_k(double a, double b, double k)
 {
 #if defined(__HIP_DEVICE_COMPILE__) && defined(MPGOS_HORNER_IN_REGISTERS)

@@ -687,7 +687,7 @@ struct Lane {
     __device__ __forceinline__ bool step(const C& a, P* sPAR, int* sPARi, bool& accepted, P* tt = nullptr)
     {
         const int NT = a.NT;
-        int update = 1, isfin = 1;
+        int update = 1;
         bool stop;
         dt = newDt;
         CP remaining;
@@ -711,11 +711,14 @@ struct Lane {
             time_terms(t + P(0.5) * h, ttm);
             time_terms(t + h, ttEnd);
             rk4(a, h, nx, inc, sPAR, sPARi, tt1, ttm, ttEnd);
+            // PT-CTL:5-20, by selection: a branch here costs every step of a lone
+            // wavefront (persistent form, 256 to 200000 Lorenz instances: 0.93
+            // times the speed)
+            bool fin = true;
 #pragma unroll
-            for (int i = 0; i < SD; i++)
-                if (!math::isfinite(nx[i])) isfin = 0;
-            // PT-CTL:5-20
-            if (isfin == 0) { term = 1; status |= MPGOS_STATUS_NONFINITE_RK4; }
+            for (int i = 0; i < SD; i++) fin = fin && math::isfinite(nx[i]);
+            term = fin ? term : 1;
+            status |= fin ? 0 : MPGOS_STATUS_NONFINITE_RK4;
             newDt = a.dt0;
             if (NE > 0) Sys::template EventFunction<P>(tid, NT, EFn, t + h, dtP, TD, nx, cPAR, sPAR, sPARi, ACC, ACCi);
             accepted = settle<CARRY>(a, h, dtP, nx, inc, EFn, update, sPAR, sPARi, tt, ttEnd);

@@ -48,10 +48,11 @@ def _doubles(out):
 @pytest.mark.parametrize("algorithm", [Algorithms.RK4, Algorithms.RKCK45])
 @pytest.mark.parametrize("system", ["lorenz", "duffing_dw"])
 def test_few_registers(gpu, oracle, system, algorithm, precision, form):
+    # variant 0: persistent RK4 kernels are built with those of few registers too
     s = _spec(system, algorithm, precision)
     ref = _doubles(run_gpu(s, precision, variant=1, **FORMS[form]))
     assert ref["nacc"].max() > 3 and (algorithm == Algorithms.RK4 or ref["nrej"].max() > 0)
     if precision == Precision.DOUBLE:
         assert_bitwise(ref, oracle.run(system, s), keys=KEYS, label="variant 1")
-    for variant in (2, 3):
+    for variant in (0, 2, 3):
         assert_bitwise(_doubles(run_gpu(s, precision, variant=variant, **FORMS[form])), ref, keys=KEYS, label=f"variant {variant}")
