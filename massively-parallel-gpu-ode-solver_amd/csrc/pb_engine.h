@@ -133,7 +133,6 @@ public:
     int nActive = 0, sharedGlobals = 1, sharedMatrix = 0, doFreq = 1;
     int couplingKernel = 0;   // 0 automatic, 1 lane-per-pair, 2 dense contraction (MFMA)
     int lastForm = -1;        // coupling form of the last launch
-    int mfmaPairs = 4;        // accepted (2 or 4); the dense-contraction form chooses its own split
     double dt0 = 1e-2, dtmax = 1.0e6, dtmin = 1.0e-12, grow = 5.0, shrink = 0.1, doMinDt = 0.0;
     std::vector<double> rtol, atol, etol;
     std::vector<int> edir;
@@ -264,8 +263,7 @@ public:
         case MPGOS_PB_SHARED_COUPLING_MATRICES: sharedMatrix = (int)v != 0; return MPGOS_OK;
         case MPGOS_PB_MFMA_UNITS_PER_LANE:
             if ((int)v != 2 && (int)v != 4) { set_error("MfmaUnitsPerLane must be 2 or 4"); return MPGOS_E_ARG; }
-            mfmaPairs = (int)v;
-            return MPGOS_OK;
+            return MPGOS_OK;   // without effect: the dense-contraction form chooses its own split
         case MPGOS_PB_COUPLING_KERNEL:
             if ((int)v < 0 || (int)v > 2) { set_error("CouplingKernel must be 0 (automatic), 1 (lane per pair) or 2 (dense contraction)"); return MPGOS_E_ARG; }
             couplingKernel = (int)v;
