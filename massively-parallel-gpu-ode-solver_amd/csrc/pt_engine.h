@@ -89,15 +89,16 @@ solve_kernel(Args<Sys, P, typename Lane<Sys, P, KAHAN, ALG>::CP> a)
     else plain_body<Sys, P, KAHAN, ALG, false, MODE == kOctetMode ? 8 : 4>(a);
 }
 
-// The kernels of launch variants 2 and 3 (128 and 64 registers), and the
-// persistent RK4 ones: in that loop the compiler keeps the polynomials'
-// coefficients in scalar registers and copies them for every use (628 steps of
-// 5000 adjoint-Duffing oscillators 0.245 ms, 0.214 ms so).  A plain function template, so that a
-// library system's can be compiled apart, with the coefficients out of vector
-// registers (mpgos_math.h).
+// In the persistent RK4 loop the compiler keeps the polynomials' coefficients in
+// scalar registers and copies them for every use: 500 steps of 1 to 200000
+// adjoint-Duffing oscillators take 1.07 times as long with them, of the other
+// Duffing forms 1.03 to 1.06 times (Keller-Miksis in FP64: 0.88).
 template <int ALG, int MODE>
 constexpr bool always_narrow() { return ALG == MPGOS_RK4 && MODE == MPGOS_KERNEL_PERSISTENT; }
 
+// The kernels of launch variants 2 and 3 (128 and 64 registers), and those above.
+// A plain function template, so that a library system's can be compiled apart,
+// with the coefficients out of vector registers (mpgos_math.h).
 template <class Sys, class P, bool KAHAN>
 auto narrow_kernel(int algorithm, int mode, int variant) -> void (*)(Args<Sys, P, typename Lane<Sys, P, KAHAN, MPGOS_RK4>::CP>)
 {
@@ -661,9 +662,14 @@ public:
     // Workgroups of the sorted form's last launch that give an instance 8 lanes:
     // the longest instances, as many as leave every wavefront a SIMD to itself,
     // and on three quarters of the SIMDs where the card is full all the same.
-    // Uneven Duffing oscillators with logged events, ms with 0, 512, 712 and 1024
-    // such wavefronts: 20000 instances 107.9, 66.1, 61.9, 62.0; 65536 35.9, 21.6,
-    // 18.5, 26.3; 131072 34.9, 28.8, 25.2, 31.6.
+    // Uneven Duffing oscillators with logged events, 64 per workgroup, on 1024
+    // SIMDs; ms with that many such wavefronts (medians; two sets of horizons
+    // agree within 5 percent):
+    //              none    512    640    704    768    832    896   1024
+    //    20000     123.9   72.3   65.8   67.5   68.5   69.3   64.5   73.3
+    //    65536      29.7   22.6   21.1   19.7   20.3   20.4   21.7   25.9
+    //   131072      15.2   13.8   13.1   12.9   13.8   13.9   14.5   16.3
+    // A flat valley: the rule's 768 costs up to 7 percent against the best.
     int octet_blocks(int B) const
     {
         if (!kGroups || algorithm != MPGOS_RKCK45 || variant != 0 || B % 64 != 0) return 0;
