@@ -322,7 +322,7 @@ __host__ __device__ constexpr size_t adjoint_shared_bytes(int preferShared)
 // wavefront; returns false, with nothing done, when the lanes' times, ends or
 // step counts differ or a segment has more than 31 steps.
 // Duffing with a quadrature state, 65536 instances x 32000 steps, K = 16 (one
-// wavefront per SIMD, bound by the instructions of a step): 407 -> 171
+// wavefront per SIMD, bound by the instructions of a step): 407 -> 174
 // instructions per step, 26.1 -> 13.2 ms.
 template <class Sys, int ALG, bool LDS_SEG, class Seg, class Restore, class Attempt, class Keep, class Back>
 __device__ __forceinline__ bool common_time_reverse(const AdjArgs<Sys>& A, Lane<Sys, double, false, ALG>& L, bool mine, bool ok,

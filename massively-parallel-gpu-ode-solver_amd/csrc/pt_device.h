@@ -884,7 +884,7 @@ struct Lane {
     // three per step; the values are those that every lane would have
     // computed, so the results do not change.  Forced Duffing oscillators, RK4,
     // 16384 instances x 64000 steps (one wavefront per compute unit, bound by the
-    // instructions of a step): 158 -> 45 vector instructions per step, 20.9 ->
+    // instructions of a step): 158 -> 49 vector instructions per step, 20.9 ->
     // 7.1 ms; 65536 instances recording adjoint checkpoints: 10.9 -> 4.4 ms.
     //
     // Called by every lane of the wavefront, lanes without an instance with term
