@@ -60,6 +60,13 @@ bool device_alloc(T*& p, size_t bytes)
     (void)hipGetLastError();
     return false;
 }
+// ... allocated by an earlier call or by this one: of several buffers an earlier
+// call may have got only the first
+template <class T>
+bool device_have(T*& p, size_t bytes)
+{
+    return p || device_alloc(p, bytes);
+}
 template <class T>
 bool host_alloc(T*& p, size_t bytes)
 {
@@ -847,12 +854,10 @@ public:
 
     int ensure_slice_buffers()
     {
-        if (!saved) {
-            if (!device_alloc(saved, lane_words() * 4 * (size_t)NT) || !device_alloc(phase, 4 * (size_t)NT) ||
-                !device_alloc(listA, 4 * (size_t)NT) || !device_alloc(listB, 4 * (size_t)NT)) {
-                set_error("time-sliced launches: allocation failed");
-                return MPGOS_E_MEMORY;
-            }
+        if (!device_have(saved, lane_words() * 4 * (size_t)NT) || !device_have(phase, 4 * (size_t)NT) ||
+            !device_have(listA, 4 * (size_t)NT) || !device_have(listB, 4 * (size_t)NT)) {
+            set_error("time-sliced launches: allocation failed");
+            return MPGOS_E_MEMORY;
         }
         if (relaunchCountsN < relaunchLaunches + 1) {
             MPGOS_HIP_TRY(hipStreamSynchronize(strm));
@@ -924,12 +929,10 @@ public:
         if (kernelMode == MPGOS_KERNEL_RELAUNCH || kernelMode == MPGOS_KERNEL_SORTED) {
             if (int rc = ensure_slice_buffers()) return rc;
         }
-        if (kernelMode == MPGOS_KERNEL_SORTED && !sortKey) {
-            if (!device_alloc(sortKey, sizeof(float) * (size_t)NT) ||
-                !device_alloc(sortHist, sizeof(unsigned) * 256)) {
-                set_error("sorted form: allocation failed");
-                return MPGOS_E_MEMORY;
-            }
+        if (kernelMode == MPGOS_KERNEL_SORTED &&
+            (!device_have(sortKey, sizeof(float) * (size_t)NT) || !device_have(sortHist, sizeof(unsigned) * 256))) {
+            set_error("sorted form: allocation failed");
+            return MPGOS_E_MEMORY;
         }
         Args<Sys, P, CP> a = make_args();
         if (ordered()) a.list = order;
