@@ -703,21 +703,26 @@ public:
         } else {
             if (K < 1 || ckcap < 1 || stepcap < 1) { set_error("per-block adjoint: interval and capacities must be >= 1"); return MPGOS_E_ARG; }
             MPGOS_HIP_TRY(hipSetDevice(device));
-            const size_t NU = (size_t)NS * UPS;
+            if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
+            const size_t NU = (size_t)NS * UPS, nx = (size_t)ckcap * UD * NU, nt = (size_t)stepcap * NS;
             MPGOS_HIP_TRY(hipStreamSynchronize(strm));
             int rc;
-            if ((rc = grow_device(recX, recXn, (size_t)ckcap * UD * NU, "checkpoints")) || (rc = grow_device(recT, recTn, (size_t)stepcap * NS, "step times")) ||
-                (rc = grow_device(recH, recHn, (size_t)stepcap * NS, "step sizes")))
+            // an earlier record goes with its buffers, and below with the launch,
+            // whether or not this call succeeds
+            if (nx > recXn || nt > recTn || nt > recHn) adjK = 0;
+            if ((rc = grow_device(recX, recXn, nx, "checkpoints")) || (rc = grow_device(recT, recTn, nt, "step times")) ||
+                (rc = grow_device(recH, recHn, nt, "step sizes")))
                 return rc;
-            adjK = K; adjCap = ckcap; adjStepCap = stepcap;
             Args<Sys, double> a = make_args();
             a.recX = recX; a.recT = recT; a.recH = recH; a.recK = K; a.recCkCap = ckcap; a.recStepCap = stepcap;
-            if (couplingKernel == 2 && !dense_request_valid()) return refuse_dense();
+            auto recorded = [&] { adjK = K; adjCap = ckcap; adjStepCap = stepcap; };
             if constexpr (NC > 0) {
                 if (coupling_form() == kDenseCoupling) {
                     MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
+                    adjK = 0;
                     if ((rc = launch_dense<true>(a))) return rc;
                     MPGOS_HIP_TRY(hipGetLastError());
+                    recorded();
                     MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
                     return MPGOS_OK;
                 }
@@ -728,8 +733,10 @@ public:
             const int threads = ((SPB * UPS + 63) / 64) * 64;
             const int grid = NS / SPB + (NS % SPB == 0 ? 0 : 1);
             MPGOS_HIP_TRY(hipEventRecord(evStart, strm));
+            adjK = 0;
             launch_lane_record<Sys>(algorithm, lane_grouped(a.sharedMatrix, grid, threads), grid, threads, lds, strm, a);
             MPGOS_HIP_TRY(hipGetLastError());
+            recorded();
             MPGOS_HIP_TRY(hipEventRecord(evStop, strm));
             return MPGOS_OK;
         }

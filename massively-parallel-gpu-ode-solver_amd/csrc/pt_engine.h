@@ -1065,6 +1065,7 @@ public:
             if (needC > ckptCount) {
                 if (ckpt) (void)hipFree(ckpt);
                 ckpt = nullptr; ckptCount = 0;
+                adjK = 0;      // the earlier record goes with them, whether or not this call succeeds
                 if (!device_alloc(ckpt, needC * sizeof(double))) { set_error("adjoint: checkpoint allocation failed"); return MPGOS_E_MEMORY; }
                 ckptCount = needC;
             }
